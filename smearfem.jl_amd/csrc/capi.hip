@@ -202,6 +202,8 @@ int sfem_ctx_create(int device, sfem_ctx** out) {
         if (nt) ctx->tune_nt = nt[0] == '1';
         const char* ws = std::getenv("SFEM_SELL_WAVE_SLICES");
         if (ws) ctx->tune_wave_slices = std::max(0, std::atoi(ws));
+        const char* sp = std::getenv("SFEM_SELL_SPLIT");
+        if (sp) ctx->tune_split = std::max(0, std::atoi(sp));
         const char* bt = std::getenv("SFEM_BARRIER_TIMEOUT_US");
         if (bt) ctx->bar_timeout_ticks = (unsigned long long)std::max(0LL, std::atoll(bt)) * 100ull;
         const char* bg = std::getenv("SFEM_BARRIER_GROUPED");

@@ -16,20 +16,30 @@
 // FP64 it costs one extra SpMV per 10x drop and keeps the recurrence honest.
 // Every mode stops only on that FP64 residual.
 //
-// Per iteration four kernels run, with no host round trip:
-//   p_update: p = zcoef z + beta p (streaming)
-//   spmv_cg : q = K_ff p, partial p.q -> alpha
-//   update  : x += alpha p, r -= alpha q, z = D^-1 r, partial r.z, r.r
-//             -> beta, replacement flag
-//   resid   : exits at once unless a replacement is due (FP64 residual);
-//             replacements that stop making progress end the solve
-//             ("stagnation": the tolerance is below what FP64 can reach)
-// The host reads the 100-byte state every `check_every` iterations.
+// Per iteration two kernels run, with no host round trip:
+//   operator pass : beta from the last update's sums; p = zcoef z + beta p
+//             (formed where a row gathers it, and written once: p is double
+//             buffered), q = K_ff p, per-block p.q.  When a replacement is
+//             due the pass forms the FP64 residual instead, with z = D^-1 r.
+//             On large systems p is a pass of its own (direction_kernel).
+//   update pass   : alpha from the pass's p.q; x += alpha p, r -= alpha q,
+//             z = D^-1 r, per-block r.z and r.r; after a residual it only
+//             takes the residual's sums (beta, the stopping tests;
+//             replacements that stop making progress end the solve:
+//             "stagnation", the tolerance is below what FP64 can reach).
+// The scalars are formed by the kernel that needs them: every block sums the
+// previous kernel's per-block partials, in one fixed order, and block 0
+// writes the state copy the next kernel reads.  Below ~100k dofs a launch is
+// bound by its chain of dependent latencies (about 1 us for each of: the
+// state, a last-block arrival, its partials), not by bytes: at 64x16x16 Hex8
+// (18.5k nodes, FP64) four kernels with last-block reductions took 41 us an
+// iteration.
+// The host reads the state every `check_every` iterations.
 //
-// Reductions are deterministic: wave64 butterfly shuffles, a fixed 4-wave
-// block combine, per-block partials, and the last block to arrive sums the
-// partials in a fixed order.  The grid is a fixed function of the problem
-// size, so results are bitwise reproducible run to run.
+// Reductions are deterministic: wave64 butterfly shuffles, a fixed combine
+// of a block's wavefronts, per-block partials summed in a fixed order.  The
+// grid is a fixed function of the problem size, so results are bitwise
+// reproducible run to run.
 #include <chrono>
 #include <cmath>
 #include <string>
@@ -42,350 +52,403 @@ namespace sfem {
 
 namespace {
 
-// ---------------------------------------------------------- p_update ---
-// p = zcoef*z + beta*p in place (zcoef = 1 except right after a residual
-// replacement, where it also makes p orthogonal to the new residual).
+// ------------------------------------------------------ state logic ----
+// After an update: beta, the replacement triggers and the stopping backstops
+// from r.z and r.r.
+__device__ __forceinline__ void cg_after_update(CgState& s, double trz, double trr) {
+    s.rz_prev = s.rz;
+    s.rz = trz;
+    s.beta = trz / s.rz_prev;
+    s.rr = trr;
+    s.iters += 1;
+    s.fold_pending = 0;
+    s.zcoef = 1.0;
+    // replacement when the recurrence converged, dropped by delta, or
+    // made no such drop for max(256, iteration of the best true residual)
+    const long long since = s.iters - s.last_upd;
+    const long long every = s.best_true_it > 256 ? s.best_true_it : 256;
+    if (trr <= s.tol2bb || trr < s.delta2 * s.maxrr || since >= every) s.need_update = 1;
+    // backstop for a recurrence that stops decreasing: no 2x drop of |r|
+    // within max(10000, 4x the iterations it took to reach the best)
+    if (trr < 0.25 * s.best_rr) {
+        s.best_rr = trr;
+        s.best_it = s.iters;
+    } else if (s.iters - s.best_it > (4 * s.best_it > 10000 ? 4 * s.best_it : 10000)) {
+        s.done = 3;
+    }
+    if (!std::isfinite(trr)) s.done = 2;
+}
+
+// After an FP64 residual: sums are r.r, r.z, r.p and the floor scale.  The
+// search direction is made orthogonal to the new residual (p <- p - gamma z,
+// gamma = r.p/r.z), folded into zcoef of the next operator pass.
+template <bool FOLD>
+__device__ __forceinline__ void cg_after_resid(CgState& s, const double (&sums)[4]) {
+    const double trr = sums[0], trz = sums[1], trp = sums[2];
+    // 16x the attainable |r|^2, (eps * || |rhs| + |K||x| ||)^2
+    const double floor_rr = 16.0 * kEps64 * kEps64 * sums[3];
+    const double rec = s.rr;  // recurrence |r|^2 that triggered this replacement
+    s.rr_true = trr;
+    s.floor_rr = floor_rr;
+    s.rr = trr;
+    s.last_upd = s.iters;
+    s.updates += 1;
+    s.need_update = 0;
+    s.fold_pending = FOLD ? 1 : 0;
+    if (trr <= s.tol2bb) {
+        s.done = 1;
+    } else {
+        const double beta = trz / s.rz_prev;
+        s.beta = beta;
+        s.zcoef = 1.0 - beta * (trp / trz);
+        s.rz = trz;
+        s.maxrr = trr;
+        // Attainable-floor test.  A replacement whose true residual does
+        // not beat the best by 10% ends the solve when it is within 4x of
+        // the rounding floor eps*|| |rhs| + |K||x| ||, and counts once
+        // when the recurrence ran 5x below it (the residual gap of finite
+        // precision; twice in a row ends the solve).  Slow progress away
+        // from the floor never stops it: the CG residual norm can plateau
+        // for thousands of iterations.
+        const bool gap = s.iters > 0 && 25.0 * rec < trr;
+        if (trr <= 0.81 * s.best_true) {
+            s.stall = 0;
+            s.best_true_it = s.iters;
+        } else if (trr <= floor_rr) {
+            s.stall += 2;
+        } else if (gap) {
+            s.stall += 1;
+        }
+        if (s.stall >= 2) s.done = 3;
+    }
+    if (trr < s.best_true) s.best_true = trr;
+    if (!std::isfinite(trr)) s.done = 2;
+    if (s.capped && !s.done) s.done = 4;
+}
+
+// What a pass tells its threads.
+struct PassGo {
+    double beta, zcoef;  // operator pass: p = zcoef z + beta p
+    int done, resid;
+};
+
+// Start of an operator pass, by every block: the last update's sums (upd:
+// r.z, r.r per block), the state after it, and what this pass has to do.
+template <int NW>
+__device__ __forceinline__ PassGo pass_begin(const CgState* __restrict__ in, CgState* __restrict__ out,
+                                             const double* __restrict__ upd, int nupd, double* sh, PassGo* shgo) {
+    double t[2] = {0.0, 0.0};
+    if (in->fresh) sum_parts_all<2, NW>(upd, nupd, t, sh);
+    if (threadIdx.x == 0) {
+        CgState s = *in;
+        if (!s.done) {
+            if (s.fresh) cg_after_update(s, t[0], t[1]);
+            if (!s.done && !s.need_update && s.iters >= s.max_iter) s.need_update = s.capped = 1;
+        }
+        s.fresh = 0;
+        s.resid = s.need_update;
+        *shgo = PassGo{s.beta, s.zcoef, s.done, s.resid};
+        if (blockIdx.x == 0) *out = s;
+    }
+    __syncthreads();
+    return *shgo;
+}
+
+// Per-block partials of an operator pass: p.q (stride 1), or the residual's
+// four sums (stride 4).
+template <int NW>
+__device__ __forceinline__ void put_parts4(double rr, double rz, double rp, double ff, double* __restrict__ parts,
+                                           double* sh) {
+    const double b0 = block_sum_waves<NW>(rr, sh), b1 = block_sum_waves<NW>(rz, sh);
+    const double b2 = block_sum_waves<NW>(rp, sh), b3 = block_sum_waves<NW>(ff, sh);
+    if (threadIdx.x == 0) {
+        parts[4 * (int64_t)blockIdx.x] = b0;
+        parts[4 * (int64_t)blockIdx.x + 1] = b1;
+        parts[4 * (int64_t)blockIdx.x + 2] = b2;
+        parts[4 * (int64_t)blockIdx.x + 3] = b3;
+    }
+}
+
+// ---------------------------------------------------- operator pass ----
+// Vectors of a pass.  Where p is formed in the gathers (FLY), p and z lie side
+// by side, a record of BS values of p then BS of z per block row: a gathered
+// row is one record, in 16-byte loads (a mesh in no particular numbering
+// gathers a cache line per row and vector).  There are two arrays of records:
+// a pass reads the one (p, z) and writes the other's p, and the update that
+// follows writes its z.  Else p and z are plain vectors, updated in place.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void p_update_kernel(T* __restrict__ p, const T* __restrict__ z, int64_t n,
-                                                            int64_t per_block, const CgState* st) {
-    if (st->done) return;
-    const T beta = (T)st->beta, zc = (T)st->zcoef;
+struct PassVecs {
+    const T* p;
+    const T* z;
+    T* pnew;
+    T* znew;
+    T* q;
+    T* r;
+    const double* x64;
+    const T* xs;  // FP32 solution increment (FOLD)
+    const double* rhs;
+    const T* dinv;
+    const T* binv;  // node-block Jacobi: planar inverse blocks, stride nrows
+};
+
+// Elements between block rows of p and z.
+template <int BS, bool FLY>
+constexpr int kRowStride = FLY ? 2 * BS : BS;
+
+template <int BS, typename T>
+struct alignas(2 * BS * sizeof(T) % 16 == 0 ? 16 : 8) PzRecord {
+    T p[BS], z[BS];
+};
+
+// p = zcoef z + beta p in place, and the pass's state: the first half of an
+// operator pass on a large system (FLY false below).  There a row's second
+// gathered vector costs more than this stream (256x64x64 Hex8, FP64 Jacobi:
+// 508 us an iteration with p formed in the gathers, 478 us so).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void direction_kernel(T* __restrict__ p, const T* __restrict__ z, int64_t n,
+                                                             int64_t per_block, const CgState* in, CgState* out,
+                                                             const double* __restrict__ upd, int nupd) {
+    constexpr int NW = kThreads / 64;
+    __shared__ double sh[NW];
+    __shared__ PassGo shgo;
+    const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
+    if (go.done || go.resid) return;
+    const T beta = (T)go.beta, zc = (T)go.zcoef;
     const int64_t i0 = (int64_t)blockIdx.x * per_block;
     const int64_t i1 = min(n, i0 + per_block);
 #pragma unroll 4  // four strides of loads in flight; the same order of operations
     for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) p[i] = fmaT<T>(beta, p[i], zc * z[i]);
 }
 
-// ---------------------------------------------------------- spmv_cg ----
-// q = K_ff p (accumulated in T), partial p.q -> last block: alpha = rz / pq.
-template <int G, typename TV, typename T>
-__global__ __launch_bounds__(kThreads) void csr_spmv_cg_kernel(const int32_t* __restrict__ rowptr,
-                                                               const int32_t* __restrict__ col,
-                                                               const TV* __restrict__ val, int64_t nrows,
-                                                               int64_t rows_per_block, const T* __restrict__ p,
-                                                               T* __restrict__ q, CgState* st,
-                                                               double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
+// Scalar CSR, G lanes per row.
+template <int G, typename TV, typename T, bool FLY, bool FOLD>
+__global__ __launch_bounds__(kThreads) void csr_pass_kernel(const int32_t* __restrict__ rowptr,
+                                                            const int32_t* __restrict__ col,
+                                                            const TV* __restrict__ val,
+                                                            const double* __restrict__ val64, int64_t nrows,
+                                                            int64_t rows_per_block, PassVecs<T> v, const CgState* in,
+                                                            CgState* out, const double* __restrict__ upd, int nupd,
+                                                            double* __restrict__ parts) {
+    constexpr int NW = kThreads / 64;
+    __shared__ double sh[NW];
+    __shared__ PassGo shgo;
+    PassGo go;
+    if constexpr (FLY) go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
+    else go = PassGo{0.0, 0.0, in->done, in->resid};  // direction_kernel has begun the pass
+    if (go.done) return;
     const int64_t r0 = logical_block() * rows_per_block;
     const int64_t r1 = min(nrows, r0 + rows_per_block);
     const int g = threadIdx.x / G, lane = threadIdx.x % G;
-    double dot = 0.0;
-    auto gx = [=](int64_t c) { return p[c]; };
-    for (int64_t row = r0 + g; row < r1; row += kThreads / G) {
-        const T s = csr_row<G, TV, T>(rowptr, col, val, row, lane, gx);
-        if (lane == 0) {
-            q[row] = s;
-            dot += (double)p[row] * (double)s;
-        }
-    }
-    const double bsum = block_sum_256(dot, sh);
-    if (threadIdx.x == 0) st_coherent(partials + 3 * blockIdx.x, bsum);
-    if (last_block_arrive(&st->arrive)) {
-        double pq, u1, u2;
-        sum_partials3(partials, gridDim.x, &pq, &u1, &u2, sh);
-        if (threadIdx.x == 0) {
-            st->alpha = st->rz / pq;
-            if (!(pq > 0.0) || !std::isfinite(st->alpha)) st->done = 2;  // breakdown
-        }
-    }
-}
-
-template <int BS, typename TV, typename T, bool NT>
-__global__ __launch_bounds__(kThreads) void sell_spmv_cg_kernel(
-    const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w, const int32_t* __restrict__ scol,
-    Vals<TV> sval, int64_t nslices, int64_t nrows, int64_t slices_per_block, const T* __restrict__ p,
-    T* __restrict__ q, CgState* st, double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
-    const int64_t s0 = logical_block() * slices_per_block;
-    const int64_t s1 = min(nslices, s0 + slices_per_block);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double dot = 0.0;
-    auto gx = [=](int64_t c) { return p[c]; };
-    for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
-        T out[BS];
-        sell_row<BS, TV, T, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, out);
-        const int64_t row = sl * 64 + lane;
-        if (row < nrows) {
-#pragma unroll
-            for (int j = 0; j < BS; ++j) {
-                const int64_t d = row * BS + j;
-                q[d] = out[j];
-                dot += (double)p[d] * (double)out[j];
+    if (!go.resid) {
+        const T beta = (T)go.beta, zc = (T)go.zcoef;
+        const T* __restrict__ p = v.p;
+        auto gx = [=](int64_t c) {
+            if constexpr (FLY) {
+                const PzRecord<1, T> w = ((const PzRecord<1, T>*)p)[c];
+                return fmaT<T>(beta, w.p[0], zc * w.z[0]);
+            } else {
+                return p[c];
+            }
+        };
+        double dot = 0.0;
+        for (int64_t row = r0 + g; row < r1; row += kThreads / G) {
+            const T s = csr_row<G, TV, T>(rowptr, col, val, row, lane, gx);
+            if (lane == 0) {
+                const T pr = gx(row);
+                if (FLY) v.pnew[row * 2] = pr;
+                v.q[row] = s;
+                dot += (double)pr * (double)s;
             }
         }
+        dot = block_sum_waves<NW>(dot, sh);
+        if (threadIdx.x == 0) parts[blockIdx.x] = dot;
+        return;
     }
-    const double bsum = block_sum_256(dot, sh);
-    if (threadIdx.x == 0) st_coherent(partials + 3 * blockIdx.x, bsum);
-    if (last_block_arrive(&st->arrive)) {
-        double pq, u1, u2;
-        sum_partials3(partials, gridDim.x, &pq, &u1, &u2, sh);
-        if (threadIdx.x == 0) {
-            st->alpha = st->rz / pq;
-            if (!(pq > 0.0) || !std::isfinite(st->alpha)) st->done = 2;
-        }
-    }
-}
-
-// Last block of an update: beta, the replacement triggers and the stopping
-// backstops from the partial sums of r.z and r.r.
-__device__ __forceinline__ void cg_update_finish(CgState* st, double* partials, double* sh) {
-    double trz, trr, u;
-    sum_partials3(partials, gridDim.x, &trz, &trr, &u, sh);
-    if (threadIdx.x == 0) {
-        st->rz_prev = st->rz;
-        st->rz = trz;
-        st->beta = trz / st->rz_prev;
-        st->rr = trr;
-        st->iters += 1;
-        st->fold_pending = 0;
-        st->zcoef = 1.0;
-        // replacement when the recurrence converged, dropped by delta, or
-        // made no such drop for max(256, iteration of the best true residual)
-        const long long since = st->iters - st->last_upd;
-        const long long every = st->best_true_it > 256 ? st->best_true_it : 256;
-        if (trr <= st->tol2bb || trr < st->delta2 * st->maxrr || since >= every) st->need_update = 1;
-        // backstop for a recurrence that stops decreasing: no 2x drop of |r|
-        // within max(10000, 4x the iterations it took to reach the best)
-        if (trr < 0.25 * st->best_rr) {
-            st->best_rr = trr;
-            st->best_it = st->iters;
-        } else if (st->iters - st->best_it > (4 * st->best_it > 10000 ? 4 * st->best_it : 10000)) {
-            st->done = 3;
-        }
-        if (!std::isfinite(trr)) st->done = 2;
-    }
-}
-
-// ----------------------------------------------------------- update ----
-// x += alpha p, r -= alpha q, z = D^-1 r, partial r.z and r.r.  With FOLD
-// (FP32 solution increment xs) a pending fold moves xs into x64 first.  The
-// last block sets beta and decides whether the FP64 residual is due.
-template <typename T, bool FOLD>
-__global__ __launch_bounds__(kThreads) void cg_update_kernel(T* __restrict__ x, double* __restrict__ x64,
-                                                             T* __restrict__ r, T* __restrict__ z,
-                                                             const T* __restrict__ p, const T* __restrict__ q,
-                                                             const T* __restrict__ dinv, int64_t n,
-                                                             int64_t per_block, CgState* st,
-                                                             double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
-    const T a = (T)st->alpha;
-    const bool fold = FOLD && st->fold_pending;
-    const int64_t i0 = (int64_t)blockIdx.x * per_block;
-    const int64_t i1 = min(n, i0 + per_block);
-    double rz = 0.0, rr = 0.0;
-#pragma unroll 4  // four strides of loads in flight; the same order of operations
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) {
-        T xi = x[i];
-        if (fold) {
-            x64[i] += (double)xi;
-            xi = 0;
-        }
-        const T ri = fmaT<T>(-a, q[i], r[i]);
-        const T zi = dinv[i] * ri;
-        x[i] = fmaT<T>(a, p[i], xi);
-        r[i] = ri;
-        z[i] = zi;
-        rz += (double)ri * (double)zi;
-        rr += (double)ri * (double)ri;
-    }
-    const double b0 = block_sum_256(rz, sh);
-    const double b1 = block_sum_256(rr, sh + 4);
-    if (threadIdx.x == 0) {
-        st_coherent(partials + 3 * blockIdx.x, b0);
-        st_coherent(partials + 3 * blockIdx.x + 1, b1);
-    }
-    if (last_block_arrive(&st->arrive)) cg_update_finish(st, partials, sh);
-}
-
-// Node-block Jacobi form of cg_update: one thread per node; z = B^-1 r with
-// B^-1 the node's inverse diagonal block (planar: binv[(j*BS+i)*nnodes + n]).
-template <int BS, typename T, bool FOLD>
-__global__ __launch_bounds__(kThreads) void cg_update_block_kernel(T* __restrict__ x, double* __restrict__ x64,
-                                                                   T* __restrict__ r, T* __restrict__ z,
-                                                                   const T* __restrict__ p, const T* __restrict__ q,
-                                                                   const T* __restrict__ binv, int64_t nnodes,
-                                                                   int64_t per_block, CgState* st,
-                                                                   double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
-    const T a = (T)st->alpha;
-    const bool fold = FOLD && st->fold_pending;
-    const int64_t n0 = (int64_t)blockIdx.x * per_block;
-    const int64_t n1 = min(nnodes, n0 + per_block);
-    double rz = 0.0, rr = 0.0;
-    for (int64_t n = n0 + threadIdx.x; n < n1; n += kThreads) {
-        T rv[BS];
-#pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            const int64_t i = n * BS + j;
-            T xi = x[i];
-            if (fold) {
-                x64[i] += (double)xi;
-                xi = 0;
-            }
-            x[i] = fmaT<T>(a, p[i], xi);
-            rv[j] = fmaT<T>(-a, q[i], r[i]);
-            r[i] = rv[j];
-            rr += (double)rv[j] * (double)rv[j];
-        }
-#pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            T zj = 0;
-#pragma unroll
-            for (int i = 0; i < BS; ++i) zj = fmaT<T>(binv[(j * BS + i) * nnodes + n], rv[i], zj);
-            z[n * BS + j] = zj;
-            rz += (double)rv[j] * (double)zj;
-        }
-    }
-    const double b0 = block_sum_256(rz, sh);
-    const double b1 = block_sum_256(rr, sh + 4);
-    if (threadIdx.x == 0) {
-        st_coherent(partials + 3 * blockIdx.x, b0);
-        st_coherent(partials + 3 * blockIdx.x + 1, b1);
-    }
-    if (last_block_arrive(&st->arrive)) cg_update_finish(st, partials, sh);
-}
-
-// ------------------------------------------- FP64 residual replacement --
-// Runs after every update; exits at once unless the FP64 residual is due.
-// r = rhs - K_ff x with x = x64 (+ xs, the FP32 increment, when FOLD), in
-// FP64; writes r and z = D^-1 r in the CG precision.  The search direction
-// is made orthogonal to the new residual (p <- p - gamma z, gamma = r.p/r.z),
-// folded into zcoef of the next spmv_cg.
-__global__ __launch_bounds__(kThreads) void fold_kernel(double* __restrict__ x64, float* __restrict__ xs, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
-        x64[i] += (double)xs[i];
-        xs[i] = 0.0f;
-    }
-}
-
-template <bool FOLD>
-__device__ __forceinline__ void resid_finish(CgState* st, double* partials, double* sh) {
-    double sums[4];
-    sum_partials4(partials, gridDim.x, sums, sh);
-    const double trr = sums[0], trz = sums[1], trp = sums[2];
-    // 16x the attainable |r|^2, (eps * || |rhs| + |K||x| ||)^2
-    const double floor_rr = 16.0 * kEps64 * kEps64 * sums[3];
-    if (threadIdx.x == 0) {
-        const double rec = st->rr;  // recurrence |r|^2 that triggered this replacement
-        st->rr_true = trr;
-        st->floor_rr = floor_rr;
-        st->rr = trr;
-        st->last_upd = st->iters;
-        st->updates += 1;
-        st->need_update = 0;
-        st->fold_pending = FOLD ? 1 : 0;
-        if (trr <= st->tol2bb) {
-            st->done = 1;
-        } else {
-            const double beta = trz / st->rz_prev;
-            st->beta = beta;
-            st->zcoef = 1.0 - beta * (trp / trz);
-            st->rz = trz;
-            st->maxrr = trr;
-            // Attainable-floor test.  A replacement whose true residual does
-            // not beat the best by 10% ends the solve when it is within 4x of
-            // the rounding floor eps*|| |rhs| + |K||x| ||, and counts once
-            // when the recurrence ran 5x below it (the residual gap of finite
-            // precision; twice in a row ends the solve).  Slow progress away
-            // from the floor never stops it: the CG residual norm can plateau
-            // for thousands of iterations.
-            const bool gap = st->iters > 0 && 25.0 * rec < trr;
-            if (trr <= 0.81 * st->best_true) {
-                st->stall = 0;
-                st->best_true_it = st->iters;
-            } else if (trr <= floor_rr) {
-                st->stall += 2;
-            } else if (gap) {
-                st->stall += 1;
-            }
-            if (st->stall >= 2) st->done = 3;
-        }
-        if (trr < st->best_true) st->best_true = trr;
-        if (!std::isfinite(trr)) st->done = 2;
-    }
-}
-
-template <int G, typename T, bool FOLD>
-__global__ __launch_bounds__(kThreads) void csr_resid_kernel(const int32_t* __restrict__ rowptr,
-                                                             const int32_t* __restrict__ col,
-                                                             const double* __restrict__ val, int64_t nrows,
-                                                             int64_t rows_per_block, const double* __restrict__ x64,
-                                                             const T* __restrict__ xs, const double* __restrict__ rhs,
-                                                             const T* __restrict__ dinv, const T* __restrict__ p,
-                                                             T* __restrict__ r, T* __restrict__ z, CgState* st,
-                                                             double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done || !st->need_update) return;
-    const int64_t r0 = logical_block() * rows_per_block;
-    const int64_t r1 = min(nrows, r0 + rows_per_block);
-    const int g = threadIdx.x / G, lane = threadIdx.x % G;
     double rr = 0.0, rz = 0.0, rp = 0.0, ff = 0.0;
+    const double* __restrict__ x64 = v.x64;
+    const T* __restrict__ xs = v.xs;
     auto gx = [=](int64_t c) { return FOLD ? x64[c] + (double)xs[c] : x64[c]; };
     for (int64_t row = r0 + g; row < r1; row += kThreads / G) {
         double a;
-        const double s = csr_row_abs<G>(rowptr, col, val, row, lane, gx, &a);
+        const double s = csr_row_abs<G>(rowptr, col, val64, row, lane, gx, &a);
         if (lane == 0) {
-            const double res = rhs[row] - s;
-            const double sc = fabs(rhs[row]) + a;
+            const double res = v.rhs[row] - s;
+            const double sc = fabs(v.rhs[row]) + a;
             ff += sc * sc;
             const T rt = (T)res;
-            const T zt = dinv[row] * rt;
-            r[row] = rt;
-            z[row] = zt;
+            const T zt = v.dinv[row] * rt;
+            constexpr int RS = kRowStride<1, FLY>;
+            const T pr = v.p[row * RS];
+            v.r[row] = rt;
+            v.znew[row * RS] = zt;
+            if (FLY) v.pnew[row * RS] = pr;
             rr += res * res;
             rz += (double)rt * (double)zt;
-            rp += (double)rt * (double)p[row];
+            rp += (double)rt * (double)pr;
         }
     }
-    const double b0 = block_sum_256(rr, sh);
-    const double b1 = block_sum_256(rz, sh + 4);
-    const double b2 = block_sum_256(rp, sh);
-    const double b3 = block_sum_256(ff, sh + 4);
-    if (threadIdx.x == 0) {
-        st_coherent(partials + 4 * blockIdx.x, b0);
-        st_coherent(partials + 4 * blockIdx.x + 1, b1);
-        st_coherent(partials + 4 * blockIdx.x + 2, b2);
-        st_coherent(partials + 4 * blockIdx.x + 3, b3);
-    }
-    if (last_block_arrive(&st->arrive)) resid_finish<FOLD>(st, partials, sh);
+    put_parts4<NW>(rr, rz, rp, ff, parts, sh);
 }
 
-// BPC: z = B^-1 r with the node's inverse diagonal block (binv, planar with
-// stride nrows) instead of the point Jacobi dinv.
-template <int BS, typename T, bool FOLD, bool BPC>
-__global__ __launch_bounds__(kThreads) void sell_resid_kernel(
+// Node-block sliced rows.  SPLIT wavefronts share a slice (64 block rows),
+// each taking every SPLIT-th block column: 1 (4 or more slices per block), or
+// 4, the whole block (slices_per_block is 1).  BPC: z = B^-1 r with the
+// node's inverse diagonal block instead of the point Jacobi dinv.
+// With a shared slice p is formed in the gathers, and the slice's column ids
+// and first values are loaded before the pass's scalars are known, so the
+// two chains of loads overlap (64x16x16 Hex8, FP64 Jacobi: 17.9 -> 15.8 us
+// an iteration; 41 us with four kernels per iteration and a wavefront per
+// slice, 0.92 TB/s of operator then, 2.4 TB/s now).
+template <int BS, typename TV, typename T, bool NT, int SPLIT, bool FOLD, bool BPC>
+__global__ __launch_bounds__(kThreads) void sell_pass_kernel(
     const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w, const int32_t* __restrict__ scol,
-    const double* __restrict__ sval, int64_t nslices, int64_t nrows, int64_t slices_per_block,
-    const double* __restrict__ x64, const T* __restrict__ xs, const double* __restrict__ rhs,
-    const T* __restrict__ dinv, const T* __restrict__ binv, const T* __restrict__ p, T* __restrict__ r,
-    T* __restrict__ z, CgState* st, double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done || !st->need_update) return;
+    Vals<TV> sval, const double* __restrict__ sval64, int64_t nslices, int64_t nrows, int64_t slices_per_block,
+    PassVecs<T> v, const CgState* in, CgState* out, const double* __restrict__ upd, int nupd,
+    double* __restrict__ parts) {
+    constexpr int NW = kThreads / 64, B2 = BS * BS;
+    static_assert(SPLIT == 1 || SPLIT == NW, "a slice belongs to a wavefront or to the block");
+    constexpr bool FLY = SPLIT > 1;
+    __shared__ double sh[NW];
+    __shared__ PassGo shgo;
+    __shared__ double buf[SPLIT > 1 ? NW : 1][2 * BS][64];
     const int64_t s0 = logical_block() * slices_per_block;
     const int64_t s1 = min(nslices, s0 + slices_per_block);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int part = wv % SPLIT;
+    if constexpr (FLY) {
+        constexpr int PRE = 4, PV = 2;  // block columns with early column ids, and early values
+        using Raw = typename Vals<TV>::Raw;
+        const int64_t sl = s0;
+        const bool live = sl < s1;
+        const int64_t base = live ? glb(sl_ptr)[sl] : 0;
+        const int w = live ? glb(sl_w)[sl] : 0;
+        int32_t pc[PRE] = {};
+        Raw pv[PV][B2] = {};
+        if (w > 0) {  // a column past the row's end repeats its last one and is dropped below
+#pragma unroll
+            for (int u = 0; u < PRE; ++u) pc[u] = ld_stream<NT>(scol + base + (int64_t)min(part + u * SPLIT, w - 1) * 64 + lane);
+#pragma unroll
+            for (int u = 0; u < PV; ++u)
+#pragma unroll
+                for (int m = 0; m < B2; ++m)
+                    pv[u][m] = sval.template raw<NT>((base + (int64_t)min(part + u * SPLIT, w - 1) * 64) * B2 + lane + m * 64);
+        }
+        const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
+        if (go.done) return;
+        if (!go.resid) {
+            const T beta = (T)go.beta, zc = (T)go.zcoef;
+            const PzRecord<BS, T>* __restrict__ pz = (const PzRecord<BS, T>*)v.p;
+            auto gx = [=](int64_t c, T(&x)[BS]) {
+                const PzRecord<BS, T> w = pz[c];
+#pragma unroll
+                for (int i = 0; i < BS; ++i) x[i] = fmaT<T>(beta, w.p[i], zc * w.z[i]);
+            };
+            T acc[BS] = {};
+            if (w > 0) {
+#pragma unroll
+                for (int u = 0; u < PRE; ++u) {
+                    const int k = part + u * SPLIT;
+                    Raw rv[B2];
+#pragma unroll
+                    for (int m = 0; m < B2; ++m)
+                        rv[m] = u < PV ? pv[u < PV ? u : 0][m]
+                                       : sval.template raw<NT>((base + (int64_t)min(k, w - 1) * 64) * B2 + lane + m * 64);
+                    T xv[BS];
+                    gx(pc[u], xv);
+#pragma unroll
+                    for (int i = 0; i < BS; ++i) xv[i] = k < w ? xv[i] : T(0);
+#pragma unroll
+                    for (int j = 0; j < BS; ++j)
+#pragma unroll
+                        for (int i = 0; i < BS; ++i) acc[j] = fmaT<T>((T)sval.decode(rv[j * BS + i]), xv[i], acc[j]);
+                }
+#pragma unroll 2
+                for (int k = part + PRE * SPLIT; k < w; k += SPLIT) {
+                    const int64_t slot = base + (int64_t)k * 64;
+                    T xv[BS];
+                    gx(ld_stream<NT>(scol + slot + lane), xv);
+#pragma unroll
+                    for (int j = 0; j < BS; ++j)
+#pragma unroll
+                        for (int i = 0; i < BS; ++i)
+                            acc[j] = fmaT<T>((T)sval.template get<NT>(slot * B2 + lane + (j * BS + i) * 64), xv[i], acc[j]);
+                }
+            }
+            sell_combine<BS, SPLIT>(acc, reinterpret_cast<T(*)[BS][64]>(&buf[0][0][0]));
+            double dot = 0.0;
+            const int64_t row = sl * 64 + lane;
+            if (part == 0 && live && row < nrows) {
+                T pr[BS];
+                gx(row, pr);
+#pragma unroll
+                for (int j = 0; j < BS; ++j) {
+                    v.pnew[row * 2 * BS + j] = pr[j];
+                    v.q[row * BS + j] = acc[j];
+                    dot += (double)pr[j] * (double)acc[j];
+                }
+            }
+            dot = block_sum_waves<NW>(dot, sh);
+            if (threadIdx.x == 0) parts[blockIdx.x] = dot;
+            return;
+        }
+    } else {
+        if (in->done) return;  // direction_kernel has begun the pass
+        if (!in->resid) {
+            const T* __restrict__ p = v.p;
+            auto gx = [=](int64_t c) { return p[c]; };
+            double dot = 0.0;
+            for (int64_t sl = s0 + wv; sl < s1; sl += NW) {
+                T acc[BS];
+                sell_row<BS, TV, T, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, acc);
+                const int64_t row = sl * 64 + lane;
+                if (row < nrows) {
+#pragma unroll
+                    for (int j = 0; j < BS; ++j) {
+                        v.q[row * BS + j] = acc[j];
+                        dot += (double)p[row * BS + j] * (double)acc[j];
+                    }
+                }
+            }
+            dot = block_sum_waves<NW>(dot, sh);
+            if (threadIdx.x == 0) parts[blockIdx.x] = dot;
+            return;
+        }
+    }
     double rr = 0.0, rz = 0.0, rp = 0.0, ff = 0.0;
-    auto gx = [=](int64_t c) { return FOLD ? x64[c] + (double)xs[c] : x64[c]; };
-    for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
-        double out[BS], aout[BS];
-        sell_row_abs<BS>(sl_ptr, sl_w, scol, sval, sl, lane, gx, out, aout);
+    const double* __restrict__ x64 = v.x64;
+    const T* __restrict__ xs = v.xs;
+    auto gx = [=](int64_t c, double(&x)[BS]) {
+#pragma unroll
+        for (int i = 0; i < BS; ++i) x[i] = FOLD ? x64[c * BS + i] + (double)xs[c * BS + i] : x64[c * BS + i];
+    };
+    auto slice = [&](int64_t sl, bool live) {
+        double acc[2 * BS] = {};
+        if (live) {
+            double o[BS], a[BS];
+            sell_row_abs_part<BS, SPLIT>(sl_ptr, sl_w, scol, sval64, sl, lane, part, gx, o, a);
+#pragma unroll
+            for (int j = 0; j < BS; ++j) {
+                acc[j] = o[j];
+                acc[BS + j] = a[j];
+            }
+        }
+        sell_combine<2 * BS, SPLIT>(acc, buf);
         const int64_t row = sl * 64 + lane;
-        if (row < nrows) {
+        if (part == 0 && live && row < nrows) {
             T rt[BS];
 #pragma unroll
             for (int j = 0; j < BS; ++j) {
                 const int64_t d = row * BS + j;
-                const double res = rhs[d] - out[j];
-                const double sc = fabs(rhs[d]) + aout[j];
+                const double res = v.rhs[d] - acc[j];
+                const double sc = fabs(v.rhs[d]) + acc[BS + j];
                 ff += sc * sc;
                 rt[j] = (T)res;
-                r[d] = rt[j];
+                const int64_t e = row * kRowStride<BS, FLY> + j;
+                const T pr = v.p[e];
+                v.r[d] = rt[j];
+                if (FLY) v.pnew[e] = pr;
                 rr += res * res;
-                rp += (double)rt[j] * (double)p[d];
+                rp += (double)rt[j] * (double)pr;
             }
 #pragma unroll
             for (int j = 0; j < BS; ++j) {
@@ -394,33 +457,204 @@ __global__ __launch_bounds__(kThreads) void sell_resid_kernel(
                 if constexpr (BPC) {
                     zt = 0;
 #pragma unroll
-                    for (int i = 0; i < BS; ++i) zt = fmaT<T>(binv[(j * BS + i) * nrows + row], rt[i], zt);
+                    for (int i = 0; i < BS; ++i) zt = fmaT<T>(v.binv[(j * BS + i) * nrows + row], rt[i], zt);
                 } else {
-                    zt = dinv[d] * rt[j];
+                    zt = v.dinv[d] * rt[j];
                 }
-                z[d] = zt;
+                v.znew[row * kRowStride<BS, FLY> + j] = zt;
                 rz += (double)rt[j] * (double)zt;
             }
         }
+    };
+    if constexpr (SPLIT == 1) {
+        for (int64_t sl = s0 + wv; sl < s1; sl += NW) slice(sl, true);
+    } else {
+        slice(s0, s0 < s1);
     }
-    const double b0 = block_sum_256(rr, sh);
-    const double b1 = block_sum_256(rz, sh + 4);
-    const double b2 = block_sum_256(rp, sh);
-    const double b3 = block_sum_256(ff, sh + 4);
+    put_parts4<NW>(rr, rz, rp, ff, parts, sh);
+}
+
+// ------------------------------------------------------ update pass ----
+// Start of an update pass: false when there is nothing to update (the solve
+// has stopped, or the operator pass was a residual, whose sums block 0
+// takes).  np: blocks of the operator pass.
+template <bool FOLD>
+__device__ __forceinline__ bool update_begin(const CgState* __restrict__ in, CgState* __restrict__ out,
+                                             const double* __restrict__ parts, int np, double* sh, double* shalpha,
+                                             double& alpha, bool& fold) {
+    constexpr int NW = kThreads / 64;
+    if (in->done || in->resid) {
+        if (blockIdx.x != 0) return false;
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        if (!in->done) sum_parts_all<4, NW>(parts, np, t, sh);
+        if (threadIdx.x == 0) {
+            CgState s = *in;
+            if (!s.done) cg_after_resid<FOLD>(s, t);
+            *out = s;
+        }
+        return false;
+    }
+    double pq[1];
+    sum_parts_all<1, NW>(parts, np, pq, sh);
     if (threadIdx.x == 0) {
-        st_coherent(partials + 4 * blockIdx.x, b0);
-        st_coherent(partials + 4 * blockIdx.x + 1, b1);
-        st_coherent(partials + 4 * blockIdx.x + 2, b2);
-        st_coherent(partials + 4 * blockIdx.x + 3, b3);
+        const double a = in->rz / pq[0];
+        const bool ok = pq[0] > 0.0 && std::isfinite(a);
+        *shalpha = ok ? a : NAN;
+        if (blockIdx.x == 0) {
+            CgState s = *in;
+            s.alpha = a;
+            if (!ok) s.done = 2;  // breakdown
+            s.fresh = ok ? 1 : 0;
+            *out = s;
+        }
     }
-    if (last_block_arrive(&st->arrive)) resid_finish<FOLD>(st, partials, sh);
+    __syncthreads();
+    alpha = *shalpha;
+    fold = FOLD && in->fold_pending;
+    return alpha == alpha;
+}
+
+// x += alpha p, r -= alpha q, z = D^-1 r, partial r.z and r.r.  With FOLD
+// (FP32 solution increment xs) a pending fold moves xs into x64 first.
+// BS: values of p (and of z) per record (FLY), 0 for plain vectors.
+template <int BS, typename T, bool FOLD>
+__global__ __launch_bounds__(kThreads) void cg_update_kernel(T* __restrict__ x, double* __restrict__ x64,
+                                                             T* __restrict__ r, T* __restrict__ z,
+                                                             const T* __restrict__ p, const T* __restrict__ q,
+                                                             const T* __restrict__ dinv, int64_t n,
+                                                             int64_t per_block, const CgState* in, CgState* out,
+                                                             const double* __restrict__ parts, int np,
+                                                             double* __restrict__ upd) {
+    constexpr int NW = kThreads / 64;
+    __shared__ double sh[NW], shalpha;
+    const int64_t i0 = (int64_t)blockIdx.x * per_block;
+    const int64_t i1 = min(n, i0 + per_block);
+    // the first stride's operands are loaded before alpha is known
+    const int64_t f0 = i0 + threadIdx.x;
+    const bool first = f0 < i1;
+    T fx = 0, fp = 0, fq = 0, fr = 0, fd = 0;
+    auto pz = [](int64_t i) {
+        if constexpr (BS == 0) return i;
+        else return (int64_t)((uint32_t)i + (uint32_t)i / (BS ? BS : 1) * BS);  // (i / BS) 2 BS + i % BS
+    };
+    if (first) fx = x[f0], fp = p[pz(f0)], fq = q[f0], fr = r[f0], fd = dinv[f0];
+    double alpha;
+    bool fold;
+    if (!update_begin<FOLD>(in, out, parts, np, sh, &shalpha, alpha, fold)) return;
+    const T a = (T)alpha;
+    double rz = 0.0, rr = 0.0;
+    auto step = [&](int64_t i, T xi, T pi, T qi, T ri0, T di) {
+        if (fold) {
+            x64[i] += (double)xi;
+            xi = 0;
+        }
+        const T ri = fmaT<T>(-a, qi, ri0);
+        const T zi = di * ri;
+        x[i] = fmaT<T>(a, pi, xi);
+        r[i] = ri;
+        z[pz(i)] = zi;
+        rz += (double)ri * (double)zi;
+        rr += (double)ri * (double)ri;
+    };
+    if (first) step(f0, fx, fp, fq, fr, fd);
+#pragma unroll 4  // four strides of loads in flight; the same order of operations
+    for (int64_t i = f0 + kThreads; i < i1; i += kThreads) step(i, x[i], p[pz(i)], q[i], r[i], dinv[i]);
+    const double b0 = block_sum_waves<NW>(rz, sh);
+    const double b1 = block_sum_waves<NW>(rr, sh);
+    if (threadIdx.x == 0) {
+        upd[2 * (int64_t)blockIdx.x] = b0;
+        upd[2 * (int64_t)blockIdx.x + 1] = b1;
+    }
+}
+
+// Node-block Jacobi form: one thread per node; z = B^-1 r with B^-1 the
+// node's inverse diagonal block (planar: binv[(j*BS+i)*nnodes + n]).
+template <int BS, bool FLY, typename T, bool FOLD>
+__global__ __launch_bounds__(kThreads) void cg_update_block_kernel(T* __restrict__ x, double* __restrict__ x64,
+                                                                   T* __restrict__ r, T* __restrict__ z,
+                                                                   const T* __restrict__ p, const T* __restrict__ q,
+                                                                   const T* __restrict__ binv, int64_t nnodes,
+                                                                   int64_t per_block, const CgState* in, CgState* out,
+                                                                   const double* __restrict__ parts, int np,
+                                                                   double* __restrict__ upd) {
+    constexpr int NW = kThreads / 64;
+    __shared__ double sh[NW], shalpha;
+    const int64_t n0 = (int64_t)blockIdx.x * per_block;
+    const int64_t n1 = min(nnodes, n0 + per_block);
+    struct In {
+        T x[BS], p[BS], q[BS], r[BS], b[BS * BS];
+    };
+    auto load = [&](int64_t n, In& o) {
+#pragma unroll
+        for (int j = 0; j < BS; ++j) {
+            const int64_t i = n * BS + j;
+            o.x[j] = x[i], o.p[j] = p[n * kRowStride<BS, FLY> + j], o.q[j] = q[i], o.r[j] = r[i];
+        }
+#pragma unroll
+        for (int m = 0; m < BS * BS; ++m) o.b[m] = binv[m * nnodes + n];
+    };
+    // the first node's operands are loaded before alpha is known
+    const int64_t f0 = n0 + threadIdx.x;
+    const bool first = f0 < n1;
+    In f{};
+    if (first) load(f0, f);
+    double alpha;
+    bool fold;
+    if (!update_begin<FOLD>(in, out, parts, np, sh, &shalpha, alpha, fold)) return;
+    const T a = (T)alpha;
+    double rz = 0.0, rr = 0.0;
+    auto step = [&](int64_t n, const In& o) {
+        T rv[BS];
+#pragma unroll
+        for (int j = 0; j < BS; ++j) {
+            const int64_t i = n * BS + j;
+            T xi = o.x[j];
+            if (fold) {
+                x64[i] += (double)xi;
+                xi = 0;
+            }
+            x[i] = fmaT<T>(a, o.p[j], xi);
+            rv[j] = fmaT<T>(-a, o.q[j], o.r[j]);
+            r[i] = rv[j];
+            rr += (double)rv[j] * (double)rv[j];
+        }
+#pragma unroll
+        for (int j = 0; j < BS; ++j) {
+            T zj = 0;
+#pragma unroll
+            for (int i = 0; i < BS; ++i) zj = fmaT<T>(o.b[j * BS + i], rv[i], zj);
+            z[n * kRowStride<BS, FLY> + j] = zj;
+            rz += (double)rv[j] * (double)zj;
+        }
+    };
+    if (first) step(f0, f);
+    for (int64_t n = f0 + kThreads; n < n1; n += kThreads) {
+        In o;
+        load(n, o);
+        step(n, o);
+    }
+    const double b0 = block_sum_waves<NW>(rz, sh);
+    const double b1 = block_sum_waves<NW>(rr, sh);
+    if (threadIdx.x == 0) {
+        upd[2 * (int64_t)blockIdx.x] = b0;
+        upd[2 * (int64_t)blockIdx.x + 1] = b1;
+    }
+}
+
+// x64 += xs, xs = 0: the FP32 increment folded at the end of a solve.
+__global__ __launch_bounds__(kThreads) void fold_kernel(double* __restrict__ x64, float* __restrict__ xs, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
+        x64[i] += (double)xs[i];
+        xs[i] = 0.0f;
+    }
 }
 
 // bb = rhs.rhs (FP64), once per solve
 __global__ __launch_bounds__(kThreads) void norm2_kernel(const double* __restrict__ v, int64_t n, int64_t per_block,
-                                                         CgState* st, double* __restrict__ partials, double rtol,
+                                                         CgStates* sts, double* __restrict__ partials, double rtol,
                                                          double delta) {
     __shared__ double sh[8];
+    CgState* st = &sts->s[0];
     const int64_t i0 = (int64_t)blockIdx.x * per_block;
     const int64_t i1 = min(n, i0 + per_block);
     double s = 0.0;
@@ -432,7 +666,7 @@ __global__ __launch_bounds__(kThreads) void norm2_kernel(const double* __restric
         st_coherent(partials + 3 * blockIdx.x + 1, 0.0);
         st_coherent(partials + 3 * blockIdx.x + 2, 0.0);
     }
-    if (last_block_arrive(&st->arrive)) {
+    if (last_block_arrive(&sts->arrive)) {
         double bb, u1, u2;
         sum_partials3(partials, gridDim.x, &bb, &u1, &u2, sh);
         if (threadIdx.x == 0) {
@@ -513,6 +747,7 @@ __global__ __launch_bounds__(kThreads) void copy_kernel(const v4f* __restrict__ 
 }
 
 // --------------------------------------------------------- host side ---
+constexpr int64_t kFlyDofs = 100000;  // scalar CSR: p formed in the gathers up to this many dofs
 constexpr int kCsrLanes = 16;  // lanes per CSR row (rows of K_ff hold up to 81 entries)
 
 struct Launch {
@@ -542,12 +777,41 @@ Launch plan_sell(int64_t nslices, unsigned cap, int wave_slices) {
     return {(unsigned)grid, per};
 }
 
+// Wavefronts per slice of an operator pass, and whether p is formed in its
+// gathers (4 of them) or by direction_kernel (1).  A wavefront per slice
+// leaves a small system with fewer wavefronts than the device holds, each
+// with up to 27 block columns of loads one after the other.  Measured on
+// MI355X, us per iteration with 1 / 4 wavefronts (1: plus direction_kernel):
+// 3D FP64 Jacobi 7 slices 19.8 / 12.6, 294 slices 24.3 / 15.8, 948 slices
+// 32.1 / 27.8, 2,196 slices 71.9 / 63.5, 4,229 slices (578 MB) 126.7 / 138.8,
+// 16,967 slices 464 / 543; mixed block Jacobi 2,196 slices 38.4 / 33.5,
+// 4,229 slices (304 MB) 71.5 / 67.8, 7,241 slices (521 MB) 111 / 128.  So the
+// line is where the operator leaves the 256 MB memory-side cache (and
+// non-temporal loads begin to pay, see stream_loads).  2D FP64 (9 block
+// columns): 30 slices 14.0 / 10.4, 711 slices 15.3 / 12.9, 1,965 slices
+// 22.9 / 23.6, 3,297 slices 30.1 / 31.6.  8 wavefronts gain nothing over 4.
+constexpr double kSharedBytes = 400e6;    // 3D: operator bytes
+constexpr int64_t kSharedSlices2 = 1536;  // 2D: slices
+int slice_split(const sfem_ctx* ctx, int64_t nslices, int bs, double operator_bytes) {
+    if (ctx->tune_split > 0) return ctx->tune_split >= 4 ? 4 : 1;
+    return (bs == 3 ? operator_bytes <= kSharedBytes : nslices <= kSharedSlices2) ? 4 : 1;
+}
+
+// Non-temporal operator loads pay once the operator no longer stays in the
+// memory-side cache between iterations (FP64, a wavefront per slice: 300 MB
+// 72.9 us without and 71.9 with, 990 MB 228 and 207).
+bool stream_loads(const sfem_ctx* ctx, double operator_bytes) {
+    return ctx->tune_nt && operator_bytes > kSharedBytes;
+}
+
 struct Ops {
     sfem_ctx* ctx;
     sfem_system* S;
     int fmt;  // SFEM_FMT_CSR / SFEM_FMT_BSR
     unsigned cap;
     Launch csr, sell, vec;
+    int split;      // wavefronts per slice
+    bool fly;       // p formed in the operator pass (double buffered)
     bool nt;        // non-temporal matrix loads in the sliced SpMV
     bool block_pc;  // node-block Jacobi preconditioner
     Launch node;    // one thread per node (block update)
@@ -556,6 +820,8 @@ struct Ops {
     double* x64;
     const double* rhs;
     int64_t n;
+    unsigned pass_grid() const { return fmt == SFEM_FMT_BSR ? sell.grid : csr.grid; }
+    unsigned update_grid() const { return block_pc ? node.grid : vec.grid; }
 };
 
 template <typename TV>
@@ -577,55 +843,83 @@ Vals<SplitVal> sell_vals<SplitVal>(const sfem_system* S) { return {S->sval32.get
 template <typename TV>
 constexpr double val_bytes() { return std::is_same<TV, SplitVal>::value ? 6.0 : (double)sizeof(TV); }
 
+// One operator pass: state st->s[0] -> st->s[1].
 template <typename TV, typename T>
-void launch_spmv_cg(const Ops& o, const T* p, T* q, CgState* st, double* partials) {
+void launch_pass(const Ops& o, const PassVecs<T>& v, CgStates* st, const double* upd, double* parts) {
+    constexpr bool FOLD = std::is_same<T, float>::value;
     sfem_system* S = o.S;
     hipStream_t s = o.ctx->stream;
+    const int nupd = (int)o.update_grid();
+    const CgState* in = &st->s[0];
+    CgState* out = &st->s[1];
+    if (!o.fly) {
+        hipLaunchKernelGGL(direction_kernel<T>, dim3(o.vec.grid), dim3(kThreads), 0, s, v.pnew, (const T*)v.z, o.n,
+                           o.vec.per_block, in, out, upd, nupd);
+        SFEM_LAUNCH_CHECK();
+        in = out;
+    }
     if (o.fmt == SFEM_FMT_BSR) {
-        auto go = [&](auto kern) {
+        auto run = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(o.sell.grid), dim3(kThreads), 0, s, S->sl_ptr.get(), S->sl_w.get(),
-                               S->scol.get(), sell_vals<TV>(S), S->nslices, S->nfb, o.sell.per_block, p, q, st,
-                               partials);
+                               S->scol.get(), sell_vals<TV>(S), S->sval64.get(), S->nslices, S->nfb, o.sell.per_block,
+                               v, in, out, upd, nupd, parts);
+        };
+        auto pick = [&](auto bs, auto bpc) {
+            constexpr int BS = decltype(bs)::value;
+            constexpr bool BPC = decltype(bpc)::value;
+            if (o.split == 4) run(sell_pass_kernel<BS, TV, T, false, 4, FOLD, BPC>);
+            else if (o.nt) run(sell_pass_kernel<BS, TV, T, true, 1, FOLD, BPC>);
+            else run(sell_pass_kernel<BS, TV, T, false, 1, FOLD, BPC>);
         };
         if (S->bs == 3) {
-            if (o.nt) go(sell_spmv_cg_kernel<3, TV, T, true>);
-            else go(sell_spmv_cg_kernel<3, TV, T, false>);
+            if (o.block_pc) pick(std::integral_constant<int, 3>(), std::true_type());
+            else pick(std::integral_constant<int, 3>(), std::false_type());
         } else {
-            if (o.nt) go(sell_spmv_cg_kernel<2, TV, T, true>);
-            else go(sell_spmv_cg_kernel<2, TV, T, false>);
+            if (o.block_pc) pick(std::integral_constant<int, 2>(), std::true_type());
+            else pick(std::integral_constant<int, 2>(), std::false_type());
         }
     } else if constexpr (!std::is_same<TV, SplitVal>::value) {
-        hipLaunchKernelGGL((csr_spmv_cg_kernel<kCsrLanes, TV, T>), dim3(o.csr.grid), dim3(kThreads), 0, s,
-                           S->rowptr.get(), S->col.get(), csr_vals<TV>(S), S->nf, o.csr.per_block, p, q, st,
-                           partials);
+        auto run = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(o.csr.grid), dim3(kThreads), 0, s, S->rowptr.get(), S->col.get(),
+                               csr_vals<TV>(S), S->val64.get(), S->nf, o.csr.per_block, v, in, out, upd, nupd, parts);
+        };
+        if (o.fly) run(csr_pass_kernel<kCsrLanes, TV, T, true, FOLD>);
+        else run(csr_pass_kernel<kCsrLanes, TV, T, false, FOLD>);
     } else {
         fail(SFEM_ERR_UNSUPPORTED, "split precision needs the node-block format");
     }
     SFEM_LAUNCH_CHECK();
 }
 
-template <typename T, bool FOLD>
-void launch_resid(const Ops& o, const T* xs, const T* dinv, const T* binv, const T* p, T* r, T* z, CgState* st,
-                  double* partials) {
-    sfem_system* S = o.S;
+// One update pass: state st->s[1] -> st->s[0].
+template <typename T>
+void launch_update(const Ops& o, const PassVecs<T>& v, T* x, double* x64, CgStates* st, const double* parts,
+                   double* upd) {
+    constexpr bool FOLD = std::is_same<T, float>::value;
     hipStream_t s = o.ctx->stream;
-    if (o.fmt == SFEM_FMT_BSR) {
-        auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(o.sell.grid), dim3(kThreads), 0, s, S->sl_ptr.get(), S->sl_w.get(),
-                               S->scol.get(), S->sval64.get(), S->nslices, S->nfb, o.sell.per_block, o.x64, xs,
-                               o.rhs, dinv, binv, p, r, z, st, partials);
-        };
-        if (S->bs == 3) {
-            if (o.block_pc) go(sell_resid_kernel<3, T, FOLD, true>);
-            else go(sell_resid_kernel<3, T, FOLD, false>);
-        } else {
-            if (o.block_pc) go(sell_resid_kernel<2, T, FOLD, true>);
-            else go(sell_resid_kernel<2, T, FOLD, false>);
-        }
+    const CgState* in = &st->s[1];
+    CgState* out = &st->s[0];
+    const int np = (int)o.pass_grid();
+    auto point = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(o.vec.grid), dim3(kThreads), 0, s, x, x64, v.r, v.znew, (const T*)v.pnew,
+                           (const T*)v.q, v.dinv, o.n, o.vec.per_block, in, out, parts, np, upd);
+    };
+    auto block = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(o.node.grid), dim3(kThreads), 0, s, x, x64, v.r, v.znew, (const T*)v.pnew,
+                           (const T*)v.q, v.binv, o.S->nfb, o.node.per_block, in, out, parts, np, upd);
+    };
+    const bool bs3 = o.S->bs == 3;
+    if (!o.block_pc) {
+        if (!o.fly) point(cg_update_kernel<0, T, FOLD>);
+        else if (o.fmt != SFEM_FMT_BSR) point(cg_update_kernel<1, T, FOLD>);
+        else if (bs3) point(cg_update_kernel<3, T, FOLD>);
+        else point(cg_update_kernel<2, T, FOLD>);
+    } else if (o.fly) {
+        if (bs3) block(cg_update_block_kernel<3, true, T, FOLD>);
+        else block(cg_update_block_kernel<2, true, T, FOLD>);
     } else {
-        hipLaunchKernelGGL((csr_resid_kernel<kCsrLanes, T, FOLD>), dim3(o.csr.grid), dim3(kThreads), 0, s,
-                           S->rowptr.get(), S->col.get(), S->val64.get(), S->nf, o.csr.per_block, S->x.get(), xs,
-                           S->rhs.get(), dinv, p, r, z, st, partials);
+        if (bs3) block(cg_update_block_kernel<3, false, T, FOLD>);
+        else block(cg_update_block_kernel<2, false, T, FOLD>);
     }
     SFEM_LAUNCH_CHECK();
 }
@@ -655,13 +949,14 @@ int resolve_format(const sfem_system* S, int fmt) {
 }
 
 // Device workspace of one solve when the caller provides it (the solve that
-// allocates nothing): four CG vectors, the FP32 solution increment, the
-// per-block partial sums and the state.
+// allocates nothing): the CG vectors r and q, the direction and z (pz: two
+// arrays of records, or p and z in the first), the FP32 solution increment,
+// the per-block partial sums and the state.
 struct CgWork {
-    void *r, *z, *q, *p, *xs;
+    void *r, *q, *pz[2], *xs;
     double* partials;
     size_t max_partials;  // doubles
-    CgState* st;
+    CgStates* st;
 };
 
 // Zeroes n elements of a vector (a kernel, not hipMemsetAsync, so that the
@@ -672,7 +967,9 @@ __global__ __launch_bounds__(kThreads) void zero_kernel(T* __restrict__ v, int64
         v[i] = T(0);
 }
 
-__global__ void cg_state_init_kernel(CgState* st) {
+__global__ __launch_bounds__(64) void cg_state_init_kernel(CgStates* st, long long max_iter) {
+    for (int k = (int)threadIdx.x; k < (int)(sizeof(st->arrive.c) / sizeof(st->arrive.c[0])); k += 64)
+        st->arrive.c[k] = 0;
     if (threadIdx.x != 0) return;
     CgState init{};
     init.rr = HUGE_VAL;
@@ -681,12 +978,8 @@ __global__ void cg_state_init_kernel(CgState* st) {
     init.best_rr = HUGE_VAL;
     init.best_true = HUGE_VAL;
     init.need_update = 1;
-    *st = init;
-}
-
-// The iteration cap was reached: the true residual of the final iterate is due.
-__global__ void cg_state_flag_update_kernel(CgState* st) {
-    if (threadIdx.x == 0) st->need_update = 1;
+    init.max_iter = max_iter;
+    st->s[0] = init;
 }
 
 template <typename T>
@@ -712,38 +1005,56 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
         fail(SFEM_ERR_UNSUPPORTED, "block-Jacobi preconditioning needs the node-block format");
     if (o->preconditioner != SFEM_PC_JACOBI && !block_pc) fail(SFEM_ERR_ARGUMENT, "solve: unknown preconditioner");
     double* x64 = padded ? S->px.get() : S->x.get();
-    Ops ops{ctx, S, fmt, (unsigned)std::max(8, ctx->n_cu * 8), {}, {}, {}, ctx->tune_nt, block_pc, {},
+    Ops ops{ctx, S, fmt, (unsigned)std::max(8, ctx->n_cu * 8), {}, {}, {}, 1, false, false, block_pc, {},
             x64, padded ? S->prhs.get() : S->rhs.get(), nf};
     if (block_pc) ops.node = plan(S->nfb, kThreads, std::max(8, ctx->n_cu * 4));
     ops.csr = plan(S->nf, kThreads / kCsrLanes, ops.cap);
-    if (S->has_block) ops.sell = plan_sell(S->nslices, ops.cap, ctx->tune_wave_slices);
+    ops.fly = nf <= kFlyDofs;
+    if (fmt == SFEM_FMT_BSR) {
+        const double op_bytes = spmv_bytes_for(S, fmt, val_bytes<TV>(), 0, 0);
+        ops.split = slice_split(ctx, S->nslices, S->bs, op_bytes);
+        ops.fly = ops.split > 1;
+        ops.nt = stream_loads(ctx, op_bytes);
+        if (ops.split > 1) {  // a block per slice
+            ops.sell = {(unsigned)std::max<int64_t>(8, (S->nslices + 7) / 8 * 8), 1};
+        } else {
+            ops.sell = plan_sell(S->nslices, ops.cap, ctx->tune_wave_slices);
+        }
+    }
     ops.vec = plan(nf, kThreads, std::max(8, ctx->n_cu * 4));
-    const unsigned maxgrid = std::max({ops.csr.grid, ops.sell.grid, ops.vec.grid, ops.node.grid});
+    // the operator pass's sums (4 per block), then the update's (2 per block;
+    // the rhs norm's first: 3 per block)
+    const size_t nparts = 4 * (size_t)ops.pass_grid();
+    const size_t nupd = std::max(2 * (size_t)ops.update_grid(), 3 * (size_t)ops.vec.grid);
 
-    DevBuf<T> rb, zb, qb, pb, xsb;
+    DevBuf<T> rb, qb, pzb[2], xsb;
     DevBuf<double> partb;
-    DevBuf<CgState> dst;
-    T *r, *z, *q, *p, *xsv = nullptr;
-    double* partials;
-    CgState* st;
+    DevBuf<CgStates> dst;
+    T *r, *q, *pz[2], *xsv = nullptr;
+    double* parts;
+    CgStates* st;
     if (ws) {
-        if (4 * (size_t)maxgrid > ws->max_partials) fail(SFEM_ERR_UNSUPPORTED, "solve: workspace too small");
-        r = (T*)ws->r, z = (T*)ws->z, q = (T*)ws->q, p = (T*)ws->p;
+        if (nparts + nupd > ws->max_partials) fail(SFEM_ERR_UNSUPPORTED, "solve: workspace too small");
+        r = (T*)ws->r, q = (T*)ws->q, pz[0] = (T*)ws->pz[0], pz[1] = (T*)ws->pz[1];
         if (FOLD) xsv = (T*)ws->xs;
-        partials = ws->partials;
+        parts = ws->partials;
         st = ws->st;
     } else {
-        rb.reset(ctx, nf), zb.reset(ctx, nf), qb.reset(ctx, nf), pb.reset(ctx, nf);
-        r = rb.get(), z = zb.get(), q = qb.get(), p = pb.get();
+        rb.reset(ctx, nf), qb.reset(ctx, nf), pzb[0].reset(ctx, 2 * nf);
+        if (ops.fly) pzb[1].reset(ctx, 2 * nf);
+        r = rb.get(), q = qb.get(), pz[0] = pzb[0].get(), pz[1] = pzb[1].get();
         if (FOLD) {
             xsb.reset(ctx, nf);
             xsv = xsb.get();
         }
-        partb.reset(ctx, 4 * (size_t)maxgrid);
-        partials = partb.get();
+        partb.reset(ctx, nparts + nupd);
+        parts = partb.get();
         dst.reset(ctx, 1);
         st = dst.get();
     }
+    // z: BS values after a record's p, or the second half of the first array
+    const int64_t zoff = !ops.fly ? nf : fmt == SFEM_FMT_BSR ? S->bs : 1;
+    double* upd = parts + nparts;
     const T* dinv = padded ? (FOLD ? (const T*)S->pdinv32.get() : (const T*)S->pdinv64.get())
                            : (FOLD ? (const T*)S->dinv32.get() : (const T*)S->dinv64.get());
     const T* binv = FOLD ? (const T*)S->binv32.get() : (const T*)S->binv64.get();
@@ -755,8 +1066,8 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     const T* xs = FOLD ? xsv : nullptr;
     if (o->x0_zero) zero_dev(ctx, S->x.get(), S->nf);
     if (padded) pad_gather(ctx, S, S->x.get(), x64);  // start from the current solution
-    zero_dev(ctx, p, nf);
-    hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(64), 0, ctx->stream, st);
+    zero_dev(ctx, pz[0], 2 * nf);
+    hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(64), 0, ctx->stream, st, (long long)o->max_iter);
     SFEM_LAUNCH_CHECK();
 
     const bool timed_run = ws == nullptr;  // events are runtime objects: none in the no-allocation solve
@@ -774,40 +1085,30 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     }
     if (timed_run) SFEM_HIP(hipEventRecord(t0, ctx->stream));
     hipLaunchKernelGGL(norm2_kernel, dim3(ops.vec.grid), dim3(kThreads), 0, ctx->stream, ops.rhs, nf,
-                       ops.vec.per_block, st, partials, o->rtol, o->reliable_delta);
+                       ops.vec.per_block, st, upd, o->rtol, o->reliable_delta);
     SFEM_LAUNCH_CHECK();
-    launch_resid<T, FOLD>(ops, xs, dinv, binv, p, r, z, st, partials);
+    T* const pz1 = ops.fly ? pz[1] : pz[0];
+    PassVecs<T> v{pz[0], pz[0] + zoff, pz1, pz1 + zoff, q, r, x64, xs, ops.rhs, dinv, binv};
 
     CgState host{};
-    int64_t enq = 0, counted = 0, timed = 0;
+    int64_t counted = 0, timed = 0;
     double spmv_ms = 0.0;
-    d2h(ctx, &host, st, sizeof(host));
-    while (!host.done && enq < o->max_iter) {
-        const int64_t chunk = std::min<int64_t>(check, o->max_iter - enq);
+    // the first step is the residual of the start; a step is an iteration or
+    // a residual replacement, and the device stops at the iteration cap
+    for (int64_t chunk = 1; !host.done; chunk = check) {
         for (int64_t k = 0; k < chunk; ++k) {
-            hipLaunchKernelGGL(p_update_kernel<T>, dim3(ops.vec.grid), dim3(kThreads), 0, ctx->stream, p, z, nf,
-                               ops.vec.per_block, st);
-            SFEM_LAUNCH_CHECK();
             if (!ev.empty()) SFEM_HIP(hipEventRecord(ev[2 * k], ctx->stream));
-            launch_spmv_cg<TV, T>(ops, p, q, st, partials);
+            launch_pass<TV, T>(ops, v, st, upd, parts);
             if (!ev.empty()) SFEM_HIP(hipEventRecord(ev[2 * k + 1], ctx->stream));
-            if (!block_pc)
-                hipLaunchKernelGGL((cg_update_kernel<T, FOLD>), dim3(ops.vec.grid), dim3(kThreads), 0, ctx->stream,
-                                   x, x64, r, z, p, q, dinv, nf, ops.vec.per_block, st, partials);
-            else if (S->bs == 3)
-                hipLaunchKernelGGL((cg_update_block_kernel<3, T, FOLD>), dim3(ops.node.grid), dim3(kThreads), 0,
-                                   ctx->stream, x, x64, r, z, p, q, binv, S->nfb, ops.node.per_block, st, partials);
-            else
-                hipLaunchKernelGGL((cg_update_block_kernel<2, T, FOLD>), dim3(ops.node.grid), dim3(kThreads), 0,
-                                   ctx->stream, x, x64, r, z, p, q, binv, S->nfb, ops.node.per_block, st, partials);
-            SFEM_LAUNCH_CHECK();
-            launch_resid<T, FOLD>(ops, xs, dinv, binv, p, r, z, st, partials);
+            launch_update<T>(ops, v, x, x64, st, parts, upd);
+            T *const po = v.pnew, *const zo = v.znew;  // in place: the same arrays
+            v.pnew = const_cast<T*>(v.p), v.znew = const_cast<T*>(v.z);
+            v.p = po, v.z = zo;
         }
-        enq += chunk;
-        d2h(ctx, &host, st, sizeof(host));
+        d2h(ctx, &host, &st->s[0], sizeof(host));
         if (!ev.empty()) {
             // launches after the stop exit at once; time only the real ones
-            const int64_t real = std::min<int64_t>(chunk, std::max<int64_t>(0, host.iters - counted));
+            const int64_t real = std::min<int64_t>(chunk, std::max<int64_t>(0, host.iters + host.updates - counted));
             for (int64_t k = 0; k < real; ++k) {
                 float ms = 0;
                 SFEM_HIP(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]));
@@ -815,13 +1116,7 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
             }
             timed += real;
         }
-        counted = host.iters;
-    }
-    if (!host.done) {  // iteration cap: evaluate the true residual of the final iterate
-        hipLaunchKernelGGL(cg_state_flag_update_kernel, dim3(1), dim3(64), 0, ctx->stream, st);
-        SFEM_LAUNCH_CHECK();
-        launch_resid<T, FOLD>(ops, xs, dinv, binv, p, r, z, st, partials);
-        d2h(ctx, &host, st, sizeof(host));
+        counted = host.iters + host.updates;
     }
     if (FOLD) {  // x = x64 + xs
         hipLaunchKernelGGL(fold_kernel, dim3(ops.vec.grid), dim3(kThreads), 0, ctx->stream, x64, (float*)xsv, nf);
@@ -853,7 +1148,7 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     stats->spmv_bytes = spmv_bytes_for(S, fmt, val_bytes<TV>(), sizeof(T), 2);
     stats->converged = host.done == 1 ? 1 : 0;
     stats->format = fmt;
-    stats->stop_reason = host.done == 0 ? 4 : host.done;
+    stats->stop_reason = host.done;
     stats->floor_residual = host.bb > 0 ? std::sqrt(host.floor_rr / 16.0 / host.bb) : 0.0;
 }
 
@@ -861,14 +1156,15 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
 
 // ---------------------------------------------- the no-allocation solve --
 // Workspace of sfem_system_solve_noalloc: a file-scope device array, one copy
-// per GPU, held until the process ends.  Layout: five CG vectors of
-// kNoAllocMaxDofs doubles (r, z, q, p, FP32 increment), the per-block
-// partial sums, the CG state.  Host code reaches it only through the address
+// per GPU, held until the process ends.  Layout: six CG vectors of
+// kNoAllocMaxDofs doubles (r, q, and p with z twice; the FP32 vectors are half
+// as long, and the increment lies behind r), the per-block partial sums, the
+// CG state.  Host code reaches it only through the address
 // hipGetSymbolAddress returns for the current device (sfem_ctx::scratch).
 namespace {
 constexpr size_t kNoAllocVec = sizeof(double) * (size_t)kNoAllocMaxDofs;
 constexpr size_t kNoAllocPartials = 4 * 16384;  // doubles: 4 per block of the largest plan
-constexpr size_t kNoAllocBytes = 5 * kNoAllocVec + sizeof(double) * kNoAllocPartials + (sizeof(CgState) + 255) / 256 * 256;
+constexpr size_t kNoAllocBytes = 6 * kNoAllocVec + sizeof(double) * kNoAllocPartials + (sizeof(CgStates) + 255) / 256 * 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 }  // namespace
 
@@ -906,9 +1202,10 @@ void system_solve_noalloc(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* 
         fail(SFEM_ERR_STATE, "solve_noalloc: the operator format these options read is not built yet; one "
                              "sfem_system_solve with the same precision and format builds it");
     unsigned char* base = static_cast<unsigned char*>(ctx->scratch);
-    CgWork ws{base, base + kNoAllocVec, base + 2 * kNoAllocVec, base + 3 * kNoAllocVec, base + 4 * kNoAllocVec,
-              reinterpret_cast<double*>(base + 5 * kNoAllocVec), kNoAllocPartials,
-              reinterpret_cast<CgState*>(base + 5 * kNoAllocVec + sizeof(double) * kNoAllocPartials)};
+    unsigned char* end = base + 6 * kNoAllocVec;
+    CgWork ws{base, base + kNoAllocVec, {base + 2 * kNoAllocVec, base + 4 * kNoAllocVec}, base + kNoAllocVec / 2,
+              reinterpret_cast<double*>(end), kNoAllocPartials,
+              reinterpret_cast<CgStates*>(end + sizeof(double) * kNoAllocPartials)};
     sfem_solve_opts oo = *o;
     oo.time_kernels = 0;
     switch (o->precision) {

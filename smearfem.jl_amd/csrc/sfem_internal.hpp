@@ -77,6 +77,7 @@ struct sfem_ctx {
     // slices over at most 8 blocks per CU).
     bool tune_nt = true;        // non-temporal matrix loads
     int tune_wave_slices = 1;   // slices per wavefront
+    int tune_split = 0;         // wavefronts per slice (1 or 4): 0 by size (SFEM_SELL_SPLIT)
     // Grid barrier of the persistent solvers: workspace, wait limit (100 MHz
     // ticks; SFEM_BARRIER_TIMEOUT_US) and whether the per-XCD grouped form may
     // be used (SFEM_BARRIER_GROUPED=0 forces the per-block form).

@@ -166,22 +166,32 @@ struct Arrivals {
 };
 }  // namespace sfem
 
-// Device scalars of one CG solve; updated only by the last block of each
-// reduction, read by every kernel of the next step.
+// Device scalars of one CG solve.  Two copies: each pass (operator, update)
+// reads one and its first block writes the other, so every block of a pass
+// sees the same values and no kernel waits for another block's scalars.
 struct CgState {
     double rz, rz_prev, beta, alpha, rr, bb, maxrr, tol2bb, delta2, rr_true;
     double zcoef;        // p_new = zcoef*z + beta*p; 1 except right after a residual replacement
     double best_rr;      // smallest recurrence |r|^2 seen (stagnation check)
     double best_true;    // smallest true |r|^2 at a replacement
     double floor_rr;     // 16 (eps || |rhs| + |K||x| ||)^2 at the last replacement
-    int done;            // 1 converged, 2 breakdown, 3 stagnated
+    int done;            // 1 converged, 2 breakdown, 3 stagnated, 4 iteration cap
     int need_update;     // the true FP64 residual is due
     int fold_pending;    // FP32 solution increment to be folded into x64
     int stall;           // replacements in a row without progress
+    int resid;           // the last operator pass was an FP64 residual
+    int fresh;           // the last update's sums (r.z, r.r) are still to be taken
+    int capped;          // the iteration cap was reached: the residual due is the last one
+    int pad0;
     long long iters, updates, best_it;
     long long last_upd;  // iteration of the latest replacement
     long long best_true_it;  // iteration of best_true
-    sfem::Arrivals arrive;
+    long long max_iter;
+};
+
+struct CgStates {
+    CgState s[2];
+    sfem::Arrivals arrive;  // the rhs norm's
 };
 
 // K_ff and its solver formats, plus the data to recombine the solution.

@@ -121,6 +121,42 @@ __device__ __forceinline__ void sum_partials3(const double* partials, int nparts
     *c = block_sum_256(s[2], sh);
 }
 
+// Sum over a block of NW wavefronts, in every thread (sh: NW slots); the
+// order is fixed: butterfly per wavefront, then the wavefronts pairwise.
+template <int NW>
+__device__ __forceinline__ double block_sum_waves(double v, double* sh) {
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0) sh[w] = v;
+    __syncthreads();
+    double t[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) t[i] = sh[i];
+#pragma unroll
+    for (int h = NW / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int i = 0; i < h; ++i) t[i] += t[i + h];
+    __syncthreads();
+    return t[0];
+}
+
+// Sums of nparts partial W-tuples (stride W) an earlier kernel on the stream
+// left, by a block of NW wavefronts, in every thread.  Every block of a
+// kernel that needs the sums calls it for itself and gets the same bits.
+template <int W, int NW>
+__device__ __forceinline__ void sum_parts_all(const double* __restrict__ partials, int nparts, double (&out)[W],
+                                              double* sh) {
+    double s[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) s[k] = 0.0;
+#pragma unroll 2
+    for (int i = threadIdx.x; i < nparts; i += NW * 64)
+#pragma unroll
+        for (int k = 0; k < W; ++k) s[k] += partials[(int64_t)W * i + k];
+#pragma unroll
+    for (int k = 0; k < W; ++k) out[k] = block_sum_waves<NW>(s[k], sh);
+}
+
 // Logical block id: consecutive logical blocks land on the same XCD (the
 // hardware deals workgroups round-robin over the 8 XCDs), so each XCD's L2
 // sees a contiguous part of the rows and of the gathered vector.
@@ -242,6 +278,57 @@ __device__ __forceinline__ void sell_row(const int64_t* __restrict__ sl_ptr, con
 #pragma unroll
             for (int i = 0; i < BS; ++i)
                 out[j] = fmaT<ACC>((ACC)vals.template get<NT>(v + (j * BS + i) * 64), xv[i], out[j]);
+    }
+}
+
+// The block columns part, part + SPLIT, ... of this lane's block row in FP64
+// (SPLIT wavefronts share a slice; their sums are added by sell_combine), and
+// aout[j] = sum |M_ji x_i|.  gx(c, x) gathers block row c of the vector.
+template <int BS, int SPLIT, typename Gather>
+__device__ __forceinline__ void sell_row_abs_part(const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w,
+                                                  const int32_t* __restrict__ scol, const double* __restrict__ sval,
+                                                  int64_t sl, int lane, int part, Gather gx, double out[BS],
+                                                  double aout[BS]) {
+    constexpr int B2 = BS * BS;
+    const int64_t base = glb(sl_ptr)[sl];
+    const int w = glb(sl_w)[sl];
+#pragma unroll
+    for (int j = 0; j < BS; ++j) out[j] = aout[j] = 0.0;
+#pragma unroll 1
+    for (int k = part; k < w; k += SPLIT) {
+        const int64_t slot = base + (int64_t)k * 64;
+        const int64_t c = ld_stream<true>(scol + slot + lane);
+        double m[B2], xv[BS];
+#pragma unroll
+        for (int i = 0; i < B2; ++i) m[i] = ld_stream<true>(sval + slot * B2 + lane + i * 64);
+        gx(c, xv);
+#pragma unroll
+        for (int j = 0; j < BS; ++j)
+#pragma unroll
+            for (int i = 0; i < BS; ++i) {
+                out[j] = fma(m[j * BS + i], xv[i], out[j]);
+                aout[j] = fma(fabs(m[j * BS + i]), fabs(xv[i]), aout[j]);
+            }
+    }
+}
+
+// Sums the W values each lane of SPLIT wavefronts holds for its row into the
+// slice's first wavefront (parts in ascending order).  buf: one W x 64 array
+// per wavefront of the block.  Every thread of the block must call it; the
+// caller's buf is free again after its next barrier.
+template <int W, int SPLIT, typename ACC>
+__device__ __forceinline__ void sell_combine(ACC (&v)[W], ACC (*buf)[W][64]) {
+    if constexpr (SPLIT > 1) {
+        const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        if (wv % SPLIT)
+#pragma unroll
+            for (int j = 0; j < W; ++j) buf[wv][j][lane] = v[j];
+        __syncthreads();
+        if (wv % SPLIT == 0)
+#pragma unroll
+            for (int h = 1; h < SPLIT; ++h)
+#pragma unroll
+                for (int j = 0; j < W; ++j) v[j] += buf[wv + h][j][lane];
     }
 }
 

@@ -211,3 +211,42 @@ def test_unattainable_tolerance_stops_on_stagnation(ctx):
         assert 0 < st["floor_residual"] < 1e-10 and st["rel_residual"] <= 20 * st["floor_residual"]
     S.close()
     K.close()
+
+
+@pytest.mark.parametrize("split", ["1", "4"])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (4, 3, 3), (7, 3, 1), (5, 4, 8), (9, 7), (1, 1), (33, 3)])
+def test_operator_pass_forms(dims, split, monkeypatch):
+    # the sliced operator pass with a wavefront per slice and with a block per
+    # slice: row counts around the 64 of a slice (4, 64, 64, 225, 72, 2, 132
+    # block rows), rows narrower than the columns loaded early, every
+    # precision, and the iteration cap met exactly
+    print(f"[case] operator pass {dims} split={split}", flush=True)
+    monkeypatch.setenv("SFEM_SELL_SPLIT", split)
+    ctx = smearfem.Context(0)
+    m = structured_mesh(dims)
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=11)
+    fixed = clamp_x0(m)
+    f = random_face_load(m, m.ndim - 1, 1, fixed, seed=12)
+    perm = np.random.default_rng(13).permutation(m.n_nodes)  # node k is numbered perm[k]
+    inv = np.argsort(perm)
+    f, fixed = f.reshape(-1, m.ndim)[inv].ravel(), fixed.reshape(-1, m.ndim)[inv].ravel()
+    nodes, ien = m.NodeList[:, inv], perm[m.IEN - 1] + 1
+    K = smearfem.assemble_system(0, nodes, ien, m.ndim, "Q1", m.ndim, m.ID, young, 0.3, ctx=ctx, device=True,
+                                 n_elem=m.n_elem)
+    Kr = O.assemble_system(0, nodes, ien, m.ndim, "Q1", m.ndim, m.ID, young, 0.3, n_elem=m.n_elem)
+    Kff, rhs = O.eliminate(Kr, fixed, f)
+    q_ref = O.recombine(fixed, None, O.dense_solve(Kff, rhs))
+    bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+    S = System(K, bc)
+    for precision, pc in (("fp64", "jacobi"), ("fp64", "block_jacobi"), ("mixed", "jacobi"),
+                          ("mixed", "block_jacobi"), ("split", "block_jacobi"), ("fp32_matrix", "jacobi")):
+        st = S.solve(precision, "bsr", rtol=1e-12, preconditioner=pc)
+        assert st["stop_reason"] == 1 and relerr(S.solution(), q_ref) <= ERR, (precision, pc)
+    full = S.solve("fp64", "bsr", rtol=1e-12)
+    if full["iterations"] > 3:
+        st = S.solve("fp64", "bsr", rtol=1e-12, max_iter=3, raise_on_fail=False)
+        assert st["iterations"] == 3 and st["stop_reason"] == 4
+    S.close()
+    bc.close()
+    K.close()
+    ctx.close()
