@@ -1100,21 +1100,45 @@ __device__ __forceinline__ void cheb_finish(int64_t row, const ChebIn<BS>& o, co
     }
 }
 
-template <int BS, int MODE, bool NT, typename TV>
+// Finest-level step on the sliced operator.  SHARED: a block per slice
+// (SharedSlice; the rule is slice_split's), the first wavefront finishes the
+// rows with operands it loaded beside its columns.
+template <int BS, int MODE, bool NT, bool SHARED, typename TV>
 __global__ __launch_bounds__(kThreads) void cheb_sell_kernel(SellOp<TV> op, const float* v, float* __restrict__ r,
                                                              float* __restrict__ x, const float* d_in,
                                                              float* __restrict__ d_out, float c1, float c2,
                                                              const float* __restrict__ binv, const int* done) {
-    if (*done) return;
-    const int64_t s0 = logical_block() * op.per_block;
-    const int64_t s1 = min(op.nslices, s0 + op.per_block);
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    auto gx = [=](int64_t c) { return v[c]; };
-    for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
-        float out[BS];
-        sell_row<BS, TV, float, NT>(op.sl_ptr, op.sl_w, op.scol, Vals<TV>{op.val}, sl, lane, gx, out);
+    if constexpr (SHARED) {
+        __shared__ float buf[kThreads / 64][BS][64];
+        const bool stop = *done != 0;  // checked before the stores
+        const int64_t sl = logical_block();
+        if (sl >= op.nslices) return;
+        SharedSlice<BS, TV, NT> cols(op.scol, Vals<TV>{op.val});
+        cols.load(op.sl_ptr, op.sl_w, sl);
         const int64_t row = sl * 64 + lane;
-        if (row < op.nrows) cheb_epilogue<BS, MODE>(row, op.nrows, out, r, x, d_in, d_out, c1, c2, binv);
+        const bool own = w == 0 && row < op.nrows;
+        ChebIn<BS> in;
+        if (own) cheb_load<BS, MODE>(row, op.nrows, r, x, d_in, binv, in);
+        auto gx = [=](int64_t c, float(&xv)[BS]) {
+#pragma unroll
+            for (int i = 0; i < BS; ++i) xv[i] = v[c * BS + i];
+        };
+        float out[BS] = {};
+        cols.apply(gx, out);
+        sell_combine<BS, kThreads / 64>(out, buf);
+        if (own && !stop) cheb_finish<BS, MODE>(row, in, out, r, x, d_in != nullptr, d_out, c1, c2);
+    } else {
+        if (*done) return;
+        const int64_t s0 = logical_block() * op.per_block;
+        const int64_t s1 = min(op.nslices, s0 + op.per_block);
+        auto gx = [=](int64_t c) { return v[c]; };
+        for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
+            float out[BS];
+            sell_row<BS, TV, float, NT>(op.sl_ptr, op.sl_w, op.scol, Vals<TV>{op.val}, sl, lane, gx, out);
+            const int64_t row = sl * 64 + lane;
+            if (row < op.nrows) cheb_epilogue<BS, MODE>(row, op.nrows, out, r, x, d_in, d_out, c1, c2, binv);
+        }
     }
 }
 
@@ -1385,6 +1409,24 @@ __global__ __launch_bounds__(kThreads) void cheb_first_kernel(const TB* __restri
     }
 }
 
+// Grid nodes fit 31 bits (the row maps are int32): the transfers index in 32
+// bits, whose divisions by the grid sizes cost a third of the 64-bit ones
+// (with 27 nodes per thread these were most of a small level's restriction).
+struct Grid32 {
+    uint32_t n0, n1, n2;
+    __device__ __forceinline__ explicit Grid32(const Grid& g)
+        : n0((uint32_t)g.n0), n1((uint32_t)g.n1), n2((uint32_t)g.n2) {}
+    __device__ __forceinline__ uint32_t at(uint32_t x, uint32_t y, uint32_t z) const { return x + n0 * (y + n1 * z); }
+};
+
+template <int ND>
+__device__ __forceinline__ void coords32(uint32_t node, const Grid32& g, uint32_t (&c)[3]) {
+    const uint32_t t = node / g.n0;
+    c[0] = node - t * g.n0;
+    c[2] = ND == 3 ? t / g.n1 : 0;
+    c[1] = t - c[2] * g.n1;
+}
+
 // b_c = P' r_f on the coarse grid (0 on fixed coarse dofs); row_of_node maps
 // fine grid nodes to rows of r_f (NULL: the identity); r_f is in units of
 // 1 / rscale.  FIRST: also the coarse level's first smoothing step
@@ -1396,32 +1438,30 @@ __device__ __forceinline__ void restrict_row(int64_t I, const float* __restrict_
                                              const float* __restrict__ binv, float c2, float cscale,
                                              float* __restrict__ rc, float* __restrict__ xc, float* __restrict__ dc,
                                              bool skip) {
-    constexpr int BS = ND;
-    int64_t ci[3];
-    coords_of<ND>(I, gc, ci);
-    // the interpolation support of I per direction (child(); the identity
-    // along directions that are not coarsened)
+    constexpr int BS = ND, NZ = ND == 3 ? 3 : 1;
+    const Grid32 f32(gf), c32(gc);
+    uint32_t ci[3];
+    coords32<ND>((uint32_t)I, c32, ci);
+    // the interpolation support of I per direction (as child(): fine nodes
+    // 2c - 1, 2c, 2c + 1 inside the grid, weights 1/2, 1, 1/2; for odd
+    // element counts the last fine node belongs to the last coarse node
+    // alone; the identity along directions that are not coarsened)
     const int f[3] = {f0, f1, f2};
-    const int64_t ef[3] = {gf.n0 - 1, gf.n1 - 1, gf.n2 - 1};
-    int64_t fi[3][3] = {};  // unused entries: node 0 (their terms are not added)
-    float fw[3][3] = {};
-    int nk[3];
+    const int ef[3] = {(int)f32.n0 - 1, (int)f32.n1 - 1, (int)f32.n2 - 1};
+    int fi[3][3];
+    float fw[3][3];
+    bool fin[3][3];
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        nk[d] = 0;
-        if (f[d] != 2) {
-            fi[d][0] = ci[d];
-            fw[d][0] = 1.0f;
-            nk[d] = 1;
-            continue;
-        }
+        const int c = (int)ci[d], e = ef[d];
+        const bool odd = e & 1;
+#pragma unroll
         for (int k = 0; k < 3; ++k) {
-            int64_t i;
-            double w;
-            if (child(ci[d], k, ef[d], i, w)) {
-                fi[d][nk[d]] = i;
-                fw[d][nk[d]] = (float)w;
-                ++nk[d];
-            }
+            const int i = f[d] != 2 ? c : odd && 2 * c > e ? e : 2 * c + k - 1;
+            const bool in = f[d] != 2 || (odd && 2 * c > e) ? k == 1 : i >= 0 && i <= e && !(odd && i == e);
+            fi[d][k] = in ? i : 0;
+            fin[d][k] = in;
+            fw[d][k] = f[d] == 2 && k != 1 ? 0.5f : 1.0f;
         }
     }
     float acc[BS];
@@ -1432,20 +1472,21 @@ __device__ __forceinline__ void restrict_row(int64_t I, const float* __restrict_
     // their term is then dropped by a select, so the sums are exactly those
     // of the support points alone, whatever that row holds (Inf / NaN too)
 #pragma unroll
-    for (int kz = 0; kz < 3; ++kz)
+    for (int kz = 0; kz < NZ; ++kz)
 #pragma unroll
         for (int ky = 0; ky < 3; ++ky)
 #pragma unroll
             for (int kx = 0; kx < 3; ++kx) {
-                const bool in = kx < nk[0] && ky < nk[1] && kz < nk[2];
-                const int64_t fn = node_at(gf, fi[0][kx], fi[1][ky], fi[2][kz]);
-                const int64_t mrow = row_of_node ? (int64_t)row_of_node[fn] : fn;
+                const int lz = ND == 3 ? kz : 1;  // 2D: the identity along z
+                const bool in = fin[0][kx] && fin[1][ky] && fin[2][lz];
+                const uint32_t fn = in ? f32.at((uint32_t)fi[0][kx], (uint32_t)fi[1][ky], (uint32_t)fi[2][lz]) : 0u;
+                const int32_t mrow = row_of_node ? row_of_node[fn] : (int32_t)fn;
                 const bool use = in && mrow >= 0;
-                const int64_t row = use ? mrow : 0;
-                const float w = fw[0][kx] * fw[1][ky] * fw[2][kz];
+                const uint32_t row = use ? (uint32_t)mrow : 0u;
+                const float w = fw[0][kx] * fw[1][ky] * fw[2][lz];
 #pragma unroll
                 for (int j = 0; j < BS; ++j) {
-                    const float t = fmaf(w, rf[row * BS + j] * rscale, acc[j]);
+                    const float t = fmaf(w, rf[(size_t)row * BS + j] * rscale, acc[j]);
                     acc[j] = use ? t : acc[j];
                 }
             }
@@ -1496,31 +1537,26 @@ __device__ __forceinline__ void prolong_row(int64_t row, const float* __restrict
                                             int f0, int f1, int f2, const int32_t* __restrict__ node_of_row,
                                             const uint8_t* __restrict__ ffix, float* __restrict__ xf,
                                             float* __restrict__ e, bool skip) {
-    constexpr int BS = ND;
-    const int64_t node = node_of_row ? (int64_t)node_of_row[row] : row;
-    int64_t cf[3];
-    coords_of<ND>(node, gf, cf);
+    constexpr int BS = ND, NZ = ND == 3 ? 2 : 1;
+    const Grid32 f32(gf), c32(gc);
+    const uint32_t node = node_of_row ? (uint32_t)node_of_row[row] : (uint32_t)row;
+    uint32_t cf[3];
+    coords32<ND>(node, f32, cf);
     const int f[3] = {f0, f1, f2};
-    int64_t p[3][2];
-    float w[3][2];
-    int np[3];
-    const int64_t ef[3] = {gf.n0 - 1, gf.n1 - 1, gf.n2 - 1};
+    uint32_t p[3][2];
+    float w[3];
+    bool two[3];  // a second parent
+    const uint32_t ef[3] = {f32.n0 - 1, f32.n1 - 1, f32.n2 - 1};
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        if (f[d] == 2 && (ef[d] & 1) && cf[d] == ef[d]) {  // odd e: the last node has one parent
-            p[d][0] = p[d][1] = (ef[d] + 1) / 2;
-            w[d][0] = w[d][1] = 1.0f;
-            np[d] = 1;
-        } else if (f[d] == 2 && (cf[d] & 1)) {
-            p[d][0] = (cf[d] - 1) / 2;
-            p[d][1] = p[d][0] + 1;
-            w[d][0] = w[d][1] = 0.5f;
-            np[d] = 2;
-        } else {
-            p[d][0] = p[d][1] = f[d] == 2 ? cf[d] / 2 : cf[d];
-            w[d][0] = w[d][1] = 1.0f;
-            np[d] = 1;
-        }
+        const bool half = f[d] == 2;
+        const bool last = half && (ef[d] & 1) && cf[d] == ef[d];  // odd e: the last node has one parent
+        two[d] = half && !last && (cf[d] & 1);
+        p[d][0] = last ? (ef[d] + 1) / 2 : half ? cf[d] / 2 : cf[d];
+        p[d][1] = two[d] ? p[d][0] + 1 : p[d][0];
+        w[d] = two[d] ? 0.5f : 1.0f;
     }
+    const float ww = w[0] * w[1] * w[2];
     float acc[BS];
 #pragma unroll
     for (int j = 0; j < BS; ++j) acc[j] = 0.0f;
@@ -1528,17 +1564,16 @@ __device__ __forceinline__ void prolong_row(int64_t row, const float* __restrict
     // exist loads the first one again and its term is dropped by a select
     // (the sums are those of the real parents, whatever the loaded value)
 #pragma unroll
-    for (int kz = 0; kz < 2; ++kz)
+    for (int kz = 0; kz < NZ; ++kz)
 #pragma unroll
         for (int ky = 0; ky < 2; ++ky)
 #pragma unroll
             for (int kx = 0; kx < 2; ++kx) {
-                const int64_t I = node_at(gc, p[0][kx], p[1][ky], p[2][kz]);
-                const bool in = kx < np[0] && ky < np[1] && kz < np[2];
-                const float ww = w[0][kx] * w[1][ky] * w[2][kz];
+                const uint32_t I = c32.at(p[0][kx], p[1][ky], p[2][kz]);
+                const bool in = (kx == 0 || two[0]) && (ky == 0 || two[1]) && (kz == 0 || two[2]);
 #pragma unroll
                 for (int j = 0; j < BS; ++j) {
-                    const float t = fmaf(ww, xc[I * BS + j], acc[j]);
+                    const float t = fmaf(ww, xc[(size_t)I * BS + j], acc[j]);
                     acc[j] = in ? t : acc[j];
                 }
             }
@@ -1564,16 +1599,21 @@ __global__ __launch_bounds__(kThreads) void prolong_kernel(const float* __restri
     prolong_row<ND>(row, xc, gc, gf, f0, f1, f2, node_of_row, ffix, xf, e, stop);
 }
 
-// coarsest level: x = A^-1 b with the dense FP64 inverse (one block)
-__global__ __launch_bounds__(kThreads) void dense_apply_kernel(const double* __restrict__ inv, int64_t nc,
+// coarsest level: x = A^-1 b with the dense FP64 inverse, a wavefront per
+// row (the row read coalesced, four strides in flight, a fixed butterfly).
+// 192 dofs (7 x 7 x 7 -> 4 x 4 x 4 nodes): one thread per row in one block
+// took 20 us, each lane walking its own row.
+__global__ __launch_bounds__(kThreads) void dense_apply_kernel(const double* __restrict__ inv, int nc,
                                                                const float* __restrict__ b, float* __restrict__ x,
                                                                const int* done) {
     const bool stop = *done != 0;  // checked before the stores
-    for (int64_t i = threadIdx.x; i < nc; i += kThreads) {
-        double s = 0.0;
-        for (int64_t j = 0; j < nc; ++j) s = fma(inv[i * nc + j], (double)b[j], s);
-        if (!stop) x[i] = (float)s;
-    }
+    const int row = (int)blockIdx.x * (kThreads / 64) + (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    if (row >= nc) return;
+    double s = 0.0;
+#pragma unroll 4
+    for (int j = lane; j < nc; j += 64) s = fma(inv[(int64_t)row * nc + j], (double)b[j], s);
+    s = wave_sum(s);
+    if (lane == 0 && !stop) x[row] = (float)s;
 }
 
 // ------------------------------------------- power iteration (setup) --
@@ -1641,22 +1681,39 @@ __device__ __forceinline__ double pow_epilogue(int64_t row, int64_t nrows, const
 }
 
 // w = B^-1 A (v / |v|), partial |w|^2
-template <int BS, typename TV>
+template <int BS, bool SHARED, typename TV>
 __global__ __launch_bounds__(kThreads) void pow_sell_kernel(SellOp<TV> op, const float* __restrict__ v,
                                                             const float* __restrict__ binv, float* __restrict__ w,
                                                             PowState* ps, double* __restrict__ partials) {
     __shared__ double sh[8];
     const float scale = (float)ps->inv;
-    const int64_t s0 = logical_block() * op.per_block;
-    const int64_t s1 = min(op.nslices, s0 + op.per_block);
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    auto gx = [=](int64_t c) { return v[c]; };
     double s = 0.0;
-    for (int64_t sl = s0 + wv; sl < s1; sl += kThreads / 64) {
-        float out[BS];
-        sell_row<BS, TV, float, false>(op.sl_ptr, op.sl_w, op.scol, Vals<TV>{op.val}, sl, lane, gx, out);
+    if constexpr (SHARED) {
+        __shared__ float buf[kThreads / 64][BS][64];
+        const int64_t sl = logical_block();
+        const bool live = sl < op.nslices;
+        SharedSlice<BS, TV> cols(op.scol, Vals<TV>{op.val});
+        if (live) cols.load(op.sl_ptr, op.sl_w, sl);
+        auto gx = [=](int64_t c, float(&xv)[BS]) {
+#pragma unroll
+            for (int i = 0; i < BS; ++i) xv[i] = v[c * BS + i];
+        };
+        float out[BS] = {};
+        cols.apply(gx, out);
+        sell_combine<BS, kThreads / 64>(out, buf);
         const int64_t row = sl * 64 + lane;
-        if (row < op.nrows) s += pow_epilogue<BS>(row, op.nrows, out, scale, binv, w);
+        if (wv == 0 && live && row < op.nrows) s = pow_epilogue<BS>(row, op.nrows, out, scale, binv, w);
+    } else {
+        const int64_t s0 = logical_block() * op.per_block;
+        const int64_t s1 = min(op.nslices, s0 + op.per_block);
+        auto gx = [=](int64_t c) { return v[c]; };
+        for (int64_t sl = s0 + wv; sl < s1; sl += kThreads / 64) {
+            float out[BS];
+            sell_row<BS, TV, float, false>(op.sl_ptr, op.sl_w, op.scol, Vals<TV>{op.val}, sl, lane, gx, out);
+            const int64_t row = sl * 64 + lane;
+            if (row < op.nrows) s += pow_epilogue<BS>(row, op.nrows, out, scale, binv, w);
+        }
     }
     const double b = block_sum_256(s, sh);
     if (threadIdx.x == 0) st_coherent(partials + blockIdx.x, b);
@@ -2124,7 +2181,7 @@ __global__ __launch_bounds__(kThreads) void mg_p_kernel(double* __restrict__ p, 
 }
 
 // q = A p (operator values TV, FP64 vectors), p.q -> alpha
-template <int BS, typename TV, bool NT>
+template <int BS, typename TV, bool NT, bool SHARED>
 __global__ __launch_bounds__(kThreads) void mg_spmv_kernel(const int64_t* __restrict__ sl_ptr,
                                                            const int32_t* __restrict__ sl_w,
                                                            const int32_t* __restrict__ scol, Vals<TV> sval,
@@ -2133,22 +2190,38 @@ __global__ __launch_bounds__(kThreads) void mg_spmv_kernel(const int64_t* __rest
                                                            MgState* st, double* __restrict__ partials) {
     __shared__ double sh[8];
     if (st->done) return;
-    const int64_t s0 = logical_block() * per_block;
-    const int64_t s1 = min(nslices, s0 + per_block);
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double dot = 0.0;
-    auto gx = [=](int64_t c) { return p[c]; };
-    for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
-        double out[BS];
-        sell_row<BS, TV, double, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, out);
-        const int64_t row = sl * 64 + lane;
-        if (row < nrows) {
+    auto finish = [&](int64_t row, const double (&out)[BS]) {
 #pragma unroll
-            for (int j = 0; j < BS; ++j) {
-                const int64_t d = row * BS + j;
-                q[d] = out[j];
-                dot = fma(p[d], out[j], dot);
-            }
+        for (int j = 0; j < BS; ++j) {
+            const int64_t d = row * BS + j;
+            q[d] = out[j];
+            dot = fma(p[d], out[j], dot);
+        }
+    };
+    if constexpr (SHARED) {
+        __shared__ double buf[kThreads / 64][BS][64];
+        const int64_t sl = logical_block();
+        const bool live = sl < nslices;
+        SharedSlice<BS, TV, NT> cols(scol, sval);
+        if (live) cols.load(sl_ptr, sl_w, sl);
+        auto gx = [=](int64_t c, double(&xv)[BS]) {
+#pragma unroll
+            for (int i = 0; i < BS; ++i) xv[i] = p[c * BS + i];
+        };
+        double out[BS] = {};
+        cols.apply(gx, out);
+        sell_combine<BS, kThreads / 64>(out, buf);
+        if (w == 0 && live && sl * 64 + lane < nrows) finish(sl * 64 + lane, out);
+    } else {
+        const int64_t s0 = logical_block() * per_block;
+        const int64_t s1 = min(nslices, s0 + per_block);
+        auto gx = [=](int64_t c) { return p[c]; };
+        for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
+            double out[BS];
+            sell_row<BS, TV, double, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, out);
+            if (sl * 64 + lane < nrows) finish(sl * 64 + lane, out);
         }
     }
     const double b = block_sum_256(dot, sh);
@@ -2241,8 +2314,12 @@ Launch plan_vec(int64_t items, unsigned cap) {
     return {(unsigned)grid, per};
 }
 
-// one slice per wavefront, four per block
-Launch plan_sell(int64_t nslices) {
+// bytes of a sliced operator of vb bytes a value
+double sell_bytes(const sfem_system* S, double vb) { return (double)S->sell_blocks * (S->bs * S->bs * vb + 4.0); }
+
+// one slice per wavefront, four per block; or a block per slice
+Launch plan_sell(int64_t nslices, bool shared) {
+    if (shared) return {(unsigned)std::max<int64_t>(8, (nslices + 7) / 8 * 8), 1};
     const int64_t per = kThreads / 64;
     int64_t grid = (nslices + per - 1) / per;
     grid = std::max<int64_t>(8, (grid + 7) / 8 * 8);
@@ -2791,7 +2868,8 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
     if (!H.mf) {
         MgLevel& v = H.L[0];
         const int64_t n = v.nrows * BS;
-        const Launch ls = plan_sell(S->nslices);
+        const bool shared = slice_split(ctx, S->nslices, BS, sell_bytes(S, H.fp16 ? 2.0 : 4.0)) > 1;
+        const Launch ls = plan_sell(S->nslices, shared);
         parts[0].reset(ctx, std::max({ls.grid, init_grid(n), 1024u}));
         double* partials = parts[0].get();
         hipLaunchKernelGGL(pow_init_kernel, dim3(init_grid(n)), dim3(kThreads), 0, s, n, v.fixed.get(), v.da.get(),
@@ -2800,16 +2878,19 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         float* vin = v.da.get();
         float* vout = v.db.get();
         for (int k = 0; k < o.power_iters; ++k) {
+            auto go = [&](auto kern, auto op, const float* binv) {
+                hipLaunchKernelGGL(kern, dim3(ls.grid), dim3(kThreads), 0, s, op, vin, binv, vout, ps.get(), partials);
+            };
             if (H.fp16) {
                 const SellOp<_Float16> op{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), H.h0.get(), S->nslices,
                                           S->nfb, ls.per_block};
-                hipLaunchKernelGGL((pow_sell_kernel<BS, _Float16>), dim3(ls.grid), dim3(kThreads), 0, s, op, vin,
-                                   (const float*)H.binv0.get(), vout, ps.get(), partials);
+                shared ? go(pow_sell_kernel<BS, true, _Float16>, op, H.binv0.get())
+                       : go(pow_sell_kernel<BS, false, _Float16>, op, H.binv0.get());
             } else {
                 const SellOp<float> op{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), S->sval32.get(), S->nslices,
                                        S->nfb, ls.per_block};
-                hipLaunchKernelGGL((pow_sell_kernel<BS, float>), dim3(ls.grid), dim3(kThreads), 0, s, op, vin,
-                                   S->binv32.get(), vout, ps.get(), partials);
+                shared ? go(pow_sell_kernel<BS, true, float>, op, S->binv32.get())
+                       : go(pow_sell_kernel<BS, false, float>, op, S->binv32.get());
             }
             SFEM_LAUNCH_CHECK();
             std::swap(vin, vout);
@@ -2835,7 +2916,8 @@ struct MgRun {
     sfem_system* S;
     MgHierarchy& H;
     hipStream_t s;
-    Launch ls;
+    Launch ls;    // the finest level's smoother (sliced)
+    bool shared;  // a block per slice
     const int* done;
     bool nt;
     std::vector<hipEvent_t>* ev = nullptr;  // non-null: time the finest-level smoothing steps
@@ -2871,8 +2953,9 @@ struct MgRun {
                 hipLaunchKernelGGL(k, dim3(ls.grid), dim3(kThreads), 0, s, op, v, L.r.get(), L.x.get(), d_in, d_out,
                                    c1, c2, (const float*)H.binv0.get(), done);
             };
-            if (mode == 0) nt ? go(cheb_sell_kernel<BS, 0, true, _Float16>) : go(cheb_sell_kernel<BS, 0, false, _Float16>);
-            else nt ? go(cheb_sell_kernel<BS, 1, true, _Float16>) : go(cheb_sell_kernel<BS, 1, false, _Float16>);
+            if (shared) mode == 0 ? go(cheb_sell_kernel<BS, 0, false, true, _Float16>) : go(cheb_sell_kernel<BS, 1, false, true, _Float16>);
+            else if (mode == 0) nt ? go(cheb_sell_kernel<BS, 0, true, false, _Float16>) : go(cheb_sell_kernel<BS, 0, false, false, _Float16>);
+            else nt ? go(cheb_sell_kernel<BS, 1, true, false, _Float16>) : go(cheb_sell_kernel<BS, 1, false, false, _Float16>);
         } else if (l == 0) {
             const SellOp<float> op{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), S->sval32.get(), S->nslices, S->nfb,
                                    ls.per_block};
@@ -2880,8 +2963,9 @@ struct MgRun {
                 hipLaunchKernelGGL(k, dim3(ls.grid), dim3(kThreads), 0, s, op, v, L.r.get(), L.x.get(), d_in, d_out,
                                    c1, c2, (const float*)S->binv32.get(), done);
             };
-            if (mode == 0) nt ? go(cheb_sell_kernel<BS, 0, true, float>) : go(cheb_sell_kernel<BS, 0, false, float>);
-            else nt ? go(cheb_sell_kernel<BS, 1, true, float>) : go(cheb_sell_kernel<BS, 1, false, float>);
+            if (shared) mode == 0 ? go(cheb_sell_kernel<BS, 0, false, true, float>) : go(cheb_sell_kernel<BS, 1, false, true, float>);
+            else if (mode == 0) nt ? go(cheb_sell_kernel<BS, 0, true, false, float>) : go(cheb_sell_kernel<BS, 0, false, false, float>);
+            else nt ? go(cheb_sell_kernel<BS, 1, true, false, float>) : go(cheb_sell_kernel<BS, 1, false, false, float>);
         } else {
             const bool grp = L.node_major;
             auto go = [&](auto k, auto op) {
@@ -2907,8 +2991,8 @@ struct MgRun {
         MgLevel& L = H.L[(size_t)l];
         const int nl = (int)H.L.size();
         if (l == nl - 1) {
-            hipLaunchKernelGGL(dense_apply_kernel, dim3(1), dim3(kThreads), 0, s, H.cinv.get(), H.nc, L.b.get(),
-                               L.x.get(), done);
+            hipLaunchKernelGGL(dense_apply_kernel, dim3((unsigned)((H.nc + 3) / 4)), dim3(kThreads), 0, s,
+                               (const double*)H.cinv.get(), (int)H.nc, (const float*)L.b.get(), L.x.get(), done);
             SFEM_LAUNCH_CHECK();
             return;
         }
@@ -2968,7 +3052,12 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
     const int64_t n = S->nfb * BS;
     double* x = padded ? S->px.get() : S->x.get();
     const double* rhs = padded ? S->prhs.get() : S->rhs.get();
-    const Launch ls = plan_sell(S->nslices);
+    constexpr double kValBytes = std::is_same<TV, SplitVal>::value ? 6.0 : (double)sizeof(TV);
+    // the outer operator's launch (and the FP64 residual's: a wavefront per slice)
+    const double outer_bytes = sell_bytes(S, kValBytes), smooth_op_bytes = sell_bytes(S, H.fp16 ? 2.0 : 4.0);
+    const bool shared = slice_split(ctx, S->nslices, BS, outer_bytes) > 1;
+    const bool shared0 = slice_split(ctx, S->nslices, BS, smooth_op_bytes) > 1;
+    const Launch ls = plan_sell(S->nslices, false), lo = plan_sell(S->nslices, shared);
     const Launch lv = plan_vec(n, (unsigned)std::max(8, ctx->n_cu * 4));
     // p: and a zero row, read for fixed nodes by the matrix-free operator
     DevBuf<double> r(ctx, (size_t)n), p(ctx, (size_t)n + BS), q(ctx, (size_t)n);
@@ -2983,7 +3072,7 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
         const MfTiles T = mf_tiles(H);
         tiles = (unsigned)((T.tx * T.ty * T.tz + 7) / 8 * 8);
     }
-    DevBuf<double> partials(ctx, 2 * (size_t)std::max({ls.grid, lv.grid, mf_grid, 2048u, xcd_rows_grid(S->nfb),
+    DevBuf<double> partials(ctx, 2 * (size_t)std::max({ls.grid, lo.grid, lv.grid, mf_grid, 2048u, xcd_rows_grid(S->nfb),
                                                         tiles}));
     DevBuf<MgState> dst(ctx, 1);
     if (o->x0_zero) memset_d(ctx, S->x.get(), 0, sizeof(double) * S->nf);
@@ -2999,7 +3088,8 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
     }
     h2d(ctx, dst.get(), &init, sizeof(init));
     MgState* st = dst.get();
-    MgRun<ND, TV> run{ctx, S, H, s, ls, &st->done, ctx->tune_nt};
+    MgRun<ND, TV> run{ctx, S, H, s, plan_sell(S->nslices, shared0), shared0, &st->done,
+                      stream_loads(ctx, smooth_op_bytes)};
     const float* z = H.L[0].x.get();
     Vals<TV> vals = outer_vals<TV>(S);
 
@@ -3059,14 +3149,15 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
                                (const MgState*)st);
             SFEM_LAUNCH_CHECK();
             auto go = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3(ls.grid), dim3(kThreads), 0, s, S->sl_ptr.get(), S->sl_w.get(),
-                                   S->scol.get(), vals, S->nslices, S->nfb, ls.per_block, (const double*)p.get(),
+                hipLaunchKernelGGL(kern, dim3(lo.grid), dim3(kThreads), 0, s, S->sl_ptr.get(), S->sl_w.get(),
+                                   S->scol.get(), vals, S->nslices, S->nfb, lo.per_block, (const double*)p.get(),
                                    q.get(), st, partials.get());
             };
             if (mf_outer) hipLaunchKernelGGL(mg_spmv_mf_kernel<ND>, dim3(mf_grid), dim3(kThreads), 0, s, mf64,
                                              (const double*)p.get(), q.get(), st, partials.get());
-            else if (ctx->tune_nt) go(mg_spmv_kernel<BS, TV, true>);
-            else go(mg_spmv_kernel<BS, TV, false>);
+            else if (shared) go(mg_spmv_kernel<BS, TV, false, true>);
+            else if (stream_loads(ctx, outer_bytes)) go(mg_spmv_kernel<BS, TV, true, false>);
+            else go(mg_spmv_kernel<BS, TV, false, false>);
             SFEM_LAUNCH_CHECK();
             hipLaunchKernelGGL(mg_update_kernel, dim3(lv.grid), dim3(kThreads), 0, s, x, r.get(),
                                (const double*)p.get(), (const double*)q.get(), n, lv.per_block, st, partials.get());

@@ -316,23 +316,10 @@ __global__ __launch_bounds__(kThreads) void sell_pass_kernel(
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int part = wv % SPLIT;
     if constexpr (FLY) {
-        constexpr int PRE = 4, PV = 2;  // block columns with early column ids, and early values
-        using Raw = typename Vals<TV>::Raw;
         const int64_t sl = s0;
         const bool live = sl < s1;
-        const int64_t base = live ? glb(sl_ptr)[sl] : 0;
-        const int w = live ? glb(sl_w)[sl] : 0;
-        int32_t pc[PRE] = {};
-        Raw pv[PV][B2] = {};
-        if (w > 0) {  // a column past the row's end repeats its last one and is dropped below
-#pragma unroll
-            for (int u = 0; u < PRE; ++u) pc[u] = ld_stream<NT>(scol + base + (int64_t)min(part + u * SPLIT, w - 1) * 64 + lane);
-#pragma unroll
-            for (int u = 0; u < PV; ++u)
-#pragma unroll
-                for (int m = 0; m < B2; ++m)
-                    pv[u][m] = sval.template raw<NT>((base + (int64_t)min(part + u * SPLIT, w - 1) * 64) * B2 + lane + m * 64);
-        }
+        SharedSlice<BS, TV, NT> row_cols(scol, sval);
+        if (live) row_cols.load(sl_ptr, sl_w, sl);
         const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
         if (go.done) return;
         if (!go.resid) {
@@ -344,36 +331,7 @@ __global__ __launch_bounds__(kThreads) void sell_pass_kernel(
                 for (int i = 0; i < BS; ++i) x[i] = fmaT<T>(beta, w.p[i], zc * w.z[i]);
             };
             T acc[BS] = {};
-            if (w > 0) {
-#pragma unroll
-                for (int u = 0; u < PRE; ++u) {
-                    const int k = part + u * SPLIT;
-                    Raw rv[B2];
-#pragma unroll
-                    for (int m = 0; m < B2; ++m)
-                        rv[m] = u < PV ? pv[u < PV ? u : 0][m]
-                                       : sval.template raw<NT>((base + (int64_t)min(k, w - 1) * 64) * B2 + lane + m * 64);
-                    T xv[BS];
-                    gx(pc[u], xv);
-#pragma unroll
-                    for (int i = 0; i < BS; ++i) xv[i] = k < w ? xv[i] : T(0);
-#pragma unroll
-                    for (int j = 0; j < BS; ++j)
-#pragma unroll
-                        for (int i = 0; i < BS; ++i) acc[j] = fmaT<T>((T)sval.decode(rv[j * BS + i]), xv[i], acc[j]);
-                }
-#pragma unroll 2
-                for (int k = part + PRE * SPLIT; k < w; k += SPLIT) {
-                    const int64_t slot = base + (int64_t)k * 64;
-                    T xv[BS];
-                    gx(ld_stream<NT>(scol + slot + lane), xv);
-#pragma unroll
-                    for (int j = 0; j < BS; ++j)
-#pragma unroll
-                        for (int i = 0; i < BS; ++i)
-                            acc[j] = fmaT<T>((T)sval.template get<NT>(slot * B2 + lane + (j * BS + i) * 64), xv[i], acc[j]);
-                }
-            }
+            row_cols.apply(gx, acc);
             sell_combine<BS, SPLIT>(acc, reinterpret_cast<T(*)[BS][64]>(&buf[0][0][0]));
             double dot = 0.0;
             const int64_t row = sl * 64 + lane;
@@ -775,33 +733,6 @@ Launch plan_sell(int64_t nslices, unsigned cap, int wave_slices) {
     int64_t grid = (nslices + per - 1) / per;
     grid = std::max<int64_t>(8, (grid + 7) / 8 * 8);
     return {(unsigned)grid, per};
-}
-
-// Wavefronts per slice of an operator pass, and whether p is formed in its
-// gathers (4 of them) or by direction_kernel (1).  A wavefront per slice
-// leaves a small system with fewer wavefronts than the device holds, each
-// with up to 27 block columns of loads one after the other.  Measured on
-// MI355X, us per iteration with 1 / 4 wavefronts (1: plus direction_kernel):
-// 3D FP64 Jacobi 7 slices 19.8 / 12.6, 294 slices 24.3 / 15.8, 948 slices
-// 32.1 / 27.8, 2,196 slices 71.9 / 63.5, 4,229 slices (578 MB) 126.7 / 138.8,
-// 16,967 slices 464 / 543; mixed block Jacobi 2,196 slices 38.4 / 33.5,
-// 4,229 slices (304 MB) 71.5 / 67.8, 7,241 slices (521 MB) 111 / 128.  So the
-// line is where the operator leaves the 256 MB memory-side cache (and
-// non-temporal loads begin to pay, see stream_loads).  2D FP64 (9 block
-// columns): 30 slices 14.0 / 10.4, 711 slices 15.3 / 12.9, 1,965 slices
-// 22.9 / 23.6, 3,297 slices 30.1 / 31.6.  8 wavefronts gain nothing over 4.
-constexpr double kSharedBytes = 400e6;    // 3D: operator bytes
-constexpr int64_t kSharedSlices2 = 1536;  // 2D: slices
-int slice_split(const sfem_ctx* ctx, int64_t nslices, int bs, double operator_bytes) {
-    if (ctx->tune_split > 0) return ctx->tune_split >= 4 ? 4 : 1;
-    return (bs == 3 ? operator_bytes <= kSharedBytes : nslices <= kSharedSlices2) ? 4 : 1;
-}
-
-// Non-temporal operator loads pay once the operator no longer stays in the
-// memory-side cache between iterations (FP64, a wavefront per slice: 300 MB
-// 72.9 us without and 71.9 with, 990 MB 228 and 207).
-bool stream_loads(const sfem_ctx* ctx, double operator_bytes) {
-    return ctx->tune_nt && operator_bytes > kSharedBytes;
 }
 
 struct Ops {

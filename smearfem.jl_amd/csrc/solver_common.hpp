@@ -281,6 +281,75 @@ __device__ __forceinline__ void sell_row(const int64_t* __restrict__ sl_ptr, con
     }
 }
 
+// A slice shared by a block of 4 wavefronts: wavefront `part` takes the block
+// columns part, part + 4, ... of the slice's 64 block rows (sell_combine adds
+// the four sums).  load() issues what does not depend on the gathered vector:
+// the first PRE column ids and PV columns of values; a column past the row's
+// end repeats its last one, and apply() drops it.
+template <int BS, typename TV, bool NT = false>
+struct SharedSlice {
+    static constexpr int B2 = BS * BS, SPLIT = kThreads / 64, PRE = 4, PV = 2;
+    using Raw = typename Vals<TV>::Raw;
+    const int32_t* scol;
+    Vals<TV> vals;
+    int64_t base = 0;
+    int w = 0, part, lane;
+    int32_t pc[PRE] = {};
+    Raw pv[PV][B2] = {};
+
+    __device__ __forceinline__ SharedSlice(const int32_t* scol_, Vals<TV> vals_) : scol(scol_), vals(vals_) {
+        part = threadIdx.x >> 6;
+        lane = threadIdx.x & 63;
+    }
+    __device__ __forceinline__ int64_t column(int u) const {
+        return base + (int64_t)min(part + u * SPLIT, w - 1) * 64;
+    }
+    __device__ __forceinline__ void load(const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w,
+                                         int64_t sl) {
+        base = glb(sl_ptr)[sl];
+        w = glb(sl_w)[sl];
+        if (w <= 0) return;
+#pragma unroll
+        for (int u = 0; u < PRE; ++u) pc[u] = ld_stream<NT>(scol + column(u) + lane);
+#pragma unroll
+        for (int u = 0; u < PV; ++u)
+#pragma unroll
+            for (int m = 0; m < B2; ++m) pv[u][m] = vals.template raw<NT>(column(u) * B2 + lane + m * 64);
+    }
+    // acc += this wavefront's columns; gx(c, x) gathers block row c
+    template <typename ACC, typename Gather>
+    __device__ __forceinline__ void apply(Gather gx, ACC (&acc)[BS]) const {
+        if (w <= 0) return;
+#pragma unroll
+        for (int u = 0; u < PRE; ++u) {
+            const bool in = part + u * SPLIT < w;
+            Raw rv[B2];
+#pragma unroll
+            for (int m = 0; m < B2; ++m)
+                rv[m] = u < PV ? pv[u < PV ? u : 0][m] : vals.template raw<NT>(column(u) * B2 + lane + m * 64);
+            ACC xv[BS];
+            gx((int64_t)pc[u], xv);
+#pragma unroll
+            for (int i = 0; i < BS; ++i) xv[i] = in ? xv[i] : ACC(0);
+#pragma unroll
+            for (int j = 0; j < BS; ++j)
+#pragma unroll
+                for (int i = 0; i < BS; ++i) acc[j] = fmaT<ACC>((ACC)vals.decode(rv[j * BS + i]), xv[i], acc[j]);
+        }
+#pragma unroll 2
+        for (int k = part + PRE * SPLIT; k < w; k += SPLIT) {
+            const int64_t slot = base + (int64_t)k * 64;
+            ACC xv[BS];
+            gx((int64_t)ld_stream<NT>(scol + slot + lane), xv);
+#pragma unroll
+            for (int j = 0; j < BS; ++j)
+#pragma unroll
+                for (int i = 0; i < BS; ++i)
+                    acc[j] = fmaT<ACC>((ACC)vals.template get<NT>(slot * B2 + lane + (j * BS + i) * 64), xv[i], acc[j]);
+        }
+    }
+};
+
 // The block columns part, part + SPLIT, ... of this lane's block row in FP64
 // (SPLIT wavefronts share a slice; their sums are added by sell_combine), and
 // aout[j] = sum |M_ji x_i|.  gx(c, x) gathers block row c of the vector.
@@ -439,6 +508,34 @@ __device__ __forceinline__ void sell_row_abs(const int64_t* __restrict__ sl_ptr,
         for (int i = 0; i < BS; ++i) x0[i] = gx(c0 * BS + i);
         step(m0, x0);
     }
+}
+
+// Wavefronts per slice of a sliced operator: 1, or 4 (a block per slice; in
+// the Jacobi CG p is then formed in the operator's gathers, else by
+// direction_kernel).  A wavefront per slice
+// leaves a small system with fewer wavefronts than the device holds, each
+// with up to 27 block columns of loads one after the other.  Measured on
+// MI355X, us per iteration with 1 / 4 wavefronts (1: plus direction_kernel):
+// 3D FP64 Jacobi 7 slices 19.8 / 12.6, 294 slices 24.3 / 15.8, 948 slices
+// 32.1 / 27.8, 2,196 slices 71.9 / 63.5, 4,229 slices (578 MB) 126.7 / 138.8,
+// 16,967 slices 464 / 543; mixed block Jacobi 2,196 slices 38.4 / 33.5,
+// 4,229 slices (304 MB) 71.5 / 67.8, 7,241 slices (521 MB) 111 / 128.  So the
+// line is where the operator leaves the 256 MB memory-side cache (and
+// non-temporal loads begin to pay, see stream_loads).  2D FP64 (9 block
+// columns): 30 slices 14.0 / 10.4, 711 slices 15.3 / 12.9, 1,965 slices
+// 22.9 / 23.6, 3,297 slices 30.1 / 31.6.  8 wavefronts gain nothing over 4.
+constexpr double kSharedBytes = 400e6;    // 3D: operator bytes
+constexpr int64_t kSharedSlices2 = 1536;  // 2D: slices
+inline int slice_split(const sfem_ctx* ctx, int64_t nslices, int bs, double operator_bytes) {
+    if (ctx->tune_split > 0) return ctx->tune_split >= 4 ? 4 : 1;
+    return (bs == 3 ? operator_bytes <= kSharedBytes : nslices <= kSharedSlices2) ? 4 : 1;
+}
+
+// Non-temporal operator loads pay once the operator no longer stays in the
+// memory-side cache between iterations (FP64, a wavefront per slice: 300 MB
+// 72.9 us without and 71.9 with, 990 MB 228 and 207).
+inline bool stream_loads(const sfem_ctx* ctx, double operator_bytes) {
+    return ctx->tune_nt && operator_bytes > kSharedBytes;
 }
 
 }  // namespace

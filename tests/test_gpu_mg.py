@@ -518,3 +518,37 @@ def test_mg_coarse_kernel_forms_same_bits(ctx, dims, monkeypatch):
         assert its[name] == its["threads"] and np.array_equal(sols[name], sols["threads"]), name
     if m.n_dof <= 6000:
         assert relerr(sols["default"], oracle_direct(oracle_K(m, young), fixed, f)) <= ERR
+
+
+@pytest.mark.parametrize("split", ["1", "4"])
+@pytest.mark.parametrize("dims", [(2, 1, 1), (4, 3, 3), (6, 5, 3), (13, 8, 5), (9, 7), (20, 3)])
+def test_sliced_finest_level_forms(dims, split, monkeypatch):
+    # the sliced smoother, power iteration and outer operator with a wavefront
+    # per slice and with a block per slice, on distorted grids with odd element
+    # counts and 12 to 756 nodes (1 to 12 slices, the last one ragged)
+    print(f"[case] sliced finest level {dims} split={split}", flush=True)
+    monkeypatch.setenv("SFEM_SELL_SPLIT", split)
+    ctx = smearfem.Context(0)
+    m = structured_mesh(dims)
+    rng = np.random.default_rng(5)
+    coords = m.NodeList + 0.1 / np.array(dims)[:, None] * rng.uniform(-1, 1, m.NodeList.shape)
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=6)
+    fixed = clamp_x0(m)
+    f = random_face_load(m, m.ndim - 1, 1, fixed, seed=7)
+    Kr = O.assemble_system(0, coords, m.IEN, m.ndim, "Q1", m.ndim, m.ID, young, 0.3, n_elem=m.n_elem)
+    Kff, rhs = O.eliminate(Kr, fixed, f)
+    q_ref = O.recombine(fixed, None, O.dense_solve(Kff, rhs))
+    K = smearfem.assemble_system(0, coords, m.IEN, m.ndim, "Q1", m.ndim, m.ID, young, 0.3, ctx=ctx, device=True,
+                                 n_elem=m.n_elem)
+    for precision in ("fp64", "split", "fp32_matrix"):
+        for fp16 in (True, False):
+            bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+            S = System(K, bc)
+            bc.close()
+            assert S.set_grid(m.dims, fine_fp16=fp16)["matrix_free"] == 0
+            st = S.solve(precision, rtol=1e-12, preconditioner="multigrid")
+            q = S.solution()
+            S.close()
+            assert st["converged"] and np.linalg.norm(q - q_ref) <= 1e-8 * np.linalg.norm(q_ref), (precision, fp16)
+    K.close()
+    ctx.close()
