@@ -18,7 +18,10 @@
 //              FP64 on 3^d-point node-block stencils (the grid gives every
 //              column, so none is stored), symmetrised, and kept in FP32 for
 //              smoothing.
-//   coarsest   dense inverse in FP64, computed on the host.
+//   direct     the first level of at most kDirectDofs dofs is solved with its
+//              dense FP64 inverse, formed on the device (blocked Gauss-Jordan);
+//              the levels below it are described (mg_info, mg_stencil) but
+//              the V-cycle does not visit them.
 //
 // Smoother: Chebyshev polynomial in B^-1 A (B = the diagonal node blocks) on
 // [lo, hi] x lambda_max, lambda_max from power iteration on every level;
@@ -42,7 +45,17 @@
 namespace sfem {
 
 constexpr int kMgMaxDegree = 8;
-constexpr int64_t kMgMaxCoarseNodes = 400;  // dense coarsest level (host inverse, O(dofs^3))
+constexpr int64_t kMgMaxCoarseNodes = 400;  // coarsest level
+// Dofs of the level solved directly, at most.  Each level below it would cost
+// a V-cycle 6 launches of 3 to 5 us, one application of the inverse costs 4 to
+// 6 us whatever its size, and the inverse takes a launch of 16 to 22 us per 32
+// dofs, partly beside the finest level's power iteration.  Measured, set-up +
+// solve in ms with the coarsest level (<= 64 nodes) / this line / 1,296 dofs:
+// 11x5x5 2.76 / 1.97 / 1.95, 16x8x8 (675 dofs) 2.53 / 2.32 / 2.33, 24x24x24
+// (1,029) 2.90 / 2.81 / 3.12, 64x16x16 (1,275) 3.91 / 3.45 / 3.92, 301x97
+// (1,092) 4.99 / 3.96 / 3.89, 256x64x64 13.6 / 13.2 / 13.7.
+constexpr int64_t kDirectDofs = 800;
+constexpr int kTile = 32;                   // Gauss-Jordan block
 
 struct MgLevel {
     int64_t n[3] = {1, 1, 1};  // nodes per grid direction
@@ -68,8 +81,10 @@ struct MgHierarchy {
     std::vector<MgLevel> L;
     DevBuf<int32_t> row_of_node;  // fine grid node -> block row (-1: every dof fixed)
     DevBuf<int32_t> node_of_row;  // block row -> fine grid node
-    DevBuf<double> cinv;          // coarsest level: dense inverse, nc x nc row-major
-    int64_t nc = 0;
+    int direct = 0;               // the level solved with its dense inverse
+    DevBuf<double> dinv;          // that inverse, row-major, ndp x ndp (padded to kTile)
+    int64_t nd_dofs = 0, ndp = 0;
+    int64_t nc = 0;               // dofs of the coarsest level
     double setup_ms = 0;
     // FP16 finest-level smoothing operator: s * K_ff (s = 2^-e, max |s a| in
     // (1/2, 1]) in the system's sliced layout, and the inverses of its
@@ -1023,6 +1038,13 @@ bool galerkin_lines_forced() {
     return e && e[0] == '1';
 }
 
+// SFEM_MG_DIRECT_DOFS overrides kDirectDofs (read when the hierarchy is
+// built; the coarsest level is solved directly whatever it says)
+int64_t direct_dofs() {
+    const char* e = std::getenv("SFEM_MG_DIRECT_DOFS");
+    return e && *e ? std::atoll(e) : kDirectDofs;
+}
+
 int64_t stencil_group_below() {
     const char* e = std::getenv("SFEM_MG_GROUP_BELOW");
     return e && *e ? std::atoll(e) : kStencilGroupBelow;
@@ -1599,21 +1621,144 @@ __global__ __launch_bounds__(kThreads) void prolong_kernel(const float* __restri
     prolong_row<ND>(row, xc, gc, gf, f0, f1, f2, node_of_row, ffix, xf, e, stop);
 }
 
-// coarsest level: x = A^-1 b with the dense FP64 inverse, a wavefront per
-// row (the row read coalesced, four strides in flight, a fixed butterfly).
-// 192 dofs (7 x 7 x 7 -> 4 x 4 x 4 nodes): one thread per row in one block
-// took 20 us, each lane walking its own row.
-__global__ __launch_bounds__(kThreads) void dense_apply_kernel(const double* __restrict__ inv, int nc,
+// direct level: x = A^-1 b with the dense FP64 inverse (row stride np), a
+// wavefront per row (the row read coalesced, the loads of eight strides in
+// flight, a fixed butterfly).  1,275 dofs: 13 MB, from the caches.
+__global__ __launch_bounds__(kThreads) void dense_apply_kernel(const double* __restrict__ inv, int nc, int np,
                                                                const float* __restrict__ b, float* __restrict__ x,
                                                                const int* done) {
     const bool stop = *done != 0;  // checked before the stores
     const int row = (int)blockIdx.x * (kThreads / 64) + (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     if (row >= nc) return;
     double s = 0.0;
-#pragma unroll 4
-    for (int j = lane; j < nc; j += 64) s = fma(inv[(int64_t)row * nc + j], (double)b[j], s);
+#pragma unroll 8
+    for (int j = lane; j < nc; j += 64) s = fma(inv[(int64_t)row * np + j], (double)b[j], s);
     s = wave_sum(s);
     if (lane == 0 && !stop) x[row] = (float)s;
+}
+
+// The direct level's operator as a dense matrix (zeroed by the caller): its
+// stencil, ones on the diagonal of fixed dofs and of the padding.
+template <int ND>
+__global__ void dense_fill_kernel(const double* __restrict__ st64, const uint8_t* __restrict__ fixed, Grid g, int np,
+                                  double* __restrict__ a) {
+    constexpr int BS = ND, B2 = BS * BS;
+    const int64_t nn = g.n0 * g.n1 * g.n2;
+    const int s = (int)blockIdx.y;
+    const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0 && I < np - nn * BS) a[(nn * BS + I) * (np + 1)] = 1.0;
+    if (I >= nn) return;
+    int64_t c[3];
+    coords_of<ND>(I, g, c);
+    int dx, dy, dz;
+    offset_of<ND>(s, dx, dy, dz);
+    if (!inside<ND>(g, c[0] + dx, c[1] + dy, c[2] + dz)) return;
+    const int64_t J = node_at(g, c[0] + dx, c[1] + dy, c[2] + dz);
+    for (int p = 0; p < BS; ++p)
+        for (int q = 0; q < BS; ++q) {
+            const bool unit = s == Sten<ND>::C && p == q && fixed[I * BS + p];
+            a[(I * BS + p) * np + J * BS + q] = unit ? 1.0 : st64[((int64_t)s * B2 + p * BS + q) * nn + I];
+        }
+}
+
+// One block step of the Gauss-Jordan inverse, A -> A' in another buffer, with
+// P = A_kk^-1: A'_kk = P, A'_kJ = P A_kJ, A'_Ik = -A_Ik P and A'_IJ = A_IJ -
+// A_Ik P A_kJ; after every k, A' is the inverse.  A workgroup per `per` tiles
+// of 32 x 32 in one tile row.  Every workgroup forms P for itself (32 pivots
+// without exchanges -- the operator is positive definite -- one barrier each,
+// about 4 us), so a step is one launch and the workgroups never wait for each
+// other; the products run on the FP64 matrix instructions (16x16x4: A[i][k]
+// in lane i + 16 k, B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 (i % 4),
+// element i / 4).
+// bad: set when a pivot is zero or not finite.
+__global__ __launch_bounds__(kThreads) void gauss_jordan_kernel(const double* __restrict__ in,
+                                                                double* __restrict__ out, int np, int k, int per,
+                                                                double* bad) {
+    typedef double double4_t __attribute__((ext_vector_type(4)));
+    constexpr int T = kTile, LD = T + 1, Q = T * T / kThreads;
+    __shared__ double P[T * LD], X[T * LD], Y[T * LD];
+    __shared__ double rowb[2][T], colb[2][T];
+    const int I = (int)blockIdx.y, J0 = (int)blockIdx.x * per, J1 = min(J0 + per, np / T), t = (int)threadIdx.x;
+    const int j = t % T, i0 = t / T;  // this thread's entries of a tile in LDS order: (i0 + 8 q, j)
+    // and of a product: wavefront w has the 16 x 16 quadrant (w / 2, w % 2)
+    const int w = t >> 6, lane = t & 63, qi = 16 * (w >> 1), qj = 16 * (w & 1), l16 = lane & 15, h = lane >> 4;
+    auto at = [&](int bi, int bj, int i) { return ((int64_t)bi * T + i) * np + (int64_t)bj * T + j; };
+    auto dat = [&](int bj, int r) { return ((int64_t)I * T + qi + h + 4 * r) * np + (int64_t)bj * T + qj + l16; };
+    double a[Q], x[Q], y[Q], c[4];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = i0 + 8 * q;
+        a[q] = in[at(k, k, i)];
+        x[q] = in[at(I, k, i)];
+        y[q] = in[at(k, J0, i)];
+        c[q] = in[dat(J0, q)];
+    }
+    bool ok = true;
+#pragma unroll 1
+    for (int p = 0; p < T; ++p) {
+        const int b = p & 1;  // two buffers: one barrier per pivot
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            if (j == p) colb[b][i0 + 8 * q] = a[q];
+            if (i0 + 8 * q == p) rowb[b][j] = a[q];
+        }
+        __syncthreads();
+        const double piv = rowb[b][p], rk = rowb[b][j];
+        ok = ok && fabs(piv) > 0.0 && isfinite(piv);
+        double rp = __builtin_amdgcn_rcp(piv);  // Newton's iteration from the hardware's estimate
+        rp = fma(fma(-piv, rp, 1.0), rp, rp);
+        rp = fma(fma(-piv, rp, 1.0), rp, rp);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = i0 + 8 * q;
+            const double ck = colb[b][i] * rp;
+            const double v = i == p ? rk * rp : fma(-ck, rk, a[q]);
+            a[q] = j == p ? (i == p ? rp : -ck) : v;
+        }
+    }
+    if (!ok && blockIdx.x == 0 && I == 0 && t == 0) *bad = 1.0;
+    auto product = [&](const double* A, const double* B) {
+        double4_t d = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < T; s += 4)
+            d = __builtin_amdgcn_mfma_f64_16x16x4f64(A[(qi + l16) * LD + s + h], B[(s + h) * LD + qj + l16], d, 0, 0, 0);
+        return d;
+    };
+    // the left factor: P in tile row k, else -A_Ik P
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        P[(i0 + 8 * q) * LD + j] = a[q];
+        X[(i0 + 8 * q) * LD + j] = x[q];
+    }
+    __syncthreads();
+    if (I != k) {
+        const double4_t m = product(X, P);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) P[(qi + h + 4 * r) * LD + qj + l16] = -m[r];
+    }
+#pragma unroll 1
+    for (int J = J0; J < J1; ++J) {
+        __syncthreads();  // P is written; Y is free
+#pragma unroll
+        for (int q = 0; q < Q; ++q) Y[(i0 + 8 * q) * LD + j] = y[q];
+        const double4_t cj = {c[0], c[1], c[2], c[3]};
+        if (J + 1 < J1)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                y[q] = in[at(k, J + 1, i0 + 8 * q)];
+                c[q] = in[dat(J + 1, q)];
+            }
+        __syncthreads();
+        if (J == k) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[dat(J, r)] = P[(qi + h + 4 * r) * LD + qj + l16];
+            continue;
+        }
+        const double4_t d = product(P, Y);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[dat(J, r)] = I == k ? d[r] : cj[r] + d[r];
+    }
 }
 
 // ------------------------------------------- power iteration (setup) --
@@ -2358,39 +2503,6 @@ MfTiles mf_tiles(const MgHierarchy& H) {
             (L0.n[2] + kTZ - 1) / kTZ};
 }
 
-// Gauss-Jordan inverse with partial pivoting (FP64); false if singular.
-bool dense_inverse(std::vector<double>& a, int64_t n, std::vector<double>& inv) {
-    inv.assign((size_t)(n * n), 0.0);
-    for (int64_t i = 0; i < n; ++i) inv[(size_t)(i * n + i)] = 1.0;
-    for (int64_t c = 0; c < n; ++c) {
-        int64_t piv = c;
-        for (int64_t i = c + 1; i < n; ++i)
-            if (std::fabs(a[(size_t)(i * n + c)]) > std::fabs(a[(size_t)(piv * n + c)])) piv = i;
-        const double pv = a[(size_t)(piv * n + c)];
-        if (!(std::fabs(pv) > 0.0) || !std::isfinite(pv)) return false;
-        if (piv != c)
-            for (int64_t j = 0; j < n; ++j) {
-                std::swap(a[(size_t)(piv * n + j)], a[(size_t)(c * n + j)]);
-                std::swap(inv[(size_t)(piv * n + j)], inv[(size_t)(c * n + j)]);
-            }
-        const double rp = 1.0 / pv;
-        for (int64_t j = 0; j < n; ++j) {
-            a[(size_t)(c * n + j)] *= rp;
-            inv[(size_t)(c * n + j)] *= rp;
-        }
-        for (int64_t i = 0; i < n; ++i) {
-            if (i == c) continue;
-            const double m = a[(size_t)(i * n + c)];
-            if (m == 0.0) continue;
-            for (int64_t j = 0; j < n; ++j) {
-                a[(size_t)(i * n + j)] -= m * a[(size_t)(c * n + j)];
-                inv[(size_t)(i * n + j)] -= m * inv[(size_t)(c * n + j)];
-            }
-        }
-    }
-    return true;
-}
-
 void cheb_coefficients(MgLevel& l, int degree, double lo, double hi) {
     const double a = lo * l.lmax, b = hi * l.lmax;
     const double theta = 0.5 * (b + a), delta = 0.5 * (b - a), sigma = theta / delta;
@@ -2515,9 +2627,15 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
     // when setup fails).  A side stream starts after an event recorded on the
     // context's stream once its buffers are allocated, so memory the cache
     // hands out again is past its earlier users.
-    DevBuf<PowState> ps(ctx, SFEM_MG_MAX_LEVELS);
-    memset_d(ctx, ps.get(), 0, sizeof(PowState) * SFEM_MG_MAX_LEVELS);
-    DevBuf<double> scales(ctx, SFEM_MG_MAX_LEVELS);  // FP16 stencil scales, 0: zero operator
+    struct SetupOut {
+        double scales[SFEM_MG_MAX_LEVELS];  // FP16 stencil scales, 0: zero operator
+        double singular;                    // 1: the direct level has a zero pivot
+        PowState ps[SFEM_MG_MAX_LEVELS];
+    };
+    DevBuf<SetupOut> setup(ctx, 1);
+    memset_d(ctx, setup.get(), 0, sizeof(SetupOut));
+    PowState* const ps = setup.get()->ps;
+    double* const scales = setup.get()->scales;
     std::vector<DevBuf<double>> parts(SFEM_MG_MAX_LEVELS);
     DevBuf<float> p0a, p0b;
     struct SideJoin {
@@ -2549,11 +2667,11 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         parts[(size_t)l].reset(ctx, std::max({nparts, init_grid(n), 1024u}));
         fork(t);
         hipLaunchKernelGGL(pow_init_kernel, dim3(init_grid(n)), dim3(kThreads), 0, t, n, v.fixed.get(), va,
-                           ps.get() + l, parts[(size_t)l].get());
+                           ps + l, parts[(size_t)l].get());
         SFEM_LAUNCH_CHECK();
     };
     auto power_coarse = [&](int l, const MgLevel& v) {
-        const hipStream_t t = side_stream(ctx, (l - 1) % (sfem_ctx::kSideStreams - 1));
+        const hipStream_t t = side_stream(ctx, (l - 1) % (sfem_ctx::kSideStreams - 2));
         const bool grp = v.node_major;
         const dim3 gp(std::min(rows_grid(v.nn * (grp ? Lanes<ND>::G : 1)), 1024u));
         power_start(l, v, v.da.get(), v.db.get(), gp.x, t);
@@ -2563,7 +2681,7 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         for (int k = 0; k < o.power_iters; ++k) {
             // grid-stride over the nodes: few blocks meet at the last-block count
             auto go = [&](auto kern, auto op) {
-                hipLaunchKernelGGL(kern, gp, dim3(kThreads), 0, t, op, vin, v.binv.get(), vout, ps.get() + l,
+                hipLaunchKernelGGL(kern, gp, dim3(kThreads), 0, t, op, vin, v.binv.get(), vout, ps + l,
                                    partials);
             };
             if (v.st16.size()) {
@@ -2595,10 +2713,38 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         float* vout = p0b.get();
         for (int k = 0; k < o.power_iters; ++k) {
             hipLaunchKernelGGL(pow_mf_kernel<ND>, dim3(gm), dim3(kThreads), 0, t, mf_op32(S, H), vin,
-                               S->binv32.get(), vout, ps.get(), parts[0].get());
+                               S->binv32.get(), vout, ps, parts[0].get());
             SFEM_LAUNCH_CHECK();
             std::swap(vin, vout);
         }
+        finish(t);
+    };
+
+    // The direct level's dense inverse, on a side stream of its own as soon
+    // as the level exists.
+    DevBuf<double> dense[2];
+    auto direct_inverse = [&](int l, const MgLevel& v) {
+        H.direct = l;
+        H.nd_dofs = v.nn * BS;
+        H.ndp = (H.nd_dofs + kTile - 1) / kTile * kTile;
+        const int np = (int)H.ndp, nb = np / kTile;
+        // tiles per workgroup: at most about three workgroups per CU, whose
+        // pivots then hide each other's latency
+        const int per = std::max(1, (nb * nb + 3 * ctx->n_cu - 1) / (3 * ctx->n_cu));
+        for (auto& d : dense) d.reset(ctx, (size_t)np * np);
+        const hipStream_t t = side_stream(ctx, sfem_ctx::kSideStreams - 2);
+        fork(t);
+        SFEM_HIP(hipMemsetAsync(dense[0].get(), 0, dense[0].bytes(), t));
+        hipLaunchKernelGGL(dense_fill_kernel<ND>, dim3(rows_grid(v.nn), NS), dim3(kThreads), 0, t,
+                           (const double*)v.st64.get(), (const uint8_t*)v.fixed.get(), grid_of(v), np, dense[0].get());
+        SFEM_LAUNCH_CHECK();
+        for (int k = 0; k < nb; ++k) {
+            hipLaunchKernelGGL(gauss_jordan_kernel, dim3((nb + per - 1) / per, nb), dim3(kThreads), 0, t,
+                               (const double*)dense[k & 1].get(), dense[(k + 1) & 1].get(), np, k, per,
+                               &setup.get()->singular);
+            SFEM_LAUNCH_CHECK();
+        }
+        H.dinv = std::move(dense[nb & 1]);
         finish(t);
     };
 
@@ -2737,7 +2883,8 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         bool more = false;
         for (int d = 0; d < ND; ++d) more = more || C.n[d] - 1 >= 2;
         const int lc = (int)H.L.size();
-        if (more && C.nn > o.coarse_nodes && lc + 1 < SFEM_MG_MAX_LEVELS) {
+        const bool coarsest = !(more && C.nn > o.coarse_nodes && lc + 1 < SFEM_MG_MAX_LEVELS);
+        if (!coarsest) {
             if (o.coarse_fp16) {
                 const int64_t nv = C.nn * NS * B2;
                 DevBuf<unsigned> mx(ctx, 1);
@@ -2746,11 +2893,11 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
                                    dim3(kThreads), 0, s, (const float*)C.st32.get(), C.nn, C.node_major, mx.get());
                 SFEM_LAUNCH_CHECK();
                 hipLaunchKernelGGL(half_scale_kernel, dim3(1), dim3(1), 0, s, (const unsigned*)mx.get(),
-                                   scales.get() + lc);
+                                   scales + lc);
                 SFEM_LAUNCH_CHECK();
                 C.st16.reset(ctx, (size_t)nv);
                 hipLaunchKernelGGL(to_half_dev_kernel, dim3(std::min(rows_grid(nv), 2048u)), dim3(kThreads), 0, s,
-                                   (const float*)C.st32.get(), nv, (const double*)scales.get() + lc, C.st16.get());
+                                   (const float*)C.st32.get(), nv, (const double*)scales + lc, C.st16.get());
                 SFEM_LAUNCH_CHECK();
                 hipLaunchKernelGGL(stencil_binv_half_kernel<ND>, dim3(rows_grid(C.nn)), dim3(kThreads), 0, s,
                                    (const _Float16*)C.st16.get(), C.nn, C.node_major, C.binv.get());
@@ -2762,13 +2909,12 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
             power_coarse(lc, C);
         }
         if (lc == 1 && H.mf) power_fine_mf();
+        if (!H.direct && C.nn <= 2 * kMgMaxCoarseNodes && (coarsest || C.nn * BS <= direct_dofs())) direct_inverse(lc, C);
         H.L.push_back(std::move(C));
         prev_st = H.L.back().st64.get();
         prev_fix = H.L.back().fixed.get();
         if ((int)H.L.size() >= SFEM_MG_MAX_LEVELS) break;
     }
-    sync(ctx);
-    stf.release();
     if (H.L.size() < 2)
         fail(SFEM_ERR_UNSUPPORTED, "multigrid: no direction has 2 or more elements to coarsen");
     MgLevel& Lc = H.L.back();
@@ -2776,47 +2922,7 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         fail(SFEM_ERR_UNSUPPORTED, "multigrid: the grid coarsens only to " + std::to_string(Lc.nn) +
                                        " nodes (at most " + std::to_string(kMgMaxCoarseNodes) +
                                        ")");
-
-    // coarsest: dense inverse on the host
-    {
-        const int64_t nn = Lc.nn, nc = nn * BS;
-        std::vector<double> st((size_t)(nn * NS * B2));
-        std::vector<uint8_t> fx((size_t)nc);
-        d2h(ctx, st.data(), Lc.st64.get(), st.size() * sizeof(double));
-        d2h(ctx, fx.data(), Lc.fixed.get(), fx.size());
-        std::vector<double> a((size_t)(nc * nc), 0.0), inv;
-        const Grid gc = grid_of(Lc);
-        for (int64_t I = 0; I < nn; ++I) {
-            int64_t c[3];
-            coords_of<ND>(I, gc, c);
-            for (int sl = 0; sl < NS; ++sl) {
-                int dx, dy, dz;
-                offset_of<ND>(sl, dx, dy, dz);
-                if (!inside<ND>(gc, c[0] + dx, c[1] + dy, c[2] + dz)) continue;
-                const int64_t J = node_at(gc, c[0] + dx, c[1] + dy, c[2] + dz);
-                for (int p = 0; p < BS; ++p)
-                    for (int q = 0; q < BS; ++q)
-                        a[(size_t)((I * BS + p) * nc + J * BS + q)] = st[(size_t)(((int64_t)sl * B2 + p * BS + q) * nn + I)];
-            }
-        }
-        for (int64_t d = 0; d < nc; ++d)
-            if (fx[(size_t)d]) a[(size_t)(d * nc + d)] = 1.0;
-        if (!dense_inverse(a, nc, inv)) fail(SFEM_ERR_SINGULAR, "multigrid: the coarsest operator is singular");
-        H.nc = nc;
-        H.cinv.reset(ctx, (size_t)(nc * nc));
-        h2d(ctx, H.cinv.get(), inv.data(), inv.size() * sizeof(double));
-    }
-
-    // FP16 smoothing operators on the levels between the finest and the
-    // coarsest (made as the levels were built): their scales
-    if (o.coarse_fp16 && H.L.size() > 2) {
-        std::vector<double> hs(H.L.size());
-        d2h(ctx, hs.data(), scales.get(), sizeof(double) * hs.size());
-        for (size_t l = 1; l + 1 < H.L.size(); ++l) {
-            if (!(hs[l] > 0.0)) fail(SFEM_ERR_SINGULAR, "multigrid: zero coarse operator");
-            H.L[l].scale = hs[l];
-        }
-    }
+    H.nc = Lc.nn * BS;
 
     // FP16 finest-level smoothing operator
     if (o.fine_fp16 && !H.mf) {
@@ -2873,13 +2979,13 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         parts[0].reset(ctx, std::max({ls.grid, init_grid(n), 1024u}));
         double* partials = parts[0].get();
         hipLaunchKernelGGL(pow_init_kernel, dim3(init_grid(n)), dim3(kThreads), 0, s, n, v.fixed.get(), v.da.get(),
-                           ps.get(), partials);
+                           ps, partials);
         SFEM_LAUNCH_CHECK();
         float* vin = v.da.get();
         float* vout = v.db.get();
         for (int k = 0; k < o.power_iters; ++k) {
             auto go = [&](auto kern, auto op, const float* binv) {
-                hipLaunchKernelGGL(kern, dim3(ls.grid), dim3(kThreads), 0, s, op, vin, binv, vout, ps.get(), partials);
+                hipLaunchKernelGGL(kern, dim3(ls.grid), dim3(kThreads), 0, s, op, vin, binv, vout, ps, partials);
             };
             if (H.fp16) {
                 const SellOp<_Float16> op{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), H.h0.get(), S->nslices,
@@ -2897,8 +3003,15 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         }
     }
     for (hipEvent_t d : join.done) SFEM_HIP(hipStreamWaitEvent(s, d, 0));
-    std::vector<PowState> hps((size_t)nl);
-    d2h(ctx, hps.data(), ps.get(), sizeof(PowState) * nl);  // the side streams joined: every level done
+    SetupOut out;  // the side streams joined: every level done
+    d2h(ctx, &out, setup.get(), offsetof(SetupOut, ps) + sizeof(PowState) * (size_t)nl);
+    const PowState* hps = out.ps;
+    if (out.singular != 0.0) fail(SFEM_ERR_SINGULAR, "multigrid: the coarsest operator is singular");
+    if (o.coarse_fp16)  // the FP16 smoothing operators' scales (made as the levels were built)
+        for (int l = 1; l + 1 < nl; ++l) {
+            if (!(out.scales[l] > 0.0)) fail(SFEM_ERR_SINGULAR, "multigrid: zero coarse operator");
+            H.L[(size_t)l].scale = out.scales[l];
+        }
     for (int l = 0; l + 1 < nl; ++l) {
         H.L[l].lmax = hps[(size_t)l].lam;
         if (!(H.L[l].lmax > 0.0) || !std::isfinite(H.L[l].lmax))
@@ -2989,10 +3102,10 @@ struct MgRun {
     // made their first smoothing step.
     void vcycle(int l, const double* r_outer) {
         MgLevel& L = H.L[(size_t)l];
-        const int nl = (int)H.L.size();
-        if (l == nl - 1) {
-            hipLaunchKernelGGL(dense_apply_kernel, dim3((unsigned)((H.nc + 3) / 4)), dim3(kThreads), 0, s,
-                               (const double*)H.cinv.get(), (int)H.nc, (const float*)L.b.get(), L.x.get(), done);
+        if (l == H.direct) {
+            hipLaunchKernelGGL(dense_apply_kernel, dim3((unsigned)((H.nd_dofs + 3) / 4)), dim3(kThreads), 0, s,
+                               (const double*)H.dinv.get(), (int)H.nd_dofs, (int)H.ndp, (const float*)L.b.get(),
+                               L.x.get(), done);
             SFEM_LAUNCH_CHECK();
             return;
         }
@@ -3018,7 +3131,7 @@ struct MgRun {
                                (const uint8_t*)C.fixed.get(), C.b.get(), (const float*)C.binv.get(), C.c2[0],
                                (float)C.scale, C.r.get(), C.x.get(), C.da.get(), done);
         };
-        if (l + 1 < nl - 1) rk(restrict_kernel<ND, true>);
+        if (l + 1 < H.direct) rk(restrict_kernel<ND, true>);
         else rk(restrict_kernel<ND, false>);
         SFEM_LAUNCH_CHECK();
         vcycle(l + 1, nullptr);

@@ -91,7 +91,7 @@ struct sfem_ctx {
     // Streams for independent work beside `stream` (default priority, made
     // on first use; joined back to `stream` by events before its results
     // are read or its buffers released).
-    static constexpr int kSideStreams = 4;
+    static constexpr int kSideStreams = 5;
     hipStream_t side[kSideStreams] = {};
 };
 

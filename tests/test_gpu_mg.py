@@ -552,3 +552,31 @@ def test_sliced_finest_level_forms(dims, split, monkeypatch):
             assert st["converged"] and np.linalg.norm(q - q_ref) <= 1e-8 * np.linalg.norm(q_ref), (precision, fp16)
     K.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("direct", ["0", "800", "1296"])
+@pytest.mark.parametrize("dims", [(1, 2, 1), (4, 4, 1), (5, 4, 3), (9, 7, 6), (17, 12, 10), (2, 2), (31, 9), (64, 33)])
+def test_direct_level(dims, direct, monkeypatch):
+    # the level solved with its dense inverse: 12 to 1,190 dofs around the
+    # 32 of a block (one block and many, the last one ragged or full), as the
+    # coarsest level alone and above it; partially fixed nodes
+    print(f"[case] direct level {dims} {direct}", flush=True)
+    monkeypatch.setenv("SFEM_MG_DIRECT_DOFS", direct)
+    ctx = smearfem.Context(0)
+    m = structured_mesh(dims)
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=8)
+    fixed = roller(m, axis=m.ndim - 1)
+    f = random_face_load(m, 0, 1, fixed, seed=9)
+    K = device_K(ctx, m, young)
+    Kff, rhs = O.eliminate(oracle_K(m, young), fixed, f)
+    q_ref = O.recombine(fixed, None, sp.linalg.spsolve(sp.csc_matrix(Kff), rhs))
+    bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+    S = System(K, bc)
+    bc.close()
+    S.set_grid(m.dims)
+    st = S.solve("fp64", rtol=1e-12, preconditioner="multigrid")
+    q = S.solution()
+    assert st["converged"] and relerr(q, q_ref) <= ERR
+    S.close()
+    K.close()
+    ctx.close()
