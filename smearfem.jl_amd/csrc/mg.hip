@@ -1052,10 +1052,14 @@ int64_t stencil_group_below() {
 
 // MODE 0: r -= A v; d_out = c1 d_in + c2 B^-1 r; x += d_out (a Chebyshev step)
 // MODE 1: r -= A v (the residual after the last step)
+// MODE 2: MODE 0, and returns the row's part of rout . x (the V-cycle's last
+// finest-level step: rout the outer residual, x the preconditioned one)
 template <int BS, int MODE>
-__device__ __forceinline__ void cheb_epilogue(int64_t row, int64_t nrows, const float (&av)[BS], float* __restrict__ r,
-                                              float* __restrict__ x, const float* d_in, float* __restrict__ d_out,
-                                              float c1, float c2, const float* __restrict__ binv) {
+__device__ __forceinline__ double cheb_epilogue(int64_t row, int64_t nrows, const float (&av)[BS],
+                                                float* __restrict__ r, float* __restrict__ x, const float* d_in,
+                                                float* __restrict__ d_out, float c1, float c2,
+                                                const float* __restrict__ binv, const double* __restrict__ rout) {
+    double rz = 0.0;
     float rv[BS];
 #pragma unroll
     for (int j = 0; j < BS; ++j) {
@@ -1063,7 +1067,7 @@ __device__ __forceinline__ void cheb_epilogue(int64_t row, int64_t nrows, const 
         rv[j] = r[d] - av[j];
         r[d] = rv[j];
     }
-    if (MODE == 1) return;
+    if (MODE == 1) return rz;
 #pragma unroll
     for (int j = 0; j < BS; ++j) {
         float z = 0.0f;
@@ -1071,9 +1075,12 @@ __device__ __forceinline__ void cheb_epilogue(int64_t row, int64_t nrows, const 
         for (int i = 0; i < BS; ++i) z = fmaf(binv[(int64_t)(j * BS + i) * nrows + row], rv[i], z);
         const int64_t d = row * BS + j;
         const float dn = fmaf(c2, z, d_in ? c1 * d_in[d] : 0.0f);
+        const float xn = x[d] + dn;
         d_out[d] = dn;
-        x[d] += dn;
+        x[d] = xn;
+        if (MODE == 2) rz = fma(rout[d], (double)xn, rz);
     }
+    return rz;
 }
 
 // The same step with its operands loaded first (cheb_load, beside the row's
@@ -1082,12 +1089,14 @@ __device__ __forceinline__ void cheb_epilogue(int64_t row, int64_t nrows, const 
 template <int BS>
 struct ChebIn {
     float r[BS], x[BS], din[BS], binv[BS * BS];
+    double rout[BS];
 };
 
 template <int BS, int MODE>
 __device__ __forceinline__ void cheb_load(int64_t row, int64_t nrows, const float* __restrict__ r,
                                           const float* __restrict__ x, const float* d_in,
-                                          const float* __restrict__ binv, ChebIn<BS>& o) {
+                                          const float* __restrict__ binv, ChebIn<BS>& o,
+                                          const double* __restrict__ rout = nullptr) {
 #pragma unroll
     for (int j = 0; j < BS; ++j) o.r[j] = r[row * BS + j];
     if (MODE == 1) return;
@@ -1098,10 +1107,13 @@ __device__ __forceinline__ void cheb_load(int64_t row, int64_t nrows, const floa
     }
 #pragma unroll
     for (int k = 0; k < BS * BS; ++k) o.binv[k] = binv[(int64_t)k * nrows + row];
+    if (MODE == 2)
+#pragma unroll
+        for (int j = 0; j < BS; ++j) o.rout[j] = rout[row * BS + j];
 }
 
 template <int BS, int MODE>
-__device__ __forceinline__ void cheb_finish(int64_t row, const ChebIn<BS>& o, const float (&av)[BS],
+__device__ __forceinline__ double cheb_finish(int64_t row, const ChebIn<BS>& o, const float (&av)[BS],
                                             float* __restrict__ r, float* __restrict__ x, bool has_din,
                                             float* __restrict__ d_out, float c1, float c2) {
     float rv[BS];
@@ -1110,16 +1122,27 @@ __device__ __forceinline__ void cheb_finish(int64_t row, const ChebIn<BS>& o, co
         rv[j] = o.r[j] - av[j];
         r[row * BS + j] = rv[j];
     }
-    if (MODE == 1) return;
+    double rz = 0.0;
+    if (MODE == 1) return rz;
 #pragma unroll
     for (int j = 0; j < BS; ++j) {
         float z = 0.0f;
 #pragma unroll
         for (int i = 0; i < BS; ++i) z = fmaf(o.binv[j * BS + i], rv[i], z);
         const float dn = fmaf(c2, z, has_din ? c1 * o.din[j] : 0.0f);
+        const float xn = o.x[j] + dn;
         d_out[row * BS + j] = dn;
-        x[row * BS + j] = o.x[j] + dn;
+        x[row * BS + j] = xn;
+        if (MODE == 2) rz = fma(o.rout[j], (double)xn, rz);
     }
+    return rz;
+}
+
+// A finest-level step's sum of r.z: the block's part, for the kernel that
+// forms beta.
+__device__ __forceinline__ void put_rz(double rz, double* __restrict__ parts, double* sh) {
+    rz = block_sum_256(rz, sh);
+    if (threadIdx.x == 0) parts[blockIdx.x] = rz;
 }
 
 // Finest-level step on the sliced operator.  SHARED: a block per slice
@@ -1129,19 +1152,23 @@ template <int BS, int MODE, bool NT, bool SHARED, typename TV>
 __global__ __launch_bounds__(kThreads) void cheb_sell_kernel(SellOp<TV> op, const float* v, float* __restrict__ r,
                                                              float* __restrict__ x, const float* d_in,
                                                              float* __restrict__ d_out, float c1, float c2,
-                                                             const float* __restrict__ binv, const int* done) {
+                                                             const float* __restrict__ binv,
+                                                             const double* __restrict__ rout,
+                                                             double* __restrict__ parts, const int* halt) {
+    __shared__ double sh[4];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    double rz = 0.0;
     if constexpr (SHARED) {
         __shared__ float buf[kThreads / 64][BS][64];
-        const bool stop = *done != 0;  // checked before the stores
+        const bool stop = *halt != 0;  // checked before the stores
         const int64_t sl = logical_block();
-        if (sl >= op.nslices) return;
+        const bool live = sl < op.nslices;
         SharedSlice<BS, TV, NT> cols(op.scol, Vals<TV>{op.val});
-        cols.load(op.sl_ptr, op.sl_w, sl);
+        if (live) cols.load(op.sl_ptr, op.sl_w, sl);
         const int64_t row = sl * 64 + lane;
-        const bool own = w == 0 && row < op.nrows;
+        const bool own = w == 0 && live && row < op.nrows;
         ChebIn<BS> in;
-        if (own) cheb_load<BS, MODE>(row, op.nrows, r, x, d_in, binv, in);
+        if (own) cheb_load<BS, MODE>(row, op.nrows, r, x, d_in, binv, in, rout);
         auto gx = [=](int64_t c, float(&xv)[BS]) {
 #pragma unroll
             for (int i = 0; i < BS; ++i) xv[i] = v[c * BS + i];
@@ -1149,9 +1176,9 @@ __global__ __launch_bounds__(kThreads) void cheb_sell_kernel(SellOp<TV> op, cons
         float out[BS] = {};
         cols.apply(gx, out);
         sell_combine<BS, kThreads / 64>(out, buf);
-        if (own && !stop) cheb_finish<BS, MODE>(row, in, out, r, x, d_in != nullptr, d_out, c1, c2);
+        if (own && !stop) rz = cheb_finish<BS, MODE>(row, in, out, r, x, d_in != nullptr, d_out, c1, c2);
     } else {
-        if (*done) return;
+        if (*halt) return;
         const int64_t s0 = logical_block() * op.per_block;
         const int64_t s1 = min(op.nslices, s0 + op.per_block);
         auto gx = [=](int64_t c) { return v[c]; };
@@ -1159,9 +1186,11 @@ __global__ __launch_bounds__(kThreads) void cheb_sell_kernel(SellOp<TV> op, cons
             float out[BS];
             sell_row<BS, TV, float, NT>(op.sl_ptr, op.sl_w, op.scol, Vals<TV>{op.val}, sl, lane, gx, out);
             const int64_t row = sl * 64 + lane;
-            if (row < op.nrows) cheb_epilogue<BS, MODE>(row, op.nrows, out, r, x, d_in, d_out, c1, c2, binv);
+            if (row < op.nrows)
+                rz += cheb_epilogue<BS, MODE>(row, op.nrows, out, r, x, d_in, d_out, c1, c2, binv, rout);
         }
     }
+    if (MODE == 2) put_rz(rz, parts, sh);
 }
 
 template <int ND, int MODE, bool GROUP, typename TV>
@@ -1353,6 +1382,45 @@ __device__ __forceinline__ void mf_row(const MfOp<T>& op, const T* kc, int64_t r
     for (int i = 0; i < ND; ++i) out[i] = o[0][i];
 }
 
+// The same row in 3D by a group of 8 lanes, lane q taking the node's cell q
+// (its corners' values times the 8 blocks of Ke(0)'s row 7 - q), summed by a
+// butterfly: every lane of the group gets the sum, unmasked (the caller puts
+// a fixed dof's own value in its place).  For small grids, where one thread
+// per row leaves the device idle and runs 576 dependent products (432 rows:
+// 7.8 us a step, 14.3 us the FP64 operator).  gather(byte offset of an FP32
+// row, x).
+template <typename T, typename Gather>
+__device__ __forceinline__ void mf_row_lanes(const MfOp<T>& op, uint32_t row, uint32_t q, Gather gather, T (&out)[3]) {
+    const uint32_t n0 = op.n0, n1 = op.n1;
+    const uint32_t P0 = n0 + 2, P1 = n1 + 2, Q0 = n0 + 1, Q1 = n1 + 1;  // padded nodes and cells per direction
+    const uint32_t node = (uint32_t)op.node_of_row[row];
+    const uint32_t yz = node / n0, cx = node - yz * n0, cz = yz / n1, cy = yz - cz * n1;
+    // the cell's lower corner is node c - 1 + (qx, qy, qz): padded c + q
+    const uint32_t x0 = cx + (q & 1), y0 = cy + ((q >> 1) & 1), z0 = cz + (q >> 2);
+    const uint32_t pn = x0 + P0 * (y0 + P1 * z0);
+    const T se = op.es[x0 + Q0 * (y0 + Q1 * z0)];
+    uint32_t o[8];
+#pragma unroll
+    for (uint32_t b = 0; b < 8; ++b) o[b] = op.offs[pn + (b & 1) + P0 * (((b >> 1) & 1) + P1 * (b >> 2))];
+    T x[8][3];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) gather(o[b], x[b]);
+    const T* k = op.kc + (7 - q) * 72;
+    T t[3] = {};
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) t[i] = fma(k[b * 9 + i * 3 + j], x[b][j], t[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) out[i] = se * t[i];
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) out[i] += __shfl_xor(out[i], off, 8);
+}
+
 // ghost-layer copies for the matrix-free operator: node rows (-1 outside)
 // and cell scales (0 outside); n: nodes or cells per direction, the copy
 // has n + 2 (directions beyond ND: 1, no layer)
@@ -1392,13 +1460,63 @@ template <int ND, int MODE>
 __global__ __launch_bounds__(kThreads) void cheb_mf_kernel(MfOp<float> op, const float* v, float* __restrict__ r,
                                                            float* __restrict__ x, const float* d_in,
                                                            float* __restrict__ d_out, float c1, float c2,
-                                                           const float* __restrict__ binv, const int* done) {
-    if (*done) return;
+                                                           const float* __restrict__ binv,
+                                                           const double* __restrict__ rout,
+                                                           double* __restrict__ parts, const int* halt) {
+    if (*halt) return;
     const int64_t row = logical_block() * kThreads + threadIdx.x;
-    if (row >= op.nrows) return;
-    float out[ND];
-    mf_row<ND, float, float>(op, op.kc, row, v, out);
-    cheb_epilogue<ND, MODE>(row, op.nrows, out, r, x, d_in, d_out, c1, c2, binv);
+    double rz = 0.0;
+    if (row < op.nrows) {
+        float out[ND];
+        mf_row<ND, float, float>(op, op.kc, row, v, out);
+        rz = cheb_epilogue<ND, MODE>(row, op.nrows, out, r, x, d_in, d_out, c1, c2, binv, rout);
+    }
+    if constexpr (MODE == 2) {
+        __shared__ double sh[4];
+        put_rz(rz, parts, sh);
+    }
+}
+
+// The step with 8 lanes per row (mf_row_lanes): small 3D grids.
+template <int MODE>
+__global__ __launch_bounds__(kThreads) void cheb_mf_lanes_kernel(MfOp<float> op, const float* v,
+                                                                 float* __restrict__ r, float* __restrict__ x,
+                                                                 const float* d_in, float* __restrict__ d_out,
+                                                                 float c1, float c2, const float* __restrict__ binv,
+                                                                 const double* __restrict__ rout,
+                                                                 double* __restrict__ parts, const int* halt) {
+    constexpr int BS = 3, G = 8;
+    const bool stop = *halt != 0;  // checked before the stores
+    const uint32_t t = blockIdx.x * kThreads + threadIdx.x, row = t / G;
+    const uint32_t q = t % G;
+    const bool live = row < op.nrows, lead = live && q == 0;
+    double rz = 0.0;
+    ChebIn<BS> in;
+    float own[BS] = {};
+    uint8_t fx[BS] = {};
+    if (lead) {
+        cheb_load<BS, MODE>(row, op.nrows, r, x, d_in, binv, in, rout);
+#pragma unroll
+        for (int j = 0; j < BS; ++j) {
+            own[j] = v[row * BS + j];
+            fx[j] = op.fixed[row * BS + j];
+        }
+    }
+    float out[BS] = {};
+    if (live)
+        mf_row_lanes<float>(op, row, q, [&](uint32_t o, float(&xv)[BS]) {
+#pragma unroll
+            for (int j = 0; j < BS; ++j) xv[j] = *(const float*)((const char*)v + (o + 4u * j));
+        }, out);
+    if (lead && !stop) {
+#pragma unroll
+        for (int j = 0; j < BS; ++j) out[j] = fx[j] ? own[j] : out[j];
+        rz = cheb_finish<BS, MODE>(row, in, out, r, x, d_in != nullptr, d_out, c1, c2);
+    }
+    if constexpr (MODE == 2) {
+        __shared__ double sh[4];
+        put_rz(rz, parts, sh);
+    }
 }
 
 // First step from x = 0: r = b, d = c2 B^-1 b, x = d.  bscale: the units of
@@ -1407,8 +1525,8 @@ template <int BS, typename TB>
 __global__ __launch_bounds__(kThreads) void cheb_first_kernel(const TB* __restrict__ b, TB bscale, int64_t nrows,
                                                               const float* __restrict__ binv, float c2,
                                                               float* __restrict__ r, float* __restrict__ x,
-                                                              float* __restrict__ d, const int* done) {
-    const bool stop = *done != 0;  // checked before the stores
+                                                              float* __restrict__ d, const int* halt) {
+    const bool stop = *halt != 0;  // checked before the stores
     const int64_t row = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (row >= nrows) return;
     float rv[BS];
@@ -1428,6 +1546,35 @@ __global__ __launch_bounds__(kThreads) void cheb_first_kernel(const TB* __restri
         const float dn = c2 * z;
         d[row * BS + j] = dn;
         x[row * BS + j] = dn;
+    }
+}
+
+// The V-cycle's first finest-level step made by the kernel that forms the
+// outer residual: r = (float)(scale rout), d = x = c2 B^-1 r.
+struct FirstStep {
+    const float* binv;
+    double scale;
+    float c2;
+    float *r, *x, *d;
+    int64_t nrows;
+};
+
+template <int BS>
+__device__ __forceinline__ void first_step_row(const FirstStep& F, int64_t row, const double (&rout)[BS]) {
+    float rv[BS];
+#pragma unroll
+    for (int j = 0; j < BS; ++j) {
+        rv[j] = (float)(rout[j] * F.scale);
+        F.r[row * BS + j] = rv[j];
+    }
+#pragma unroll
+    for (int j = 0; j < BS; ++j) {
+        float z = 0.0f;
+#pragma unroll
+        for (int i = 0; i < BS; ++i) z = fmaf(F.binv[(int64_t)(j * BS + i) * F.nrows + row], rv[i], z);
+        const float dn = F.c2 * z;
+        F.d[row * BS + j] = dn;
+        F.x[row * BS + j] = dn;
     }
 }
 
@@ -1621,13 +1768,56 @@ __global__ __launch_bounds__(kThreads) void prolong_kernel(const float* __restri
     prolong_row<ND>(row, xc, gc, gf, f0, f1, f2, node_of_row, ffix, xf, e, stop);
 }
 
+// ------------------------------------------------------- outer CG ----
+// The scalars are formed by the kernels that need them: each sums the
+// previous kernel's per-block partials itself, and its first block stores
+// what later kernels read.
+struct MgState {
+    double bb, tol2bb;
+    double rz[2];   // r.z of the iterations, by parity
+    double rr, rr_true, best_true, floor_rr;
+    long long iters, trues;
+    int done;       // 1 converged, 2 breakdown, 3 stagnation
+    int halt;       // done, or the FP64 check is due: the V-cycle's kernels exit
+    int restart;    // next direction is z (after a residual replacement)
+    int need_true;  // the recurrence claims convergence: check the FP64 residual
+    int fresh;      // the last update's r.r is still to be taken
+    int stall;
+    Arrivals arrive;
+};
+
+// By one block: the iteration count and the claim of convergence from the
+// last update's per-block r.r.
+__device__ __forceinline__ void take_rr(MgState* st, const double* __restrict__ upd, int nupd, double* sh) {
+    if (st->done || !st->fresh) return;  // uniform
+    double rr[1];
+    sum_parts_all<1, kThreads / 64>(upd, nupd, rr, sh);
+    if (threadIdx.x == 0) {
+        st->fresh = 0;
+        st->rr = rr[0];
+        st->iters += 1;
+        if (rr[0] <= st->tol2bb) st->need_true = st->halt = 1;
+        if (!isfinite(rr[0])) st->done = st->halt = 2;
+    }
+}
+
+// After the last update of the enqueued iterations.
+__global__ __launch_bounds__(kThreads) void mg_check_kernel(MgState* st, const double* __restrict__ upd, int nupd) {
+    __shared__ double sh[4];
+    take_rr(st, upd, nupd, sh);
+}
+
 // direct level: x = A^-1 b with the dense FP64 inverse (row stride np), a
 // wavefront per row (the row read coalesced, the loads of eight strides in
 // flight, a fixed butterfly).  1,275 dofs: 13 MB, from the caches.
+// Its first block also takes the last update's r.r (take_rr).
 __global__ __launch_bounds__(kThreads) void dense_apply_kernel(const double* __restrict__ inv, int nc, int np,
                                                                const float* __restrict__ b, float* __restrict__ x,
-                                                               const int* done) {
-    const bool stop = *done != 0;  // checked before the stores
+                                                               MgState* st, const double* __restrict__ upd,
+                                                               int nupd) {
+    __shared__ double sh[4];
+    const bool stop = st->halt != 0;  // checked before the stores
+    if (blockIdx.x == 0) take_rr(st, upd, nupd, sh);
     const int row = (int)blockIdx.x * (kThreads / 64) + (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     if (row >= nc) return;
     double s = 0.0;
@@ -1889,6 +2079,33 @@ __global__ __launch_bounds__(kThreads, 4) void pow_stencil_kernel(StOp<TV> op, c
     if (last_block_arrive(&ps->arrive)) pow_finish(ps, partials, sh);
 }
 
+__global__ __launch_bounds__(kThreads) void pow_mf_lanes_kernel(MfOp<float> op, const float* __restrict__ v,
+                                                                const float* __restrict__ binv,
+                                                                float* __restrict__ w, PowState* ps,
+                                                                double* __restrict__ partials) {
+    constexpr int BS = 3, G = 8;
+    __shared__ double sh[8];
+    const float scale = (float)ps->inv;
+    const uint32_t t = blockIdx.x * kThreads + threadIdx.x, row = t / G;
+    const uint32_t q = t % G;
+    double sum = 0.0;
+    if (row < op.nrows) {
+        float out[BS];
+        mf_row_lanes<float>(op, row, q, [&](uint32_t o, float(&xv)[BS]) {
+#pragma unroll
+            for (int j = 0; j < BS; ++j) xv[j] = *(const float*)((const char*)v + (o + 4u * j));
+        }, out);
+        if (q == 0) {
+#pragma unroll
+            for (int j = 0; j < BS; ++j) out[j] = op.fixed[row * BS + j] ? v[row * BS + j] : out[j];
+            sum = pow_epilogue<BS>(row, op.nrows, out, scale, binv, w);
+        }
+    }
+    const double b = block_sum_256(sum, sh);
+    if (threadIdx.x == 0) st_coherent(partials + blockIdx.x, b);
+    if (last_block_arrive(&ps->arrive)) pow_finish(ps, partials, sh);
+}
+
 template <int ND>
 __global__ __launch_bounds__(kThreads) void pow_mf_kernel(MfOp<float> op, const float* __restrict__ v,
                                                           const float* __restrict__ binv, float* __restrict__ w,
@@ -1907,19 +2124,6 @@ __global__ __launch_bounds__(kThreads) void pow_mf_kernel(MfOp<float> op, const 
     if (last_block_arrive(&ps->arrive)) pow_finish(ps, partials, sh);
 }
 
-// ------------------------------------------------------- outer CG ----
-struct MgState {
-    double bb, tol2bb;
-    double rz, rz_old, alpha, beta;
-    double rr, rr_true, best_true, floor_rr;
-    long long iters, trues;
-    int done;       // 1 converged, 2 breakdown, 3 stagnation
-    int restart;    // next direction is z (after a residual replacement)
-    int need_true;  // the recurrence claims convergence: check the FP64 residual
-    int stall;
-    Arrivals arrive;
-};
-
 __global__ __launch_bounds__(kThreads) void mg_norm_kernel(const double* __restrict__ rhs, int64_t n,
                                                            int64_t per_block, MgState* st,
                                                            double* __restrict__ partials, double rtol) {
@@ -1936,7 +2140,7 @@ __global__ __launch_bounds__(kThreads) void mg_norm_kernel(const double* __restr
             st->bb = bb;
             st->tol2bb = rtol * rtol * bb;
             if (bb == 0.0) {
-                st->done = 1;
+                st->done = st->halt = 1;
                 st->rr_true = 0.0;
             }
         }
@@ -1959,7 +2163,8 @@ __global__ __launch_bounds__(kThreads) void mg_true_k_kernel(const int64_t* __re
                                                              const int32_t* __restrict__ free_of, int64_t nrows,
                                                              const double* __restrict__ x,
                                                              const double* __restrict__ rhs, double* __restrict__ r,
-                                                             MgState* st, double* __restrict__ partials) {
+                                                             FirstStep first, MgState* st,
+                                                             double* __restrict__ partials) {
     constexpr int B2 = BS * BS, G = 32;
     __shared__ double sh[8];
     if (st->done || !st->need_true) return;
@@ -2006,11 +2211,12 @@ __global__ __launch_bounds__(kThreads) void mg_true_k_kernel(const int64_t* __re
                     aout[j] = fabs(x[d]);
                 }
                 const double res = rhs[d] - out[j];
-                r[d] = res;
+                r[d] = out[j] = res;
                 rr = fma(res, res, rr);
                 const double sc = fabs(rhs[d]) + aout[j];
                 ff = fma(sc, sc, ff);
             }
+            first_step_row<BS>(first, row, out);
         }
     }
     true_finish(st, partials, sh, rr, ff);
@@ -2026,7 +2232,8 @@ __global__ __launch_bounds__(kThreads) void mg_true_kernel(const int64_t* __rest
                                                            int64_t nrows, int64_t per_block,
                                                            const double* __restrict__ x,
                                                            const double* __restrict__ rhs, double* __restrict__ r,
-                                                           MgState* st, double* __restrict__ partials) {
+                                                           FirstStep first, MgState* st,
+                                                           double* __restrict__ partials) {
     __shared__ double sh[8];
     if (st->done || !st->need_true) return;
     const int64_t s0 = logical_block() * per_block;
@@ -2043,11 +2250,12 @@ __global__ __launch_bounds__(kThreads) void mg_true_kernel(const int64_t* __rest
             for (int j = 0; j < BS; ++j) {
                 const int64_t d = row * BS + j;
                 const double res = rhs[d] - out[j];
-                r[d] = res;
+                r[d] = out[j] = res;
                 rr = fma(res, res, rr);
                 const double sc = fabs(rhs[d]) + aout[j];
                 ff = fma(sc, sc, ff);
             }
+            first_step_row<BS>(first, row, out);
         }
     }
     true_finish(st, partials, sh, rr, ff);
@@ -2089,40 +2297,25 @@ __device__ void true_finish(MgState* st, double* __restrict__ partials, double* 
                     if (trr <= st->floor_rr || st->stall >= 3) st->done = 3;
                 }
             }
+            st->halt = st->done;
         }
     }
 }
 
-// r.z -> beta (0 after a restart)
-// block partials of r.z; the last block to arrive forms rz and beta
-__device__ void rz_finish(MgState* st, double* __restrict__ partials, double* sh, double s) {
-    const double b = block_sum_256(s, sh);
-    if (threadIdx.x == 0) st_coherent(partials + blockIdx.x, b);
-    if (last_block_arrive(&st->arrive)) {
-        const double rz = sum_parts(partials, gridDim.x, sh);
-        if (threadIdx.x == 0) {
-            if (!(rz > 0.0) || !isfinite(rz)) {
-                st->done = 2;
-            } else {
-                st->beta = st->restart ? 0.0 : rz / st->rz_old;
-                st->rz_old = rz;
-            }
-            st->rz = rz;
-            st->restart = 0;
-        }
+// Start of the pass that forms the direction, by every block: beta from the
+// V-cycle's last step's r.z (0 after a restart).  False: nothing to do.
+__device__ __forceinline__ bool direction_begin(MgState* st, int parity, const double* __restrict__ zparts, int nz,
+                                                double* sh, double& beta) {
+    if (st->halt || st->done) return false;
+    double rz[1];
+    sum_parts_all<1, kThreads / 64>(zparts, nz, rz, sh);
+    const bool ok = rz[0] > 0.0 && isfinite(rz[0]);
+    beta = st->restart ? 0.0 : rz[0] / st->rz[parity ^ 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->rz[parity] = rz[0];
+        if (!ok) st->done = 2;  // the other blocks find it for themselves
     }
-}
-
-__global__ __launch_bounds__(kThreads) void mg_rz_kernel(const double* __restrict__ r, const float* __restrict__ z,
-                                                         int64_t n, int64_t per_block, MgState* st,
-                                                         double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
-    const int64_t i0 = (int64_t)blockIdx.x * per_block, i1 = min(n, i0 + per_block);
-    double s = 0.0;
-#pragma unroll 4  // four strides of loads in flight; the same order of operations
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) s = fma(r[i], (double)z[i], s);
-    rz_finish(st, partials, sh, s);
+    return ok;
 }
 
 // ------------------------------- matrix-free finest level on MFMA (3D) --
@@ -2164,12 +2357,12 @@ template <int MODE>
 __global__ __launch_bounds__(kThreads) void cheb_mf_mfma_kernel(
     MfOp<float> op, MfTiles T, const half4_t* __restrict__ kfrag, float kscale, const float* v,
     float* __restrict__ r, float* __restrict__ x, const float* d_in, float* __restrict__ d_out, float c1, float c2,
-    const float* __restrict__ binv, const int* done) {
+    const float* __restrict__ binv, const double* __restrict__ rout, double* __restrict__ parts, const int* halt) {
     __shared__ _Float16 xh[kHN * 3], xl[kHN * 3];
     __shared__ float zc[kCN * kZS];
     __shared__ float scell[kCN];
     __shared__ float wmax[kThreads / 64];
-    if (*done != 0) return;  // uniform over the grid
+    if (*halt != 0) return;  // uniform over the grid
     const int tid = threadIdx.x;
     const int64_t t = logical_block();
     const bool live = t < T.tx * T.ty * T.tz;
@@ -2195,12 +2388,12 @@ __global__ __launch_bounds__(kThreads) void cheb_mf_mfma_kernel(
             rv[j] = r[r3 + j];
             own[j] = v[r3 + j];
             fx[j] = op.fixed[r3 + j];
-            if (MODE == 0) {
+            if (MODE != 1) {
                 xv[j] = x[r3 + j];
                 dv[j] = d_in ? d_in[r3 + j] : 0.0f;
             }
         }
-        if (MODE == 0)
+        if (MODE != 1)
 #pragma unroll
             for (int m = 0; m < 9; ++m) bv[m] = binv[(int64_t)m * op.nrows + row];
     }
@@ -2285,7 +2478,7 @@ __global__ __launch_bounds__(kThreads) void cheb_mf_mfma_kernel(
     __syncthreads();
     // C: a tile node sums its 8 cells (ascending corner code), then the
     // Chebyshev epilogue on the values loaded at the start
-    double s = 0.0;
+    double rz = 0.0;
     if (row >= 0) {
         float acc[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -2303,91 +2496,119 @@ __global__ __launch_bounds__(kThreads) void cheb_mf_mfma_kernel(
             res[j] = rv[j] - (fx[j] ? own[j] : acc[j]);
             r[r3 + j] = res[j];
         }
-        if (MODE == 0)
+        if (MODE != 1)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 float z = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 3; ++i) z = fmaf(bv[j * 3 + i], res[i], z);
                 const float dn = fmaf(c2, z, d_in ? c1 * dv[j] : 0.0f);
+                const float xn = xv[j] + dn;
                 d_out[r3 + j] = dn;
-                x[r3 + j] = xv[j] + dn;
+                x[r3 + j] = xn;
+                if (MODE == 2) rz = fma(rout[r3 + j], (double)xn, rz);
             }
+    }
+    if constexpr (MODE == 2) {
+        __shared__ double sh[4];
+        put_rz(rz, parts, sh);
     }
 }
 
+// p = z + beta p in place: the direction as a pass of its own (large systems).
 __global__ __launch_bounds__(kThreads) void mg_p_kernel(double* __restrict__ p, const float* __restrict__ z, int64_t n,
-                                                        int64_t per_block, const MgState* st) {
-    if (st->done) return;
-    const double beta = st->beta;
+                                                        int64_t per_block, MgState* st, int parity,
+                                                        const double* __restrict__ zparts, int nz) {
+    __shared__ double sh[4];
+    double beta;
+    if (!direction_begin(st, parity, zparts, nz, sh, beta)) return;
     const int64_t i0 = (int64_t)blockIdx.x * per_block, i1 = min(n, i0 + per_block);
 #pragma unroll 4  // four strides of loads in flight; the same order of operations
     for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) p[i] = fma(beta, p[i], (double)z[i]);
 }
 
-// q = A p (operator values TV, FP64 vectors), p.q -> alpha
+// Operands of the outer operator pass.  FLY: p = z + beta p formed where a row
+// gathers it and written once (p is double buffered), as in the Jacobi CG;
+// else p is read (pnew unused).
+struct OuterVecs {
+    const double* p;
+    const float* z;
+    double* pnew;
+    double* q;
+    const double* zparts;
+    int nz, parity;
+};
+
+// q = A p (operator values TV, FP64 vectors), per-block p.q
 template <int BS, typename TV, bool NT, bool SHARED>
 __global__ __launch_bounds__(kThreads) void mg_spmv_kernel(const int64_t* __restrict__ sl_ptr,
                                                            const int32_t* __restrict__ sl_w,
                                                            const int32_t* __restrict__ scol, Vals<TV> sval,
                                                            int64_t nslices, int64_t nrows, int64_t per_block,
-                                                           const double* __restrict__ p, double* __restrict__ q,
-                                                           MgState* st, double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
+                                                           OuterVecs v, MgState* st, double* __restrict__ parts) {
+    __shared__ double sh[4];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double dot = 0.0;
-    auto finish = [&](int64_t row, const double (&out)[BS]) {
-#pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            const int64_t d = row * BS + j;
-            q[d] = out[j];
-            dot = fma(p[d], out[j], dot);
-        }
-    };
-    if constexpr (SHARED) {
+    if constexpr (SHARED) {  // FLY
         __shared__ double buf[kThreads / 64][BS][64];
         const int64_t sl = logical_block();
         const bool live = sl < nslices;
         SharedSlice<BS, TV, NT> cols(scol, sval);
         if (live) cols.load(sl_ptr, sl_w, sl);
+        double beta;
+        if (!direction_begin(st, v.parity, v.zparts, v.nz, sh, beta)) return;
+        const double* __restrict__ p = v.p;
+        const float* __restrict__ z = v.z;
         auto gx = [=](int64_t c, double(&xv)[BS]) {
 #pragma unroll
-            for (int i = 0; i < BS; ++i) xv[i] = p[c * BS + i];
+            for (int i = 0; i < BS; ++i) xv[i] = fma(beta, p[c * BS + i], (double)z[c * BS + i]);
         };
         double out[BS] = {};
         cols.apply(gx, out);
         sell_combine<BS, kThreads / 64>(out, buf);
-        if (w == 0 && live && sl * 64 + lane < nrows) finish(sl * 64 + lane, out);
+        const int64_t row = sl * 64 + lane;
+        if (w == 0 && live && row < nrows) {
+            double pr[BS];
+            gx(row, pr);
+#pragma unroll
+            for (int j = 0; j < BS; ++j) {
+                v.pnew[row * BS + j] = pr[j];
+                v.q[row * BS + j] = out[j];
+                dot = fma(pr[j], out[j], dot);
+            }
+        }
     } else {
+        if (st->halt || st->done) return;
         const int64_t s0 = logical_block() * per_block;
         const int64_t s1 = min(nslices, s0 + per_block);
+        const double* __restrict__ p = v.p;
         auto gx = [=](int64_t c) { return p[c]; };
         for (int64_t sl = s0 + w; sl < s1; sl += kThreads / 64) {
             double out[BS];
             sell_row<BS, TV, double, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, out);
-            if (sl * 64 + lane < nrows) finish(sl * 64 + lane, out);
+            const int64_t row = sl * 64 + lane;
+            if (row < nrows) {
+#pragma unroll
+                for (int j = 0; j < BS; ++j) {
+                    const int64_t d = row * BS + j;
+                    v.q[d] = out[j];
+                    dot = fma(p[d], out[j], dot);
+                }
+            }
         }
     }
-    const double b = block_sum_256(dot, sh);
-    if (threadIdx.x == 0) st_coherent(partials + blockIdx.x, b);
-    if (last_block_arrive(&st->arrive)) {
-        const double pq = sum_parts(partials, gridDim.x, sh);
-        if (threadIdx.x == 0) {
-            st->alpha = st->rz_old / pq;
-            if (!(pq > 0.0) || !isfinite(st->alpha)) st->done = 2;
-        }
-    }
+    dot = block_sum_256(dot, sh);
+    if (threadIdx.x == 0) parts[blockIdx.x] = dot;
 }
 
-// q = K_ff p matrix-free in FP64, p.q -> alpha (4 waves per SIMD: <= 128
+// q = K_ff p matrix-free in FP64, per-block p.q (4 waves per SIMD: <= 128
 // registers)
 template <int ND>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void mg_spmv_mf_kernel(MfOp<double> op, const double* __restrict__ p,
-                                                              double* __restrict__ q, MgState* st,
-                                                              double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void mg_spmv_mf_kernel(
+    MfOp<double> op, OuterVecs v, MgState* st, double* __restrict__ parts) {
+    __shared__ double sh[4];
+    if (st->halt || st->done) return;
+    const double* __restrict__ p = v.p;
     double dot = 0.0;
     for (int64_t row = logical_block() * kThreads + threadIdx.x; row < op.nrows;
          row += (int64_t)gridDim.x * kThreads) {
@@ -2396,51 +2617,89 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 #pragma unroll
         for (int j = 0; j < ND; ++j) {
             const int64_t d = row * ND + j;
-            q[d] = out[j];
+            v.q[d] = out[j];
             dot = fma(p[d], out[j], dot);
         }
     }
-    const double b = block_sum_256(dot, sh);
-    if (threadIdx.x == 0) st_coherent(partials + blockIdx.x, b);
-    if (last_block_arrive(&st->arrive)) {
-        const double pq = sum_parts(partials, gridDim.x, sh);
-        if (threadIdx.x == 0) {
-            st->alpha = st->rz_old / pq;
-            if (!(pq > 0.0) || !isfinite(st->alpha)) st->done = 2;
-        }
-    }
+    dot = block_sum_256(dot, sh);
+    if (threadIdx.x == 0) parts[blockIdx.x] = dot;
 }
 
-// x += alpha p, r -= alpha q, r.r; a recurrence at the tolerance asks for
-// the FP64 check
-__global__ __launch_bounds__(kThreads) void mg_update_kernel(double* __restrict__ x, double* __restrict__ r,
-                                                             const double* __restrict__ p,
-                                                             const double* __restrict__ q, int64_t n,
-                                                             int64_t per_block, MgState* st,
-                                                             double* __restrict__ partials) {
-    __shared__ double sh[8];
-    if (st->done) return;
-    const double a = st->alpha;
-    const int64_t i0 = (int64_t)blockIdx.x * per_block, i1 = min(n, i0 + per_block);
-    double rr = 0.0;
-#pragma unroll 4  // four strides of loads in flight; the same order of operations
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) {
-        x[i] = fma(a, p[i], x[i]);
-        const double ri = fma(-a, q[i], r[i]);
-        r[i] = ri;
-        rr = fma(ri, ri, rr);
-    }
-    const double b = block_sum_256(rr, sh);
-    if (threadIdx.x == 0) st_coherent(partials + blockIdx.x, b);
-    if (last_block_arrive(&st->arrive)) {
-        const double trr = sum_parts(partials, gridDim.x, sh);
-        if (threadIdx.x == 0) {
-            st->rr = trr;
-            st->iters += 1;
-            if (trr <= st->tol2bb) st->need_true = 1;
-            if (!isfinite(trr)) st->done = 2;
+// The same with 8 lanes per row and p formed in the gathers (small 3D grids).
+__global__ __launch_bounds__(kThreads) void mg_spmv_mf_lanes_kernel(MfOp<double> op, OuterVecs v, MgState* st,
+                                                                    double* __restrict__ parts) {
+    constexpr int BS = 3, G = 8;
+    __shared__ double sh[4];
+    double beta;
+    if (!direction_begin(st, v.parity, v.zparts, v.nz, sh, beta)) return;
+    const uint32_t t = blockIdx.x * kThreads + threadIdx.x, row = t / G;
+    const uint32_t q = t % G;
+    double dot = 0.0;
+    if (row < op.nrows) {
+        auto gather = [&](uint32_t o, double(&xv)[BS]) {  // o: bytes of an FP32 row
+            const float* z = (const float*)((const char*)v.z + o);
+            const double* p = (const double*)((const char*)v.p + 2u * o);
+#pragma unroll
+            for (int j = 0; j < BS; ++j) xv[j] = fma(beta, p[j], (double)z[j]);
+        };
+        double out[BS];
+        mf_row_lanes<double>(op, row, q, gather, out);
+        if (q == 0) {
+            double pr[BS];
+            gather(row * (uint32_t)(BS * sizeof(float)), pr);
+#pragma unroll
+            for (int j = 0; j < BS; ++j) {
+                const int64_t d = (int64_t)row * BS + j;
+                if (op.fixed[d]) out[j] = pr[j];
+                v.pnew[d] = pr[j];
+                v.q[d] = out[j];
+                dot = fma(pr[j], out[j], dot);
+            }
         }
     }
+    dot = block_sum_256(dot, sh);
+    if (threadIdx.x == 0) parts[blockIdx.x] = dot;
+}
+
+// x += alpha p, r -= alpha q, per-block r.r, and the next V-cycle's first
+// finest-level step on the new r (one thread per block row); parts: the
+// operator pass's p.q.
+template <int BS>
+__global__ __launch_bounds__(kThreads) void mg_update_kernel(double* __restrict__ x, double* __restrict__ r,
+                                                             const double* __restrict__ p,
+                                                             const double* __restrict__ q, int64_t per_block,
+                                                             FirstStep first, MgState* st, int parity,
+                                                             const double* __restrict__ parts, int np,
+                                                             double* __restrict__ upd) {
+    __shared__ double sh[4];
+    if (st->halt || st->done) return;
+    double pq[1];
+    sum_parts_all<1, kThreads / 64>(parts, np, pq, sh);
+    const double a = st->rz[parity] / pq[0];
+    const bool ok = pq[0] > 0.0 && isfinite(a);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->restart = 0;
+        st->fresh = ok ? 1 : 0;
+        if (!ok) st->done = 2;  // breakdown: the other blocks find it for themselves
+    }
+    if (!ok) return;
+    const int64_t i0 = (int64_t)blockIdx.x * per_block, i1 = min(first.nrows, i0 + per_block);
+    double rr = 0.0;
+#pragma unroll 2
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += kThreads) {
+        double rv[BS];
+#pragma unroll
+        for (int j = 0; j < BS; ++j) {
+            const int64_t d = i * BS + j;
+            x[d] = fma(a, p[d], x[d]);
+            rv[j] = fma(-a, q[d], r[d]);
+            r[d] = rv[j];
+            rr = fma(rv[j], rv[j], rr);
+        }
+        first_step_row<BS>(first, i, rv);
+    }
+    rr = block_sum_256(rr, sh);
+    if (threadIdx.x == 0) upd[blockIdx.x] = rr;
 }
 
 // ---------------------------------------------------------- host ----
@@ -2477,6 +2736,18 @@ unsigned rows_grid(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + kThre
 // rows (a z-slab of the grid), and the neighbour rows it gathers are mostly
 // in its own L2.  Blocks past the last row return.
 unsigned xcd_rows_grid(int64_t n) { return (rows_grid(n) + 7u) / 8u * 8u; }
+
+// 3D rows up to which the matrix-free finest level takes 8 lanes per row
+// (SFEM_MF_LANES overrides it; read when a hierarchy is built or solved
+// with).  us per iteration with one thread / 8 lanes per row on MI355X: 27
+// nodes 65.8 / 45.4, 432 70.8 / 52.8, 1,377 73.2 / 54.5, 3,549 92.3 / 73.6,
+// 15,625 118.0 / 113.9, 18,785 120.2 / 129.3, 40,625 129.3 / 169.4.  In 2D (36
+// products a row) four lanes gain 4 % at 272 nodes and lose 3 % at 11,011.
+constexpr int64_t kLaneRows = 16384;
+int64_t mf_lane_rows(int nd) {
+    const char* e = std::getenv("SFEM_MF_LANES");
+    return nd != 3 ? 0 : e && *e ? std::atoll(e) : kLaneRows;
+}
 
 Grid grid_of(const MgLevel& l) { return Grid{l.n[0], l.n[1], l.n[2]}; }
 
@@ -2706,14 +2977,19 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
         memset_d(ctx, p0a.get(), 0, p0a.bytes());
         memset_d(ctx, p0b.get(), 0, p0b.bytes());
         // a row per thread, blocks mapped XCD-contiguously as in the smoothing step
-        const unsigned gm = xcd_rows_grid(L0.nrows);
+        const bool lanes = L0.nrows <= mf_lane_rows(ND);
+        const unsigned gm = lanes ? rows_grid(L0.nrows * 8) : xcd_rows_grid(L0.nrows);
         const hipStream_t t = side_stream(ctx, sfem_ctx::kSideStreams - 1);
         power_start(0, L0, p0a.get(), p0b.get(), gm, t);
         float* vin = p0a.get();
         float* vout = p0b.get();
         for (int k = 0; k < o.power_iters; ++k) {
-            hipLaunchKernelGGL(pow_mf_kernel<ND>, dim3(gm), dim3(kThreads), 0, t, mf_op32(S, H), vin,
-                               S->binv32.get(), vout, ps, parts[0].get());
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(gm), dim3(kThreads), 0, t, mf_op32(S, H), vin, S->binv32.get(), vout,
+                                   ps, parts[0].get());
+            };
+            if (lanes) go(pow_mf_lanes_kernel);
+            else go(pow_mf_kernel<ND>);
             SFEM_LAUNCH_CHECK();
             std::swap(vin, vout);
         }
@@ -3031,59 +3307,76 @@ struct MgRun {
     hipStream_t s;
     Launch ls;    // the finest level's smoother (sliced)
     bool shared;  // a block per slice
-    const int* done;
+    bool lanes;   // 8 lanes per row (matrix-free)
+    MgState* st;
     bool nt;
+    const double* rout;  // the outer residual, for the last step's r.z
+    double* zparts;
+    const double* upd;   // the update's r.r
+    int nupd;
     std::vector<hipEvent_t>* ev = nullptr;  // non-null: time the finest-level smoothing steps
     size_t ev_next = 0;
     bool time_vc = false;  // time this V-cycle's steps
+    // blocks of a finest-level step: the count of its r.z partials
+    unsigned fine_grid() const {
+        if (H.mf && H.mfma) {
+            const MfTiles T = mf_tiles(H);
+            return (unsigned)((T.tx * T.ty * T.tz + 7) / 8 * 8);
+        }
+        if (H.mf) return lanes ? rows_grid(H.L[0].nrows * 8) : xcd_rows_grid(H.L[0].nrows);
+        return ls.grid;
+    }
+    // mode: 0 a step, 1 the residual, 2 (finest level) the V-cycle's last step
     void step(int l, int mode, const float* v, const float* d_in, float* d_out, float c1, float c2) {
         MgLevel& L = H.L[(size_t)l];
+        const int* halt = &st->halt;
         // timed: the finest-level smoothing steps
-        const bool timed = ev && time_vc && l == 0 && mode == 0 && 2 * ev_next + 1 < ev->size();
+        const bool timed = ev && time_vc && l == 0 && mode != 1 && 2 * ev_next + 1 < ev->size();
         if (timed) SFEM_HIP(hipEventRecord((*ev)[2 * ev_next], s));
-        if (l == 0 && H.mf && H.mfma) {  // the matrix cores (3D)
-            const MfTiles T = mf_tiles(H);
-            const dim3 grid((unsigned)((T.tx * T.ty * T.tz + 7) / 8 * 8));
-            const half4_t* kf = (const half4_t*)H.kfrag.get();
-            const float* bi = (const float*)S->binv32.get();
-            if (mode == 0)
-                hipLaunchKernelGGL((cheb_mf_mfma_kernel<0>), grid, dim3(kThreads), 0, s, mf_op32(S, H), T, kf,
-                                   H.kscale, v, L.r.get(), L.x.get(), d_in, d_out, c1, c2, bi, done);
-            else
-                hipLaunchKernelGGL((cheb_mf_mfma_kernel<1>), grid, dim3(kThreads), 0, s, mf_op32(S, H), T, kf,
-                                   H.kscale, v, L.r.get(), L.x.get(), d_in, d_out, c1, c2, bi, done);
-        } else if (l == 0 && H.mf) {
-            auto go = [&](auto k) {
-                hipLaunchKernelGGL(k, dim3(xcd_rows_grid(L.nrows)), dim3(kThreads), 0, s, mf_op32(S, H), v, L.r.get(),
-                                   L.x.get(), d_in, d_out, c1, c2, (const float*)S->binv32.get(), done);
+        if (l == 0) {
+            const float* bi = H.fp16 ? H.binv0.get() : S->binv32.get();
+            auto go = [&](auto k, auto... op) {
+                hipLaunchKernelGGL(k, dim3(fine_grid()), dim3(kThreads), 0, s, op..., v, L.r.get(), L.x.get(), d_in,
+                                   d_out, c1, c2, bi, rout, zparts, halt);
             };
-            if (mode == 0) go(cheb_mf_kernel<ND, 0>);
-            else go(cheb_mf_kernel<ND, 1>);
-        } else if (l == 0 && H.fp16) {
-            const SellOp<_Float16> op{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), H.h0.get(), S->nslices, S->nfb,
-                                      ls.per_block};
-            auto go = [&](auto k) {
-                hipLaunchKernelGGL(k, dim3(ls.grid), dim3(kThreads), 0, s, op, v, L.r.get(), L.x.get(), d_in, d_out,
-                                   c1, c2, (const float*)H.binv0.get(), done);
+            auto sell = [&](auto tv, auto op) {
+                using TS = decltype(tv);
+                auto pick = [&](auto m) {
+                    constexpr int M = decltype(m)::value;
+                    if (shared) go(cheb_sell_kernel<BS, M, false, true, TS>, op);
+                    else if (nt) go(cheb_sell_kernel<BS, M, true, false, TS>, op);
+                    else go(cheb_sell_kernel<BS, M, false, false, TS>, op);
+                };
+                if (mode == 0) pick(std::integral_constant<int, 0>());
+                else if (mode == 1) pick(std::integral_constant<int, 1>());
+                else pick(std::integral_constant<int, 2>());
             };
-            if (shared) mode == 0 ? go(cheb_sell_kernel<BS, 0, false, true, _Float16>) : go(cheb_sell_kernel<BS, 1, false, true, _Float16>);
-            else if (mode == 0) nt ? go(cheb_sell_kernel<BS, 0, true, false, _Float16>) : go(cheb_sell_kernel<BS, 0, false, false, _Float16>);
-            else nt ? go(cheb_sell_kernel<BS, 1, true, false, _Float16>) : go(cheb_sell_kernel<BS, 1, false, false, _Float16>);
-        } else if (l == 0) {
-            const SellOp<float> op{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), S->sval32.get(), S->nslices, S->nfb,
-                                   ls.per_block};
-            auto go = [&](auto k) {
-                hipLaunchKernelGGL(k, dim3(ls.grid), dim3(kThreads), 0, s, op, v, L.r.get(), L.x.get(), d_in, d_out,
-                                   c1, c2, (const float*)S->binv32.get(), done);
-            };
-            if (shared) mode == 0 ? go(cheb_sell_kernel<BS, 0, false, true, float>) : go(cheb_sell_kernel<BS, 1, false, true, float>);
-            else if (mode == 0) nt ? go(cheb_sell_kernel<BS, 0, true, false, float>) : go(cheb_sell_kernel<BS, 0, false, false, float>);
-            else nt ? go(cheb_sell_kernel<BS, 1, true, false, float>) : go(cheb_sell_kernel<BS, 1, false, false, float>);
+            if (H.mf && H.mfma) {  // the matrix cores (3D)
+                const MfTiles T = mf_tiles(H);
+                const half4_t* kf = (const half4_t*)H.kfrag.get();
+                if (mode == 0) go(cheb_mf_mfma_kernel<0>, mf_op32(S, H), T, kf, H.kscale);
+                else if (mode == 1) go(cheb_mf_mfma_kernel<1>, mf_op32(S, H), T, kf, H.kscale);
+                else go(cheb_mf_mfma_kernel<2>, mf_op32(S, H), T, kf, H.kscale);
+            } else if (H.mf && lanes) {
+                if (mode == 0) go(cheb_mf_lanes_kernel<0>, mf_op32(S, H));
+                else if (mode == 1) go(cheb_mf_lanes_kernel<1>, mf_op32(S, H));
+                else go(cheb_mf_lanes_kernel<2>, mf_op32(S, H));
+            } else if (H.mf) {
+                if (mode == 0) go(cheb_mf_kernel<ND, 0>, mf_op32(S, H));
+                else if (mode == 1) go(cheb_mf_kernel<ND, 1>, mf_op32(S, H));
+                else go(cheb_mf_kernel<ND, 2>, mf_op32(S, H));
+            } else if (H.fp16) {
+                sell(_Float16(0), SellOp<_Float16>{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), H.h0.get(),
+                                                   S->nslices, S->nfb, ls.per_block});
+            } else {
+                sell(0.0f, SellOp<float>{S->sl_ptr.get(), S->sl_w.get(), S->scol.get(), S->sval32.get(), S->nslices,
+                                         S->nfb, ls.per_block});
+            }
         } else {
             const bool grp = L.node_major;
             auto go = [&](auto k, auto op) {
                 hipLaunchKernelGGL(k, dim3(rows_grid(L.nn * (grp ? Lanes<ND>::G : 1))), dim3(kThreads), 0, s, op, v,
-                                   L.r.get(), L.x.get(), d_in, d_out, c1, c2, (const float*)L.binv.get(), done);
+                                   L.r.get(), L.x.get(), d_in, d_out, c1, c2, (const float*)L.binv.get(), halt);
             };
             auto pick = [&](auto op, auto tv) {
                 using TS = decltype(tv);
@@ -3097,23 +3390,18 @@ struct MgRun {
         if (timed) SFEM_HIP(hipEventRecord((*ev)[2 * ev_next++ + 1], s));
     }
 
-    // x_l = V-cycle(b_l); level 0's right-hand side is the outer residual.
-    // Levels below 0 start after the restriction that formed b_l, which also
-    // made their first smoothing step.
-    void vcycle(int l, const double* r_outer) {
+    // x_l = V-cycle(b_l).  The finest level's first step is made by the
+    // kernel that formed the outer residual, those of the levels below by the
+    // restriction that formed b_l.
+    void vcycle(int l) {
         MgLevel& L = H.L[(size_t)l];
+        const int* halt = &st->halt;
         if (l == H.direct) {
             hipLaunchKernelGGL(dense_apply_kernel, dim3((unsigned)((H.nd_dofs + 3) / 4)), dim3(kThreads), 0, s,
                                (const double*)H.dinv.get(), (int)H.nd_dofs, (int)H.ndp, (const float*)L.b.get(),
-                               L.x.get(), done);
+                               L.x.get(), st, upd, nupd);
             SFEM_LAUNCH_CHECK();
             return;
-        }
-        if (l == 0) {
-            const float* binv = H.fp16 ? H.binv0.get() : S->binv32.get();
-            hipLaunchKernelGGL((cheb_first_kernel<BS, double>), dim3(rows_grid(L.nrows)), dim3(kThreads), 0, s, r_outer,
-                               H.scale0, L.nrows, binv, L.c2[0], L.r.get(), L.x.get(), L.da.get(), done);
-            SFEM_LAUNCH_CHECK();
         }
         float* dp = L.da.get();
         float* dn = L.db.get();
@@ -3129,22 +3417,23 @@ struct MgRun {
                                (float)(1.0 / (l == 0 ? H.scale0 : L.scale)), gf,
                                l == 0 ? (const int32_t*)H.row_of_node.get() : nullptr, gc, C.f[0], C.f[1], C.f[2],
                                (const uint8_t*)C.fixed.get(), C.b.get(), (const float*)C.binv.get(), C.c2[0],
-                               (float)C.scale, C.r.get(), C.x.get(), C.da.get(), done);
+                               (float)C.scale, C.r.get(), C.x.get(), C.da.get(), halt);
         };
         if (l + 1 < H.direct) rk(restrict_kernel<ND, true>);
         else rk(restrict_kernel<ND, false>);
         SFEM_LAUNCH_CHECK();
-        vcycle(l + 1, nullptr);
+        vcycle(l + 1);
         hipLaunchKernelGGL(prolong_kernel<ND>, dim3(rows_grid(L.nrows)), dim3(kThreads), 0, s,
                            (const float*)C.x.get(), gc, gf, C.f[0], C.f[1], C.f[2],
                            l == 0 ? (const int32_t*)H.node_of_row.get() : nullptr, L.nrows,
-                           (const uint8_t*)L.fixed.get(), L.x.get(), L.da.get(), done);
+                           (const uint8_t*)L.fixed.get(), L.x.get(), L.da.get(), halt);
         SFEM_LAUNCH_CHECK();
-        step(l, 0, L.da.get(), nullptr, L.db.get(), 0.0f, L.c2[0]);
+        const int last = l == 0 ? 2 : 0;  // the V-cycle's last step also sums r.z
+        step(l, L.degree == 1 ? last : 0, L.da.get(), nullptr, L.db.get(), 0.0f, L.c2[0]);
         dp = L.db.get();
         dn = L.da.get();
         for (int k = 1; k < L.degree; ++k) {
-            step(l, 0, dp, dp, dn, L.c1[k], L.c2[k]);
+            step(l, k + 1 == L.degree ? last : 0, dp, dp, dn, L.c1[k], L.c2[k]);
             std::swap(dp, dn);
         }
     }
@@ -3172,64 +3461,79 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
     const bool shared0 = slice_split(ctx, S->nslices, BS, smooth_op_bytes) > 1;
     const Launch ls = plan_sell(S->nslices, false), lo = plan_sell(S->nslices, shared);
     const Launch lv = plan_vec(n, (unsigned)std::max(8, ctx->n_cu * 4));
-    // p: and a zero row, read for fixed nodes by the matrix-free operator
-    DevBuf<double> r(ctx, (size_t)n), p(ctx, (size_t)n + BS), q(ctx, (size_t)n);
+    const Launch lr = plan_vec(S->nfb, (unsigned)std::max(8, ctx->n_cu * 4));  // a block row per thread
     // FP64 outer operator matrix-free when the hierarchy allows it
     const bool mf_outer = H.mf == 2 && std::is_same<TV, double>::value;
-    const unsigned mf_grid = std::min(xcd_rows_grid(S->nfb), 8192u);
+    const bool lanes = H.mf && S->nfb <= mf_lane_rows(ND);
+    const bool fly = mf_outer ? lanes : shared;  // p formed in the operator's gathers (double buffered)
+    // p: and a zero row, read for fixed nodes by the matrix-free operator
+    DevBuf<double> r(ctx, (size_t)n), p(ctx, (size_t)(n + BS) * (fly ? 2 : 1)), q(ctx, (size_t)n);
+    const unsigned mf_grid = lanes ? rows_grid(S->nfb * 8) : std::min(xcd_rows_grid(S->nfb), 8192u);
     MfOp<double> mf64{};
     if (mf_outer) mf64 = mf_op<double>(S, H, H.kc64.get(), H.es64.get());
     else ensure_sell(ctx, S);  // the outer operator reads the sliced values
-    unsigned tiles = 0;
-    if (H.mfma) {
-        const MfTiles T = mf_tiles(H);
-        tiles = (unsigned)((T.tx * T.ty * T.tz + 7) / 8 * 8);
-    }
-    DevBuf<double> partials(ctx, 2 * (size_t)std::max({ls.grid, lo.grid, lv.grid, mf_grid, 2048u, xcd_rows_grid(S->nfb),
-                                                        tiles}));
+    MgRun<ND, TV> run{ctx, S, H, s, plan_sell(S->nslices, shared0), shared0, lanes, nullptr,
+                      stream_loads(ctx, smooth_op_bytes), r.get(), nullptr, nullptr, (int)lr.grid};
+    // per-block partials: r.z of the V-cycle's last step, p.q, r.r, and the
+    // sums of the residual and norm kernels
+    const unsigned nz = run.fine_grid(), npq = mf_outer ? mf_grid : lo.grid;
+    const unsigned tk_grid = std::min(rows_grid(S->nfb * 32), 2048u);  // 32 lanes per row
+    DevBuf<double> partials(ctx, (size_t)nz + npq + lr.grid + 2 * (size_t)std::max({ls.grid, lv.grid, tk_grid}));
+    double *const zparts = partials.get(), *const qparts = zparts + nz, *const upd = qparts + npq,
+                  *const sums = upd + lr.grid;
     DevBuf<MgState> dst(ctx, 1);
     if (o->x0_zero) memset_d(ctx, S->x.get(), 0, sizeof(double) * S->nf);
     if (padded) pad_gather(ctx, S, S->x.get(), x);
-    memset_d(ctx, p.get(), 0, sizeof(double) * (n + BS));
+    memset_d(ctx, p.get(), 0, p.bytes());
     MgState init{};
     init.best_true = HUGE_VAL;
-    init.need_true = 1;
+    init.need_true = init.halt = 1;
     init.restart = 1;
     if (o->x0_zero) {  // x = 0: the residual is rhs, no operator pass
         SFEM_HIP(hipMemcpyAsync(r.get(), rhs, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-        init.need_true = 0;
+        init.need_true = init.halt = 0;
     }
     h2d(ctx, dst.get(), &init, sizeof(init));
     MgState* st = dst.get();
-    MgRun<ND, TV> run{ctx, S, H, s, plan_sell(S->nslices, shared0), shared0, &st->done,
-                      stream_loads(ctx, smooth_op_bytes)};
-    const float* z = H.L[0].x.get();
+    run.st = st;
+    run.zparts = zparts;
+    run.upd = upd;
+    const MgLevel& L0 = H.L[0];
+    const float* z = L0.x.get();
     Vals<TV> vals = outer_vals<TV>(S);
+    const float* binv0 = H.fp16 ? H.binv0.get() : S->binv32.get();
+    const FirstStep first{binv0, H.scale0, L0.c2[0], L0.r.get(), L0.x.get(), L0.da.get(), S->nfb};
 
     hipEvent_t t0, t1;
     SFEM_HIP(hipEventCreate(&t0));
     SFEM_HIP(hipEventCreate(&t1));
     SFEM_HIP(hipEventRecord(t0, s));
-    hipLaunchKernelGGL(mg_norm_kernel, dim3(lv.grid), dim3(kThreads), 0, s, rhs, n, lv.per_block, st, partials.get(),
-                       o->rtol);
+    hipLaunchKernelGGL(mg_norm_kernel, dim3(lv.grid), dim3(kThreads), 0, s, rhs, n, lv.per_block, st, sums, o->rtol);
     SFEM_LAUNCH_CHECK();
     // FP64 residual of the assembled K: from K's block columns when the
     // finest level is matrix-free (K assembled on the grid, exactly
     // symmetric; the sliced values need not exist), else the sliced values
-    const unsigned tk_grid = std::min(rows_grid(S->nfb * 32), 2048u);  // 32 lanes per row
     auto true_resid = [&] {
         if (H.mf)
             hipLaunchKernelGGL(mg_true_k_kernel<BS>, dim3(tk_grid), dim3(kThreads), 0, s, S->K->bcolptr.get(),
                                S->K->browidx.get(), S->K->bval.get(), H.node_of_row.get(), H.row_of_node.get(),
-                               S->free_of.get(), S->nfb, (const double*)x, rhs, r.get(), st, partials.get());
+                               S->free_of.get(), S->nfb, (const double*)x, rhs, r.get(), first, st, sums);
         else
             hipLaunchKernelGGL(mg_true_kernel<BS>, dim3(ls.grid), dim3(kThreads), 0, s, S->sl_ptr.get(),
                                S->sl_w.get(), S->scol.get(), S->sval64.get(), S->nslices, S->nfb, ls.per_block,
-                               (const double*)x, rhs, r.get(), st, partials.get());
+                               (const double*)x, rhs, r.get(), first, st, sums);
         SFEM_LAUNCH_CHECK();
     };
+    if (o->x0_zero) {
+        hipLaunchKernelGGL((cheb_first_kernel<BS, double>), dim3(rows_grid(S->nfb)), dim3(kThreads), 0, s,
+                           (const double*)r.get(), H.scale0, S->nfb, binv0, first.c2, first.r, first.x, first.d,
+                           (const int*)&st->halt);
+        SFEM_LAUNCH_CHECK();
+    } else {
+        true_resid();
+    }
     MgState host{};
-    int64_t enq = 0, counted = 0, timed = 0;
+    int64_t counted = 0, timed = 0, launched = 0;
     double smooth_ms = 0.0;
     const int chunk_max = std::max(1, std::min(o->check_every, 8));
     // finest-level smoothing steps per V-cycle; with time_kernels those of
@@ -3242,43 +3546,52 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
         for (auto& e : ev) SFEM_HIP(hipEventCreate(&e));
         run.ev = &ev;
     }
-    d2h(ctx, &host, st, sizeof(host));
+    d2h(ctx, &host, st, offsetof(MgState, arrive));
     // iterations enqueued per poll: chunk_max, then the count the observed
     // contraction of r.r predicts to the stop (V-cycles enqueued past the
-    // stop exit at once but still cost their launches)
+    // stop exit at once but still cost their launches).  The FP64 check a
+    // converged recurrence asks for runs at the end of a chunk; until then
+    // the kernels exit.
     int64_t next = chunk_max, seen_iters = 0;
     double seen_rr = host.bb;
-    while (!host.done && enq < o->max_iter) {
-        const int64_t chunk = std::min<int64_t>(next, o->max_iter - enq);
+    OuterVecs ov{p.get(), z, fly ? p.get() + n + BS : p.get(), q.get(), zparts, (int)nz, 0};
+    while (!host.done && host.iters < o->max_iter) {
+        const int64_t chunk = std::min<int64_t>(next, o->max_iter - host.iters);
         run.ev_next = 0;
         for (int64_t k = 0; k < chunk; ++k) {
-            true_resid();
             run.time_vc = k % kTimeEvery == 0;
-            run.vcycle(0, r.get());
-            hipLaunchKernelGGL(mg_rz_kernel, dim3(lv.grid), dim3(kThreads), 0, s, (const double*)r.get(), z, n,
-                               lv.per_block, st, partials.get());
-            SFEM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(mg_p_kernel, dim3(lv.grid), dim3(kThreads), 0, s, p.get(), z, n, lv.per_block,
-                               (const MgState*)st);
-            SFEM_LAUNCH_CHECK();
+            ov.parity = (int)(launched++ & 1);
+            run.vcycle(0);
+            if (!fly) {
+                hipLaunchKernelGGL(mg_p_kernel, dim3(lv.grid), dim3(kThreads), 0, s, ov.pnew, z, n, lv.per_block, st,
+                                   ov.parity, (const double*)zparts, (int)nz);
+                SFEM_LAUNCH_CHECK();
+            }
             auto go = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3(lo.grid), dim3(kThreads), 0, s, S->sl_ptr.get(), S->sl_w.get(),
-                                   S->scol.get(), vals, S->nslices, S->nfb, lo.per_block, (const double*)p.get(),
-                                   q.get(), st, partials.get());
+                                   S->scol.get(), vals, S->nslices, S->nfb, lo.per_block, ov, st, qparts);
             };
-            if (mf_outer) hipLaunchKernelGGL(mg_spmv_mf_kernel<ND>, dim3(mf_grid), dim3(kThreads), 0, s, mf64,
-                                             (const double*)p.get(), q.get(), st, partials.get());
+            if (mf_outer && lanes)
+                hipLaunchKernelGGL(mg_spmv_mf_lanes_kernel, dim3(mf_grid), dim3(kThreads), 0, s, mf64, ov, st,
+                                   qparts);
+            else if (mf_outer)
+                hipLaunchKernelGGL(mg_spmv_mf_kernel<ND>, dim3(mf_grid), dim3(kThreads), 0, s, mf64, ov, st, qparts);
             else if (shared) go(mg_spmv_kernel<BS, TV, false, true>);
             else if (stream_loads(ctx, outer_bytes)) go(mg_spmv_kernel<BS, TV, true, false>);
             else go(mg_spmv_kernel<BS, TV, false, false>);
             SFEM_LAUNCH_CHECK();
-            hipLaunchKernelGGL(mg_update_kernel, dim3(lv.grid), dim3(kThreads), 0, s, x, r.get(),
-                               (const double*)p.get(), (const double*)q.get(), n, lv.per_block, st, partials.get());
+            hipLaunchKernelGGL(mg_update_kernel<BS>, dim3(lr.grid), dim3(kThreads), 0, s, x, r.get(),
+                               (const double*)ov.pnew, (const double*)q.get(), lr.per_block, first, st, ov.parity,
+                               (const double*)qparts, (int)npq, upd);
             SFEM_LAUNCH_CHECK();
+            double* const po = ov.pnew;  // in place: the same array
+            ov.pnew = const_cast<double*>(ov.p);
+            ov.p = po;
         }
+        hipLaunchKernelGGL(mg_check_kernel, dim3(1), dim3(kThreads), 0, s, st, (const double*)upd, (int)lr.grid);
+        SFEM_LAUNCH_CHECK();
         true_resid();  // the check a converged recurrence asked for
-        enq += chunk;
-        d2h(ctx, &host, st, sizeof(host));
+        d2h(ctx, &host, st, offsetof(MgState, arrive));
         if (o->time_kernels) {
             // V-cycles after the stop exit at once; time those of real iterations
             const int64_t real = std::min<int64_t>(chunk, std::max<int64_t>(0, host.iters - counted));
@@ -3305,9 +3618,9 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
     if (!host.done) {  // iteration cap: the true residual of the final iterate
         MgState h2 = host;
         h2.need_true = 1;
-        h2d(ctx, st, &h2, sizeof(h2));
+        h2d(ctx, st, &h2, offsetof(MgState, arrive));
         true_resid();
-        d2h(ctx, &host, st, sizeof(host));
+        d2h(ctx, &host, st, offsetof(MgState, arrive));
         if (host.done != 1) host.done = 0;  // reported as the iteration cap
     }
     if (padded) pad_scatter(ctx, S, x, S->x.get());

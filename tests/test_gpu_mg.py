@@ -580,3 +580,39 @@ def test_direct_level(dims, direct, monkeypatch):
     S.close()
     K.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("lanes", ["0", "100000"])
+@pytest.mark.parametrize("dims", [(2, 1, 1), (3, 3, 1), (7, 3, 3), (8, 8, 8), (13, 6, 5)])
+def test_matrix_free_row_forms(dims, lanes, monkeypatch):
+    # the matrix-free rows with one thread and with 8 lanes each: 8 to 729
+    # rows around the 32 rows of a block, clamped and partially fixed nodes
+    # (their own values), prescribed values, and a warm start (the FP64 check
+    # and the first step on its residual come before the first V-cycle)
+    print(f"[case] matrix-free rows {dims} lanes={lanes}", flush=True)
+    monkeypatch.setenv("SFEM_MF_LANES", lanes)
+    ctx = smearfem.Context(0)
+    m = structured_mesh(dims)
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=14)
+    for fixed in (clamp_x0(m), roller(m)):
+        f = random_face_load(m, 0, 1, fixed, seed=15)
+        q_d = np.where(fixed == 1, 1e-3, 0.0)
+        q_ref = oracle_direct(oracle_K(m, young), fixed, f, q_d)
+        mesh = smearfem.Mesh(ctx, m.n_elem, m.NodeList, m.IEN, m.ndim, "Q1", m.ndim, m.ID, young, 0.3)
+        mesh.set_grid(m.dims)
+        K = mesh.assemble()
+        bc = BoundaryConditions(ctx, K.shape[0], f, fixed, q_d)
+        S = System(K, bc)
+        bc.close()
+        assert S.set_grid()["matrix_free"] == 2
+        st = S.solve("fp64", rtol=1e-12, preconditioner="multigrid")
+        assert st["converged"] and relerr(S.solution(), q_ref) <= ERR
+        st = S.solve("fp64", rtol=1e-12, preconditioner="multigrid", x0_zero=False)
+        assert st["converged"] and st["iterations"] == 0 and relerr(S.solution(), q_ref) <= ERR
+        if S.n_free > 60:
+            st = S.solve("fp64", rtol=1e-12, preconditioner="multigrid", max_iter=2, raise_on_fail=False)
+            assert st["iterations"] == 2 and st["stop_reason"] == 4
+        S.close()
+        K.close()
+        mesh.close()
+    ctx.close()
