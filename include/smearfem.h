@@ -511,8 +511,9 @@ int  sfem_batch_create_specs(sfem_ctx* ctx, int64_t nprob, const sfem_problem_sp
 /* n_total = ndim*N_total; n_padded = dofs of the padded operator; slices of 64 node rows. */
 int  sfem_batch_info(const sfem_batch* b, int64_t* n_total, int64_t* n_padded, int64_t* slices,
                      double* assemble_ms, double* eliminate_ms);
-/* Solve every problem.  item_slices: slices per work item (changes the
- * reduction order, so results are bitwise reproducible per item_slices);
+/* Solve every problem.  item_slices: active 64-row slices per block up to
+ * which a block's wavefronts share each slice (more: a wavefront per slice);
+ * results do not depend on it;
  * blocks_per_cu: persistent grid = blocks_per_cu * CUs (0 = default; capped
  * at residency).  opts->check_every > 0 splits the solve into launches of
  * that many iterations; <= 0 runs it in one launch.  per: nprob entries or

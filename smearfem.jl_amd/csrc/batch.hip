@@ -10,12 +10,12 @@
 // padding rows have zero matrix rows, zero rhs and unit diagonal, so they
 // stay exactly zero through the iteration).
 //
-// The solver keeps one CG state per problem.  A problem's rows are cut into
-// work items of `item_slices` slices; each per-problem dot product is formed
-// from that problem's item partials by one block in a fixed order.  A
-// problem's arithmetic therefore depends only on its own data and on
-// item_slices: it is bitwise the same alone, in this batch, in any other
-// batch, for any grid size and for any split of its iterations over launches.
+// The solver keeps one CG state per problem.  Every per-problem dot product is
+// formed from that problem's slice partials in a fixed order, whichever blocks
+// made them.  A problem's arithmetic therefore depends only on its own data:
+// it is bitwise the same alone, in this batch, in any other batch, for any
+// grid size, for any item_slices and for any split of its iterations over
+// launches.
 //
 // Reference: the per-problem maths is smearFEM's assemble_system
 // (src/fem.jl:135-256) and the example's elimination and solve
@@ -260,43 +260,108 @@ __global__ void fold_all_kernel(double* __restrict__ x64, float* __restrict__ xs
 }
 
 // ----------------------------------------------------- persistent PCG ---
-// Block-uniform OR of pred over the table's problems.
-template <typename F>
-__device__ __forceinline__ bool block_any(int nprob, F pred) {
-    __shared__ int flag;
-    if (threadIdx.x == 0) flag = 0;
-    __syncthreads();
-    int mine = 0;
-    for (int i = threadIdx.x; i < nprob; i += kThreads) mine |= pred(i) ? 1 : 0;
-    if (mine) atomicOr(&flag, 1);
-    __syncthreads();
-    const bool r = flag != 0;
-    __syncthreads();
-    return r;
+// One launch iterates every problem of a table; between the passes of an
+// iteration the grid meets at a barrier, and a problem's scalars are formed by
+// the blocks that need them.  Per iteration:
+//
+//   A  per run of slices of one problem: the sums the last pass left (r.z, r.r
+//      and p.q of an update, or the sums of an FP64 residual) give beta, the
+//      stopping tests and what comes next; then either the FP64 residual of
+//      the run's rows, if it is due, or q = K p with p = zcoef z + beta p
+//      formed in the gathers (p has two buffers), and the slice partials of p.q
+//   U  alpha from the partials of p.q; x += alpha p; r -= alpha q;
+//      z = M^-1 r; slice partials of r.z and r.r
+//
+// The block that holds a problem's first slice writes its new state to the
+// other of two state slots, so no block reads what another one writes.  What
+// bounds a small table is the chain barrier - partials - operator - barrier,
+// not bytes: the form before this one had four barriers an iteration (six
+// with a residual due), a wavefront per slice and skipped finished problems
+// item by item.  24 Hex8 problems of 180 to 20,000 nodes, mixed precision,
+// 1,229 iterations: 95.5 ms before, 48.3 now; 256 problems up to 31,700
+// nodes, split precision, 808 iterations: 314 ms before, 259 now.
+//
+// A table with more than item_slices active slices per block is bound by HBM
+// instead: there p is formed by a pass of its own (a third barrier; the
+// gathers then read one vector, not two) and each wavefront takes a whole
+// slice with non-temporal operator loads, the residuals that are due spread
+// over all blocks (in one block's run they kept the rest waiting: 399 ms).
+// Both forms add the same numbers in the same order, so the active problems
+// may move from one to the other as others finish.  The line at 8 slices a
+// block, 24 / 256 problems as above: always the second form 56.5 / 260 ms, at
+// 8 slices 48.3 / 259, at 64 48.3 / 338.
+
+enum TableFlags : int32_t { kFlagDone = 1, kFlagResid = 2, kFlagBuf = 4 };  // what a pass needs of a state
+
+constexpr int kMaxGroups = 2048;  // problems, or groups of them, whose activity a block tracks
+
+// The slices still iterated, in table order: groups of `gs` problems, their
+// slice counts (0 once all problems of the group are done) and the prefix sums.
+struct ActiveSet {
+    int pre[kMaxGroups + 1];
+    int w[kMaxGroups];
+};
+
+// Descriptors do not change during a launch: read as constants, so that what
+// they hold (the same in every lane) stays in scalar registers.
+using DescPtr = const ProbDesc __attribute__((address_space(4)))*;
+
+// A value that is the same in every lane of the wavefront, in scalar registers.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uniform(double v) {
+    const int2 u = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(double, make_int2(uniform(u.x), uniform(u.y)));
 }
 
-// Sum of partial slot k over items [i0, i1), fixed order for a 256-thread block.
-__device__ __forceinline__ double items_sum(const double* part, int stride, int k, int i0, int i1, double* sh) {
-    double s = 0.0;
-    for (int i = i0 + threadIdx.x; i < i1; i += kThreads) s += glb(part)[(int64_t)stride * i + k];
-    return block_sum_256(s, sh);
+// Prefix sums of set.w; returns the total.  Every thread of the block calls.
+__device__ __forceinline__ int active_prefix(ActiveSet& set, int ng) {
+    constexpr int PER = kMaxGroups / kThreads;
+    __shared__ int tot[kThreads / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int g = threadIdx.x * PER + i;
+        s += g < ng ? set.w[g] : 0;
+    }
+    int inc = s;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += v;
+    }
+    if (lane == 63) tot[wv] = inc;
+    __syncthreads();
+    int base = inc - s;
+    for (int i = 0; i < wv; ++i) base += tot[i];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int g = threadIdx.x * PER + i;
+        if (g < ng) {
+            set.pre[g] = base;
+            base += set.w[g];
+            if (g == ng - 1) set.pre[ng] = base;
+        }
+    }
+    __syncthreads();
+    return uniform(set.pre[ng]);
 }
 
 // The operator values of a descriptor as the launch's value source.
 template <typename TV>
-__device__ __forceinline__ Vals<TV> desc_vals(const ProbDesc& D) {
-    if constexpr (std::is_same<TV, SplitVal>::value) return Vals<SplitVal>{(const float*)D.sval, D.sval16};
-    else return Vals<TV>{(const TV*)D.sval};
+__device__ __forceinline__ Vals<TV> desc_vals(DescPtr D) {
+    if constexpr (std::is_same<TV, SplitVal>::value) return Vals<SplitVal>{(const float*)D->sval, D->sval16};
+    else return Vals<TV>{(const TV*)D->sval};
 }
 
 // z = preconditioner(r) for the BS dofs of node row `row`
 template <int BS, typename T>
-__device__ __forceinline__ void apply_pc(const ProbDesc& D, int64_t row, const T (&rv)[BS], T (&zv)[BS]) {
-    if (D.block_pc) {
-        const SFEM_GLOBAL T* binv = glb((const T*)D.binv);
+__device__ __forceinline__ void apply_pc(DescPtr D, int64_t row, const T (&rv)[BS], T (&zv)[BS]) {
+    if (D->block_pc) {
+        const SFEM_GLOBAL T* binv = glb((const T*)D->binv);
         T m[BS * BS];
 #pragma unroll
-        for (int v = 0; v < BS * BS; ++v) m[v] = binv[v * D.binv_stride + row];
+        for (int v = 0; v < BS * BS; ++v) m[v] = binv[v * D->binv_stride + row];
 #pragma unroll
         for (int j = 0; j < BS; ++j) {
             T acc = 0;
@@ -305,79 +370,246 @@ __device__ __forceinline__ void apply_pc(const ProbDesc& D, int64_t row, const T
             zv[j] = acc;
         }
     } else {
-        const SFEM_GLOBAL T* dinv = glb((const T*)D.dinv);
+        const SFEM_GLOBAL T* dinv = glb((const T*)D->dinv);
 #pragma unroll
         for (int j = 0; j < BS; ++j) zv[j] = dinv[row * BS + j] * rv[j];
     }
 }
 
-// Update phase of one work item: x += al p, r -= al q, z = M^-1 r, one node
-// per thread; returns the thread's r.z and r.r.
+// Update of one node row: x += al p, r -= al q, z = M^-1 r; returns its r.z
+// and r.r.
 template <int BS, typename T, bool FOLD>
-__device__ __forceinline__ void update_item(const ProbDesc& D, const WorkItem& I, T al, bool fold, double& rz,
-                                            double& rr) {
-    SFEM_GLOBAL double* x64 = glb(D.x64);
-    SFEM_GLOBAL T* xs = glb((T*)D.xs);
-    SFEM_GLOBAL T* r = glb((T*)D.r);
-    SFEM_GLOBAL T* z = glb((T*)D.z);
-    const SFEM_GLOBAL T* p = glb((const T*)D.p);
-    const SFEM_GLOBAL T* q = glb((const T*)D.q);
-    for (int64_t n = I.slice0 * 64 + threadIdx.x; n < I.slice1 * 64; n += kThreads) {
-        T pv[BS], qv[BS], rv[BS], zv[BS];
+__device__ __forceinline__ void update_row(DescPtr D, int64_t n, const T* p_, T al, bool fold, double& rz,
+                                           double& rr) {
+    SFEM_GLOBAL double* x64 = glb(D->x64);
+    SFEM_GLOBAL T* xs = glb((T*)D->xs);
+    SFEM_GLOBAL T* r = glb((T*)D->r);
+    SFEM_GLOBAL T* z = glb((T*)D->z);
+    const SFEM_GLOBAL T* p = glb(p_);
+    const SFEM_GLOBAL T* q = glb((const T*)D->q);
+    T pv[BS], qv[BS], rv[BS], zv[BS];
 #pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            pv[j] = p[n * BS + j];
-            qv[j] = q[n * BS + j];
-            rv[j] = r[n * BS + j];
-        }
+    for (int j = 0; j < BS; ++j) {
+        pv[j] = p[n * BS + j];
+        qv[j] = q[n * BS + j];
+        rv[j] = r[n * BS + j];
+    }
 #pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            const int64_t i = n * BS + j;
-            if constexpr (FOLD) {
-                T xi = xs[i];
-                if (fold) {
-                    x64[i] += (double)xi;
-                    xi = 0;
-                }
-                xs[i] = fmaT<T>(al, pv[j], xi);
-            } else {
-                x64[i] = fma((double)al, (double)pv[j], x64[i]);
+    for (int j = 0; j < BS; ++j) {
+        const int64_t i = n * BS + j;
+        if constexpr (FOLD) {
+            T xi = xs[i];
+            if (fold) {
+                x64[i] += (double)xi;
+                xi = 0;
             }
-            rv[j] = fmaT<T>(-al, qv[j], rv[j]);
-            r[i] = rv[j];
-            rr += (double)rv[j] * (double)rv[j];
+            xs[i] = fmaT<T>(al, pv[j], xi);
+        } else {
+            x64[i] = fma((double)al, (double)pv[j], x64[i]);
         }
-        apply_pc<BS, T>(D, n, rv, zv);
+        rv[j] = fmaT<T>(-al, qv[j], rv[j]);
+        r[i] = rv[j];
+        rr += (double)rv[j] * (double)rv[j];
+    }
+    apply_pc<BS, T>(D, n, rv, zv);
 #pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            z[n * BS + j] = zv[j];
-            rz += (double)rv[j] * (double)zv[j];
-        }
+    for (int j = 0; j < BS; ++j) {
+        z[n * BS + j] = zv[j];
+        rz += (double)rv[j] * (double)zv[j];
     }
 }
 
-// FP64 residual of one work item: r = rhs - K x, z = M^-1 r; accumulates
-// |r|^2, r.z, r.p and the rounding-floor scale.
-template <int BS, typename T, bool FOLD>
-__device__ __forceinline__ void resid_item(const ProbDesc& D, const WorkItem& I, int w, int lane, double& rr,
-                                           double& rz, double& rp, double& ff) {
-    const SFEM_GLOBAL double* x64 = glb((const double*)D.x64);
-    const SFEM_GLOBAL T* xs = glb((const T*)D.xs);
-    const SFEM_GLOBAL T* p = glb((const T*)D.p);
-    const SFEM_GLOBAL double* rhs = glb(D.rhs);
-    SFEM_GLOBAL T* r = glb((T*)D.r);
-    SFEM_GLOBAL T* z = glb((T*)D.z);
-    auto gx = [&](int64_t c) { return FOLD ? x64[c] + (double)xs[c] : x64[c]; };
-    for (int64_t sl = I.slice0 + w; sl < I.slice1; sl += kThreads / 64) {
+// The scalars of a problem from the sums its last pass left: `v` holds p.q,
+// r.z, r.r of an update, r.r, r.z, r.p and the rounding-floor scale of an
+// FP64 residual, or |rhs|^2 on the first visit.
+template <bool FOLD>
+__device__ void consume(ProbState& S, const double* v) {
+    if (S.init_pending) {
+        S.bb = v[0];
+        S.tol2bb = S.rtol * S.rtol * S.bb;
+        S.delta2 = S.delta * S.delta;
+        S.maxrr = S.bb;
+        S.rz = 0.0;
+        S.rz_prev = HUGE_VAL;
+        S.beta = 0.0;
+        S.zcoef = 1.0;
+        S.best_rr = HUGE_VAL;
+        S.best_true = HUGE_VAL;
+        S.rr_true = S.bb;
+        S.need_update = 1;
+        S.capped = S.max_iter <= 0 ? 1 : 0;
+        S.init_pending = 0;
+    } else if (S.pending == kUpdateSums) {
+        const double pq = v[0], trz = v[1], trr = v[2];
+        S.rz_prev = S.rz;
+        S.rz = trz;
+        S.beta = trz / S.rz_prev;
+        S.iters += 1;
+        S.fold_pending = 0;
+        S.zcoef = 1.0;
+        S.rr_rec = trr;
+        const int64_t since = S.iters - S.last_upd;
+        if (trr <= S.tol2bb || trr < S.delta2 * S.maxrr || since >= (S.best_true_it > 256 ? S.best_true_it : 256))
+            S.need_update = 1;
+        // backstop for a recurrence that stops decreasing: no 2x drop of |r|
+        // within max(10000, 4x the iterations it took to reach the best)
+        if (trr < 0.25 * S.best_rr) {
+            S.best_rr = trr;
+            S.best_it = S.iters;
+        } else if (S.iters - S.best_it > (4 * S.best_it > 10000 ? 4 * S.best_it : 10000)) {
+            S.done = 3;
+        }
+        if (S.iters >= S.max_iter && !S.done) {  // final FP64 residual, then stop
+            S.need_update = 1;
+            S.capped = 1;
+        }
+        if (!(pq > 0.0) || !isfinite(trr)) S.done = 2;
+    } else if (S.pending == kResidSums) {
+        const double trr = v[0], trz = v[1], trp = v[2];
+        // 16x the attainable |r|^2, (eps * || |rhs| + |K||x| ||)^2
+        const double floor_rr = 16.0 * kEps64 * kEps64 * v[3];
+        S.rr_true = trr;
+        S.floor_rr = floor_rr;
+        S.updates += 1;
+        S.last_upd = S.iters;
+        S.need_update = 0;
+        S.fold_pending = FOLD ? 1 : 0;
+        if (trr <= S.tol2bb) {
+            S.done = 1;
+        } else if (S.capped) {
+            S.done = 4;
+        } else {
+            S.beta = trz / S.rz_prev;
+            S.zcoef = 1.0 - S.beta * (trp / trz);
+            S.rz = trz;
+            S.maxrr = trr;
+            // attainable floor: no 10% gain on the best true residual
+            // within 4x of the rounding floor, or twice in a row while
+            // the recurrence ran 5x below it
+            const bool gap = S.iters > 0 && 25.0 * S.rr_rec < trr;
+            if (trr <= 0.81 * S.best_true) {
+                S.stall = 0;
+                S.best_true_it = S.iters;
+            } else if (trr <= floor_rr) {
+                S.stall += 2;
+            } else if (gap) {
+                S.stall += 1;
+            }
+            if (S.stall >= 2) S.done = 3;
+        }
+        if (trr < S.best_true) S.best_true = trr;
+        if (!isfinite(trr)) S.done = 2;
+    }
+    S.pending = kNoSums;
+}
+
+// This lane's block row of slice `sl` by one wavefront, with the sums of a
+// slice shared by four (SharedSlice, sell_combine): one accumulator per
+// residue of the block column modulo 4, added in ascending order.  Per pair of
+// block columns the column ids and all value loads are issued before any of
+// them is used, then the gathers, then the arithmetic; scheduling barriers
+// keep the compiler from interleaving loads with their uses, which would leave
+// one load in flight per wavefront.
+template <int BS, typename TV, typename ACC, bool NT, typename Gather>
+__device__ __forceinline__ void sell_row_quads(const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w,
+                                               const int32_t* __restrict__ scol, Vals<TV> vals, int64_t sl, int lane,
+                                               Gather gx, ACC out[BS]) {
+    constexpr int B2 = BS * BS;
+    using Raw = typename Vals<TV>::Raw;
+    const int64_t base = glb(sl_ptr)[sl];
+    const int w = glb(sl_w)[sl];
+    ACC acc[4][BS];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int j = 0; j < BS; ++j) acc[h][j] = 0;
+    auto add = [&](const Raw (&rv)[B2], const ACC (&xv)[BS], ACC (&s)[BS]) {
+#pragma unroll
+        for (int j = 0; j < BS; ++j)
+#pragma unroll
+            for (int i = 0; i < BS; ++i) s[j] = fmaT<ACC>((ACC)vals.decode(rv[j * BS + i]), xv[i], s[j]);
+    };
+    auto pair = [&](int k, ACC (&sa)[BS], ACC (&sb)[BS]) {
+        const int64_t s0 = base + (int64_t)k * 64, s1 = s0 + 64;
+        const int64_t c0 = ld_stream<NT>(scol + s0 + lane), c1 = ld_stream<NT>(scol + s1 + lane);
+        Raw r0[B2], r1[B2];
+#pragma unroll
+        for (int m = 0; m < B2; ++m) r0[m] = vals.template raw<NT>(s0 * B2 + lane + m * 64);
+#pragma unroll
+        for (int m = 0; m < B2; ++m) r1[m] = vals.template raw<NT>(s1 * B2 + lane + m * 64);
+        __builtin_amdgcn_sched_barrier(0);
+        ACC x0[BS], x1[BS];
+        gx(c0, x0);
+        gx(c1, x1);
+        __builtin_amdgcn_sched_barrier(0);
+        add(r0, x0, sa);
+        add(r1, x1, sb);
+    };
+    auto single = [&](int k, ACC (&s)[BS]) {
+        const int64_t s0 = base + (int64_t)k * 64;
+        const int64_t c0 = ld_stream<NT>(scol + s0 + lane);
+        Raw r0[B2];
+#pragma unroll
+        for (int m = 0; m < B2; ++m) r0[m] = vals.template raw<NT>(s0 * B2 + lane + m * 64);
+        ACC x0[BS];
+        gx(c0, x0);
+        add(r0, x0, s);
+    };
+    int k = 0;
+    for (; k + 4 <= w; k += 4) {
+        pair(k, acc[0], acc[1]);
+        pair(k + 2, acc[2], acc[3]);
+    }
+    if (k + 2 <= w) {
+        pair(k, acc[0], acc[1]);
+        if (k + 3 <= w) single(k + 2, acc[2]);
+    } else if (k < w) {
+        single(k, acc[0]);
+    }
+#pragma unroll
+    for (int j = 0; j < BS; ++j) out[j] = ((acc[0][j] + acc[1][j]) + acc[2][j]) + acc[3][j];
+}
+
+// FP64 residual of one slice: r = rhs - K x, z = M^-1 r; slice partials of
+// |r|^2, r.z, r.p and the rounding-floor scale (stride `ps`).  SHARED: by the
+// block, each wavefront a quarter of the block columns; otherwise by one
+// wavefront, the quarters one after the other and added in the same order.
+template <int BS, typename T, bool FOLD, bool SHARED>
+__device__ __forceinline__ void resid_slice(DescPtr D, int64_t s, const T* p_, double* part, int64_t ps,
+                                            double (*buf)[6][64]) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const SFEM_GLOBAL double* x64 = glb((const double*)D->x64);
+    const SFEM_GLOBAL T* xs = glb((const T*)D->xs);
+    const SFEM_GLOBAL T* p = glb(p_);
+    const SFEM_GLOBAL double* rhs = glb(D->rhs);
+    SFEM_GLOBAL T* r = glb((T*)D->r);
+    SFEM_GLOBAL T* z = glb((T*)D->z);
+    auto gx = [&](int64_t c, double (&x)[BS]) {
+#pragma unroll
+        for (int i = 0; i < BS; ++i) x[i] = FOLD ? x64[c * BS + i] + (double)xs[c * BS + i] : x64[c * BS + i];
+    };
+    const int64_t sl = D->slice0 + s;
+    double v[2 * BS] = {};
+#pragma unroll 1
+    for (int h = 0; h < (SHARED ? 1 : 4); ++h) {
         double out[BS], aout[BS];
-        sell_row_abs<BS>(D.sl_ptr, D.sl_w, D.scol, D.sval64, sl, lane, gx, out, aout);
+        sell_row_abs_part<BS, 4>(D->sl_ptr, D->sl_w, D->scol, D->sval64, sl, lane, SHARED ? wv : h, gx, out, aout);
+#pragma unroll
+        for (int j = 0; j < BS; ++j) {
+            v[j] = h ? v[j] + out[j] : out[j];
+            v[BS + j] = h ? v[BS + j] + aout[j] : aout[j];
+        }
+    }
+    if constexpr (SHARED) sell_combine<2 * BS, 4>(v, reinterpret_cast<double (*)[2 * BS][64]>(buf));
+    if (!SHARED || wv == 0) {
         const int64_t row = sl * 64 + lane;
+        double rr = 0.0, rz = 0.0, rp = 0.0, ff = 0.0;
         T rt[BS], zt[BS];
 #pragma unroll
         for (int j = 0; j < BS; ++j) {
             const int64_t d = row * BS + j;
-            const double res = rhs[d] - out[j];
-            const double sc = fabs(rhs[d]) + aout[j];
+            const double res = rhs[d] - v[j];
+            const double sc = fabs(rhs[d]) + v[BS + j];
             ff += sc * sc;
             rt[j] = (T)res;
             r[d] = rt[j];
@@ -390,221 +622,433 @@ __device__ __forceinline__ void resid_item(const ProbDesc& D, const WorkItem& I,
             z[row * BS + j] = zt[j];
             rz += (double)rt[j] * (double)zt[j];
         }
+        const double b0 = wave_sum(rr), b1 = wave_sum(rz), b2 = wave_sum(rp), b3 = wave_sum(ff);
+        if (lane == 0) {
+            const int64_t t = D->t0 + s;
+            glb(part)[t] = b0;
+            glb(part)[ps + t] = b1;
+            glb(part)[2 * ps + t] = b2;
+            glb(part)[3 * ps + t] = b3;
+        }
+    }
+    if constexpr (SHARED) __syncthreads();
+}
+
+// q = K p of slices [s0, s1), each shared by the block, and the slice
+// partials of p.q.  FLY: p = zc z + beta pold, written to pnew; otherwise
+// pold is p.  `sl` holds the first slice's early loads.
+template <int BS, typename TV, typename T, bool FLY>
+__device__ __forceinline__ void shared_run(SharedSlice<BS, TV, !FLY>& sl, DescPtr D, int64_t s0, int64_t s1,
+                                           T beta, T zc, const T* pold_, T* pnew_, double* part,
+                                           double (*buf)[6][64]) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const SFEM_GLOBAL T* z = glb((const T*)D->z);
+    const SFEM_GLOBAL T* pold = glb(pold_);
+    SFEM_GLOBAL T* pnew = glb(pnew_);
+    SFEM_GLOBAL T* q = glb((T*)D->q);
+    auto gx = [&](int64_t c, T (&x)[BS]) {
+#pragma unroll
+        for (int i = 0; i < BS; ++i)
+            x[i] = FLY ? fmaT<T>(beta, pold[c * BS + i], zc * z[c * BS + i]) : pold[c * BS + i];
+    };
+    for (int64_t s = s0; s < s1; ++s) {
+        const int64_t row = (D->slice0 + s) * 64 + lane;
+        T own[BS] = {};
+        if (wv == 0) gx(row, own);
+        T acc[BS] = {};
+        sl.apply(gx, acc);
+        if (s + 1 < s1) sl.load(D->sl_ptr, D->sl_w, D->slice0 + s + 1);
+        sell_combine<BS, 4>(acc, reinterpret_cast<T (*)[BS][64]>(buf));
+        if (wv == 0) {
+            double dot = 0.0;
+#pragma unroll
+            for (int j = 0; j < BS; ++j) {
+                if (FLY) pnew[row * BS + j] = own[j];
+                q[row * BS + j] = acc[j];
+                dot += (double)own[j] * (double)acc[j];
+            }
+            dot = wave_sum(dot);
+            if (lane == 0) glb(part)[D->t0 + s] = dot;
+        }
+        __syncthreads();
     }
 }
 
+// A run of slices of one problem inside a block's part of the active slices.
+struct RunCursor {
+    int g, pos, left;  // group, slices of it passed, slices of the part left
+    int prob, off;     // problem of the group reached, slices of it passed
+};
+
 template <typename TV, typename T, bool FOLD>
-__global__ __launch_bounds__(kThreads) void table_pcg_kernel(TableLaunch a) {
+__global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
     GridBarrier grid{a.bar_ws, a.bar_timeout, 0u, false};
     if (!grid.start(a.bar_grouped != 0)) return;
-    __shared__ double sh[8];
-    const int G = gridDim.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const ProbDesc* probs = a.probs;
+    __shared__ ActiveSet set;
+    __shared__ ProbState S;  // the state of the problem at hand
+    __shared__ double sh[16];
+    __shared__ double buf[kThreads / 64][6][64];
+    const int G = gridDim.x, w = uniform((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const DescPtr probs = (DescPtr)a.probs;
+    DescPtr D = probs;
+    const int64_t ps = a.nslices;
+    double* const partu = a.part + 8 * ps;  // r.z, r.r of the update
+    const int gs = (a.nprob + kMaxGroups - 1) / kMaxGroups, ng = (a.nprob + gs - 1) / gs;
 
-    // ---- I: first launch of a problem: |rhs|^2 and the initial state ----
-    if (block_any(a.nprob, [&](int i) { return probs[i].st->init_pending != 0; })) {
-        for (int it = blockIdx.x; it < a.nitems; it += G) {
-            const WorkItem I = a.items[it];
-            const ProbDesc& D = probs[I.prob];
-            if (!D.st->init_pending) continue;
-            double s = 0.0;
-            const SFEM_GLOBAL double* rhs = glb(D.rhs);
-            for (int64_t i = I.slice0 * 64 * D.bs + threadIdx.x; i < I.slice1 * 64 * D.bs; i += kThreads)
-                s = fma(rhs[i], rhs[i], s);
-            const double b = block_sum_256(s, sh);
-            if (threadIdx.x == 0) glb(a.part)[4 * (int64_t)it + 3] = b;
+    // ---- the active problems ----
+    int init = 0;
+    for (int g = threadIdx.x; g < ng; g += kThreads) {
+        int n = 0;
+        bool any = false;
+        for (int p = g * gs; p < min(a.nprob, (g + 1) * gs); ++p) {
+            ProbState* st = probs[p].st;
+            const bool open = !st->done && probs[p].nslices > 0;
+            n += probs[p].nslices;
+            any |= open;
+            init |= open && st->init_pending ? 1 : 0;
         }
-        if (!grid.sync()) return;
-        for (int pr = blockIdx.x; pr < a.nprob; pr += G) {
-            ProbState* st = probs[pr].st;
-            if (!st->init_pending) continue;
-            const double bb = items_sum(a.part, 4, 3, probs[pr].item0, probs[pr].item1, sh);
-            if (threadIdx.x == 0) {
-                ProbState S = *st;
-                S.bb = bb;
-                S.tol2bb = S.rtol * S.rtol * bb;
-                S.delta2 = S.delta * S.delta;
-                S.maxrr = bb;
-                S.rz = 0.0;
-                S.rz_prev = HUGE_VAL;
-                S.beta = 0.0;
-                S.zcoef = 1.0;
-                S.best_rr = HUGE_VAL;
-                S.best_true = HUGE_VAL;
-                S.rr_true = bb;
-                S.need_update = 1;
-                S.capped = S.max_iter <= 0 ? 1 : 0;
-                S.init_pending = 0;
-                *st = S;
+        set.w[g] = any ? n : 0;
+    }
+    init = __syncthreads_or(init);
+
+    // this block's part of the active slices; consecutive parts share an XCD
+    int total = 0, first = 0, count = 0, g0 = 0;
+    auto cut = [&] {
+        total = active_prefix(set, ng);
+        const int64_t lb = logical_block();
+        first = (int)(lb * total / G);
+        count = (int)((lb + 1) * total / G) - first;
+        int lo = 0, hi = ng;  // the last group whose prefix is <= first
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) / 2;
+            if (uniform(set.pre[mid]) <= first) lo = mid;
+            else hi = mid;
+        }
+        g0 = lo;
+    };
+    cut();
+    auto runs = [&] {
+        const int off = first - uniform(set.pre[g0]);
+        return RunCursor{g0, off, count, g0 * gs, off};
+    };
+    auto next = [&](RunCursor& c, int& p, int& s0, int& s1) {
+        while (c.left > 0) {
+            const int gw = uniform(set.w[c.g]);
+            if (c.pos >= gw) {  // next group that has slices
+                ++c.g;
+                c.pos = c.off = 0;
+                c.prob = c.g * gs;
+                continue;
+            }
+            const int ns = gs == 1 ? gw : probs[c.prob].nslices;
+            if (c.off >= ns) {
+                c.off -= ns;
+                ++c.prob;
+                continue;
+            }
+            const int len = min(ns - c.off, c.left);
+            p = c.prob;
+            s0 = c.off;
+            s1 = c.off + len;
+            c.pos += len;
+            c.off += len;
+            c.left -= len;
+            return true;
+        }
+        return false;
+    };
+
+    // ---- the problem at hand: descriptor and state (slot i & 1), the
+    // state kept in LDS while a block stays with one problem ----
+    int have = -1;
+    int64_t have_slot = -1;
+    auto copy_words = [&](void* dst, const void* src, int words) {
+        for (int i = threadIdx.x; i < words; i += kThreads) ((uint32_t*)dst)[i] = glb((const uint32_t*)src)[i];
+    };
+    auto take_desc = [&](int p) {
+        if (have != p) have_slot = -1;
+        have = p;
+        D = probs + p;
+    };
+    auto take_state = [&](int p, int64_t slot) {
+        if (have_slot == slot) return;
+        __syncthreads();
+        copy_words(&S, (slot & 1) ? a.alt + p : D->st, sizeof(ProbState) / 4);
+        __syncthreads();
+        have_slot = slot;
+    };
+    // pass A of iteration k reaches a run: state, sums, scalars; the run with
+    // the problem's first slice records the new state
+    auto advance = [&](int p, int s0, int64_t k, bool fly) {
+        take_state(p, k);
+        const double* pa = a.part + ((k + 1) & 1) * 4 * ps + D->t0;
+        const double* pu = partu + D->t0;
+        const int ns = D->nslices;
+        if (!S.done && (S.init_pending || S.pending != kNoSums)) {
+            double v[4] = {};
+            if (S.init_pending) {
+                for (int i = threadIdx.x; i < ns; i += kThreads) v[0] += glb(pa)[i];
+            } else if (S.pending == kUpdateSums) {
+                for (int i = threadIdx.x; i < ns; i += kThreads) {
+                    v[0] += glb(pa)[i];
+                    v[1] += glb(pu)[i];
+                    v[2] += glb(pu)[ps + i];
+                }
+            } else {
+                for (int i = threadIdx.x; i < ns; i += kThreads)
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) v[m] += glb(pa)[m * ps + i];
+            }
+#pragma unroll
+            for (int m = 0; m < 4; ++m) v[m] = wave_sum(v[m]);
+            if (lane == 0)
+#pragma unroll
+                for (int m = 0; m < 4; ++m) sh[w * 4 + m] = v[m];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0 && !S.done) {
+            if (S.init_pending || S.pending != kNoSums) {
+                double v[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) v[m] = (sh[m] + sh[4 + m]) + (sh[8 + m] + sh[12 + m]);
+                consume<FOLD>(S, v);
+            }
+            if (!S.done) {
+                S.pending = S.need_update ? kResidSums : kUpdateSums;
+                if (!S.need_update && fly) S.pbuf ^= 1;
+            }
+        }
+        __syncthreads();
+        have_slot = k + 1;
+        if (s0 == 0) {
+            uint32_t* dst = (uint32_t*)(((k + 1) & 1) ? a.alt + p : D->st);
+            for (int i = threadIdx.x; i < (int)(sizeof(ProbState) / 4); i += kThreads)
+                glb(dst)[i] = ((const uint32_t*)&S)[i];
+            if (threadIdx.x == 0)
+                glb(a.flags)[((k + 1) & 1) * a.nprob + p] =
+                    (S.done ? kFlagDone : 0) | (S.need_update ? kFlagResid : 0) | (S.pbuf ? kFlagBuf : 0);
+        }
+    };
+
+    // ---- first launch of a problem: slice partials of |rhs|^2 ----
+    if (init) {
+        RunCursor c = runs();
+        for (int p, s0, s1; next(c, p, s0, s1);) {
+            take_desc(p);
+            take_state(p, 0);
+            if (!S.init_pending) continue;
+            const SFEM_GLOBAL double* rhs = glb(D->rhs);
+            const int n = 64 * D->bs;
+            for (int64_t s = s0 + w; s < s1; s += kThreads / 64) {
+                double v = 0.0;
+                for (int i = lane; i < n; i += 64) {
+                    const double b = rhs[(D->slice0 + s) * n + i];
+                    v = fma(b, b, v);
+                }
+                v = wave_sum(v);
+                if (lane == 0) glb(a.part)[4 * ps + D->t0 + s] = v;
             }
         }
         if (!grid.sync()) return;
     }
 
-    for (int64_t k = 0; k < a.iters; ++k) {
-        // ---- R: FP64 residual replacement for the problems that are due ----
-        if (block_any(a.nprob, [&](int i) { return probs[i].st->need_update && !probs[i].st->done; })) {
-            for (int it = blockIdx.x; it < a.nitems; it += G) {
-                const WorkItem I = a.items[it];
-                const ProbDesc& D = probs[I.prob];
-                if (!D.st->need_update || D.st->done) continue;
-                double rr = 0.0, rz = 0.0, rp = 0.0, ff = 0.0;
-                if (D.bs == 3) resid_item<3, T, FOLD>(D, I, w, lane, rr, rz, rp, ff);
-                else resid_item<2, T, FOLD>(D, I, w, lane, rr, rz, rp, ff);
-                const double b0 = block_sum_256(rr, sh), b1 = block_sum_256(rz, sh + 4);
-                const double b2 = block_sum_256(rp, sh), b3 = block_sum_256(ff, sh + 4);
-                if (threadIdx.x == 0) {
-                    glb(a.partr)[4 * (int64_t)it] = b0;
-                    glb(a.partr)[4 * (int64_t)it + 1] = b1;
-                    glb(a.partr)[4 * (int64_t)it + 2] = b2;
-                    glb(a.partr)[4 * (int64_t)it + 3] = b3;
+    int64_t k = 0;
+    for (; k < a.iters && total > 0; ++k) {
+        double* pa = a.part + (k & 1) * 4 * ps;
+        if ((int64_t)total <= (int64_t)a.item_slices * G) {
+            // ---- A, slices shared by the block ----
+            auto run = [&](auto bs, int p, int s0, int s1) {
+                constexpr int BS = decltype(bs)::value;
+                SharedSlice<BS, TV> sl(D->scol, desc_vals<TV>(D));
+                sl.load(D->sl_ptr, D->sl_w, D->slice0 + s0);
+                advance(p, s0, k, true);
+                if (uniform(S.done)) return;
+                const int pb = uniform(S.pbuf);
+                if (uniform(S.need_update)) {
+                    for (int s = s0; s < s1; ++s)
+                        resid_slice<BS, T, FOLD, true>(D, s, (const T*)D->p[pb], pa, ps, buf);
+                } else {
+                    shared_run<BS, TV, T, true>(sl, D, s0, s1, (T)uniform(S.beta), (T)uniform(S.zcoef), (const T*)D->p[pb ^ 1],
+                                                (T*)D->p[pb], pa, buf);
                 }
+            };
+            RunCursor c = runs();
+            for (int p, s0, s1; next(c, p, s0, s1);) {
+                take_desc(p);
+                if (D->bs == 3) run(std::integral_constant<int, 3>{}, p, s0, s1);
+                else run(std::integral_constant<int, 2>{}, p, s0, s1);
+            }
+        } else {
+            // ---- A, p by a pass of its own ----
+            RunCursor c = runs();
+            for (int p, s0, s1; next(c, p, s0, s1);) {
+                take_desc(p);
+                advance(p, s0, k, false);
+                if (uniform(S.done)) continue;
+                const int pb = uniform(S.pbuf);
+                if (uniform(S.need_update)) continue;
+                const T beta = (T)uniform(S.beta), zc = (T)uniform(S.zcoef);
+                SFEM_GLOBAL T* pv = glb((T*)D->p[pb]);
+                const SFEM_GLOBAL T* z = glb((const T*)D->z);
+                const int64_t n = 64 * D->bs;
+                for (int64_t i = (D->slice0 + s0) * n + threadIdx.x; i < (D->slice0 + s1) * n; i += kThreads)
+                    pv[i] = fmaT<T>(beta, pv[i], zc * z[i]);
             }
             if (!grid.sync()) return;
-            for (int pr = blockIdx.x; pr < a.nprob; pr += G) {
-                ProbState* st = probs[pr].st;
-                if (!st->need_update || st->done) continue;
-                const int i0 = probs[pr].item0, i1 = probs[pr].item1;
-                const double trr = items_sum(a.partr, 4, 0, i0, i1, sh);
-                const double trz = items_sum(a.partr, 4, 1, i0, i1, sh);
-                const double trp = items_sum(a.partr, 4, 2, i0, i1, sh);
-                // 16x the attainable |r|^2, (eps * || |rhs| + |K||x| ||)^2
-                const double floor_rr = 16.0 * kEps64 * kEps64 * items_sum(a.partr, 4, 3, i0, i1, sh);
-                if (threadIdx.x == 0) {
-                    ProbState S = *st;
-                    S.rr_true = trr;
-                    S.floor_rr = floor_rr;
-                    S.updates += 1;
-                    S.last_upd = S.iters;
-                    S.need_update = 0;
-                    S.fold_pending = FOLD ? 1 : 0;
-                    if (trr <= S.tol2bb) {
-                        S.done = 1;
-                    } else if (S.capped) {
-                        S.done = 4;
-                    } else {
-                        S.beta = trz / S.rz_prev;
-                        S.zcoef = 1.0 - S.beta * (trp / trz);
-                        S.rz = trz;
-                        S.maxrr = trr;
-                        // attainable floor: no 10% gain on the best true residual
-                        // within 4x of the rounding floor, or twice in a row while
-                        // the recurrence ran 5x below it
-                        const bool gap = S.iters > 0 && 25.0 * S.rr_rec < trr;
-                        if (trr <= 0.81 * S.best_true) {
-                            S.stall = 0;
-                            S.best_true_it = S.iters;
-                        } else if (trr <= floor_rr) {
-                            S.stall += 2;
-                        } else if (gap) {
-                            S.stall += 1;
-                        }
-                        if (S.stall >= 2) S.done = 3;
+            // ---- q = K p or the residual: the blocks of an XCD go through
+            // its part of the active slices together, a slice per wavefront (a
+            // residual pass, twice the bytes, so meets all blocks alike); what
+            // is left after the last whole round is shared slice by slice ----
+            const int xn = G % 8 ? 1 : 8, xb = G / xn, bx = blockIdx.x / xn;
+            const int x0 = (int)((int64_t)(blockIdx.x % xn) * total / xn);
+            const int xs = (int)((int64_t)(blockIdx.x % xn + 1) * total / xn) - x0;
+            const int rest = xs % (4 * xb);
+            const int whole = rest > 3 * xb ? xs : xs - rest;
+            auto spmv = [&](auto bs, DescPtr P, int64_t s, int buf_of) {
+                constexpr int BS = decltype(bs)::value;
+                const SFEM_GLOBAL T* pv = glb((const T*)P->p[buf_of]);
+                SFEM_GLOBAL T* q = glb((T*)P->q);
+                auto gx = [&](int64_t col, T (&x)[BS]) {
+#pragma unroll
+                    for (int i = 0; i < BS; ++i) x[i] = pv[col * BS + i];
+                };
+                const int64_t row = (P->slice0 + s) * 64 + lane;
+                T out[BS];
+                sell_row_quads<BS, TV, T, true>(P->sl_ptr, P->sl_w, P->scol, desc_vals<TV>(P), P->slice0 + s, lane, gx,
+                                                out);
+                double dot = 0.0;
+#pragma unroll
+                for (int j = 0; j < BS; ++j) {
+                    q[row * BS + j] = out[j];
+                    dot += (double)pv[row * BS + j] * (double)out[j];
+                }
+                dot = wave_sum(dot);
+                if (lane == 0) glb(pa)[P->t0 + s] = dot;
+            };
+            auto find = [&](int at, int& off) {  // problem and slice of an active position
+                int lo = 0, hi = ng;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) / 2;
+                    if (uniform(set.pre[mid]) <= at) lo = mid;
+                    else hi = mid;
+                }
+                off = at - uniform(set.pre[lo]);
+                int q = lo * gs;
+                if (gs > 1)
+                    while (off >= probs[q].nslices) off -= probs[q++].nslices;
+                return q;
+            };
+            const SFEM_GLOBAL int32_t* fl = glb(a.flags) + ((k + 1) & 1) * a.nprob;
+            for (int i = 4 * bx + w; i < whole; i += 4 * xb) {
+                int off;
+                const int q = find(x0 + i, off);
+                const int f = uniform(fl[q]);
+                if (f & kFlagDone) continue;
+                const DescPtr P = probs + q;
+                if (f & kFlagResid) {
+                    const T* pv = (const T*)P->p[f & kFlagBuf ? 1 : 0];
+                    if (P->bs == 3) resid_slice<3, T, FOLD, false>(P, off, pv, pa, ps, buf);
+                    else resid_slice<2, T, FOLD, false>(P, off, pv, pa, ps, buf);
+                } else if (P->bs == 3) spmv(std::integral_constant<int, 3>{}, P, off, f & kFlagBuf ? 1 : 0);
+                else spmv(std::integral_constant<int, 2>{}, P, off, f & kFlagBuf ? 1 : 0);
+            }
+            for (int i = whole + bx; i < xs; i += xb) {
+                int off;
+                const int q = find(x0 + i, off);
+                const int f = uniform(fl[q]);
+                if (f & kFlagDone) continue;
+                const DescPtr P = probs + q;
+                auto run = [&](auto bs) {
+                    constexpr int BS = decltype(bs)::value;
+                    if (f & kFlagResid) {
+                        resid_slice<BS, T, FOLD, true>(P, off, (const T*)P->p[f & kFlagBuf ? 1 : 0], pa, ps, buf);
+                        return;
                     }
-                    if (trr < S.best_true) S.best_true = trr;
-                    if (!isfinite(trr)) S.done = 2;
-                    *st = S;
-                }
+                    SharedSlice<BS, TV, true> sl(P->scol, desc_vals<TV>(P));
+                    sl.load(P->sl_ptr, P->sl_w, P->slice0 + off);
+                    shared_run<BS, TV, T, false>(sl, P, off, off + 1, T(0), T(0), (const T*)P->p[f & kFlagBuf ? 1 : 0],
+                                                 nullptr, pa, buf);
+                };
+                if (P->bs == 3) run(std::integral_constant<int, 3>{});
+                else run(std::integral_constant<int, 2>{});
             }
-            if (!grid.sync()) return;
-        }
-        if (!block_any(a.nprob, [&](int i) { return !probs[i].st->done; })) break;
-
-        // ---- P: p = zcoef z + beta p ----
-        for (int it = blockIdx.x; it < a.nitems; it += G) {
-            const WorkItem I = a.items[it];
-            const ProbDesc& D = probs[I.prob];
-            if (D.st->done) continue;
-            const T beta = (T)D.st->beta, zc = (T)D.st->zcoef;
-            SFEM_GLOBAL T* p = glb((T*)D.p);
-            const SFEM_GLOBAL T* z = glb((const T*)D.z);
-            for (int64_t i = I.slice0 * 64 * D.bs + threadIdx.x; i < I.slice1 * 64 * D.bs; i += kThreads)
-                p[i] = fmaT<T>(beta, p[i], zc * z[i]);
         }
         if (!grid.sync()) return;
 
-        // ---- S: q = K p and the item partials of p.q ----
-        for (int it = blockIdx.x; it < a.nitems; it += G) {
-            const WorkItem I = a.items[it];
-            const ProbDesc& D = probs[I.prob];
-            if (D.st->done) continue;
-            const SFEM_GLOBAL T* p = glb((const T*)D.p);
-            SFEM_GLOBAL T* q = glb((T*)D.q);
-            const Vals<TV> vals = desc_vals<TV>(D);
-            const int bs = D.bs;
-            double dot = 0.0;
-            auto gx = [&](int64_t c) { return p[c]; };
-            for (int64_t sl = I.slice0 + w; sl < I.slice1; sl += kThreads / 64) {
-                T out[3];
-                if (bs == 3) sell_row_staged<3, TV, T, true>(D.sl_ptr, D.sl_w, D.scol, vals, sl, lane, gx, out);
-                else sell_row_staged<2, TV, T, true>(D.sl_ptr, D.sl_w, D.scol, vals, sl, lane, gx, out);
-                for (int j = 0; j < bs; ++j) {
-                    const int64_t d = (sl * 64 + lane) * bs + j;
-                    q[d] = out[j];
-                    dot += (double)p[d] * (double)out[j];
+        // ---- U, a wavefront per slice ----
+        // problems that were done before this iteration leave the active set:
+        // both state slots hold their final state (one group per thread and
+        // iteration in turn)
+        const int gd = (int)(k % ((ng + kThreads - 1) / kThreads)) * kThreads + threadIdx.x;
+        int gone = 0;
+        if (k > 0 && gd < ng && set.w[gd] > 0) {
+            gone = 1;
+            for (int p = gd * gs; p < min(a.nprob, (gd + 1) * gs); ++p)
+                gone &= (gs > 1 && probs[p].nslices == 0) || (glb(a.flags)[(k & 1) * a.nprob + p] & kFlagDone) ? 1 : 0;
+        }
+        RunCursor c = runs();
+        for (int p, s0, s1; next(c, p, s0, s1);) {
+            take_desc(p);
+            take_state(p, k + 1);
+            if (uniform(S.done | S.need_update)) continue;
+            const int pb = uniform(S.pbuf);
+            double v = 0.0;
+            for (int i = threadIdx.x; i < D->nslices; i += kThreads) v += glb(pa)[D->t0 + i];
+            const double pq = block_sum_256(v, sh);
+            const T al = (T)uniform(S.rz / pq);
+            const bool fold = FOLD && uniform(S.fold_pending);
+            const T* pv = (const T*)D->p[pb];
+            for (int64_t s = s0 + w; s < s1; s += kThreads / 64) {
+                const int64_t row = (D->slice0 + s) * 64 + lane;
+                double rz = 0.0, rr = 0.0;
+                if (D->bs == 3) update_row<3, T, FOLD>(D, row, pv, al, fold, rz, rr);
+                else update_row<2, T, FOLD>(D, row, pv, al, fold, rz, rr);
+                rz = wave_sum(rz);
+                rr = wave_sum(rr);
+                if (lane == 0) {
+                    glb(partu)[D->t0 + s] = rz;
+                    glb(partu)[ps + D->t0 + s] = rr;
                 }
             }
-            const double b = block_sum_256(dot, sh);
-            if (threadIdx.x == 0) glb(a.part)[4 * (int64_t)it] = b;
         }
         if (!grid.sync()) return;
+        if (__syncthreads_or(gone)) {
+            if (gone) set.w[gd] = 0;
+            __syncthreads();
+            cut();
+        }
+    }
 
-        // ---- U: alpha; x += alpha p; r -= alpha q; z = M^-1 r (per node) ----
-        for (int it = blockIdx.x; it < a.nitems; it += G) {
-            const WorkItem I = a.items[it];
-            const ProbDesc& D = probs[I.prob];
-            if (D.st->done) continue;
-            const double pq = items_sum(a.part, 4, 0, D.item0, D.item1, sh);
-            const T al = (T)(D.st->rz / pq);
-            const bool fold = FOLD && D.st->fold_pending;
-            double rz = 0.0, rr = 0.0;
-            if (D.bs == 3) update_item<3, T, FOLD>(D, I, al, fold, rz, rr);
-            else update_item<2, T, FOLD>(D, I, al, fold, rz, rr);
-            const double b0 = block_sum_256(rz, sh), b1 = block_sum_256(rr, sh + 4);
+    // ---- the sums the last pass left, and the state back to the host's slot ----
+    for (int p = blockIdx.x; p < a.nprob; p += G) {
+        take_desc(p);
+        have_slot = -1;
+        take_state(p, 0);
+        if (S.done) continue;
+        if (D->nslices == 0) {  // no rows: solved
             if (threadIdx.x == 0) {
-                glb(a.part)[4 * (int64_t)it + 1] = b0;
-                glb(a.part)[4 * (int64_t)it + 2] = b1;
+                D->st->init_pending = D->st->need_update = 0;
+                D->st->updates = 1;
+                D->st->done = 1;
             }
+            continue;
         }
-        if (!grid.sync()) return;
-
-        // ---- F: per-problem scalars and stopping tests ----
-        for (int pr = blockIdx.x; pr < a.nprob; pr += G) {
-            ProbState* st = probs[pr].st;
-            if (st->done) continue;
-            const int i0 = probs[pr].item0, i1 = probs[pr].item1;
-            const double pq = items_sum(a.part, 4, 0, i0, i1, sh);
-            const double trz = items_sum(a.part, 4, 1, i0, i1, sh);
-            const double trr = items_sum(a.part, 4, 2, i0, i1, sh);
-            if (threadIdx.x == 0) {
-                ProbState S = *st;
-                S.rz_prev = S.rz;
-                S.rz = trz;
-                S.beta = trz / S.rz_prev;
-                S.iters += 1;
-                S.fold_pending = 0;
-                S.zcoef = 1.0;
-                S.rr_rec = trr;
-                const int64_t since = S.iters - S.last_upd;
-                if (trr <= S.tol2bb || trr < S.delta2 * S.maxrr || since >= (S.best_true_it > 256 ? S.best_true_it : 256))
-                    S.need_update = 1;
-                // backstop for a recurrence that stops decreasing: no 2x drop of |r|
-                // within max(10000, 4x the iterations it took to reach the best)
-                if (trr < 0.25 * S.best_rr) {
-                    S.best_rr = trr;
-                    S.best_it = S.iters;
-                } else if (S.iters - S.best_it > (4 * S.best_it > 10000 ? 4 * S.best_it : 10000)) {
-                    S.done = 3;
-                }
-                if (S.iters >= S.max_iter && !S.done) {  // final FP64 residual, then stop
-                    S.need_update = 1;
-                    S.capped = 1;
-                }
-                if (!(pq > 0.0) || !isfinite(trr)) S.done = 2;
-                *st = S;
-            }
+        have_slot = -1;
+        take_state(p, k);
+        const double* pa = a.part + ((k + 1) & 1) * 4 * ps + D->t0;
+        const bool upd = S.pending == kUpdateSums;
+        double v[4];
+        for (int m = 0; m < 4; ++m) {
+            const double* src = upd && m > 0 ? partu + (m - 1) * ps + D->t0 : pa + m * ps;
+            double t = 0.0;
+            if (S.pending != kNoSums && !(upd && m == 3))
+                for (int i = threadIdx.x; i < D->nslices; i += kThreads) t += glb(src)[i];
+            v[m] = block_sum_256(t, sh);
         }
-        if (!grid.sync()) return;
+        if (threadIdx.x == 0) {
+            if (!S.done && !S.init_pending && S.pending != kNoSums) consume<FOLD>(S, v);
+            *D->st = S;
+        }
     }
 }
 
@@ -638,7 +1082,7 @@ int table_max_blocks_per_cu(int precision) {
 }
 
 void table_launch(sfem_ctx* ctx, int precision, const TableLaunch& a0, int grid) {
-    if (a0.nitems <= 0 || a0.nprob <= 0) return;
+    if (a0.nprob <= 0) return;
     if (!ctx->bar_ws) ctx->bar_ws = static_cast<unsigned*>(ctx->alloc->alloc(sizeof(unsigned) * kBarWords));
     TableLaunch a = a0;
     a.bar_ws = ctx->bar_ws;
@@ -656,6 +1100,31 @@ void table_launch(sfem_ctx* ctx, int precision, const TableLaunch& a0, int grid)
     d2h(ctx, flags, a.bar_ws + kBarFlags, sizeof(flags));
     ctx->bar_last_grouped = a.bar_grouped && flags[0] == 0u;
     if (flags[1]) fail(SFEM_ERR_DEVICE, "persistent solver: a grid barrier wait exceeded its time limit");
+}
+
+TableLaunch table_prepare(sfem_ctx* ctx, TableWork& W, std::vector<ProbDesc>& descs, int item_slices) {
+    const size_t np = descs.size();
+    int64_t t0 = 0;
+    for (ProbDesc& D : descs) {
+        D.t0 = t0;
+        t0 += D.nslices;
+    }
+    if (W.descs.size() < np) {
+        W.descs.reset(ctx, np * 2);
+        W.alt.reset(ctx, np * 2);
+        W.flags.reset(ctx, np * 4);
+    }
+    if (W.part.size() < (size_t)t0 * kTableSums) W.part.reset(ctx, (size_t)t0 * kTableSums * 2);
+    h2d(ctx, W.descs.get(), descs.data(), sizeof(ProbDesc) * np);
+    TableLaunch a{};
+    a.probs = W.descs.get();
+    a.nprob = (int)np;
+    a.item_slices = item_slices;
+    a.nslices = t0;
+    a.part = W.part.get();
+    a.alt = W.alt.get();
+    a.flags = W.flags.get();
+    return a;
 }
 
 void table_fold(sfem_ctx* ctx, double* x64, void* xs, int64_t n) {
@@ -786,30 +1255,13 @@ void batch_build(sfem_ctx* ctx, sfem_batch* B) {
     (void)hipEventDestroy(e1);
 }
 
-void batch_items(const sfem_batch* B, int item_slices, std::vector<WorkItem>* items,
-                 std::vector<std::pair<int, int>>* ranges) {
-    items->clear();
-    ranges->clear();
-    for (size_t p = 0; p < B->hprobs.size(); ++p) {
-        const BatchProb& P = B->hprobs[p];
-        const int i0 = (int)items->size();
-        for (int64_t s = P.slice0; s < P.slice1; s += item_slices) {
-            WorkItem I{};
-            I.prob = (int32_t)p;
-            I.slice0 = s;
-            I.slice1 = std::min(P.slice1, s + item_slices);
-            items->push_back(I);
-        }
-        ranges->push_back({i0, (int)items->size()});
-    }
-}
-
 void batch_ensure_work(sfem_ctx* ctx, sfem_batch* B, int precision) {
     const size_t vb = prec_vec_bytes(precision);
     if (B->work_vb != vb) {
         B->wr.reset(ctx, vb * B->npad);
         B->wz.reset(ctx, vb * B->npad);
         B->wp.reset(ctx, vb * B->npad);
+        B->wp2.reset(ctx, vb * B->npad);
         B->wq.reset(ctx, vb * B->npad);
         B->work_vb = vb;
     }
@@ -817,7 +1269,7 @@ void batch_ensure_work(sfem_ctx* ctx, sfem_batch* B, int precision) {
         B->wxs.reset(ctx, sizeof(float) * B->npad);
 }
 
-ProbDesc batch_desc(sfem_batch* B, int precision, int preconditioner, ProbState* st, int item0, int item1) {
+ProbDesc batch_desc(sfem_batch* B, int precision, int preconditioner, ProbState* st, const BatchProb& P) {
     ProbDesc D{};
     D.sl_ptr = B->sl_ptr.get();
     D.sl_w = B->sl_w.get();
@@ -830,7 +1282,8 @@ ProbDesc batch_desc(sfem_batch* B, int precision, int preconditioner, ProbState*
     D.xs = precision == SFEM_PREC_MIXED ? (void*)B->wxs.get() : nullptr;
     D.r = B->wr.get();
     D.z = B->wz.get();
-    D.p = B->wp.get();
+    D.p[0] = B->wp.get();
+    D.p[1] = B->wp2.get();
     D.q = B->wq.get();
     D.dinv = precision == SFEM_PREC_MIXED ? (const void*)B->dinv32.get() : (const void*)B->dinv64.get();
     D.binv = precision == SFEM_PREC_MIXED ? (const void*)B->binv32.get() : (const void*)B->binv64.get();
@@ -838,8 +1291,8 @@ ProbDesc batch_desc(sfem_batch* B, int precision, int preconditioner, ProbState*
     D.block_pc = preconditioner == SFEM_PC_BLOCK_JACOBI ? 1 : 0;
     D.st = st;
     D.bs = B->bs;
-    D.item0 = item0;
-    D.item1 = item1;
+    D.slice0 = P.slice0;
+    D.nslices = (int32_t)(P.slice1 - P.slice0);
     return D;
 }
 
@@ -875,31 +1328,17 @@ double batch_run(sfem_ctx* ctx, sfem_batch* B, const sfem_solve_opts& o, int ite
     if (o.max_iter < 0) fail(SFEM_ERR_ARGUMENT, "batch solve: max_iter must be >= 0");
     if (B->st.size() != (size_t)B->nprob) B->st.reset(ctx, (size_t)B->nprob);
     batch_reset(ctx, B, prec, o, B->st.get());
-    std::vector<WorkItem> items;
-    std::vector<std::pair<int, int>> ranges;
-    batch_items(B, item_slices, &items, &ranges);
     std::vector<ProbDesc> descs((size_t)B->nprob);
     for (int64_t p = 0; p < B->nprob; ++p)
-        descs[(size_t)p] = batch_desc(B, prec, o.preconditioner, B->st.get() + p, ranges[(size_t)p].first,
-                                      ranges[(size_t)p].second);
-    DevBuf<ProbDesc> ddesc(ctx, descs.size());
-    DevBuf<WorkItem> ditems(ctx, items.size());
-    DevBuf<double> part(ctx, 4 * items.size()), partr(ctx, 4 * items.size());
-    h2d(ctx, ddesc.get(), descs.data(), sizeof(ProbDesc) * descs.size());
-    h2d(ctx, ditems.get(), items.data(), sizeof(WorkItem) * items.size());
-    TableLaunch a{};
-    a.probs = ddesc.get();
-    a.nprob = (int)B->nprob;
-    a.items = ditems.get();
-    a.nitems = (int)items.size();
-    a.part = part.get();
-    a.partr = partr.get();
+        descs[(size_t)p] = batch_desc(B, prec, o.preconditioner, B->st.get() + p, B->hprobs[(size_t)p]);
+    TableWork work;
+    TableLaunch a = table_prepare(ctx, work, descs, item_slices);
     const int grid = table_grid(ctx, prec, blocks_per_cu);
     // One launch holds the whole solve unless a per-launch iteration budget
     // (check_every > 0) splits it; the state lives in memory either way.  A
-    // problem needs at most max_iter + 1 loop passes (the last one is the
-    // final FP64 residual of an iteration-capped problem).
-    const int64_t need = o.max_iter + 2;
+    // problem needs at most 2 max_iter + 2 loop passes: an FP64 residual at the
+    // start and after every iteration; the last sums are taken as a launch ends.
+    const int64_t need = 2 * std::min<int64_t>(o.max_iter, INT64_MAX / 4) + 3;
     const int64_t budget = o.check_every > 0 ? std::min<int64_t>(o.check_every, need) : need;
     hipEvent_t e0, e1;
     SFEM_HIP(hipEventCreate(&e0));
@@ -1030,7 +1469,7 @@ sfem_batch* batch_create(sfem_ctx* ctx, int64_t nprob, int ndim, int n_dof, cons
 int64_t batch_device_bytes(const sfem_batch* B, int precision) {
     const int64_t b2 = (int64_t)B->bs * B->bs;
     const int64_t vb = (int64_t)prec_vec_bytes(precision);
-    return B->sell_blocks * (4 + b2 * 14) + B->nslices * 12 + B->npad * (8 * 3 + 4 + 4 * vb + (vb == 4 ? 4 : 0)) +
+    return B->sell_blocks * (4 + b2 * 14) + B->nslices * 12 + B->npad * (8 * 3 + 4 + 5 * vb + (vb == 4 ? 4 : 0)) +
            B->nslices * 64 * b2 * 12 + (int64_t)B->pad_of.size() * 4 + B->n * 9;
 }
 

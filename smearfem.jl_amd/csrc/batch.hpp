@@ -17,8 +17,11 @@ struct ProbState {
     double rr_true, best_rr, best_true, rr_rec, floor_rr;
     int64_t max_iter, iters, updates, best_it, last_upd, best_true_it;
     int32_t init_pending, need_update, fold_pending, done;  // done: 0 running, 1 converged, 2 breakdown,
-    int32_t stall, capped, pad0, pad1;                      // 3 stagnation, 4 iteration cap
+    int32_t stall, capped;                                  // 3 stagnation, 4 iteration cap
+    int32_t pending, pbuf;  // sums the last pass left (TableSums); buffer that holds p
 };
+
+enum TableSums : int32_t { kNoSums = 0, kUpdateSums = 1, kResidSums = 2 };
 
 // One problem of a table: its sliced operator and vectors (padded layout,
 // 64-row slices, vectors of nslices*64*bs entries).  Pointers are typed by the
@@ -38,33 +41,41 @@ struct ProbDesc {
     void* xs;
     void* r;
     void* z;
-    void* p;
+    void* p[2];
     void* q;
     const void* dinv;
     const void* binv;
     ProbState* st;
     int64_t binv_stride;
-    int32_t bs, item0, item1, block_pc;
-};
-
-// A run of slices [slice0, slice1) of one problem, processed by one block.
-struct WorkItem {
-    int32_t prob, pad;
-    int64_t slice0, slice1;
+    int64_t slice0, t0;  // first slice in the operator; in the table's slice order
+    int32_t nslices, bs, block_pc, pad;
 };
 
 struct TableLaunch {
     const ProbDesc* probs;
     int nprob;
-    const WorkItem* items;
-    int nitems;
-    double* part;   // 4 per item
-    double* partr;  // 4 per item
-    int64_t iters;  // loop passes in this launch
+    int item_slices;   // slices a block may hold for its wavefronts to share each of them
+    int64_t nslices;   // of all problems
+    double* part;      // kTableSums per slice
+    ProbState* alt;    // second state slot per problem
+    int32_t* flags;    // 2 per problem: done, by state slot
+    int64_t iters;     // loop passes in this launch (an iteration or an FP64 residual)
     unsigned* bar_ws;                 // grid barrier workspace (kBarWords, zeroed per launch)
     unsigned long long bar_timeout;   // barrier wait limit, 100 MHz ticks
     int bar_grouped;                  // allow the per-XCD grouped barrier
 };
+
+constexpr int kTableSums = 10;  // 2 x 4 of pass A (by iteration parity), 2 of the update
+
+// Workspace of a table's launches, grown as needed.
+struct TableWork {
+    DevBuf<ProbDesc> descs;
+    DevBuf<double> part;
+    DevBuf<ProbState> alt;
+    DevBuf<int32_t> flags;
+};
+// Uploads the descriptors (their t0 is set here) and fills in the launch.
+TableLaunch table_prepare(sfem_ctx* ctx, TableWork& W, std::vector<ProbDesc>& descs, int item_slices);
 
 struct BatchProb {
     int64_t slice0, slice1, n_free;
@@ -100,7 +111,7 @@ struct sfem_batch {
     sfem::DevBuf<double> binv64;  // planar, stride nslices * 64
     // CG work vectors, typed by the last precision (work_vb bytes per entry)
     size_t work_vb = 0;
-    sfem::DevBuf<uint8_t> wr, wz, wp, wq, wxs;
+    sfem::DevBuf<uint8_t> wr, wz, wp, wp2, wq, wxs;
     sfem::DevBuf<sfem::ProbState> st;
     double t_assemble_ms = 0, t_eliminate_ms = 0;
     ~sfem_batch();
@@ -121,10 +132,8 @@ sfem_batch* batch_from_device(sfem_ctx* ctx, int64_t nprob, sfem_mesh* mesh, sfe
 void spec_build(sfem_ctx* ctx, int64_t nprob, const sfem_problem_spec* specs, sfem_mesh** mesh, sfem_bc** bc,
                 std::vector<int64_t>* node_off);
 int64_t spec_free_dofs(const sfem_problem_spec& s);
-void batch_items(const sfem_batch* B, int item_slices, std::vector<WorkItem>* items,
-                 std::vector<std::pair<int, int>>* ranges);
 void batch_ensure_work(sfem_ctx* ctx, sfem_batch* B, int precision);
-ProbDesc batch_desc(sfem_batch* B, int precision, int preconditioner, ProbState* st, int item0, int item1);
+ProbDesc batch_desc(sfem_batch* B, int precision, int preconditioner, ProbState* st, const BatchProb& P);
 void batch_reset(sfem_ctx* ctx, sfem_batch* B, int precision, const sfem_solve_opts& o, ProbState* d_st);
 void batch_solution(sfem_ctx* ctx, const sfem_batch* B, double* q);
 int64_t batch_device_bytes(const sfem_batch* B, int precision);

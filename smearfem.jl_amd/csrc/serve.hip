@@ -10,8 +10,8 @@
 // device memory back to the allocator.  Requests that arrive while others
 // run join at the next step and share the launch with them.
 //
-// A request's arithmetic depends only on its own operator, item_slices and
-// precision (per-problem reductions over its own items, state in memory), so
+// A request's arithmetic depends only on its own operator and precision
+// (per-problem reductions over its own slices, state in memory), so
 // its result is bitwise the same alone or in any mix.
 //
 // Multigrid servers solve requests that come with their grid (or as a spec,
@@ -92,9 +92,7 @@ struct sfem_server {
     std::vector<int> free_slots;
     sfem::DevBuf<sfem::ProbState> pool;
     std::vector<sfem::ProbState> hpool;
-    sfem::DevBuf<sfem::ProbDesc> ddesc;
-    sfem::DevBuf<sfem::WorkItem> ditems;
-    sfem::DevBuf<double> part, partr;
+    sfem::TableWork work;
     int64_t bytes_in_use = 0, next_id = 0;
     int grid = 0;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -143,7 +141,7 @@ void estimate_bytes(Request& r, int precision) {
     const int64_t rows = (r.n_nodes + 63) / 64 * 64;
     const int64_t slots = rows * maxdeg;
     const int64_t b2 = (int64_t)bs * bs, vb = (int64_t)prec_vec_bytes(precision);
-    r.est_resident = slots * (4 + 14 * b2) + rows / 64 * 12 + rows * bs * (8 * 3 + 4 + 4 * vb + 4) +
+    r.est_resident = slots * (4 + 14 * b2) + rows / 64 * 12 + rows * bs * (8 * 3 + 4 + 5 * vb + 4) +
                      rows * b2 * 12 + r.n_nodes * 4 + r.n_nodes * bs * 8;
     const int64_t ke = (int64_t)nen * bs * nen * bs;
     r.est_transient = r.est_resident + r.n_elem * (ke * 8 + (int64_t)nen * nen * 24) + slots * (8 + b2 * 8);
@@ -448,35 +446,11 @@ void step(sfem_server* S, int* n_finished, double* ms) {
     lk.unlock();
     if (S->active.empty()) return;
     std::vector<ProbDesc> descs;
-    std::vector<WorkItem> items;
     for (int64_t id : S->active) {
         Request& r = S->reqs.at(id);
-        std::vector<WorkItem> its;
-        std::vector<std::pair<int, int>> ranges;
-        batch_items(r.B, S->o.item_slices, &its, &ranges);
-        const int base = (int)items.size();
-        for (WorkItem w : its) {
-            w.prob = (int32_t)descs.size();
-            items.push_back(w);
-        }
-        descs.push_back(batch_desc(r.B, S->o.precision, S->table_pc, S->pool.get() + r.slot, base,
-                                   (int)items.size()));
+        descs.push_back(batch_desc(r.B, S->o.precision, S->table_pc, S->pool.get() + r.slot, r.B->hprobs[0]));
     }
-    if (S->ddesc.size() < descs.size()) S->ddesc.reset(ctx, descs.size() * 2);
-    if (S->ditems.size() < items.size()) {
-        S->ditems.reset(ctx, items.size() * 2);
-        S->part.reset(ctx, items.size() * 8);
-        S->partr.reset(ctx, items.size() * 8);
-    }
-    h2d(ctx, S->ddesc.get(), descs.data(), sizeof(ProbDesc) * descs.size());
-    h2d(ctx, S->ditems.get(), items.data(), sizeof(WorkItem) * items.size());
-    TableLaunch a{};
-    a.probs = S->ddesc.get();
-    a.nprob = (int)descs.size();
-    a.items = S->ditems.get();
-    a.nitems = (int)items.size();
-    a.part = S->part.get();
-    a.partr = S->partr.get();
+    TableLaunch a = table_prepare(ctx, S->work, descs, S->o.item_slices);
     a.iters = S->o.iters_per_step;
     SFEM_HIP(hipEventRecord(S->e0, ctx->stream));
     table_launch(ctx, S->o.precision, a, S->grid);

@@ -285,11 +285,14 @@ __device__ __forceinline__ void sell_row(const int64_t* __restrict__ sl_ptr, con
 // columns part, part + 4, ... of the slice's 64 block rows (sell_combine adds
 // the four sums).  load() issues what does not depend on the gathered vector:
 // the first PRE column ids and PV columns of values; a column past the row's
-// end repeats its last one, and apply() drops it.
+// end repeats its last one, and apply() drops it.  PRE is 8 (all ids of a Hex8
+// row) where the values take 32 bits: 96x24x24, mixed, 72 -> 69 ms; with
+// 64-bit values the registers cost a wavefront per SIMD (64x16x16, FP64,
+// 24.8 -> 26.8 ms).
 template <int BS, typename TV, bool NT = false>
 struct SharedSlice {
-    static constexpr int B2 = BS * BS, SPLIT = kThreads / 64, PRE = 4, PV = 2;
     using Raw = typename Vals<TV>::Raw;
+    static constexpr int B2 = BS * BS, SPLIT = kThreads / 64, PRE = sizeof(Raw) == 4 ? 8 : 4, PV = 2;
     const int32_t* scol;
     Vals<TV> vals;
     int64_t base = 0;
@@ -322,6 +325,7 @@ struct SharedSlice {
         if (w <= 0) return;
 #pragma unroll
         for (int u = 0; u < PRE; ++u) {
+            if (u == 4 && u * SPLIT >= w) return;
             const bool in = part + u * SPLIT < w;
             Raw rv[B2];
 #pragma unroll
@@ -363,14 +367,7 @@ __device__ __forceinline__ void sell_row_abs_part(const int64_t* __restrict__ sl
     const int w = glb(sl_w)[sl];
 #pragma unroll
     for (int j = 0; j < BS; ++j) out[j] = aout[j] = 0.0;
-#pragma unroll 1
-    for (int k = part; k < w; k += SPLIT) {
-        const int64_t slot = base + (int64_t)k * 64;
-        const int64_t c = ld_stream<true>(scol + slot + lane);
-        double m[B2], xv[BS];
-#pragma unroll
-        for (int i = 0; i < B2; ++i) m[i] = ld_stream<true>(sval + slot * B2 + lane + i * 64);
-        gx(c, xv);
+    auto add = [&](const double (&m)[B2], const double (&xv)[BS]) {
 #pragma unroll
         for (int j = 0; j < BS; ++j)
 #pragma unroll
@@ -378,6 +375,32 @@ __device__ __forceinline__ void sell_row_abs_part(const int64_t* __restrict__ sl
                 out[j] = fma(m[j * BS + i], xv[i], out[j]);
                 aout[j] = fma(fabs(m[j * BS + i]), fabs(xv[i]), aout[j]);
             }
+    };
+    // two block columns at a time: both columns' ids and values are in flight
+    // before either gather
+    int k = part;
+#pragma unroll 1
+    for (; k + SPLIT < w; k += 2 * SPLIT) {
+        const int64_t s0 = base + (int64_t)k * 64, s1 = s0 + SPLIT * 64;
+        const int64_t c0 = ld_stream<true>(scol + s0 + lane), c1 = ld_stream<true>(scol + s1 + lane);
+        double m0[B2], m1[B2], x0[BS], x1[BS];
+#pragma unroll
+        for (int i = 0; i < B2; ++i) m0[i] = ld_stream<true>(sval + s0 * B2 + lane + i * 64);
+#pragma unroll
+        for (int i = 0; i < B2; ++i) m1[i] = ld_stream<true>(sval + s1 * B2 + lane + i * 64);
+        gx(c0, x0);
+        gx(c1, x1);
+        add(m0, x0);
+        add(m1, x1);
+    }
+    if (k < w) {
+        const int64_t s0 = base + (int64_t)k * 64;
+        const int64_t c0 = ld_stream<true>(scol + s0 + lane);
+        double m0[B2], x0[BS];
+#pragma unroll
+        for (int i = 0; i < B2; ++i) m0[i] = ld_stream<true>(sval + s0 * B2 + lane + i * 64);
+        gx(c0, x0);
+        add(m0, x0);
     }
 }
 
@@ -401,66 +424,10 @@ __device__ __forceinline__ void sell_combine(ACC (&v)[W], ACC (*buf)[W][64]) {
     }
 }
 
-// sell_row with explicit staging, for kernels whose register budget is set
-// elsewhere (the persistent solvers): per pair of block columns, the column
-// ids and all value loads are issued before any of them is used, then the
-// gathers, then the arithmetic.  Scheduling barriers keep the compiler from
-// interleaving loads with their uses, which would leave one load in flight
-// per wavefront.  Same arithmetic, in the same order, as sell_row.
-template <int BS, typename TV, typename ACC, bool NT = false, typename Gather>
-__device__ __forceinline__ void sell_row_staged(const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w,
-                                                const int32_t* __restrict__ scol, Vals<TV> vals, int64_t sl,
-                                                int lane, Gather gx, ACC out[BS]) {
-    constexpr int B2 = BS * BS;
-    using Raw = typename Vals<TV>::Raw;
-    const int64_t base = glb(sl_ptr)[sl];
-    const int w = glb(sl_w)[sl];
-#pragma unroll
-    for (int j = 0; j < BS; ++j) out[j] = 0;
-    int k = 0;
-    for (; k + 2 <= w; k += 2) {
-        const int64_t s0 = base + (int64_t)k * 64, s1 = s0 + 64;
-        const int64_t c0 = ld_stream<NT>(scol + s0 + lane), c1 = ld_stream<NT>(scol + s1 + lane);
-        Raw r0[B2], r1[B2];
-#pragma unroll
-        for (int m = 0; m < B2; ++m) r0[m] = vals.template raw<NT>(s0 * B2 + lane + m * 64);
-#pragma unroll
-        for (int m = 0; m < B2; ++m) r1[m] = vals.template raw<NT>(s1 * B2 + lane + m * 64);
-        __builtin_amdgcn_sched_barrier(0);
-        ACC x0[BS], x1[BS];
-#pragma unroll
-        for (int i = 0; i < BS; ++i) x0[i] = gx(c0 * BS + i);
-#pragma unroll
-        for (int i = 0; i < BS; ++i) x1[i] = gx(c1 * BS + i);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < BS; ++j)
-#pragma unroll
-            for (int i = 0; i < BS; ++i) out[j] = fmaT<ACC>((ACC)vals.decode(r0[j * BS + i]), x0[i], out[j]);
-#pragma unroll
-        for (int j = 0; j < BS; ++j)
-#pragma unroll
-            for (int i = 0; i < BS; ++i) out[j] = fmaT<ACC>((ACC)vals.decode(r1[j * BS + i]), x1[i], out[j]);
-    }
-    if (k < w) {
-        const int64_t s0 = base + (int64_t)k * 64;
-        const int64_t c0 = ld_stream<NT>(scol + s0 + lane);
-        Raw r0[B2];
-#pragma unroll
-        for (int m = 0; m < B2; ++m) r0[m] = vals.template raw<NT>(s0 * B2 + lane + m * 64);
-        ACC x0[BS];
-#pragma unroll
-        for (int i = 0; i < BS; ++i) x0[i] = gx(c0 * BS + i);
-#pragma unroll
-        for (int j = 0; j < BS; ++j)
-#pragma unroll
-            for (int i = 0; i < BS; ++i) out[j] = fmaT<ACC>((ACC)vals.decode(r0[j * BS + i]), x0[i], out[j]);
-    }
-}
-
-// sell_row in FP64 plus aout[j] = sum |M_ji x_i| over the row's blocks,
-// staged like sell_row_staged (pairs of block columns; the arithmetic order
-// per row is k, then j, then i).
+// sell_row in FP64 plus aout[j] = sum |M_ji x_i| over the row's blocks.  Per
+// pair of block columns the ids and all values are loaded before any of them
+// is used, then the gathers (scheduling barriers keep that order); the
+// arithmetic order per row is k, then j, then i.
 template <int BS, typename Gather>
 __device__ __forceinline__ void sell_row_abs(const int64_t* __restrict__ sl_ptr, const int32_t* __restrict__ sl_w,
                                              const int32_t* __restrict__ scol, const double* __restrict__ sval,
