@@ -332,6 +332,83 @@ __global__ void fin_true_kernel(ColumnState* cs, int kp, const double* part, int
     cs[j] = c;
 }
 
+// Small systems: lanes that share a row (or node row) of a column, each with
+// every L-th block of it.  A lane with all 27 blocks of a node goes through
+// seven rounds of dependent loads (ids, free dofs, P) while most of the chip
+// is idle; with four lanes it is two.
+template <int KP>
+constexpr int kRowLanes = KP >= 64 ? 1 : KP == 32 ? 2 : KP == 16 ? 4 : 8;
+
+// Q = K_ff P and partials of P.Q, kRowLanes lanes to a row of a column.
+template <int KP, bool BLK>
+__global__ __launch_bounds__(kThreadsM) void many_pass_kernel(
+    const int64_t* __restrict__ bcolptr, const int32_t* __restrict__ browidx, const double* __restrict__ bval,
+    const int32_t* __restrict__ free_of, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ col,
+    int64_t nunits, int64_t chunk, const double* __restrict__ P, double* __restrict__ Q, double* __restrict__ part) {
+    constexpr int L = kRowLanes<KP>, UPB = kThreadsM / (KP * L);
+    __shared__ double sh[kThreadsM];
+    const int64_t lb = logical_block();
+    const int j = threadIdx.x % KP, h = threadIdx.x / KP % L, ul = threadIdx.x / (KP * L);
+    auto dir = [&](int64_t row) { return P[row * KP + j]; };
+    double dot = 0.0;
+    for (int64_t u = lb * chunk + ul; u < min(nunits, (lb + 1) * chunk); u += UPB) {
+        constexpr int W = BLK ? 3 : 1;
+        int32_t f[W];
+        double a[W];
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            f[i] = BLK ? free_of[3 * u + i] : (int32_t)u;
+            a[i] = 0.0;
+        }
+        if constexpr (BLK) {
+            if (f[0] < 0 && f[1] < 0 && f[2] < 0) continue;
+            const int64_t e1 = bcolptr[u + 1];
+            for (int64_t e = bcolptr[u] + h; e < e1; e += 4 * L) {
+                int64_t r[4];
+                double v[4][9], x[4][3];
+                int32_t g[4][3];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) r[t] = browidx[min(e + t * L, e1 - 1)];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int m = 0; m < 9; ++m) v[t][m] = bval[min(e + t * L, e1 - 1) * 9 + m];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) g[t][i] = e + t * L < e1 ? free_of[3 * r[t] + i] : -1;
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) x[t][i] = g[t][i] >= 0 ? dir(g[t][i]) : 0.0;
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        a[i] = fma(v[t][i], x[t][0], fma(v[t][3 + i], x[t][1], fma(v[t][6 + i], x[t][2], a[i])));
+            }
+        } else {
+            const int32_t e1 = rowptr[u + 1];
+#pragma unroll 4
+            for (int32_t e = rowptr[u] + h; e < e1; e += L) a[0] = fma(bval[e], dir(col[e]), a[0]);
+        }
+#pragma unroll
+        for (int off = KP; off < KP * L; off <<= 1)
+#pragma unroll
+            for (int i = 0; i < W; ++i) a[i] += __shfl_xor(a[i], off, 64);
+        if (h == 0)
+#pragma unroll
+            for (int i = 0; i < W; ++i)
+                if (f[i] >= 0) {
+                    Q[(int64_t)f[i] * KP + j] = a[i];
+                    dot = fma(dir(f[i]), a[i], dot);
+                }
+    }
+    block_partial<KP>(dot, sh, part + lb * KP);
+}
+
 __global__ void recombine_many_kernel(const int32_t* __restrict__ free_of, const double* __restrict__ X, int kp,
                                       const double* __restrict__ qd, int64_t n, int k, double* __restrict__ q) {
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -340,6 +417,14 @@ __global__ void recombine_many_kernel(const int32_t* __restrict__ free_of, const
     for (int j = 0; j < k; ++j)
         q[(int64_t)j * n + s] = row >= 0 ? X[(int64_t)row * kp + j] : (qd ? qd[(int64_t)j * n + s] : 0.0);
 }
+
+// Node rows (or rows) x columns up to which a row is spread over lanes.
+// Measured, a sweep's call on a cube of ne^3 Hex8 with k columns, one lane /
+// several: ne 8, k 1, 4, 16: 3.3 / 2.5, 3.1 / 2.4, 3.5 / 2.8 ms; ne 16: 6.9 /
+// 4.8, 6.5 / 4.8, 10.1 / 8.4; ne 24: 10.8 / 7.3 (k 1), 10.0 / 10.4 (k 4,
+// 62,500 entries), 19.5 / 22.1 (k 16, 250,000); ne 32: 15.4 / 14.3 (k 1), 18.5
+// / 26.4 (k 4, 143,748).
+constexpr int64_t kLaneEntries = 100000;
 
 template <int KP>
 struct ManyRun {
@@ -368,8 +453,17 @@ struct ManyRun {
                 hipLaunchKernelGGL(spmm_kernel<KP>, dim3(nb), dim3(kThreadsM), 0, ctx->stream, S->rowptr.get(),
                                    S->col.get(), S->val64.get(), nf, chunk, src, dst, prt);
         };
+        // several lanes to a row while one lane to a row fills the chip less
+        // than about three times over
+        constexpr int UPB = kThreadsM / (KP * kRowLanes<KP>);
+        const int64_t units = blk ? nunits : nf;
+        const bool lanes = ctx->tune_split > 0 ? ctx->tune_split >= 4 : units * KP <= kLaneEntries;
+        const int nbp =
+            lanes ? (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)ctx->n_cu * 16, (units + UPB - 1) / UPB)) : nb;
+        const int64_t pchunk = ((units + nbp - 1) / nbp + UPB - 1) / UPB * UPB;
         const size_t nv = (size_t)std::max<int64_t>(nf, 1) * KP;
         DevBuf<double> X(ctx, nv), R(ctx, nv), Z(ctx, nv), P(ctx, nv), Q(ctx, nv), RHS(ctx, nv);
+        DevBuf<double> partp(ctx, (size_t)nbp * KP);
         DevBuf<double> part(ctx, (size_t)nb * 2 * KP);
         DevBuf<ColumnState> cs(ctx, KP);
         memset_d(ctx, X.get(), 0, sizeof(double) * nv);
@@ -390,11 +484,19 @@ struct ManyRun {
         const long long max_iter = std::max<int64_t>(o.max_iter, 1);
         const int max_restarts = 64;
         const int64_t max_checks = max_iter / every + 2 * max_restarts + 8;
+        auto pass = [&] {
+            auto kern = blk ? many_pass_kernel<KP, true> : many_pass_kernel<KP, false>;
+            hipLaunchKernelGGL(kern, dim3(nbp), b, 0, ctx->stream, K->bcolptr.get(), K->browidx.get(),
+                               blk ? K->bval.get() : S->val64.get(), S->free_of.get(), S->rowptr.get(),
+                               S->col.get(), units, pchunk, P.get(), Q.get(), partp.get());
+        };
         hcs.assign(KP, ColumnState{});
         for (int64_t check = 0;; ++check) {
             for (int it = 0; it < every; ++it) {
-                spmm(P.get(), Q.get(), part.get());
-                hipLaunchKernelGGL(fin_alpha_kernel, dim3(KP), dim3(256), 0, ctx->stream, cs.get(), KP, part.get(), nb);
+                if (lanes) pass();
+                else spmm(P.get(), Q.get(), partp.get());
+                hipLaunchKernelGGL(fin_alpha_kernel, dim3(KP), dim3(256), 0, ctx->stream, cs.get(), KP, partp.get(),
+                                   nbp);
                 hipLaunchKernelGGL(update_kernel<KP>, g, b, 0, ctx->stream, nf, chunk, cs.get(), X.get(), R.get(), Z.get(),
                                    P.get(), Q.get(), dinv, part.get());
                 hipLaunchKernelGGL(fin_beta_kernel, dim3(KP), dim3(256), 0, ctx->stream, cs.get(), KP, part.get(), nb,

@@ -8,6 +8,8 @@ scipy's sum; each sweep solution within 1e-8 relative of a direct FP64 solve
 of the oracle's K_free; a sweep step after set_bc bitwise equal to a fresh
 elimination with the same data.
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -248,6 +250,43 @@ def test_solve_many_vs_oracle(ctx, k):
         h.close()
 
 
+@pytest.mark.parametrize("dims,scalar", [((1, 1, 1), False), ((9, 6, 5), False), ((9, 6, 5), True), ((12, 10), False)])
+def test_solve_many_row_forms(dims, scalar, monkeypatch):
+    """A row spread over lanes (small systems; forced with SFEM_SELL_SPLIT=4)
+    against a lane to a row (=1) and the oracle, for every width of the
+    columns, node blocks and scalar rows.  Both reach a true residual of
+    1e-12, so they differ by at most twice 1e-12 times the condition number
+    (below 1e4 here)."""
+    print(f"[case] solve_many forms {dims} scalar={scalar}", flush=True)
+    nd = len(dims)
+    m = smearfem.structured_mesh(dims)
+    fixed = smearfem.clamp_x0(m)
+    Ko = O.assemble_system(0, m.NodeList, m.IEN, nd, "Q1", nd, m.ID, 1.0, 0.3, n_elem=m.n_elem)
+    F = np.random.default_rng(3).standard_normal((m.n_dof, 64))
+    out = []
+    for split in ("4", "1"):
+        monkeypatch.setenv("SFEM_SELL_SPLIT", split)
+        c = smearfem.Context(0)
+        monkeypatch.delenv("SFEM_SELL_SPLIT")
+        K = smearfem.assemble_system(0, m.NodeList, m.IEN, nd, "Q1", nd, m.ID, 1.0, 0.3, n_elem=m.n_elem, ctx=c,
+                                     device=True, force_scalar=scalar)
+        S = System(K, smearfem.BoundaryConditions(c, m.n_dof, None, fixed))
+        qs = []
+        for k in (1, 2, 3, 7, 16, 33):
+            q, per, _ = S.solve_many(f=F[:, :k], rtol=1e-12)
+            assert all(p["stop_reason"] == 1 and p["rel_residual"] <= 1e-12 for p in per)
+            qs.append(q)
+        with pytest.raises(smearfem.NotConvergedError):
+            S.solve_many(f=F[:, :3], rtol=1e-12, max_iter=1)
+        for h in (S, K, c):
+            h.close()
+        out.append(qs)
+    for a, b in zip(*out):
+        assert relerr(a, b) <= 2e-8
+    Kff, rhs = O.eliminate(Ko, fixed, F[:, 32])
+    assert relerr(out[0][-1][:, 32], O.recombine(fixed, None, O.dense_solve(Kff, rhs))) <= ERR
+
+
 def test_solve_many_loads_and_errors(ctx):
     print("[case] solve_many loads", flush=True)
     m = smearfem.structured_mesh((6, 3, 3))
@@ -304,4 +343,32 @@ def test_apply_and_face_traction_loads(ctx):
     assert np.allclose(f, area[:, None] * t[None, :], rtol=1e-13, atol=1e-15)
     assert np.allclose(f.sum(axis=0), 2 * L[0] * L[1] * t, rtol=1e-13)
     for h in (K, mesh, faces):
+        h.close()
+
+
+@pytest.mark.parametrize("ne", [510, 511, 512, 723, 886, 887, 1000])
+def test_large_download(ctx, ne):
+    """Downloads around the staging threshold (4 MiB: the coordinates of 512 x
+    512 nodes), of whole and broken chunks of 1 MiB, and past the 12 buffers of
+    the ring, from three threads of which two share a context: every
+    coordinate is the grid's."""
+    print(f"[case] download ne={ne}", flush=True)
+    other = smearfem.Context(0)
+    meshes = [meshgrid(0, 1, 0, 1, 0, 0, ne, 2, faces=False, ctx=c) for c in (ctx, ctx, other)]
+    meshes = [m[0] if isinstance(m, tuple) else m for m in meshes]
+    got = [[] for _ in meshes]
+    threads = [threading.Thread(target=lambda m=m, g=g: g.extend(m.export()[0] for _ in range(2)))
+               for m, g in zip(meshes, got)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g in got:
+        assert len(g) == 2
+        for nodes in g:
+            x, y = nodes[0].reshape(ne + 1, ne + 1), nodes[1].reshape(ne + 1, ne + 1)
+            # the coordinate is start + k (end - start) / ne: within 2 ulp of 1
+            assert np.abs(x[0] - np.arange(ne + 1) / ne).max() <= 4.5e-16 and (x == x[0]).all()
+            assert np.array_equal(y[:, 0], x[0]) and (y.T == x[0]).all()
+    for h in (*meshes, other):
         h.close()
