@@ -59,6 +59,8 @@ private:
     int64_t in_use_ = 0, held_ = 0, limit_ = -1;
 };
 
+struct Staging;  // capi.hip
+
 }  // namespace sfem
 
 // A context lives until sfem_ctx_destroy has been called and every object
@@ -71,6 +73,7 @@ struct sfem_ctx {
     hipStream_t stream = nullptr;
     std::string last_error;
     sfem::Allocator* alloc = nullptr;
+    sfem::Staging* staging = nullptr;  // pinned buffers of large downloads (made by the first one)
     // Sliced-SpMV launch shape (measured on MI355X, 256x64x64 Hex8, FP64:
     // 392 us with both defaults vs 494 us with neither).  Overrides at
     // creation: SFEM_SPMV_NT=0/1, SFEM_SELL_WAVE_SLICES=n (0 = spread the
