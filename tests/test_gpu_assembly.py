@@ -304,3 +304,25 @@ def test_grid_declared_non_blocked_numbering(ctx):
     K.close()
     mesh.close()
     assert_parity(g, oracle_csc(m, 3, young=young, ID=idp))
+
+
+@pytest.mark.parametrize("gap", [1, 7, 8, 9, 63, 64, 65, 1000])
+def test_columns_without_blocks(ctx, gap):
+    """Runs of nodes that no element uses, before, between and after those that
+    are used: the column pointers of the empty columns (filled by a thread or
+    by a whole wavefront) against the oracle's CSC."""
+    print(f"[case] empty columns gap={gap}", flush=True)
+    n_el = 70  # more first blocks than a wavefront has lanes
+    first = gap + np.arange(n_el) * (4 + gap)
+    n_nodes = int(first[-1]) + 4 + gap
+    nodes = np.zeros((2, n_nodes))
+    ien = np.zeros((n_el, 4), dtype=np.int64)
+    for e, a in enumerate(first):
+        nodes[:, a:a + 4] = [[0, 1, 1, 0], [0, 0, 1 + 0.01 * e, 1]]
+        ien[e] = np.arange(a, a + 4) + 1
+    ident = np.arange(1, 2 * n_nodes + 1, dtype=np.int64).reshape(n_nodes, 2)
+    K = smearfem.assemble_system(0, nodes, ien, 2, "Q1", 2, ident, 1.0, 0.3, n_elem=n_el, ctx=ctx).tocsc()
+    Ko = O.assemble_system(0, nodes, ien, 2, "Q1", 2, ident, 1.0, 0.3, n_elem=n_el).tocsc()
+    assert K.shape == Ko.shape
+    assert np.array_equal(K.indptr, Ko.indptr) and np.array_equal(K.indices, Ko.indices)
+    assert np.abs(K.data - Ko.data).max() <= 1e-12 * np.abs(Ko.data).max()
