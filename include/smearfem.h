@@ -282,8 +282,9 @@ int  sfem_system_solution(sfem_ctx* ctx, const sfem_system* sys, double* q,
  *   Levels: the grid coarsened by 2 along each direction whose element count
  *   is even, until a level has at most coarse_nodes nodes (at least once);
  *   coarse operators are Galerkin products P'AP with multilinear P on the
- *   free dofs; the coarsest (at most 400 nodes, else SFEM_ERR_UNSUPPORTED)
- *   is solved with a dense inverse.  Smoothing: `degree` Chebyshev steps in
+ *   free dofs; the coarsest has at most 400 nodes (else
+ *   SFEM_ERR_UNSUPPORTED).  A V-cycle ends at the first level of at most 800
+ *   dofs, solved with its dense inverse.  Smoothing: `degree` Chebyshev steps in
  *   (node diagonal block)^-1 K on [lo, hi] x lambda_max before and after the
  *   coarse correction, lambda_max by power_iters power iterations.
  * The hierarchy depends on K and the fixed set only: sfem_system_set_bc keeps
