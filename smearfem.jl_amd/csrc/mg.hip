@@ -1771,7 +1771,11 @@ __global__ __launch_bounds__(kThreads) void prolong_kernel(const float* __restri
 // ------------------------------------------------------- outer CG ----
 // The scalars are formed by the kernels that need them: each sums the
 // previous kernel's per-block partials itself, and its first block stores
-// what later kernels read.
+// what later kernels read.  No kernel stores what its own blocks branch on
+// before a barrier: a block may start after the store, and its wavefronts
+// could read either value.  So a breakdown goes into a field of its own
+// (bad_dir, bad_upd), which the kernels after it read and take_rr turns into
+// done and halt.
 struct MgState {
     double bb, tol2bb;
     double rz[2];   // r.z of the iterations, by parity
@@ -1782,14 +1786,22 @@ struct MgState {
     int restart;    // next direction is z (after a residual replacement)
     int need_true;  // the recurrence claims convergence: check the FP64 residual
     int fresh;      // the last update's r.r is still to be taken
+    int bad_dir;    // breakdown found while the direction was formed (r.z)
+    int bad_upd;    // breakdown found by the update (p.q)
     int stall;
     Arrivals arrive;
 };
 
-// By one block: the iteration count and the claim of convergence from the
-// last update's per-block r.r.
+// By one block: a breakdown ends the solve; else the iteration count and the
+// claim of convergence from the last update's per-block r.r.
 __device__ __forceinline__ void take_rr(MgState* st, const double* __restrict__ upd, int nupd, double* sh) {
-    if (st->done || !st->fresh) return;  // uniform
+    const int bad = st->bad_dir | st->bad_upd, idle = st->done | !st->fresh;
+    __syncthreads();  // read by every wavefront before any store below
+    if (bad) {
+        if (threadIdx.x == 0) st->done = st->halt = 2;
+        return;
+    }
+    if (idle) return;
     double rr[1];
     sum_parts_all<1, kThreads / 64>(upd, nupd, rr, sh);
     if (threadIdx.x == 0) {
@@ -2323,7 +2335,8 @@ __device__ void true_finish(MgState* st, double* __restrict__ partials, double* 
 }
 
 // Start of the pass that forms the direction, by every block: beta from the
-// V-cycle's last step's r.z (0 after a restart).  False: nothing to do.
+// V-cycle's last step's r.z (0 after a restart).  False: nothing to do, in
+// every thread of the grid alike.
 __device__ __forceinline__ bool direction_begin(MgState* st, int parity, const double* __restrict__ zparts, int nz,
                                                 double* sh, double& beta) {
     if (st->halt || st->done) return false;
@@ -2333,7 +2346,7 @@ __device__ __forceinline__ bool direction_begin(MgState* st, int parity, const d
     beta = st->restart ? 0.0 : rz[0] / st->rz[parity ^ 1];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st->rz[parity] = rz[0];
-        if (!ok) st->done = 2;  // the other blocks find it for themselves
+        if (!ok) st->bad_dir = 1;  // the other blocks find it for themselves
     }
     return ok;
 }
@@ -2598,7 +2611,7 @@ __global__ __launch_bounds__(kThreads) void mg_spmv_kernel(const int64_t* __rest
             }
         }
     } else {
-        if (st->halt || st->done) return;
+        if (st->halt || st->done || st->bad_dir) return;
         const int64_t s0 = logical_block() * per_block;
         const int64_t s1 = min(nslices, s0 + per_block);
         const double* __restrict__ p = v.p;
@@ -2627,7 +2640,7 @@ template <int ND>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void mg_spmv_mf_kernel(
     MfOp<double> op, OuterVecs v, MgState* st, double* __restrict__ parts) {
     __shared__ double sh[4];
-    if (st->halt || st->done) return;
+    if (st->halt || st->done || st->bad_dir) return;
     const double* __restrict__ p = v.p;
     double dot = 0.0;
     for (int64_t row = logical_block() * kThreads + threadIdx.x; row < op.nrows;
@@ -2692,7 +2705,7 @@ __global__ __launch_bounds__(kThreads) void mg_update_kernel(double* __restrict_
                                                              const double* __restrict__ parts, int np,
                                                              double* __restrict__ upd) {
     __shared__ double sh[4];
-    if (st->halt || st->done) return;
+    if (st->halt || st->done || st->bad_dir) return;
     double pq[1];
     sum_parts_all<1, kThreads / 64>(parts, np, pq, sh);
     const double a = st->rz[parity] / pq[0];
@@ -2700,7 +2713,7 @@ __global__ __launch_bounds__(kThreads) void mg_update_kernel(double* __restrict_
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st->restart = 0;
         st->fresh = ok ? 1 : 0;
-        if (!ok) st->done = 2;  // breakdown: the other blocks find it for themselves
+        if (!ok) st->bad_upd = 1;  // breakdown: the other blocks find it for themselves
     }
     if (!ok) return;
     const int64_t i0 = (int64_t)blockIdx.x * per_block, i1 = min(first.nrows, i0 + per_block);

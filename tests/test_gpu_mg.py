@@ -616,3 +616,42 @@ def test_matrix_free_row_forms(dims, lanes, monkeypatch):
         K.close()
         mesh.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("form", ["lanes", "rows", "sliced_shared", "sliced"])
+@pytest.mark.parametrize("dims", [(9, 6, 5), (20, 14), (64, 48, 48)])
+def test_breakdown_keeps_the_iterate(dims, form, monkeypatch):
+    # an indefinite K (some moduli negative) ends the solve by breakdown: with
+    # every modulus negative r.z < 0 at once and x stays 0; else after k
+    # iterations, whose iterate is kept bit for bit (compared with a solve
+    # capped at k iterations).  Up to 588 blocks an update, so that some start
+    # after the first has found the breakdown
+    print(f"[case] breakdown {dims} {form}", flush=True)
+    monkeypatch.setenv("SFEM_MF_LANES", "1000000" if form == "lanes" else "0")
+    monkeypatch.setenv("SFEM_SELL_SPLIT", "1" if form == "sliced" else "4")
+    ctx = smearfem.Context(0)
+    m = structured_mesh(dims)
+    fixed = clamp_x0(m)
+    f = random_face_load(m, m.ndim - 1, 1, fixed, seed=4)
+    for every in (1, 7):
+        young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=3)
+        young[::every] *= -1.0 if every == 1 else -0.2
+        mesh = smearfem.Mesh(ctx, m.n_elem, m.NodeList, m.IEN, m.ndim, "Q1", m.ndim, m.ID, young, 0.3)
+        if not form.startswith("sliced"):
+            mesh.set_grid(m.dims)
+        K = mesh.assemble()
+        bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+        S = System(K, bc)
+        S.set_grid(m.dims)
+        opts = dict(rtol=1e-12, preconditioner="multigrid", raise_on_fail=False)
+        st = S.solve("fp64", max_iter=100, **opts)
+        q = S.solution()
+        assert st["stop_reason"] == 2 and np.isfinite(q).all()
+        if every == 1:
+            assert st["iterations"] == 0 and not q.any()
+        else:
+            capped = S.solve("fp64", max_iter=st["iterations"], **opts)
+            assert capped["iterations"] == st["iterations"] and np.array_equal(S.solution(), q)
+        for h in (S, bc, K, mesh):
+            h.close()
+    ctx.close()
