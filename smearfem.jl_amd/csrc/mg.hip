@@ -2928,7 +2928,8 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
     // exists, while the next levels are built: the finest level's first when
     // it is matrix-free.  Every level has its own vectors, sums and PowState;
     // all of them live until the side streams are joined (join syncs them
-    // when setup fails).  A side stream starts after an event recorded on the
+    // when setup fails: what a side stream uses is declared before it, or
+    // belongs to a level of H).  A side stream starts after an event recorded on the
     // context's stream once its buffers are allocated, so memory the cache
     // hands out again is past its earlier users.
     struct SetupOut {
@@ -2942,6 +2943,7 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
     double* const scales = setup.get()->scales;
     std::vector<DevBuf<double>> parts(SFEM_MG_MAX_LEVELS);
     DevBuf<float> p0a, p0b;
+    DevBuf<double> dense[2];  // the direct level's matrix and its inverse, by turns
     struct SideJoin {
         std::vector<hipStream_t> streams;
         std::vector<hipEvent_t> done;
@@ -3031,7 +3033,6 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
 
     // The direct level's dense inverse, on a side stream of its own as soon
     // as the level exists.
-    DevBuf<double> dense[2];
     auto direct_inverse = [&](int l, const MgLevel& v) {
         H.direct = l;
         H.nd_dofs = v.nn * BS;
@@ -3215,13 +3216,14 @@ void build_levels(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_mg_o
             }
             C.da.reset(ctx, (size_t)C.nn * BS);
             C.db.reset(ctx, (size_t)C.nn * BS);
-            power_coarse(lc, C);
         }
-        if (lc == 1 && H.mf) power_fine_mf();
-        if (!H.direct && C.nn <= 2 * kMgMaxCoarseNodes && (coarsest || C.nn * BS <= direct_dofs())) direct_inverse(lc, C);
         H.L.push_back(std::move(C));
-        prev_st = H.L.back().st64.get();
-        prev_fix = H.L.back().fixed.get();
+        const MgLevel& V = H.L.back();
+        if (!coarsest) power_coarse(lc, V);
+        if (lc == 1 && H.mf) power_fine_mf();
+        if (!H.direct && V.nn <= 2 * kMgMaxCoarseNodes && (coarsest || V.nn * BS <= direct_dofs())) direct_inverse(lc, V);
+        prev_st = V.st64.get();
+        prev_fix = V.fixed.get();
         if ((int)H.L.size() >= SFEM_MG_MAX_LEVELS) break;
     }
     if (H.L.size() < 2)

@@ -655,3 +655,28 @@ def test_breakdown_keeps_the_iterate(dims, form, monkeypatch):
         for h in (S, bc, K, mesh):
             h.close()
     ctx.close()
+
+
+def test_refused_hierarchy_leaves_the_context_usable(ctx):
+    # a coarsest level of more than 400 nodes is refused once its dense inverse
+    # is under way on a side stream: that work ends before its buffers go back
+    # to the context, so a solve right after it is not disturbed
+    print("[case] refused hierarchy", flush=True)
+    m = structured_mesh((50, 51))
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=8)
+    fixed = clamp_x0(m)
+    f = random_face_load(m, 1, 1, fixed, seed=9)
+    K = device_K(ctx, m, young)
+    Kff, rhs = O.eliminate(oracle_K(m, young), fixed, f)
+    q_ref = O.recombine(fixed, None, sp.linalg.spsolve(sp.csc_matrix(Kff), rhs))
+    bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+    S = System(K, bc)
+    bc.close()
+    for _ in range(4):
+        with pytest.raises(smearfem.UnsupportedError):
+            S.set_grid(m.dims, coarse_nodes=10000)
+        S.set_grid(m.dims)
+        st = S.solve("fp64", rtol=1e-12, preconditioner="multigrid")
+        assert st["converged"] and relerr(S.solution(), q_ref) <= ERR
+    S.close()
+    K.close()
