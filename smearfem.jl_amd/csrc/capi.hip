@@ -114,11 +114,12 @@ struct Staging {
     }
     bool ready() {  // made on first use; false if the pinned memory is not to be had
         if (buf) return true;
+        bool ok = true;
         for (hipEvent_t& e : ev)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-        if (hipHostMalloc((void**)&buf, kSlotBytes * kSlots, hipHostMallocDefault) != hipSuccess) {
+            ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+        if (!ok || hipHostMalloc((void**)&buf, kSlotBytes * kSlots, hipHostMallocDefault) != hipSuccess) {
             buf = nullptr;
-            (void)hipGetLastError();
+            (void)hipGetLastError();  // the caller copies directly: nothing failed
             return false;
         }
         return true;
@@ -171,6 +172,8 @@ void staged_d2h(sfem_ctx* ctx, Staging& st, char* dst, const char* src, size_t b
     }
     if (err != hipSuccess) stop.store(true);
     for (std::thread& t : pool) t.join();
+    // copies still under way write the ring: they end before it is used again
+    if (err != hipSuccess) (void)hipStreamSynchronize(ctx->stream);
     SFEM_HIP(err);
 }
 
