@@ -4,6 +4,7 @@
 // message retrievable with sfem_last_error(); nothing prints or exits.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -139,9 +140,12 @@ void staged_d2h(sfem_ctx* ctx, Staging& st, char* dst, const char* src, size_t b
         for (;;) {
             const int64_t c = next.fetch_add(1);
             if (c >= n) return;
-            while (landed.load(std::memory_order_acquire) <= c) {
+            int64_t have;
+            for (int spins = 0; (have = landed.load(std::memory_order_acquire)) <= c; ++spins) {
                 if (stop.load()) return;
-                std::this_thread::yield();
+                // before the first chunk, work queued ahead of the copy may run for long
+                if (have || spins < 2000) std::this_thread::yield();
+                else std::this_thread::sleep_for(std::chrono::microseconds(50));
             }
             std::memcpy(dst + (size_t)c * kSlotBytes, st.buf + (size_t)(c % kSlots) * kSlotBytes, size_of(c));
             copied[(size_t)c].store(1, std::memory_order_release);
