@@ -58,6 +58,7 @@ struct TableLaunch {
     int64_t nslices;   // of all problems
     double* part;      // kTableSums per slice
     ProbState* alt;    // second state slot per problem
+    double* pq;        // per problem: p.q of the last update
     int32_t* flags;    // 2 per problem: done, by state slot
     int64_t iters;     // loop passes in this launch (an iteration or an FP64 residual)
     unsigned* bar_ws;                 // grid barrier workspace (kBarWords, zeroed per launch)
@@ -72,6 +73,7 @@ struct TableWork {
     DevBuf<ProbDesc> descs;
     DevBuf<double> part;
     DevBuf<ProbState> alt;
+    DevBuf<double> pq;
     DevBuf<int32_t> flags;
 };
 // Uploads the descriptors (their t0 is set here) and fills in the launch.
