@@ -289,17 +289,28 @@ __global__ void fold_all_kernel(double* __restrict__ x64, float* __restrict__ xs
 // Both forms add the same numbers in the same order, so the active problems
 // may move from one to the other as others finish.  The line at 8 slices a
 // block, 24 / 256 problems as above: always the second form 56.5 / 260 ms, at
-// 8 slices 48.3 / 259, at 64 48.3 / 338.
+// 8 slices 48.3 / 259, at 64 48.3 / 338.  For 3D slices of 64-bit values it
+// lies lower (kShareSlices64).
 
 enum TableFlags : int32_t { kFlagDone = 1, kFlagResid = 2, kFlagBuf = 4 };  // what a pass needs of a state
+
+// Slices per block up to which the first form is taken where an operator value
+// takes more than 32 bits (FP64, split) in 3D, at most.  One problem, us an
+// iteration with the first / the second form on 512 blocks: FP64 1,369 slices
+// 66 / 89, 1,839 102 / 70, 3,602 197 / 119; split 63 / 85, 77 / 60, 185 / 100;
+// FP32 values 2,532 slices 57 / 65, 3,602 89 / 82, mixed 70 / 77, 5,585 slices
+// 125 / 106.  In 2D (9 block columns) FP64 4,697 slices 57 / 59, 11,265 129 /
+// 106: item_slices alone decides.
+constexpr int kShareSlices64 = 3;
 
 constexpr int kMaxGroups = 2048;  // problems, or groups of them, whose activity a block tracks
 
 // The slices still iterated, in table order: groups of `gs` problems, their
-// slice counts (0 once all problems of the group are done) and the prefix sums.
+// slice counts (0 once all problems of the group are done) and the prefix
+// sums; w3, pre3 the same for the slices of 3D problems alone.
 struct ActiveSet {
-    int pre[kMaxGroups + 1];
-    int w[kMaxGroups];
+    int pre[kMaxGroups + 1], pre3[kMaxGroups + 1];
+    int w[kMaxGroups], w3[kMaxGroups];
 };
 
 // Descriptors do not change during a launch: read as constants, so that what
@@ -313,8 +324,8 @@ __device__ __forceinline__ double uniform(double v) {
     return __builtin_bit_cast(double, make_int2(uniform(u.x), uniform(u.y)));
 }
 
-// Prefix sums of set.w; returns the total.  Every thread of the block calls.
-__device__ __forceinline__ int active_prefix(ActiveSet& set, int ng) {
+// Prefix sums of w[0..ng); returns the total.  Every thread of the block calls.
+__device__ __forceinline__ int active_prefix(const int* w, int* pre, int ng) {
     constexpr int PER = kMaxGroups / kThreads;
     __shared__ int tot[kThreads / 64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -322,7 +333,7 @@ __device__ __forceinline__ int active_prefix(ActiveSet& set, int ng) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int g = threadIdx.x * PER + i;
-        s += g < ng ? set.w[g] : 0;
+        s += g < ng ? w[g] : 0;
     }
     int inc = s;
 #pragma unroll
@@ -338,13 +349,13 @@ __device__ __forceinline__ int active_prefix(ActiveSet& set, int ng) {
     for (int i = 0; i < PER; ++i) {
         const int g = threadIdx.x * PER + i;
         if (g < ng) {
-            set.pre[g] = base;
-            base += set.w[g];
-            if (g == ng - 1) set.pre[ng] = base;
+            pre[g] = base;
+            base += w[g];
+            if (g == ng - 1) pre[ng] = base;
         }
     }
     __syncthreads();
-    return uniform(set.pre[ng]);
+    return uniform(pre[ng]);
 }
 
 // The operator values of a descriptor as the launch's value source.
@@ -727,23 +738,26 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
     // ---- the active problems ----
     int init = 0;
     for (int g = threadIdx.x; g < ng; g += kThreads) {
-        int n = 0;
+        int n = 0, n3 = 0;
         bool any = false;
         for (int p = g * gs; p < min(a.nprob, (g + 1) * gs); ++p) {
             ProbState* st = probs[p].st;
             const bool open = !st->done && probs[p].nslices > 0;
             n += probs[p].nslices;
+            n3 += probs[p].bs == 3 ? probs[p].nslices : 0;
             any |= open;
             init |= open && st->init_pending ? 1 : 0;
         }
         set.w[g] = any ? n : 0;
+        set.w3[g] = any ? n3 : 0;
     }
     init = __syncthreads_or(init);
 
     // this block's part of the active slices; consecutive parts share an XCD
-    int total = 0, first = 0, count = 0, g0 = 0;
+    int total = 0, total3 = 0, first = 0, count = 0, g0 = 0;
     auto cut = [&] {
-        total = active_prefix(set, ng);
+        total = active_prefix(set.w, set.pre, ng);
+        total3 = active_prefix(set.w3, set.pre3, ng);
         const int64_t lb = logical_block();
         first = (int)(lb * total / G);
         count = (int)((lb + 1) * total / G) - first;
@@ -877,7 +891,8 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
     int64_t k = 0;
     for (; k < a.iters && total > 0; ++k) {
         double* pa = a.part + (k & 1) * 4 * ps;
-        if ((int64_t)total <= (int64_t)a.item_slices * G) {
+        if ((int64_t)a.item_slices * total3 + (int64_t)a.item_slices3 * (total - total3) <=
+            (int64_t)a.item_slices * a.item_slices3 * G) {
             // ---- A, slices shared by the block ----
             auto run = [&](auto bs, int p, int s0, int s1) {
                 constexpr int BS = decltype(bs)::value;
@@ -1036,7 +1051,7 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
         }
         if (!grid.sync()) return;
         if (__syncthreads_or(gone)) {
-            if (gone) set.w[gd] = 0;
+            if (gone) set.w[gd] = set.w3[gd] = 0;
             __syncthreads();
             cut();
         }
@@ -1107,6 +1122,9 @@ void table_launch(sfem_ctx* ctx, int precision, const TableLaunch& a0, int grid)
     a.bar_ws = ctx->bar_ws;
     a.bar_timeout = ctx->bar_timeout_ticks;
     a.bar_grouped = ctx->bar_grouped ? 1 : 0;
+    a.item_slices = std::min(a.item_slices, 1 << 20);  // more than any grid has to share
+    const bool wide = precision == SFEM_PREC_FP64 || precision == SFEM_PREC_SPLIT;
+    a.item_slices3 = wide ? std::min(a.item_slices, kShareSlices64) : a.item_slices;
     SFEM_HIP(hipMemsetAsync(a.bar_ws, 0, sizeof(unsigned) * kBarWords, ctx->stream));
     switch (precision) {
         case SFEM_PREC_FP64: launch_table<double, double, false>(ctx, a, grid); break;

@@ -55,6 +55,7 @@ struct TableLaunch {
     const ProbDesc* probs;
     int nprob;
     int item_slices;   // slices a block may hold for its wavefronts to share each of them
+    int item_slices3;  // the same for slices of 3D problems
     int64_t nslices;   // of all problems
     double* part;      // kTableSums per slice
     ProbState* alt;    // second state slot per problem

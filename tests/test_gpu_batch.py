@@ -223,51 +223,70 @@ def test_autotune_picks_a_measured_candidate(ctx, tmp_path, monkeypatch):
     B.close()
 
 
+@pytest.mark.parametrize("ndim", [2, 3])
 @pytest.mark.parametrize("precision,pc", [("fp64", "jacobi"), ("mixed", "block_jacobi"), ("fp32_matrix", "jacobi"),
                                           ("split", "block_jacobi")])
-def test_batch_table_forms_bitwise(ctx, precision, pc):
+def test_batch_table_forms_bitwise(ctx, precision, pc, ndim):
     """The two forms of a pass (a block's wavefronts share each slice and form
     p in the gathers; a wavefront per slice after a pass over p) add the same
-    numbers in the same order: item_slices 64 keeps the first, 1 starts in the
-    second on 256 blocks (at least 300 slices here) and changes over as
-    problems finish, also between launches of 5 passes."""
-    print(f"[case] batch table forms {precision} {pc}", flush=True)
+    numbers in the same order.  item_slices 64 on 512 blocks keeps the first
+    (at most 3 slices a block); 1 starts in the second on 256 blocks, of which
+    32 share an XCD's part of the slices (more than 4 x 32: whole rounds of a
+    slice per wavefront, and a remainder shared slice by slice), and changes
+    over as problems finish, also between launches of 5 passes."""
+    print(f"[case] batch table forms {precision} {pc} {ndim}D", flush=True)
     rng = np.random.default_rng(12)
-    probs = uneven_hex8_problems(36, 21, lo=6, hi=11)
-    for dims in ((3, 6, 2), (4, 3, 3), (1, 12, 4), (3, 15, 3)):  # 63, 64, 65 and 192 free nodes
+    if ndim == 3:
+        probs = uneven_hex8_problems(90, 21, lo=6, hi=12)
+        odd = ((3, 6, 2), (4, 3, 3), (1, 12, 4), (3, 15, 3))  # 63, 64, 65 and 192 free nodes
+    else:
+        probs = []
+        for nx, ny in rng.integers(36, 54, (38, 2)):
+            m = structured_mesh((int(nx), int(ny)))
+            probs.append(make_problem(m, 1.0, 0.3, face_load(m, 0, 1, 1, -1.0), clamp_x0(m)))
+        odd = ((9, 6), (8, 7), (5, 12), (12, 15))  # 63, 64, 65 and 192 free nodes
+    first_odd = len(probs)
+    for dims in odd:
         m = structured_mesh(dims)
-        probs.append(make_problem(m, 1.0, 0.3, face_load(m, 0, 1, 2, -1.0), clamp_x0(m)))
-    m = structured_mesh((2, 2, 2))  # no free dofs: the answer is q_d
+        probs.append(make_problem(m, 1.0, 0.3, face_load(m, 0, 1, ndim - 1, -1.0), clamp_x0(m)))
+    m = structured_mesh((2,) * ndim)  # no free dofs: the answer is q_d
     q_d = rng.standard_normal(m.n_dof)
     probs.append(make_problem(m, 1.0, 0.3, np.zeros(m.n_dof), np.ones(m.n_dof, dtype=clamp_x0(m).dtype), q_d))
     B = Batch(probs, ctx)
+    assert 8 * (4 * 32 + 8) <= B.slices <= 3 * 512
     want = None
-    for isl, check_every in ((64, 0), (1, 0), (1, 5)):
-        st, per = B.solve(precision, rtol=1e-11, item_slices=isl, blocks_per_cu=1, check_every=check_every,
+    for isl, per_cu, check_every in ((64, 2, 0), (1, 1, 0), (1, 1, 5)):
+        st, per = B.solve(precision, rtol=1e-11, item_slices=isl, blocks_per_cu=per_cu, check_every=check_every,
                           preconditioner=pc)
+        assert st["grid"] == per_cu * ctx.device_info()["n_cu"]
         q = B.solution()
         if want is None:
             want = q
         assert all(np.array_equal(a, b) for a, b in zip(q, want)), (isl, check_every)
     B.close()
     assert np.array_equal(want[-1], q_d)
-    for i in (0, 17, 36, 37):
+    for i in (0, 17, first_odd, first_odd + 1):
         assert relerr(want[i], oracle_solution(probs[i])) <= ERR
 
 
 def test_batch_more_problems_than_groups(ctx):
     """More problems than a block tracks one by one (2,048): they are tracked
-    in groups, each problem with the bits it has alone."""
+    in groups, each problem with the bits it has alone, in both forms of a
+    pass (2,100 slices on 512 blocks, and item_slices 1 on 256)."""
     print("[case] batch of 2,100 problems", flush=True)
     probs = []
     for k in range(2100):
         m = structured_mesh((8 + k % 2, 7) if k % 700 == 349 else (1 + k % 5, 1 + k % 3))  # 64 or 72, or few free nodes
         probs.append(make_problem(m, 1.0 + k % 7, 0.3, face_load(m, 0, 1, 1, -1.0), clamp_x0(m)))
     B = Batch(probs, ctx)
+    assert B.slices >= len(probs)
     st, per = B.solve("fp64", rtol=1e-11, item_slices=8)
     qs = B.solution()
-    B.close()
     assert st["not_converged"] == 0
+    st, per = B.solve("fp64", rtol=1e-11, item_slices=1, blocks_per_cu=1)
+    assert st["not_converged"] == 0
+    assert all(np.array_equal(a, b) for a, b in zip(B.solution(), qs))
+    B.close()
     for k in (0, 1, 2, 1049, 2099):
         assert relerr(qs[k], oracle_solution(probs[k])) <= ERR
         A = Batch([probs[k]], ctx)
