@@ -67,6 +67,32 @@ def test_alone_equals_in_mix(ctx, precision, pc):
     S.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_plane_and_solid_requests_share_a_table(ctx, precision):
+    """A table of 2D and 3D requests whose parts are cut by the slices' work
+    (about 1,300 slices on 256 blocks, a slice per wavefront): each has the
+    bits it has alone, in any order of submission."""
+    print(f"[case] serve 2D and 3D {precision}", flush=True)
+    reqs = [request(d, 30 + i) for i, d in enumerate([(200, 120), (40, 20, 20), (4, 2, 2), (150, 160), (36, 22, 18),
+                                                      (9, 7)])]
+    opts = dict(precision=precision, rtol=1e-9, preconditioner="block_jacobi")
+    alone = []
+    for p in reqs:
+        S = Server(ctx, **opts)
+        rid = S.submit(p)
+        S.drain()
+        assert S.poll(rid)["stop_reason"] == 1
+        alone.append(S.take(rid, p.n_dof))
+        S.close()
+    for order in (range(6), (4, 1, 2, 5, 0, 3), (1, 0, 4, 3, 5, 2)):
+        S = Server(ctx, item_slices=1, blocks_per_cu=1, **opts)
+        ids = {i: S.submit(reqs[i]) for i in order}
+        S.drain()
+        for i, rid in ids.items():
+            assert np.array_equal(S.take(rid, reqs[i].n_dof), alone[i]), (tuple(order), i)
+        S.close()
+
+
 def test_partially_fixed_request_in_mix(ctx):
     """A request with a roller plane (only u_z fixed on z = 0) is served next
     to plain cantilevers: same bits alone and in the mix, oracle parity."""
