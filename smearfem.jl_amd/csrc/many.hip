@@ -418,13 +418,19 @@ __global__ void recombine_many_kernel(const int32_t* __restrict__ free_of, const
         q[(int64_t)j * n + s] = row >= 0 ? X[(int64_t)row * kp + j] : (qd ? qd[(int64_t)j * n + s] : 0.0);
 }
 
-// Node rows (or rows) x columns up to which a row is spread over lanes.
-// Measured, a sweep's call on a cube of ne^3 Hex8 with k columns, one lane /
-// several: ne 8, k 1, 4, 16: 3.3 / 2.5, 3.1 / 2.4, 3.5 / 2.8 ms; ne 16: 6.9 /
-// 4.8, 6.5 / 4.8, 10.1 / 8.4; ne 24: 10.8 / 7.3 (k 1), 10.0 / 10.4 (k 4,
-// 62,500 entries), 19.5 / 22.1 (k 16, 250,000); ne 32: 15.4 / 14.3 (k 1), 18.5
-// / 26.4 (k 4, 143,748).
-constexpr int64_t kLaneEntries = 100000;
+// Node rows (or rows) x columns up to which a row is spread over lanes, for
+// rows of 3D operators: KP < 8 and KP >= 8 columns.  Measured with one lane /
+// several.  A sweep's call on a cube of ne^3 Hex8 with k columns, ms: ne 16, k
+// 16 (78,608 entries) 8.5 / 7.9; ne 20, k 4 7.2 / 6.7, k 8 (74,088) 9.1 / 9.1;
+// ne 22, k 6 (97,336) 9.8 / 10.7; ne 24, k 1 10.0 / 6.6, k 4 (62,500) 9.5 /
+// 9.8, k 8 12.4 / 14.7; ne 28, k 2 11.0 / 10.6, k 4 (97,556) 13.4 / 14.3; ne
+// 32, k 1 14.4 / 11.8, k 2 (71,874) 15.2 / 14.7.  A clamped cube, us an
+// iteration: ne 22, k 6 46.7 / 51.7; ne 24, k 4 44.6 / 36.5, k 8 49 / 59; ne
+// 28, k 4 66 / 48; scalar rows, ne 24, k 2 (93,750) 38.6 / 33.1, k 4 36 / 49.
+// Rows of a 2D operator (up to 18 entries) gain nothing at any size: 100 x 100
+// Q4, k 1 20.7 / 22.0, k 4 21.5 / 25.1; 160 x 160, k 1 21.3 / 24.0.
+constexpr int64_t kLaneEntries = 100000, kLaneEntriesWide = 80000;
+constexpr int64_t kLaneRowEntries = 32;  // mean entries of a scalar row from which lanes are taken
 
 template <int KP>
 struct ManyRun {
@@ -457,7 +463,9 @@ struct ManyRun {
         // than about three times over
         constexpr int UPB = kThreadsM / (KP * kRowLanes<KP>);
         const int64_t units = blk ? nunits : nf;
-        const bool lanes = ctx->tune_split > 0 ? ctx->tune_split >= 4 : units * KP <= kLaneEntries;
+        const bool lanes = ctx->tune_split > 0 ? ctx->tune_split >= 4
+                                               : (blk || S->nnz >= kLaneRowEntries * nf) &&
+                                                     units * KP <= (KP < 8 ? kLaneEntries : kLaneEntriesWide);
         const int nbp =
             lanes ? (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)ctx->n_cu * 16, (units + UPB - 1) / UPB)) : nb;
         const int64_t pchunk = ((units + nbp - 1) / nbp + UPB - 1) / UPB * UPB;
