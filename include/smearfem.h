@@ -214,8 +214,9 @@ typedef struct {
     double  rtol;            /* stop when ||rhs - K_ff x||_2 <= rtol ||rhs||_2 (FP64)   */
     int64_t max_iter;        /* cap on CG iterations (all precisions)                    */
     double  reliable_delta;  /* mixed: FP64 update when the FP32 residual drops by this  */
-    int     check_every;     /* iterations enqueued between host convergence polls      */
-    int     time_kernels;    /* 1: time every SpMV launch with HIP events                */
+    int     check_every;     /* iterations (and FP64 residuals) enqueued between host polls;
+                                at most 64 with time_kernels                             */
+    int     time_kernels;    /* 1: time every operator pass with HIP events              */
     int     x0_zero;         /* 1: start from x = 0 (else from the system's current x)   */
     int     preconditioner;  /* SFEM_PC_*                                                */
 } sfem_solve_opts;
@@ -232,9 +233,10 @@ typedef struct {
     int64_t spmv64_launches; /* FP64 residual SpMVs                                      */
     double  rel_residual;    /* final ||rhs - K_ff x|| / ||rhs|| evaluated in FP64       */
     double  solve_ms;        /* device time of the solve (HIP events)                    */
-    double  spmv_ms;         /* summed device time of timed SpMV launches                */
-    double  spmv_bytes;      /* algorithmic bytes of one iteration SpMV                  */
-    int64_t spmv_timed;      /* number of SpMV launches that were timed                  */
+    double  spmv_ms;         /* summed device time of the iterations' operator passes    */
+    double  spmv_bytes;      /* algorithmic bytes of one such pass (on small systems the
+                                pass also forms the direction: z read, p written)        */
+    int64_t spmv_timed;      /* number of those passes (FP64 residuals are left out)     */
     int     converged;
     int     format;          /* format actually used                                     */
     int     stop_reason;     /* 1 converged, 2 breakdown, 3 stagnation, 4 iteration cap  */

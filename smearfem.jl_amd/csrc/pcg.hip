@@ -147,6 +147,10 @@ __device__ __forceinline__ PassGo pass_begin(const CgState* __restrict__ in, CgS
         }
         s.fresh = 0;
         s.resid = s.need_update;
+        if (!s.done) {
+            s.passes += 1;
+            s.resid_bits = s.resid_bits << 1 | (unsigned long long)s.resid;
+        }
         *shgo = PassGo{s.beta, s.zcoef, s.done, s.resid};
         if (blockIdx.x == 0) *out = s;
     }
@@ -774,9 +778,11 @@ Vals<SplitVal> sell_vals<SplitVal>(const sfem_system* S) { return {S->sval32.get
 template <typename TV>
 constexpr double val_bytes() { return std::is_same<TV, SplitVal>::value ? 6.0 : (double)sizeof(TV); }
 
-// One operator pass: state st->s[0] -> st->s[1].
+// One operator pass: state st->s[0] -> st->s[1].  begin: an event recorded in
+// front of the operator's own kernel, or NULL.
 template <typename TV, typename T>
-void launch_pass(const Ops& o, const PassVecs<T>& v, CgStates* st, const double* upd, double* parts) {
+void launch_pass(const Ops& o, const PassVecs<T>& v, CgStates* st, const double* upd, double* parts,
+                 hipEvent_t begin) {
     constexpr bool FOLD = std::is_same<T, float>::value;
     sfem_system* S = o.S;
     hipStream_t s = o.ctx->stream;
@@ -789,6 +795,7 @@ void launch_pass(const Ops& o, const PassVecs<T>& v, CgStates* st, const double*
         SFEM_LAUNCH_CHECK();
         in = out;
     }
+    if (begin) SFEM_HIP(hipEventRecord(begin, s));
     if (o.fmt == SFEM_FMT_BSR) {
         auto run = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(o.sell.grid), dim3(kThreads), 0, s, S->sl_ptr.get(), S->sl_w.get(),
@@ -1008,9 +1015,11 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
         SFEM_HIP(hipEventCreate(&t1));
     }
     const auto w0 = std::chrono::steady_clock::now();
-    const int check = std::max(1, o->check_every);
+    const bool time_passes = o->time_kernels && timed_run;
+    // the state tells which of the last 64 passes were residuals
+    const int check = std::max(1, time_passes ? std::min(o->check_every, 64) : o->check_every);
     std::vector<hipEvent_t> ev;
-    if (o->time_kernels && timed_run) {
+    if (time_passes) {
         ev.resize(2 * (size_t)check);
         for (auto& e : ev) SFEM_HIP(hipEventCreate(&e));
     }
@@ -1028,26 +1037,27 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     // a residual replacement, and the device stops at the iteration cap
     for (int64_t chunk = 1; !host.done; chunk = check) {
         for (int64_t k = 0; k < chunk; ++k) {
-            if (!ev.empty()) SFEM_HIP(hipEventRecord(ev[2 * k], ctx->stream));
-            launch_pass<TV, T>(ops, v, st, upd, parts);
-            if (!ev.empty()) SFEM_HIP(hipEventRecord(ev[2 * k + 1], ctx->stream));
+            launch_pass<TV, T>(ops, v, st, upd, parts, time_passes ? ev[2 * k] : nullptr);
+            if (time_passes) SFEM_HIP(hipEventRecord(ev[2 * k + 1], ctx->stream));
             launch_update<T>(ops, v, x, x64, st, parts, upd);
             T *const po = v.pnew, *const zo = v.znew;  // in place: the same arrays
             v.pnew = const_cast<T*>(v.p), v.znew = const_cast<T*>(v.z);
             v.p = po, v.z = zo;
         }
         d2h(ctx, &host, &st->s[0], sizeof(host));
-        if (!ev.empty()) {
-            // launches after the stop exit at once; time only the real ones
-            const int64_t real = std::min<int64_t>(chunk, std::max<int64_t>(0, host.iters + host.updates - counted));
+        if (time_passes) {
+            // launches after the stop exit at once: the first `real` of the
+            // chunk ran; residuals among them are another operator
+            const int64_t real = host.passes - counted;
             for (int64_t k = 0; k < real; ++k) {
+                if (host.resid_bits >> (real - 1 - k) & 1) continue;
                 float ms = 0;
                 SFEM_HIP(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]));
                 spmv_ms += ms;
+                ++timed;
             }
-            timed += real;
         }
-        counted = host.iters + host.updates;
+        counted = host.passes;
     }
     if (FOLD) {  // x = x64 + xs
         hipLaunchKernelGGL(fold_kernel, dim3(ops.vec.grid), dim3(kThreads), 0, ctx->stream, x64, (float*)xsv, nf);
@@ -1075,8 +1085,9 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     stats->solve_ms = total;
     stats->spmv_ms = spmv_ms;
     stats->spmv_timed = timed;
-    // spmv_cg: matrix once, p read once, q written
-    stats->spmv_bytes = spmv_bytes_for(S, fmt, val_bytes<TV>(), sizeof(T), 2);
+    // the operator pass: matrix once, p read once, q written; where it also
+    // forms p, z read and the new p written
+    stats->spmv_bytes = spmv_bytes_for(S, fmt, val_bytes<TV>(), sizeof(T), ops.fly ? 4 : 2);
     stats->converged = host.done == 1 ? 1 : 0;
     stats->format = fmt;
     stats->stop_reason = host.done;

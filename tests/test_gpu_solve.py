@@ -250,3 +250,35 @@ def test_operator_pass_forms(dims, split, monkeypatch):
     bc.close()
     K.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("split,fmt", [("1", "bsr"), ("4", "bsr"), ("1", "csr")])
+def test_operator_pass_timing(split, fmt, monkeypatch):
+    # time_kernels: every iteration's operator pass is timed, FP64 residuals
+    # are not, whatever the polling interval; the bytes are those of one pass:
+    # the matrix, p and q, and z and the new p where the pass forms p
+    print(f"[case] pass timing split={split} {fmt}", flush=True)
+    monkeypatch.setenv("SFEM_SELL_SPLIT", split)
+    ctx = smearfem.Context(0)
+    m = structured_mesh((24, 8, 8))
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=17)
+    fixed = clamp_x0(m)
+    K = device_K(ctx, m, young)
+    bc = BoundaryConditions(ctx, K.shape[0], random_face_load(m, 2, 1, fixed, seed=18), fixed)
+    S = System(K, bc)
+    n, nnz, slices = S.n_free, S.nnz, -(-(S.n_free // 3) // 64)
+    vecs = 4 if split == "4" or fmt == "csr" else 2  # CSR forms p in its gathers up to 100,000 dofs
+    modes = [("fp64", 8, 8), ("mixed", 4, 4)] + ([("split", 6, 8)] if fmt == "bsr" else [])
+    for precision, vb, xb in modes:
+        plain = S.solve(precision, fmt, rtol=1e-10)
+        for every in (1, 7, 64, 200):
+            st = S.solve(precision, fmt, rtol=1e-10, check_every=every, time_kernels=True)
+            assert st["iterations"] == plain["iterations"] and st["fp64_updates"] == plain["fp64_updates"] > 2
+            assert st["spmv_timed"] == st["iterations"] and 0.0 < st["spmv_ms"] < st["solve_ms"]
+        if fmt == "bsr":
+            op = nnz // 9 * (9 * vb + 4) + 12 * slices + 8
+        else:
+            op = nnz * (vb + 4) + 4 * (n + 1)
+        assert st["spmv_bytes"] == op + vecs * n * xb
+    for h in (S, bc, K, ctx):
+        h.close()
