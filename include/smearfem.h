@@ -245,7 +245,8 @@ typedef struct {
     double  smooth_ms;       /* multigrid, time_kernels: summed device time of the timed
                                 finest-level smoothing steps (FP32 operator)             */
     int64_t smooth_timed;    /* number of those launches                                 */
-    double  smooth_bytes;    /* algorithmic bytes of one finest-level smoothing step     */
+    double  smooth_bytes;    /* algorithmic bytes of one finest-level smoothing step (the
+                                mean over a V-cycle's steps)                             */
 } sfem_solve_stats;
 
 void sfem_solve_opts_default(sfem_solve_opts* opts);

@@ -3684,7 +3684,8 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
     // a smoothing step: FP16 or FP32 operator once (matrix-free: the node map,
     // ghost-layer row and one cell scale per row, the fixed flags), v
     // gathered, r and x read and written, d read and written, the 3x3 (2x2)
-    // inverse blocks read
+    // inverse blocks read; of a V-cycle's per_iter steps the last also reads
+    // the outer FP64 residual
     stats->smooth_ms = smooth_ms;
     stats->smooth_timed = timed;
     if (H.mf)
@@ -3692,6 +3693,7 @@ void mg_pcg(sfem_ctx* ctx, sfem_system* S, MgHierarchy& H, const sfem_solve_opts
     else
         stats->smooth_bytes = (double)S->nnzb * (BS * BS * (H.fp16 ? 2.0 : 4.0) + 4.0) +
                               (double)(S->nslices + 1) * 8.0 + (double)S->nslices * 4.0 + (double)n * 4.0 * (7.0 + BS);
+    stats->smooth_bytes += 8.0 * (double)n / per_iter;
 }
 
 template <int ND>

@@ -680,3 +680,29 @@ def test_refused_hierarchy_leaves_the_context_usable(ctx):
         assert st["converged"] and relerr(S.solution(), q_ref) <= ERR
     S.close()
     K.close()
+
+
+@pytest.mark.parametrize("grid", [True, False])
+@pytest.mark.parametrize("degree", [1, 2, 3])
+def test_smoothing_step_bytes(ctx, grid, degree):
+    # the mean bytes of a V-cycle's 2 degree - 1 finest-level steps: operator,
+    # vectors and inverse blocks, and in the last step the outer FP64 residual
+    print(f"[case] smoothing bytes grid={grid} degree={degree}", flush=True)
+    m = structured_mesh((24, 8, 8))
+    young = element_young_loguniform(m.n_elem, 0.1, 10.0, seed=17)
+    fixed = clamp_x0(m)
+    mesh = smearfem.Mesh(ctx, m.n_elem, m.NodeList, m.IEN, m.ndim, "Q1", m.ndim, m.ID, young, 0.3)
+    if grid:
+        mesh.set_grid(m.dims)
+    K = mesh.assemble()
+    bc = BoundaryConditions(ctx, K.shape[0], random_face_load(m, 2, 1, fixed, seed=18), fixed)
+    S = System(K, bc)
+    S.set_grid(m.dims, degree=degree)
+    st = S.solve("fp64", rtol=1e-10, preconditioner="multigrid", time_kernels=True)
+    n, rows = S.n_free, S.n_free // 3
+    slices = -(-rows // 64)
+    step = rows * (12 + 3) + n * 4 * 9 if grid else S.nnz // 9 * (9 * 2 + 4) + 12 * slices + 8 + n * 4 * 10
+    assert st["smooth_timed"] > 0 and st["smooth_ms"] > 0.0
+    assert st["smooth_bytes"] == pytest.approx(step + 8 * n / (2 * degree - 1), rel=1e-12)
+    for h in (S, bc, K, mesh):
+        h.close()
