@@ -709,7 +709,12 @@ __global__ __launch_bounds__(kThreads) void copy_kernel(const v4f* __restrict__ 
 }
 
 // --------------------------------------------------------- host side ---
-constexpr int64_t kFlyDofs = 100000;  // scalar CSR: p formed in the gathers up to this many dofs
+// Scalar CSR: p formed in the gathers up to this many dofs.  us an iteration
+// with p in the gathers / by direction_kernel, FP64 Jacobi: 3D, 1,944 dofs 12.1
+// / 15.1, 20,808 16.2 / 18.7, 60,000 29.2 / 26.9, 90,000 36.8 / 33.1, 322,752
+// 128 / 100; 2D, 7,320 dofs 13.3 / 15.0, 45,300 21.5 / 19.0, 97,240 25.8 /
+// 21.7; mixed precision turns at the same sizes.
+constexpr int64_t kFlyDofs = 30000;
 constexpr int kCsrLanes = 16;  // lanes per CSR row (rows of K_ff hold up to 81 entries)
 
 struct Launch {

@@ -267,7 +267,7 @@ def test_operator_pass_timing(split, fmt, monkeypatch):
     bc = BoundaryConditions(ctx, K.shape[0], random_face_load(m, 2, 1, fixed, seed=18), fixed)
     S = System(K, bc)
     n, nnz, slices = S.n_free, S.nnz, -(-(S.n_free // 3) // 64)
-    vecs = 4 if split == "4" or fmt == "csr" else 2  # CSR forms p in its gathers up to 100,000 dofs
+    vecs = 4 if split == "4" or fmt == "csr" else 2  # CSR forms p in its gathers up to 30,000 dofs
     modes = [("fp64", 8, 8), ("mixed", 4, 4)] + ([("split", 6, 8)] if fmt == "bsr" else [])
     for precision, vb, xb in modes:
         plain = S.solve(precision, fmt, rtol=1e-10)
@@ -281,4 +281,26 @@ def test_operator_pass_timing(split, fmt, monkeypatch):
             op = nnz * (vb + 4) + 4 * (n + 1)
         assert st["spmv_bytes"] == op + vecs * n * xb
     for h in (S, bc, K, ctx):
+        h.close()
+
+
+@pytest.mark.parametrize("dims", [(121, 122), (122, 122), (122, 123), (25, 19, 19)])
+def test_csr_pass_forms(ctx, dims):
+    # the scalar CSR operator pass on both sides of the 30,000 dofs up to which
+    # it forms p in its gathers (29,766, 30,012, 30,256 and 30,000 dofs)
+    print(f"[case] csr pass {dims}", flush=True)
+    m = structured_mesh(dims)
+    fixed = clamp_x0(m)
+    f = random_face_load(m, m.ndim - 1, 1, fixed, seed=21)
+    q_ref, Kr = oracle_direct(m, fixed, f)
+    K = device_K(ctx, m)
+    bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+    S = System(K, bc)
+    for precision in ("fp64", "mixed", "fp32_matrix"):
+        st = S.solve(precision, "csr", rtol=1e-11, time_kernels=True)
+        assert st["stop_reason"] in (1, 3) and relerr(S.solution(), q_ref) <= ERR, precision
+        vecs = 4 if S.n_free <= 30000 else 2
+        vb, xb = {"fp64": (8, 8), "mixed": (4, 4), "fp32_matrix": (4, 8)}[precision]
+        assert st["spmv_bytes"] == S.nnz * (vb + 4) + 4 * (S.n_free + 1) + vecs * S.n_free * xb
+    for h in (S, bc, K):
         h.close()
