@@ -3776,6 +3776,14 @@ void mg_solve(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solv
     else mg_solve_nd<2>(ctx, S, o, st);
 }
 
+int64_t mg_direct_bound(int64_t n) {
+    sfem_mg_opts o;
+    mg_opts_default(&o);
+    // the first level of at most direct_dofs() dofs, or the coarsest
+    const int64_t most = std::max<int64_t>(direct_dofs(), 3 * o.coarse_nodes);
+    return (std::min(n, std::min<int64_t>(most, 3 * 2 * kMgMaxCoarseNodes)) + kTile - 1) / kTile * kTile;
+}
+
 void mg_info(const sfem_system* S, sfem_mg_info* info) {
     *info = sfem_mg_info{};
     if (!S->mg) fail(SFEM_ERR_STATE, "multigrid: no hierarchy (sfem_system_set_grid)");

@@ -54,6 +54,7 @@ struct Request {
     std::vector<int64_t> ien;
     std::vector<uint8_t> fixed;
     int64_t est_resident = 0, est_transient = 0, bytes = 0;
+    int64_t est_inverse = 0;  // multigrid: the direct level's two dense matrices
     sfem_batch* B = nullptr;
     int slot = -1;
     std::vector<double> result;
@@ -145,6 +146,8 @@ void estimate_bytes(Request& r, int precision) {
                      rows * b2 * 12 + r.n_nodes * 4 + r.n_nodes * bs * 8;
     const int64_t ke = (int64_t)nen * bs * nen * bs;
     r.est_transient = r.est_resident + r.n_elem * (ke * 8 + (int64_t)nen * nen * 24) + slots * (8 + b2 * 8);
+    const int64_t np = mg_direct_bound(r.n_nodes * bs);
+    r.est_inverse = 2 * np * np * (int64_t)sizeof(double);
 }
 
 double launch_ms(sfem_server* S) {
@@ -398,10 +401,12 @@ void step_grid(sfem_server* S, int* n_finished, double* ms) {
         }
         if (!idle) break;
         Request& r = S->reqs.at(S->gqueue.front());
-        // the request's build and hierarchy are held only while it is solved
-        const int64_t need = r.est_transient + r.est_transient / 2;
-        if (S->bytes_in_use + need > S->o.hbm_budget) {
-            if (!S->active.empty() || busy) break;  // wait for memory to free up
+        // the request's build and hierarchy are held only while it is solved;
+        // on an idle device the dense inverse alone turns no request away
+        const int64_t built = r.est_transient + r.est_transient / 2, need = built + r.est_inverse;
+        const bool idle_device = S->active.empty() && !busy;
+        if (S->bytes_in_use + (idle_device ? built : need) > S->o.hbm_budget) {
+            if (!idle_device) break;  // wait for memory to free up
             r.state = SFEM_REQ_FAILED;
             r.error = "request does not fit the HBM budget";
             r.t_fin = S->now_ms();

@@ -285,6 +285,9 @@ void stream_copy_bench(sfem_ctx* ctx, int64_t bytes, int reps, double* avg_ms);
 void mg_opts_default(sfem_mg_opts* o);
 void system_set_grid(sfem_ctx* ctx, sfem_system* S, int ndim, const int64_t* dims, const sfem_mg_opts* opts);
 void mg_solve(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve_stats* st);
+// Order of the direct level's dense matrix, at most, for a system of n dofs
+// with the default options.
+int64_t mg_direct_bound(int64_t n);
 void mg_info(const sfem_system* S, sfem_mg_info* info);
 void mg_stencil(sfem_ctx* ctx, const sfem_system* S, int level, double* stencil, uint8_t* fixed);
 }  // namespace sfem

@@ -176,6 +176,35 @@ def test_hbm_budget_admission(ctx):
     S.close()
 
 
+@pytest.mark.parametrize("dims,order", [((38, 38), 800), ((12, 9), 288), ((40, 20, 20), 800)])
+def test_multigrid_reservation_holds_the_dense_inverse(ctx, dims, order):
+    """A multigrid request reserves the direct level's two dense matrices (at
+    most 800 dofs, or the request's own, to whole blocks of 32) with its build;
+    on an idle device they turn no request away."""
+    print(f"[case] serve reservation {dims}", flush=True)
+    p = request(dims, 40)
+    opts = dict(precision="fp64", rtol=1e-10, preconditioner="multigrid", mg_workers=1)
+
+    def reserved(budget):
+        for _ in range(20):  # a request may be done within its own step
+            S = Server(ctx, hbm_budget=budget, **opts)
+            rid = S.submit(p)
+            S.step()
+            held = S.info()["bytes"]
+            S.drain()
+            state = S.poll(rid)["state"]
+            S.close()
+            if held or state == "failed":
+                break
+        return held, state
+
+    held, state = reserved(64 << 30)
+    inverse = 2 * order ** 2 * 8
+    assert state == "done" and held > inverse
+    assert reserved(held - inverse) == (held, "done")
+    assert reserved(held - inverse - 1) == (0, "failed")
+
+
 def test_poisson_stream_small(ctx):
     print("[case] serve poisson", flush=True)
     rng = np.random.Generator(np.random.PCG64(7))
