@@ -516,11 +516,14 @@ int  sfem_batch_create_specs(sfem_ctx* ctx, int64_t nprob, const sfem_problem_sp
 int  sfem_batch_info(const sfem_batch* b, int64_t* n_total, int64_t* n_padded, int64_t* slices,
                      double* assemble_ms, double* eliminate_ms);
 /* Solve every problem.  item_slices: active 64-row slices per block up to
- * which a block's wavefronts share each slice (more: a wavefront per slice);
- * results do not depend on it;
+ * which a block's wavefronts share each slice (more: a wavefront per slice;
+ * 3 at most count for 3D slices in precision FP64 and SPLIT); results do not
+ * depend on it;
  * blocks_per_cu: persistent grid = blocks_per_cu * CUs (0 = default; capped
  * at residency).  opts->check_every > 0 splits the solve into launches of
- * that many iterations; <= 0 runs it in one launch.  per: nprob entries or
+ * that many steps, an iteration or an FP64 residual of a problem each (a
+ * residual is due at the start, at a 10x drop by default and to confirm the
+ * end); <= 0 runs it in one launch.  per: nprob entries or
  * NULL.  Returns SFEM_ERR_NOT_CONVERGED if any problem did not converge. */
 int  sfem_batch_solve(sfem_ctx* ctx, sfem_batch* b, const sfem_solve_opts* opts, int item_slices,
                       int blocks_per_cu, sfem_batch_problem_stats* per, sfem_batch_stats* stats);
@@ -535,8 +538,8 @@ void sfem_batch_destroy(sfem_batch* b);
  * inputs as a one-problem batch) queue on the host; each step admits queued
  * requests in arrival order while their device footprint fits the HBM
  * budget and a slot is free (assembly + elimination on the device), runs
- * iters_per_step iterations of every active request in one persistent
- * launch, and retires the finished ones (solution copied to the host, device
+ * iters_per_step steps (an iteration or an FP64 residual each) of every
+ * active request in one persistent launch, and retires the finished ones (solution copied to the host, device
  * memory released).  A request's result does not depend on what else is
  * active: it is bitwise the result it gets alone.
  * With preconditioner = SFEM_PC_MULTIGRID, requests submitted with their
@@ -561,7 +564,7 @@ typedef struct {
     int     blocks_per_cu;
     int64_t hbm_budget;       /* bytes admitted requests may hold on the device           */
     int     max_active;       /* cap on concurrently active requests                      */
-    int     iters_per_step;   /* CG iterations per persistent launch                      */
+    int     iters_per_step;   /* steps per persistent launch (iterations and residuals)   */
     int     preconditioner;   /* SFEM_PC_*                                                */
     int     mg_workers;       /* multigrid servers: requests solved at once, each by a host
                                  thread with its own stream (4)                            */

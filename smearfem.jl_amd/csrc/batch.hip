@@ -264,13 +264,13 @@ __global__ void fold_all_kernel(double* __restrict__ x64, float* __restrict__ xs
 // iteration the grid meets at a barrier, and a problem's scalars are formed by
 // the blocks that need them.  Per iteration:
 //
-//   A  per run of slices of one problem: the sums the last pass left (r.z, r.r
-//      and p.q of an update, or the sums of an FP64 residual) give beta, the
+//   A  per run of slices of one problem: the sums the last pass left (r.z and
+//      r.r of an update, or the sums of an FP64 residual) give beta, the
 //      stopping tests and what comes next; then either the FP64 residual of
 //      the run's rows, if it is due, or q = K p with p = zcoef z + beta p
 //      formed in the gathers (p has two buffers), and the slice partials of p.q
-//   U  alpha from the partials of p.q; x += alpha p; r -= alpha q;
-//      z = M^-1 r; slice partials of r.z and r.r
+//   U  alpha from the partials of p.q, whose sum is left for the next A;
+//      x += alpha p; r -= alpha q; z = M^-1 r; slice partials of r.z and r.r
 //
 // The block that holds a problem's first slice writes its new state to the
 // other of two state slots, so no block reads what another one writes.  What

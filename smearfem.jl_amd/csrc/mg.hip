@@ -1821,7 +1821,7 @@ __global__ __launch_bounds__(kThreads) void mg_check_kernel(MgState* st, const d
 
 // direct level: x = A^-1 b with the dense FP64 inverse (row stride np), a
 // wavefront per row (the row read coalesced, the loads of eight strides in
-// flight, a fixed butterfly).  1,275 dofs: 13 MB, from the caches.
+// flight, a fixed butterfly).  800 dofs: 5 MB, from the caches; a launch.
 // Its first block also takes the last update's r.r (take_rr).
 __global__ __launch_bounds__(kThreads) void dense_apply_kernel(const double* __restrict__ inv, int nc, int np,
                                                                const float* __restrict__ b, float* __restrict__ x,

@@ -34,7 +34,8 @@
 // state, a last-block arrival, its partials), not by bytes: at 64x16x16 Hex8
 // (18.5k nodes, FP64) four kernels with last-block reductions took 41 us an
 // iteration.
-// The host reads the state every `check_every` iterations.
+// The host reads the state every `check_every` steps (an iteration or an FP64
+// residual each).
 //
 // Reductions are deterministic: wave64 butterfly shuffles, a fixed combine
 // of a block's wavefronts, per-block partials summed in a fixed order.  The

@@ -5,10 +5,11 @@
 // arrival order while a slot is free and their device footprint fits the HBM
 // budget -- each admitted request is assembled and eliminated on the device
 // into its own padded sliced operator (a one-problem batch) and gets a CG
-// state slot; (2) run iters_per_step iterations of every active request in
-// one cooperative launch; (3) retire finished requests: solution to the host,
-// device memory back to the allocator.  Requests that arrive while others
-// run join at the next step and share the launch with them.
+// state slot; (2) run iters_per_step steps (an iteration or an FP64 residual
+// each) of every active request in one cooperative launch; (3) retire
+// finished requests: solution to the host, device memory back to the
+// allocator.  Requests that arrive while others run join at the next step and
+// share the launch with them.
 //
 // A request's arithmetic depends only on its own operator and precision
 // (per-problem reductions over its own slices, state in memory), so

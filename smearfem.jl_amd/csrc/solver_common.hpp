@@ -101,16 +101,6 @@ __device__ __forceinline__ void thread_partials(const double* partials, int npar
         for (int k = 0; k < W; ++k) s[k] += ld_coherent(partials + (int64_t)W * i + k);
 }
 
-// Fixed-order sum of nparts partial quadruples (stride 4) by one block.
-__device__ __forceinline__ void sum_partials4(const double* partials, int nparts, double out[4], double* sh) {
-    double s[4];
-    thread_partials<4>(partials, nparts, s);
-    out[0] = block_sum_256(s[0], sh);
-    out[1] = block_sum_256(s[1], sh + 4);
-    out[2] = block_sum_256(s[2], sh);
-    out[3] = block_sum_256(s[3], sh + 4);
-}
-
 // Fixed-order sum of nparts partial triples (stride 3) by one block.
 __device__ __forceinline__ void sum_partials3(const double* partials, int nparts, double* a, double* b, double* c,
                                               double* sh) {

@@ -3,8 +3,9 @@
 No counterpart in the reference.  ``Server`` wraps ``sfem_server_*``
 (serve.hip): requests queue on the host, each ``step`` admits queued
 requests in arrival order while a slot is free and their device footprint
-fits the HBM budget, runs ``iters_per_step`` CG iterations of every active
-request in one persistent launch and retires the finished ones.  A request's
+fits the HBM budget, runs ``iters_per_step`` steps (a CG iteration or an FP64
+residual each) of every active request in one persistent launch and retires
+the finished ones.  A request's
 result is bitwise the same alone or in any mix.
 
 ``run_poisson`` drives a server with a Poisson arrival stream in wall-clock

@@ -3,8 +3,8 @@
 Bar: every problem's displacement within 1e-8 relative of a direct FP64 solve
 of the oracle's K for that problem alone (rtol 1e-12), in every precision.
 Invariance: a problem's solution is bitwise the same alone, inside a batch,
-for any persistent grid size and for any split of the solve over launches
-(same item_slices).
+for any persistent grid size and item_slices and for any split of the solve
+over launches.
 """
 import numpy as np
 import pytest
