@@ -710,6 +710,30 @@ __global__ __launch_bounds__(kThreads) void copy_kernel(const v4f* __restrict__ 
 }
 
 // --------------------------------------------------------- host side ---
+// Slices up to which a block's four wavefronts share a slice and form p in the
+// gathers; above, a wavefront takes a slice and direction_kernel forms p.  A
+// small system else has fewer wavefronts than the device holds, each with up
+// to 27 block columns of loads one after the other; on a larger one the second
+// gathered vector costs more, most of all where the nodes are numbered in no
+// particular order.  Node-block Jacobi, us an iteration, one wavefront / four:
+//   grid numbering  FP64 276 slices 28.8 / 19.1, 625 30.7 / 26.2, 1,225 49.6 /
+//     42.2, 1,541 51.6 / 51.3, 3,038 99.6 / 107.7; FP32 values (fp32_matrix)
+//     1,225 36.1 / 33.8, 1,541 38.4 / 40.0, 4,802 98.5 / 117.5
+//   shuffled  FP64 1,225 61.6 / 56.9, 1,369 62.2 / 66.2, 1,712 75.6 / 83.2;
+//     split 1,225 59.0 / 51.4, 1,541 60.1 / 68.3; fp32_matrix 1,225 49.3 / 49.3,
+//     1,369 48.8 / 56.3, 4,802 155.6 / 224.3; mixed 1,369 44.1 / 43.7, 1,712
+//     46.7 / 52.1, 4,802 128.3 / 174.4
+//   2D, shuffled  FP64 1,177 26.4 / 25.2, 1,449 27.7 / 28.2; split 1,177 24.4 /
+//     24.8, 1,355 25.9 / 28.8
+constexpr int64_t kSharedSlices = 1280;
+
+// Operator bytes from which its loads are non-temporal (a wavefront per slice):
+// where it no longer stays in the 256 MB memory-side cache between iterations.
+// us an iteration without / with: 211 MB (split) 60.7 / 67.2, 259 MB (mixed)
+// 64.8 / 66.7, 276 MB (FP64) 77.7 / 79.3, 305 MB (split) 78.6 / 76.3, 332 MB
+// (mixed) 91.8 / 84.2, 376 MB (split) 104.8 / 94.6, 399 MB (FP64) 99.6 / 91.7.
+constexpr double kStreamBytes = 290e6;
+
 // Scalar CSR: p formed in the gathers up to this many dofs.  us an iteration
 // with p in the gathers / by direction_kernel, FP64 Jacobi: 3D, 1,944 dofs 12.1
 // / 15.1, 20,808 16.2 / 18.7, 60,000 29.2 / 26.9, 90,000 36.8 / 33.1, 322,752
@@ -956,9 +980,10 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     ops.fly = nf <= kFlyDofs;
     if (fmt == SFEM_FMT_BSR) {
         const double op_bytes = spmv_bytes_for(S, fmt, val_bytes<TV>(), 0, 0);
-        ops.split = slice_split(ctx, S->nslices, S->bs, op_bytes);
+        const bool share = ctx->tune_split > 0 ? ctx->tune_split >= 4 : S->nslices <= kSharedSlices;
+        ops.split = share ? 4 : 1;
         ops.fly = ops.split > 1;
-        ops.nt = stream_loads(ctx, op_bytes);
+        ops.nt = ctx->tune_nt && op_bytes > kStreamBytes;
         if (ops.split > 1) {  // a block per slice
             ops.sell = {(unsigned)std::max<int64_t>(8, (S->nslices + 7) / 8 * 8), 1};
         } else {

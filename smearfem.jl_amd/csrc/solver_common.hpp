@@ -467,20 +467,17 @@ __device__ __forceinline__ void sell_row_abs(const int64_t* __restrict__ sl_ptr,
     }
 }
 
-// Wavefronts per slice of a sliced operator: 1, or 4 (a block per slice; in
-// the Jacobi CG p is then formed in the operator's gathers, else by
-// direction_kernel).  A wavefront per slice
-// leaves a small system with fewer wavefronts than the device holds, each
-// with up to 27 block columns of loads one after the other.  Measured on
-// MI355X, us per iteration with 1 / 4 wavefronts (1: plus direction_kernel):
-// 3D FP64 Jacobi 7 slices 19.8 / 12.6, 294 slices 24.3 / 15.8, 948 slices
-// 32.1 / 27.8, 2,196 slices 71.9 / 63.5, 4,229 slices (578 MB) 126.7 / 138.8,
-// 16,967 slices 464 / 543; mixed block Jacobi 2,196 slices 38.4 / 33.5,
-// 4,229 slices (304 MB) 71.5 / 67.8, 7,241 slices (521 MB) 111 / 128.  So the
-// line is where the operator leaves the 256 MB memory-side cache (and
-// non-temporal loads begin to pay, see stream_loads).  2D FP64 (9 block
-// columns): 30 slices 14.0 / 10.4, 711 slices 15.3 / 12.9, 1,965 slices
-// 22.9 / 23.6, 3,297 slices 30.1 / 31.6.  8 wavefronts gain nothing over 4.
+// Wavefronts per slice of a sliced operator in the multigrid solve: 1, or 4 (a
+// block per slice; in the outer CG p is then formed in the operator's
+// gathers).  A wavefront per slice leaves a small system with fewer wavefronts
+// than the device holds, each with up to 27 block columns of loads one after
+// the other.  Distorted 3D grids, FP64, us per iteration with 1 / 4 wavefronts
+// for the outer operator and the FP16 smoother alike: 276 slices 133 / 109,
+// 1,089 174 / 149, 2,102 264 / 246, 3,752 329 / 360, 4,802 407 / 430, 8,450
+// 743 / 756; with this rule (the smoother's 22 bytes a block still shared) 326,
+// 389 and 717 at the last three.  2D (9 block columns): 190 slices 93 / 84,
+// 1,177 130 / 126, 2,468 160 / 159, 8,452 279 / 307.  8 wavefronts gain nothing
+// over 4.
 constexpr double kSharedBytes = 400e6;    // 3D: operator bytes
 constexpr int64_t kSharedSlices2 = 1536;  // 2D: slices
 inline int slice_split(const sfem_ctx* ctx, int64_t nslices, int bs, double operator_bytes) {
@@ -488,9 +485,8 @@ inline int slice_split(const sfem_ctx* ctx, int64_t nslices, int bs, double oper
     return (bs == 3 ? operator_bytes <= kSharedBytes : nslices <= kSharedSlices2) ? 4 : 1;
 }
 
-// Non-temporal operator loads pay once the operator no longer stays in the
-// memory-side cache between iterations (FP64, a wavefront per slice: 300 MB
-// 72.9 us without and 71.9 with, 990 MB 228 and 207).
+// Non-temporal operator loads in the multigrid solve: once the operator no
+// longer stays in the memory-side cache between iterations.
 inline bool stream_loads(const sfem_ctx* ctx, double operator_bytes) {
     return ctx->tune_nt && operator_bytes > kSharedBytes;
 }

@@ -304,3 +304,31 @@ def test_csr_pass_forms(ctx, dims):
         assert st["spmv_bytes"] == S.nnz * (vb + 4) + 4 * (S.n_free + 1) + vecs * S.n_free * xb
     for h in (S, bc, K):
         h.close()
+
+
+@pytest.mark.parametrize("dims", [(320, 255), (320, 256)])
+def test_operator_pass_line(ctx, dims):
+    # 1,280 slices, the last size whose slices a block's wavefronts share, and
+    # 1,285: both against a direct solve, in a shuffled numbering, and the
+    # bytes of the pass tell the form (z read and p written, or not)
+    print(f"[case] operator pass line {dims}", flush=True)
+    m = structured_mesh(dims, lengths=tuple(d / max(dims) for d in dims))
+    fixed = clamp_x0(m)
+    f = random_face_load(m, 1, 1, fixed, seed=22)
+    perm = np.random.default_rng(23).permutation(m.n_nodes)
+    inv = np.argsort(perm)
+    f, fixed = f.reshape(-1, 2)[inv].ravel(), fixed.reshape(-1, 2)[inv].ravel()
+    mesh = (0, m.NodeList[:, inv], perm[m.IEN - 1] + 1, 2, "Q1", 2, m.ID, 1.0, 0.3)
+    K = smearfem.assemble_system(*mesh, ctx=ctx, device=True, n_elem=m.n_elem)
+    Kff, rhs = O.eliminate(O.assemble_system(*mesh, n_elem=m.n_elem), fixed, f)
+    q_ref = O.recombine(fixed, None, spla.spsolve(Kff.tocsc(), rhs))
+    bc = BoundaryConditions(ctx, K.shape[0], f, fixed)
+    S = System(K, bc)
+    slices = -(-S.n_free // 128)
+    for precision, vb, xb in (("fp64", 8, 8), ("mixed", 4, 4), ("fp32_matrix", 4, 8), ("split", 6, 8)):
+        st = S.solve(precision, "bsr", rtol=1e-12, raise_on_fail=False, preconditioner="block_jacobi")
+        assert st["stop_reason"] in (1, 3) and relerr(S.solution(), q_ref) <= ERR, precision
+        vecs = 4 if slices <= 1280 else 2
+        assert st["spmv_bytes"] == S.nnz // 4 * (4 * vb + 4) + 12 * slices + 8 + vecs * S.n_free * xb
+    for h in (S, bc, K):
+        h.close()
