@@ -133,11 +133,16 @@ struct PassGo {
     int done, resid;
 };
 
+// What a timed pass was (the host leaves residuals out of the times).
+enum PassKind : int { kPassNone = 0, kPassIteration = 1, kPassResidual = 2 };
+
 // Start of an operator pass, by every block: the last update's sums (upd:
 // r.z, r.r per block), the state after it, and what this pass has to do.
+// kind: where a timed pass records it, else NULL.
 template <int NW>
 __device__ __forceinline__ PassGo pass_begin(const CgState* __restrict__ in, CgState* __restrict__ out,
-                                             const double* __restrict__ upd, int nupd, double* sh, PassGo* shgo) {
+                                             const double* __restrict__ upd, int nupd, double* sh, PassGo* shgo,
+                                             int* kind) {
     double t[2] = {0.0, 0.0};
     if (in->fresh) sum_parts_all<2, NW>(upd, nupd, t, sh);
     if (threadIdx.x == 0) {
@@ -148,10 +153,7 @@ __device__ __forceinline__ PassGo pass_begin(const CgState* __restrict__ in, CgS
         }
         s.fresh = 0;
         s.resid = s.need_update;
-        if (!s.done) {
-            s.passes += 1;
-            s.resid_bits = s.resid_bits << 1 | (unsigned long long)s.resid;
-        }
+        if (kind && blockIdx.x == 0) *kind = s.done ? kPassNone : s.resid ? kPassResidual : kPassIteration;
         *shgo = PassGo{s.beta, s.zcoef, s.done, s.resid};
         if (blockIdx.x == 0) *out = s;
     }
@@ -194,6 +196,7 @@ struct PassVecs {
     const double* rhs;
     const T* dinv;
     const T* binv;  // node-block Jacobi: planar inverse blocks, stride nrows
+    int* kind;      // a timed pass records what it was here, else NULL
 };
 
 // Elements between block rows of p and z.
@@ -212,11 +215,11 @@ struct alignas(2 * BS * sizeof(T) % 16 == 0 ? 16 : 8) PzRecord {
 template <typename T>
 __global__ __launch_bounds__(kThreads) void direction_kernel(T* __restrict__ p, const T* __restrict__ z, int64_t n,
                                                              int64_t per_block, const CgState* in, CgState* out,
-                                                             const double* __restrict__ upd, int nupd) {
+                                                             const double* __restrict__ upd, int nupd, int* kind) {
     constexpr int NW = kThreads / 64;
     __shared__ double sh[NW];
     __shared__ PassGo shgo;
-    const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
+    const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo, kind);
     if (go.done || go.resid) return;
     const T beta = (T)go.beta, zc = (T)go.zcoef;
     const int64_t i0 = (int64_t)blockIdx.x * per_block;
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(kThreads) void csr_pass_kernel(const int32_t* __res
     __shared__ double sh[NW];
     __shared__ PassGo shgo;
     PassGo go;
-    if constexpr (FLY) go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
+    if constexpr (FLY) go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo, v.kind);
     else go = PassGo{0.0, 0.0, in->done, in->resid};  // direction_kernel has begun the pass
     if (go.done) return;
     const int64_t r0 = logical_block() * rows_per_block;
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(kThreads) void sell_pass_kernel(
         const bool live = sl < s1;
         SharedSlice<BS, TV, NT> row_cols(scol, sval);
         if (live) row_cols.load(sl_ptr, sl_w, sl);
-        const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo);
+        const PassGo go = pass_begin<NW>(in, out, upd, nupd, sh, &shgo, v.kind);
         if (go.done) return;
         if (!go.resid) {
             const T beta = (T)go.beta, zc = (T)go.zcoef;
@@ -821,7 +824,7 @@ void launch_pass(const Ops& o, const PassVecs<T>& v, CgStates* st, const double*
     CgState* out = &st->s[1];
     if (!o.fly) {
         hipLaunchKernelGGL(direction_kernel<T>, dim3(o.vec.grid), dim3(kThreads), 0, s, v.pnew, (const T*)v.z, o.n,
-                           o.vec.per_block, in, out, upd, nupd);
+                           o.vec.per_block, in, out, upd, nupd, v.kind);
         SFEM_LAUNCH_CHECK();
         in = out;
     }
@@ -1047,10 +1050,13 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
     }
     const auto w0 = std::chrono::steady_clock::now();
     const bool time_passes = o->time_kernels && timed_run;
-    // the state tells which of the last 64 passes were residuals
     const int check = std::max(1, time_passes ? std::min(o->check_every, 64) : o->check_every);
     std::vector<hipEvent_t> ev;
+    DevBuf<int> dkinds;
+    std::vector<int> kinds;
     if (time_passes) {
+        dkinds.reset(ctx, (size_t)check);
+        kinds.resize((size_t)check);
         ev.resize(2 * (size_t)check);
         for (auto& e : ev) SFEM_HIP(hipEventCreate(&e));
     }
@@ -1059,15 +1065,16 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
                        ops.vec.per_block, st, upd, o->rtol, o->reliable_delta);
     SFEM_LAUNCH_CHECK();
     T* const pz1 = ops.fly ? pz[1] : pz[0];
-    PassVecs<T> v{pz[0], pz[0] + zoff, pz1, pz1 + zoff, q, r, x64, xs, ops.rhs, dinv, binv};
+    PassVecs<T> v{pz[0], pz[0] + zoff, pz1, pz1 + zoff, q, r, x64, xs, ops.rhs, dinv, binv, nullptr};
 
     CgState host{};
-    int64_t counted = 0, timed = 0;
+    int64_t timed = 0;
     double spmv_ms = 0.0;
     // the first step is the residual of the start; a step is an iteration or
     // a residual replacement, and the device stops at the iteration cap
     for (int64_t chunk = 1; !host.done; chunk = check) {
         for (int64_t k = 0; k < chunk; ++k) {
+            if (time_passes) v.kind = dkinds.get() + k;
             launch_pass<TV, T>(ops, v, st, upd, parts, time_passes ? ev[2 * k] : nullptr);
             if (time_passes) SFEM_HIP(hipEventRecord(ev[2 * k + 1], ctx->stream));
             launch_update<T>(ops, v, x, x64, st, parts, upd);
@@ -1077,18 +1084,16 @@ void run_pcg(sfem_ctx* ctx, sfem_system* S, const sfem_solve_opts* o, sfem_solve
         }
         d2h(ctx, &host, &st->s[0], sizeof(host));
         if (time_passes) {
-            // launches after the stop exit at once: the first `real` of the
-            // chunk ran; residuals among them are another operator
-            const int64_t real = host.passes - counted;
-            for (int64_t k = 0; k < real; ++k) {
-                if (host.resid_bits >> (real - 1 - k) & 1) continue;
+            // launches after the stop exit at once, and residuals are another operator
+            d2h(ctx, kinds.data(), dkinds.get(), sizeof(int) * (size_t)chunk);
+            for (int64_t k = 0; k < chunk; ++k) {
+                if (kinds[(size_t)k] != kPassIteration) continue;
                 float ms = 0;
                 SFEM_HIP(hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]));
                 spmv_ms += ms;
                 ++timed;
             }
         }
-        counted = host.passes;
     }
     if (FOLD) {  // x = x64 + xs
         hipLaunchKernelGGL(fold_kernel, dim3(ops.vec.grid), dim3(kThreads), 0, ctx->stream, x64, (float*)xsv, nf);

@@ -187,8 +187,6 @@ struct CgState {
     long long last_upd;  // iteration of the latest replacement
     long long best_true_it;  // iteration of best_true
     long long max_iter;
-    long long passes;                // operator passes begun, residuals among them
-    unsigned long long resid_bits;   // which of the last 64 were residuals (bit 0: the last)
 };
 
 struct CgStates {
