@@ -133,6 +133,7 @@ void staged_d2h(sfem_ctx* ctx, Staging& st, char* dst, const char* src, size_t b
     const int64_t n = (int64_t)((bytes + kSlotBytes - 1) / kSlotBytes);
     std::atomic<int64_t> landed{0}, next{0};  // chunks in their slots; next chunk to copy
     std::atomic<bool> stop{false};
+    const auto patience = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
     std::vector<std::atomic<int>> copied((size_t)n);
     for (auto& c : copied) c.store(0, std::memory_order_relaxed);
     auto size_of = [&](int64_t c) { return std::min(kSlotBytes, bytes - (size_t)c * kSlotBytes); };
@@ -140,12 +141,14 @@ void staged_d2h(sfem_ctx* ctx, Staging& st, char* dst, const char* src, size_t b
         for (;;) {
             const int64_t c = next.fetch_add(1);
             if (c >= n) return;
-            int64_t have;
-            for (int spins = 0; (have = landed.load(std::memory_order_acquire)) <= c; ++spins) {
+            // before the first chunk, work queued ahead of the copy may run for
+            // long: after 5 ms of it the thread sleeps between looks
+            for (int spins = 1;; ++spins) {
+                const int64_t have = landed.load(std::memory_order_acquire);
+                if (have > c) break;
                 if (stop.load()) return;
-                // before the first chunk, work queued ahead of the copy may run for long
-                if (have || spins < 2000) std::this_thread::yield();
-                else std::this_thread::sleep_for(std::chrono::microseconds(50));
+                if (have || spins % 64 || std::chrono::steady_clock::now() < patience) std::this_thread::yield();
+                else std::this_thread::sleep_for(std::chrono::microseconds(100));
             }
             std::memcpy(dst + (size_t)c * kSlotBytes, st.buf + (size_t)(c % kSlots) * kSlotBytes, size_of(c));
             copied[(size_t)c].store(1, std::memory_order_release);
