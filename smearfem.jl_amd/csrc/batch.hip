@@ -762,12 +762,13 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
     // this block's part of the active slices; consecutive parts share an XCD,
     // and the XCD's part [x0, x0 + xs) by the work of the slices
     const int xn = G % 8 ? 1 : 8, xb = G / xn, bx = blockIdx.x / xn;
-    int total = 0, total3 = 0, first = 0, count = 0, g0 = 0, x0 = 0, xs = 0;
+    int total = 0, first = 0, count = 0, g0 = 0, x0 = 0, xs = 0;
+    bool shared = false;  // the first form
     auto work_before = [&](int g) {
         return (int64_t)uniform(set.pre[g]) + (int64_t)(kWork3 - 1) * uniform(set.pre3[g]);
     };
-    auto share = [&](int x) {  // active position at which x of xn equal shares of the work end
-        if (x == 0 || x == xn || total3 == 0 || total3 == total) return (int)((int64_t)total * x / xn);
+    auto share = [&](int x, bool mixed) {  // active position at which x of xn equal shares of the work end
+        if (x == 0 || x == xn || !mixed) return (int)((int64_t)total * x / xn);
         const int64_t W = work_before(ng) * x / xn;
         int lo = 0, hi = ng;  // the last group that begins at or before W: it has slices
         while (hi - lo > 1) {
@@ -780,7 +781,9 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
     };
     auto cut = [&] {
         total = active_prefix(set.w, set.pre, ng);
-        total3 = active_prefix(set.w3, set.pre3, ng);
+        const int total3 = active_prefix(set.w3, set.pre3, ng);
+        shared = (int64_t)a.item_slices * total3 + (int64_t)a.item_slices3 * (total - total3) <=
+                 (int64_t)a.item_slices * a.item_slices3 * G;
         const int64_t lb = logical_block();
         first = (int)(lb * total / G);
         count = (int)((lb + 1) * total / G) - first;
@@ -791,8 +794,11 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
             else hi = mid;
         }
         g0 = lo;
-        x0 = share(blockIdx.x % xn);
-        xs = share(blockIdx.x % xn + 1) - x0;
+        if (!shared) {
+            const bool mixed = total3 > 0 && total3 < total;
+            x0 = share(blockIdx.x % xn, mixed);
+            xs = share(blockIdx.x % xn + 1, mixed) - x0;
+        }
     };
     cut();
     auto runs = [&] {
@@ -916,8 +922,7 @@ __global__ __launch_bounds__(kThreads, 2) void table_pcg_kernel(TableLaunch a) {
     int64_t k = 0;
     for (; k < a.iters && total > 0; ++k) {
         double* pa = a.part + (k & 1) * 4 * ps;
-        if ((int64_t)a.item_slices * total3 + (int64_t)a.item_slices3 * (total - total3) <=
-            (int64_t)a.item_slices * a.item_slices3 * G) {
+        if (shared) {
             // ---- A, slices shared by the block ----
             auto run = [&](auto bs, int p, int s0, int s1) {
                 constexpr int BS = decltype(bs)::value;
