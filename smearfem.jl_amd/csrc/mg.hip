@@ -53,7 +53,8 @@ constexpr int64_t kMgMaxCoarseNodes = 400;  // coarsest level
 // solve in ms with the coarsest level (<= 64 nodes) / this line / 1,296 dofs:
 // 11x5x5 2.76 / 1.97 / 1.95, 16x8x8 (675 dofs) 2.53 / 2.32 / 2.33, 24x24x24
 // (1,029) 2.90 / 2.81 / 3.12, 64x16x16 (1,275) 3.91 / 3.45 / 3.92, 301x97
-// (1,092) 4.99 / 3.96 / 3.89, 256x64x64 13.6 / 13.2 / 13.7.
+// (1,092) 4.99 / 3.96 / 3.89, 256x64x64 13.6 / 13.2 / 13.7 (no more than two
+// runs differ).
 constexpr int64_t kDirectDofs = 800;
 constexpr int kTile = 32;                   // Gauss-Jordan block
 
