@@ -1562,7 +1562,9 @@ struct FirstStep {
 
 template <int BS>
 __device__ __forceinline__ void first_step_row(const FirstStep& F, int64_t row, const double (&rout)[BS]) {
-    float rv[BS];
+    float rv[BS], b[BS * BS];  // b is loaded before the stores, which may alias for all the compiler knows
+#pragma unroll
+    for (int k = 0; k < BS * BS; ++k) b[k] = F.binv[(int64_t)k * F.nrows + row];
 #pragma unroll
     for (int j = 0; j < BS; ++j) {
         rv[j] = (float)(rout[j] * F.scale);
@@ -1572,7 +1574,7 @@ __device__ __forceinline__ void first_step_row(const FirstStep& F, int64_t row, 
     for (int j = 0; j < BS; ++j) {
         float z = 0.0f;
 #pragma unroll
-        for (int i = 0; i < BS; ++i) z = fmaf(F.binv[(int64_t)(j * BS + i) * F.nrows + row], rv[i], z);
+        for (int i = 0; i < BS; ++i) z = fmaf(b[j * BS + i], rv[i], z);
         const float dn = F.c2 * z;
         F.d[row * BS + j] = dn;
         F.x[row * BS + j] = dn;
@@ -2622,11 +2624,13 @@ __global__ __launch_bounds__(kThreads) void mg_spmv_kernel(const int64_t* __rest
             sell_row<BS, TV, double, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, out);
             const int64_t row = sl * 64 + lane;
             if (row < nrows) {
+                double pr[BS];  // before the stores, which may alias for all the compiler knows
+#pragma unroll
+                for (int j = 0; j < BS; ++j) pr[j] = p[row * BS + j];
 #pragma unroll
                 for (int j = 0; j < BS; ++j) {
-                    const int64_t d = row * BS + j;
-                    v.q[d] = out[j];
-                    dot = fma(p[d], out[j], dot);
+                    v.q[row * BS + j] = out[j];
+                    dot = fma(pr[j], out[j], dot);
                 }
             }
         }
@@ -2648,11 +2652,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
          row += (int64_t)gridDim.x * kThreads) {
         double out[ND];
         mf_row<ND, double, double>(op, op.kc, row, p, out);
+        double pr[ND];  // before the stores, which may alias for all the compiler knows
+#pragma unroll
+        for (int j = 0; j < ND; ++j) pr[j] = p[row * ND + j];
 #pragma unroll
         for (int j = 0; j < ND; ++j) {
-            const int64_t d = row * ND + j;
-            v.q[d] = out[j];
-            dot = fma(p[d], out[j], dot);
+            v.q[row * ND + j] = out[j];
+            dot = fma(pr[j], out[j], dot);
         }
     }
     dot = block_sum_256(dot, sh);

@@ -368,10 +368,13 @@ __global__ __launch_bounds__(kThreads) void sell_pass_kernel(
                 sell_row<BS, TV, T, NT>(sl_ptr, sl_w, scol, sval, sl, lane, gx, acc);
                 const int64_t row = sl * 64 + lane;
                 if (row < nrows) {
+                    T pr[BS];  // loaded before the stores, which may alias for all the compiler knows
+#pragma unroll
+                    for (int j = 0; j < BS; ++j) pr[j] = p[row * BS + j];
 #pragma unroll
                     for (int j = 0; j < BS; ++j) {
                         v.q[row * BS + j] = acc[j];
-                        dot += (double)p[row * BS + j] * (double)acc[j];
+                        dot += (double)pr[j] * (double)acc[j];
                     }
                 }
             }
